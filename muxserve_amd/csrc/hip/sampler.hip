@@ -43,7 +43,12 @@ union SmFrag {
 };
 
 constexpr int kSmTile = 256;              // the hidden size must be a multiple of this
-constexpr int kSmMaxRowsPerPass = 64;
+constexpr int kSmMaxRowsPerPass = 256;
+// Up to 32 sampled rows the narrow kernel, beyond them the wide one (32000 rows of
+// 4096, us, narrow / wide: 8 rows 46.8 / 48.0, 32 rows 47.7 / 47.1, 33 rows
+// 54.3 / 47.1, 64 rows 55.7 / 47.4; with 128 and 256 rows 112 / 57 and 221 / 84,
+// the narrow one passing over the matrix once per 64 rows).
+constexpr int kSmNarrowRows = 32;
 #ifndef MUX_SM_PREFETCH_TILES
 #define MUX_SM_PREFETCH_TILES 2
 #endif
@@ -79,6 +84,67 @@ __device__ __forceinline__ void take_better(float &v, int &i, float ov, int oi) 
     v = ov;
     i = oi;
   }
+}
+
+// The workgroup's result per sampled row goes to its line of the table as a
+// 64-bit key (ordered logit bits << 32 | ~index: a larger key is a better
+// logit or, between equal logits, a lower index).
+__device__ __forceinline__ void store_key(const LmHeadParams &P, int64_t at, float v, int i) {
+  const unsigned long long key =
+      (static_cast<unsigned long long>(ordered_bits(v)) << 32) | (0xffffffffu - static_cast<uint32_t>(i));
+  __hip_atomic_store(&P.table[at], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Announces this workgroup's line of the table; true in the workgroup that came
+// last.  The table is written and read with device-coherent accesses (they
+// bypass the per-XCD L2), so ordering them against the counter takes only a wait
+// for this wave's table stores to be acknowledged before the workgroup meets
+// and bumps the counter.  A device-scope fence would also write back and
+// invalidate this XCD's L2, which holds the hidden states every other
+// workgroup is still reading (measured: +30 us per launch).
+__device__ __forceinline__ bool last_to_arrive(const LmHeadParams &P, int *s_last) {
+  wait_own_vector_memory();
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *s_last = __hip_atomic_fetch_add(P.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  __syncthreads();
+  if (!*s_last) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return true;
+}
+
+// Last workgroup to arrive: thread -> (sampled row tid % ROWS, slice tid / ROWS
+// of the workgroups), sixteen loads in flight.  fin: THREADS keys of LDS.
+template <int ROWS, int THREADS>
+__device__ __forceinline__ void reduce_table(const LmHeadParams &P, unsigned long long *fin) {
+  constexpr int SLICES = THREADS / ROWS;
+  const int tid = threadIdx.x;
+  const int row = tid % ROWS, slice = tid / ROWS;
+  unsigned long long best = 0;
+  const int n_wg = gridDim.x;
+  for (int b0 = slice; b0 < n_wg && slice < SLICES; b0 += 16 * SLICES) {
+    unsigned long long v[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int b = b0 + j * SLICES;
+      v[j] = b < n_wg ? __hip_atomic_load(&P.table[static_cast<int64_t>(b) * ROWS + row], __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT)
+                      : 0ull;
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) best = v[j] > best ? v[j] : best;
+  }
+  fin[tid] = best;
+  __syncthreads();
+  if (tid < P.num_rows) {
+    unsigned long long k = fin[tid];
+#pragma unroll
+    for (int sl = 1; sl < SLICES; ++sl) k = fin[sl * ROWS + tid] > k ? fin[sl * ROWS + tid] : k;
+    const uint32_t idx = 0xffffffffu - static_cast<uint32_t>(k);
+    P.next_tokens[tid] = idx < static_cast<uint32_t>(P.vocab) ? idx : 0;   // every logit NaN: token 0
+  }
+  if (tid == 0) __hip_atomic_store(P.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <typename T, int NB, int NW, int RB>
@@ -249,62 +315,216 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
     }
   }
   __syncthreads();
-  // The workgroup's result per sampled row goes to its line of the table as a
-  // 64-bit key (ordered logit bits << 32 | ~index: a larger key is a better
-  // logit or, between equal logits, a lower index).
   if (tid < ROWS) {
     float bv = red_v[0][tid];
     int bi = red_i[0][tid];
 #pragma unroll
     for (int w = 1; w < NW; ++w) take_better(bv, bi, red_v[w][tid], red_i[w][tid]);
-    const unsigned long long key = (static_cast<unsigned long long>(ordered_bits(bv)) << 32) |
-                                   (0xffffffffu - static_cast<uint32_t>(bi));
-    __hip_atomic_store(&P.table[static_cast<int64_t>(blockIdx.x) * ROWS + tid], key, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    store_key(P, static_cast<int64_t>(blockIdx.x) * ROWS + tid, bv, bi);
   }
-  // The table is written and read with device-coherent accesses (they bypass
-  // the per-XCD L2), so ordering them against the counter takes only a wait
-  // for this wave's table stores to be acknowledged before the workgroup meets
-  // and bumps the counter.  A device-scope fence would also write back and
-  // invalidate this XCD's L2, which holds the hidden states every other
-  // workgroup is still reading (measured: +30 us per launch).
-  wait_own_vector_memory();
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __syncthreads();
-  if (tid == 0)
-    s_last = __hip_atomic_fetch_add(P.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
-  __syncthreads();
-  if (!s_last) return;
-  // Last workgroup to arrive: thread -> (sampled row tid % ROWS, slice
-  // tid / ROWS of the workgroups), sixteen loads in flight.
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  constexpr int SLICES = 64 * NW / ROWS;
-  __shared__ unsigned long long fin[SLICES][ROWS];
-  const int row = tid % ROWS, slice = tid / ROWS;
-  unsigned long long best = 0;
-  const int n_wg = gridDim.x;
-  for (int b0 = slice; b0 < n_wg; b0 += 16 * SLICES) {
-    unsigned long long v[16];
+  if (!last_to_arrive(P, &s_last)) return;
+  __shared__ unsigned long long fin[64 * NW];
+  reduce_table<ROWS, 64 * NW>(P, fin);
+}
+
+// ---------------------------------------------------------------------------
+// More than 32 sampled rows: a matrix product with both operands through LDS.
+// The kernel above reads one fragment of hidden states from LDS per MFMA (its
+// waves are 16 vocabulary rows tall), which slows it from 33 rows on, and past
+// 64 rows it would have to pass over the matrix once per 64.  Here eight waves
+// share a tile of 128 vocabulary rows x 64 NB sampled rows as 2 x 4 waves of
+// 64 x 16 NB, so that a fragment from LDS feeds NB (embedding) or four (hidden
+// states) MFMAs.
+//   * 128 rows per workgroup: a 32000-row vocabulary is 250 workgroups, one per
+//     compute unit, one round.
+//   * The hidden dimension is walked in tiles of 64 (a 128-byte line per row).  A
+//     tile goes global -> registers -> LDS (two LDS buffers, one barrier per tile;
+//     16-byte chunk c of a row at position c ^ (row % 8): no bank conflicts), and
+//     PD further tiles are in flight in registers.
+// Up to 64 rows it is bound by HBM (262 MB of a 32000 x 4096 matrix in 47 us =
+// 5.6 TB/s).  With 256 rows (84 us: 3.1 TB/s, 0.8 PFLOP/s) the clock is 1.66 GHz,
+// the matrix cores are busy half and the LDS 44 % of the time; the memory is not
+// what it waits for (every tile from the L1: 77 us), and a third LDS buffer with
+// a barrier that waits for the writes only changes nothing.
+// The reduction is the one above with 64 NB columns per table line.
+template <typename T, int NB, int PD>
+__global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHeadParams P) {
+  constexpr int KT = 64;                   // hidden elements per tile
+  constexpr int ROWS = 64 * NB;            // sampled rows
+  constexpr int VR = 128;                  // vocabulary rows
+  constexpr int NW = 8;
+  constexpr int kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;   // instruction classes of the scheduler
+  constexpr int TILE = (VR + ROWS) * KT;   // elements of one LDS buffer: embedding rows, then hidden rows
+  __shared__ __attribute__((aligned(16))) uint16_t tile[2][TILE];
+  __shared__ float red_v[2][ROWS];
+  __shared__ int red_i[2][ROWS];
+  __shared__ int s_last;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int r16 = lane & 15, g = lane >> 4;
+  const int n_tiles = P.hidden_size / KT;
+  const int t_start = blockIdx.x % n_tiles;            // (see the kernel above)
+  const int vrow0 = blockIdx.x * VR;
+
+  // Staging: thread -> row tid / 8 (+ 64 j), chunk tid % 8.  Every load is
+  // unconditional - behind a branch the compiler waits for all loads in flight
+  // instead of the oldest: rows past the vocabulary re-read its last row (masked
+  // at the end), sampled rows past the last re-read a valid one (not stored).
+  const int srow = tid >> 3, schunk = tid & 7;
+  const uint16_t *wsrc[2], *hsrc[NB];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int b = b0 + j * SLICES;
-      v[j] = b < n_wg ? __hip_atomic_load(&P.table[static_cast<int64_t>(b) * ROWS + row], __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT)
-                      : 0ull;
+  for (int j = 0; j < 2; ++j)
+    wsrc[j] = P.weight + static_cast<int64_t>(min(vrow0 + srow + 64 * j, P.vocab - 1)) * P.weight_stride + 8 * schunk;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int row = min(srow + 64 * j, P.num_rows - 1);
+    const int src = P.row_index ? min(max(P.row_index[row], 0), P.hidden_rows - 1) : row;
+    hsrc[j] = P.hidden + static_cast<int64_t>(src) * P.hidden_stride + 8 * schunk;
+  }
+  const int soff = srow * KT + 8 * (schunk ^ (srow & 7));     // (rows 64 apart swizzle alike)
+  struct Staged {
+    sm_u32x4 w[2], h[NB];
+  };
+  auto load = [&](Staged &r, int t) {
+    int x = t + t_start;
+    x = (x >= n_tiles ? x - n_tiles : x) * KT;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) r.h[j] = *reinterpret_cast<const sm_u32x4 *>(hsrc[j] + x);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) r.w[j] = __builtin_nontemporal_load(reinterpret_cast<const sm_u32x4 *>(wsrc[j] + x));
+  };
+  auto store = [&](const Staged &r, int buf) {
+    uint16_t *const dst = &tile[buf][soff];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) *reinterpret_cast<sm_u32x4 *>(dst + (VR + 64 * j) * KT) = r.h[j];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<sm_u32x4 *>(dst + 64 * j * KT) = r.w[j];
+  };
+
+  sm_v4f32 acc[4][NB];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = sm_v4f32{0.f, 0.f, 0.f, 0.f};
+  // Fragments of one half (32 of the 64 hidden elements) of a tile, and their products.
+  struct Half {
+    SmFrag a[4], b[NB];
+  };
+  auto read_half = [&](Half &f, int buf, int kk) {
+    const int chunk = 8 * ((4 * kk + g) ^ (r16 & 7));
+    const uint16_t *const wt = &tile[buf][(64 * wm + r16) * KT + chunk];
+    const uint16_t *const ht = &tile[buf][(VR + 16 * NB * wn + r16) * KT + chunk];
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) f.a[mb].u = *reinterpret_cast<const sm_u32x4 *>(wt + 16 * mb * KT);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) f.b[nb].u = *reinterpret_cast<const sm_u32x4 *>(ht + 16 * nb * KT);
+  };
+  auto multiply = [&](const Half &f) {
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        if constexpr (__is_same(T, F16))
+          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.a[mb].h, f.b[nb].h, acc[mb][nb], 0, 0, 0);
+        else
+          acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[mb].b, f.b[nb].b, acc[mb][nb], 0, 0, 0);
+      }
+  };
+
+  // Register set s holds the tile t with t % PD == s that comes next.
+  Staged st[PD];
+  load(st[0], 0);
+  store(st[0], 0);
+#pragma unroll
+  for (int s = 1; s <= PD; ++s) load(st[s % PD], min(s, n_tiles - 1));
+  __syncthreads();
+  int buf = 0;
+  // One tile.  Each half's fragments are on their way while the half before it is
+  // being multiplied: the second half's behind the first, the next tile's first
+  // half behind the second (which is therefore multiplied after the barrier that
+  // completes the next tile); LDS accesses and MFMAs are dealt one by one, since a
+  // wave that issues its reads in a row waits for the LDS queue with the matrix
+  // cores idle (256 rows: 88 -> 83 us).
+  Half f0, f1;
+  read_half(f0, 0, 0);
+  auto step = [&](Staged &next, int t, bool store_next, bool load_next) {
+    read_half(f1, buf, 1);
+    multiply(f0);
+    if (store_next) store(next, buf ^ 1);
+    if (load_next) load(next, t + 1 + PD);
+#pragma unroll
+    for (int i = 0; i < 4 + NB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
     }
 #pragma unroll
-    for (int j = 0; j < 16; ++j) best = v[j] > best ? v[j] : best;
-  }
-  fin[slice][row] = best;
-  __syncthreads();
-  if (tid < P.num_rows) {
-    unsigned long long k = fin[0][tid];
+    for (int i = 0; i < 2 + NB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kMfma, 4 * NB, 0);
+    __builtin_amdgcn_sched_group_barrier(kVmemRead, 2 + NB, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    buf ^= 1;
+    if (store_next) read_half(f0, buf, 0);
+    multiply(f1);
 #pragma unroll
-    for (int sl = 1; sl < SLICES; ++sl) k = fin[sl][tid] > k ? fin[sl][tid] : k;
-    const uint32_t idx = 0xffffffffu - static_cast<uint32_t>(k);
-    P.next_tokens[tid] = idx < static_cast<uint32_t>(P.vocab) ? idx : 0;   // every logit NaN: token 0
+    for (int i = 0; i < 4 + NB; ++i) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kMfma, 4 * NB, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int t0 = 0;
+  for (; t0 + 2 * PD < n_tiles; t0 += PD) {
+#pragma unroll
+    for (int s = 0; s < PD; ++s) step(st[(s + 1) % PD], t0 + s, true, true);
   }
-  if (tid == 0) __hip_atomic_store(P.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (; t0 < n_tiles; t0 += PD) {
+#pragma unroll
+    for (int s = 0; s < PD; ++s) {
+      const int t = t0 + s;
+      if (t < n_tiles) step(st[(s + 1) % PD], t, t + 1 < n_tiles, t + 1 + PD < n_tiles);
+    }
+  }
+
+  // Lane holds logits[vocab row vrow0 + 64 wm + 16 mb + 4 g + i][sampled row 16 (NB wn + nb) + r16].
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    float bv = -__builtin_inff();
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int vr = vrow0 + 64 * wm + 16 * mb + 4 * g + i;
+        const float val = sm_round<T>(acc[mb][nb][i]);
+        if (vr < P.vocab) take_better(bv, bi, val, vr);
+      }
+#pragma unroll
+    for (int off = 16; off <= 32; off <<= 1) {
+      const float ov = __shfl_xor(bv, off);
+      const int oi = __shfl_xor(bi, off);
+      take_better(bv, bi, ov, oi);
+    }
+    if (g == 0) {
+      red_v[wm][16 * (NB * wn + nb) + r16] = bv;
+      red_i[wm][16 * (NB * wn + nb) + r16] = bi;
+    }
+  }
+  __syncthreads();
+  if (tid < ROWS) {
+    float bv = red_v[0][tid];
+    int bi = red_i[0][tid];
+    take_better(bv, bi, red_v[1][tid], red_i[1][tid]);
+    store_key(P, static_cast<int64_t>(blockIdx.x) * ROWS + tid, bv, bi);
+  }
+  if (!last_to_arrive(P, &s_last)) return;
+  reduce_table<ROWS, 64 * NW>(P, reinterpret_cast<unsigned long long *>(&tile[0][0]));
 }
 
 __global__ void sampler_zero_kernel(uint32_t *p, int n) {
@@ -322,7 +542,8 @@ constexpr int kSmEightWaveMinWgs = MUX_SM_EIGHT_WAVE_MIN_WGS;
 
 extern "C" size_t mux_greedy_sample_workspace_bytes(int32_t vocab_size) {
   if (vocab_size <= 0) return 0;
-  const size_t n_wg = (static_cast<size_t>(vocab_size) + 63) / 64;            // the most workgroups a launch uses
+  // The largest table: 128 vocabulary rows per workgroup, a key per sampled row of a pass.
+  const size_t n_wg = (static_cast<size_t>(vocab_size) + 127) / 128;
   return mux::kSmCounterBytes + n_wg * mux::kSmMaxRowsPerPass * sizeof(unsigned long long);
 }
 
@@ -366,7 +587,7 @@ extern "C" int32_t mux_greedy_sample(int64_t *next_tokens, const void *hidden_st
   const bool wide = (vocab_size + 127) / 128 >= kSmEightWaveMinWgs;
   const int rows_per_wg = wide ? 128 : 64;
   const int n_wg = (vocab_size + rows_per_wg - 1) / rows_per_wg;
-  // At most 64 sampled rows per pass over the matrix; larger batches take
+  // At most 256 sampled rows per pass over the matrix; larger batches take
   // several passes, one after the other on the stream.
   for (int r0 = 0; r0 < num_rows; r0 += kSmMaxRowsPerPass) {
     const int rows = min(num_rows - r0, kSmMaxRowsPerPass);
@@ -383,19 +604,31 @@ extern "C" int32_t mux_greedy_sample(int64_t *next_tokens, const void *hidden_st
     P.counter = static_cast<uint32_t *>(workspace);
     P.table = reinterpret_cast<unsigned long long *>(static_cast<char *>(workspace) + kSmCounterBytes);
     P.next_tokens = next_tokens + r0;
-    const int nb = rows <= 16 ? 1 : (rows <= 32 ? 2 : 4);
+    const int nb = rows <= 16 ? 1 : 2;
+    if (rows > kSmNarrowRows) {
+      const dim3 wide_grid((vocab_size + 127) / 128);
+#define MUX_LM_WIDE(TT)                                                                                            \
+  do {                                                                                                            \
+    if (rows <= 64) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 1, 4>), wide_grid, dim3(512), 0, st, P);   \
+    else if (rows <= 128) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 2, 3>), wide_grid, dim3(512), 0, st, P); \
+    else if (rows <= 192) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 3, 2>), wide_grid, dim3(512), 0, st, P); \
+    else hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 4, 2>), wide_grid, dim3(512), 0, st, P);              \
+  } while (0)
+      if (dtype == MUXA_DTYPE_F16) MUX_LM_WIDE(F16);
+      else MUX_LM_WIDE(BF16);
+#undef MUX_LM_WIDE
+      continue;
+    }
     const dim3 grid(n_wg);
 #define MUX_LM_GO(TT, NBV, NWV, RBV) \
   hipLaunchKernelGGL((lm_head_argmax_kernel<TT, NBV, NWV, RBV>), grid, dim3(64 * NWV), 0, st, P)
-#define MUX_LM_LAUNCH(TT)                  \
-  do {                                     \
-    if (!wide) {                           \
-      if (nb == 1) MUX_LM_GO(TT, 1, 4, 1); \
-      else if (nb == 2) MUX_LM_GO(TT, 2, 4, 1); \
-      else MUX_LM_GO(TT, 4, 4, 1);         \
+#define MUX_LM_LAUNCH(TT)                       \
+  do {                                          \
+    if (!wide) {                                \
+      if (nb == 1) MUX_LM_GO(TT, 1, 4, 1);      \
+      else MUX_LM_GO(TT, 2, 4, 1);              \
     } else if (nb == 1) MUX_LM_GO(TT, 1, 8, 1); \
-    else if (nb == 2) MUX_LM_GO(TT, 2, 8, 1);   \
-    else MUX_LM_GO(TT, 4, 8, 1);           \
+    else MUX_LM_GO(TT, 2, 8, 1);                \
   } while (0)
     if (dtype == MUXA_DTYPE_F16) MUX_LM_LAUNCH(F16);
     else MUX_LM_LAUNCH(BF16);

@@ -161,6 +161,30 @@ def test_greedy_sample_planted_winners_vocab_cut_and_ties(dtype, Hd):
     assert toks == lo.greedy_sample(emb, hid, [], len(ids) + 1, V)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R,V,Hd,gathered", [
+    (33, 129, 256, False), (64, 128, 512, True), (65, 1000, 256, False), (127, 255, 768, True), (128, 1031, 256, False),
+    (129, 257, 512, False), (192, 5003, 256, True), (193, 1000, 1280, False), (256, 385, 256, True),
+    (257, 1031, 512, False), (300, 24593, 256, True)])
+def test_greedy_sample_many_rows_planted_winners(dtype, R, V, Hd, gathered):
+    """Batches beyond 32 rows, at the edges of the 64-row steps and of the
+    256-row passes, with every row's winner planted (its logit is about Hd / 2,
+    the others' below 0.02 sqrt(Hd) x 6): the answer is exact, no tolerance."""
+    print(f"[case] greedy_sample many rows {dtype} R={R} V={V} hidden={Hd} gathered={gathered}", flush=True)
+    g = torch.Generator().manual_seed(R * 1000 + V)
+    emb = (torch.randn((V + 3, Hd), generator=g) * 0.02).to(dtype)
+    rows = 2 * R if gathered else R
+    hid = torch.randn((rows, Hd), generator=g).to(dtype)
+    index = torch.randperm(rows, generator=g)[:R].to(torch.int32) if gathered else torch.arange(R, dtype=torch.int32)
+    ids = torch.randperm(V, generator=g)[:R] if R <= V else torch.arange(R) % V
+    if R > V:
+        hid[V:] = hid[:R - V]                                  # rows that share a winner share a hidden state
+    emb[ids] = (hid[index.long()].float() * 0.5).to(dtype)
+    emb[V:] = 4.0                                              # outside the vocabulary
+    toks = ops.greedy_sample(emb.to(DEV), hid.to(DEV), V, R, row_index=index.to(DEV) if gathered else None)
+    assert toks.cpu().tolist() == ids.tolist()
+
+
 def test_greedy_sampler_module_prompt_and_decode_steps():
     print("[case] GreedySampler module", flush=True)
     g = torch.Generator().manual_seed(11)

@@ -21,7 +21,21 @@
 // same key order (two groups of four keys), which costs nothing because V^T is
 // read from LDS anyway.
 // The next tile's global loads are issued before the current tile's math.
-#include "mux_common.h"
+//
+// The step form (STEP = true, mux_rope_prefill_and_cache) is a whole prompt step
+// of the attention layer behind the rotation of k: it also rotates q and writes
+// k and v to the pool.  As kernels of their own these passes are bound by
+// memory and run 1:1 beside an attention that leaves the memory idle - at
+// 16 x 2048 tokens, 32 heads: rotation of q and k 193 us, cache write 248 us,
+// attention 600 us.  Here the query fragments are rotated in the registers they
+// are loaded into (one workgroup reads each of them once; a lane holds both
+// halves of a pair), and a workgroup scatters the 128 rows of K and V that its
+// last four tiles bring into LDS anyway, so k and v are not read again and the
+// stores go out under the matrix work.  Measured, whole step: 16 x 2048 tokens
+// f16 1031 -> 845 us (the kernel 740 us of it: attention alone 620, pool stores
+// 75, rotation of q 35), three bf16 prompts of 700 - 4000 tokens on 64 / 8 heads
+// 528 -> 506 us.
+#include "cache_write.h"
 
 #include <algorithm>
 #include <vector>
@@ -110,7 +124,19 @@ struct PrefillParams {
   int32_t slots_per_pair;
   uint32_t pairs[kMaxPairs];
 };
-static_assert(sizeof(PrefillParams) <= 4096, "kernel argument segment");
+
+// The step form's part: one model's rotation and cache write.
+struct PrefillStep {
+  const int64_t *positions;
+  const float *cos_sin;          // [max_position, 128] = [cos | sin]
+  const int64_t *slots;          // layer slice of the slot mapping
+  int64_t slot_stride;
+  uint16_t *k_pool, *v_pool;
+  int64_t pool_slots;
+  int32_t max_position;
+  int32_t block_size;
+};
+static_assert(sizeof(PrefillParams) + sizeof(PrefillStep) <= 4096, "kernel argument segment");
 constexpr int kPairTileBits = 12;       // tile in bits 0-11, prompt in bits 12-27, model in bits 28-30
 
 // K and V tiles go from global memory straight into LDS
@@ -141,8 +167,87 @@ constexpr int kTileElems = kBN * kHeadSize;          // one unpadded row-major t
 // every V^T read.)
 __device__ __forceinline__ int swz(int row) { return ((row & 3) << 1) | ((row >> 2) & 1) | (row & 8); }
 
-template <typename T>
-__global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillParams P) {
+// 16 tokens (rows row0 .. row0 + 15 of the K and V tile in LDS) to the pool, by
+// the four waves of a workgroup together.  slot: lane's token row0 + lane % 16,
+// -1 for none.  K: a thread stores one token's chunk, the 16 tokens of a chunk
+// side by side, so a wave fills 1 KiB of a 16-token block.  V: the transposing
+// read hands a lane 8 consecutive tokens of one dim, which is a chunk of the pool
+// where those tokens are a run (consecutive slots from a multiple of 8: every
+// prompt behind a block table, up to its last few tokens); the others go element
+// by element.  The LDS reads are written out with their wait: for a transposing
+// read of its own the compiler first waits for every load in flight, the next
+// tile's among them.
+// True if exactly two vector-memory instructions were issued (both 8-token
+// halves are runs): the caller's wait for older loads can then leave them.
+__device__ __forceinline__ bool write_tokens_to_pool(const uint16_t *Kt, const uint16_t *Vr, int row0, int64_t slot,
+                                                     int wave, int lane, const PrefillStep &S) {
+  constexpr int D = kHeadSize;
+  // (kept from the tile loop's registers: the compiler would hoist the addresses
+  // below out of it and spill)
+  asm volatile("" : "+v"(lane));
+  typedef const __attribute__((address_space(3))) uint16_t lds_u16;
+  const int bs = S.block_size, bs_shift = __builtin_ctz(static_cast<unsigned>(bs));
+  const int i = lane & 15, c = 4 * wave + (lane >> 4);      // this thread's token and chunk (8 dims)
+  const int kr = row0 + i;
+  // Group of 16 lanes: dims 8 c .. 8 c + 7 of both halves.  Lane 4 j + m points at
+  // four dims (m & 1) of token j (and j + 4) of half m >> 1, and receives dim
+  // lane % 8 of half (lane / 8) % 2.
+  const int j = i >> 2, m = i & 3;
+  const int r0 = row0 + 8 * (m >> 1) + j, r1 = r0 + 4;
+  const uint32_t ka = (uint32_t)(uintptr_t)(lds_u16 *)(Kt + kr * D + 8 * (c ^ swz(kr)));
+  const uint32_t va0 = (uint32_t)(uintptr_t)(lds_u16 *)(Vr + r0 * D + 8 * (c ^ swz(r0)) + 4 * (m & 1));
+  const uint32_t va1 = (uint32_t)(uintptr_t)(lds_u16 *)(Vr + r1 * D + 8 * (c ^ swz(r1)) + 4 * (m & 1));
+  u32x4 kx;
+  u32x2 v0, v1;
+  asm volatile("ds_read_b128 %0, %3\n\tds_read_b64_tr_b16 %1, %4\n\tds_read_b64_tr_b16 %2, %5\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(kx), "=&v"(v0), "=&v"(v1)
+               : "v"(ka), "v"(va0), "v"(va1)
+               : "memory");
+  // Runs: the previous lane's slot plus one, from a multiple of 8.
+  const uint32_t slot_lo = static_cast<uint32_t>(slot), slot_hi = static_cast<uint32_t>(slot >> 32);
+  const uint32_t prev_lo = __builtin_amdgcn_update_dpp(0, slot_lo, 0x111, 0xf, 0xf, true);      // row_shr:1
+  const uint32_t prev_hi = __builtin_amdgcn_update_dpp(0, slot_hi, 0x111, 0xf, 0xf, true);
+  const int64_t prev = static_cast<int64_t>((static_cast<uint64_t>(prev_hi) << 32) | prev_lo);
+  const bool chained = slot >= 0 && ((lane & 7) == 0 ? (slot & 7) == 0 : slot == prev + 1);
+  const uint32_t runs = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(chained));
+  const bool run_a = (runs & 0xff) == 0xff, run_b = (runs & 0xff00) == 0xff00;      // (the four groups agree)
+  auto slot_of = [&](int l) {
+    const uint32_t lo = __builtin_amdgcn_readlane(slot_lo, l), hi = __builtin_amdgcn_readlane(slot_hi, l);
+    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+  };
+  const int64_t a = slot_of(0), b = slot_of(8), base = i < 8 ? a : b;
+  const int d = 8 * c + (lane & 7);
+  uint16_t *const kp = S.k_pool + (((slot >> bs_shift) * (D / 8) + c) * bs + (slot & (bs - 1))) * 8;
+  uint16_t *const vp = S.v_pool + ((base >> bs_shift) * D + d) * bs + (base & (bs - 1));
+  const u32x4 vx = {v0.x, v0.y, v1.x, v1.y};
+  if (run_a && run_b) {
+    // (K rows are whole lines; V rows are where the halves fill the block's rows:
+    // those stream past the L2, as in the cache-write kernel, and the wait states
+    // between a 16-byte store and a write of its data are spelled out as there)
+    asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 4" ::"v"(kp), "v"(kx) : "memory");
+    if (bs == 8 || (bs == 16 && b == a + 8 && (a & 15) == 0))
+      asm volatile("global_store_dwordx4 %0, %1, off nt\n\ts_nop 4" ::"v"(vp), "v"(vx) : "memory");
+    else
+      asm volatile("global_store_dwordx4 %0, %1, off\n\ts_nop 4" ::"v"(vp), "v"(vx) : "memory");
+    return true;
+  }
+  if (slot >= 0) *reinterpret_cast<u32x4 *>(kp) = kx;
+  if (i < 8 ? run_a : run_b) {
+    *reinterpret_cast<u32x4 *>(vp) = vx;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int64_t sa = slot_of(e), sb = slot_of(8 + e), sl = i < 8 ? sa : sb;
+      if (sl >= 0)
+        S.v_pool[((sl >> bs_shift) * D + d) * bs + (sl & (bs - 1))] =
+            static_cast<uint16_t>(vx[e >> 1] >> (16 * (e & 1)));
+    }
+  }
+  return false;
+}
+
+template <typename T, bool STEP>
+__device__ __forceinline__ void prefill_body(const PrefillParams &P, const PrefillStep &S) {
   constexpr int D = kHeadSize;
   // K[2], V[2] tile buffers.  The epilogue reuses the memory for the output rows
   // (4 waves x 32 rows of 272 bytes), which is the larger of the two.
@@ -211,9 +316,14 @@ __global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillPar
   const int wq0 = q0 + wave * 32;        // first query row of this wave
   const int my_q = wq0 + qcol;           // this lane's query position inside the prompt
 
+  // The query heads of a kv head share its K and V: the one whose turn it is by
+  // the query tile writes them (each writes as many tiles as the others).
+  bool writes_pool = false;
+  if constexpr (STEP) writes_pool = hq - hk * I.ratio == (q0 / kBM) % I.ratio;
+
   // ---- Q^T fragments: Q[my_q][16 s + 8 half .. +7], s = 0..7 ------------------------
   Frag qf[8];
-  {
+  if constexpr (!STEP) {
     const bool ok = my_q < len;
     const uint16_t *qp = I.q + static_cast<int64_t>(seq_begin + (ok ? my_q : 0)) * I.q_stride + hq * D + 8 * half;
 #pragma unroll
@@ -275,172 +385,279 @@ __global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillPar
     v_lane_base[1] = rl * D + 8 * (cl ^ swz(rl) ^ 4) + 4 * (m & 1);
   }
   dma_tile(0);
+  if constexpr (STEP) {
+    // Rotation of the wave's 32 query rows: a lane takes the chunks c and c + 8
+    // (the two halves of the same pairs) of one row, 8 rows at a time, so that
+    // rows, table and the write-back go as whole lines, and the fragments come
+    // back through the second tile buffers, 16 rows (4 KiB per wave) at a time.
+    // Rows past the prompt stand for its last one (the same value stored twice,
+    // by the one wave that holds the row, after all its loads); a wave that has
+    // only such rows does nothing.
+#pragma unroll
+    for (int f = 0; f < 8; ++f) qf[f].u = u32x4{0, 0, 0, 0};
+    if (wq0 < len) {
+      const int c = lane & 7, r8 = lane >> 3;
+      u32x4 lo[4], hi[4], cs4[4][2], sn4[4][2];
+      int64_t pos[4];
+      uint16_t *qp[4];
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int64_t row = seq_begin + min(wq0 + 8 * it + r8, len - 1);
+        pos[it] = S.positions[row];
+        qp[it] = const_cast<uint16_t *>(I.q) + row * I.q_stride + hq * D + 8 * c;
+        lo[it] = *reinterpret_cast<const u32x4 *>(qp[it]);
+        hi[it] = *reinterpret_cast<const u32x4 *>(qp[it] + D / 2);
+      }
+      __builtin_amdgcn_sched_barrier(0);   // the rows are requested before the wait for the positions
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int64_t p = pos[it] < 0 ? 0 : (pos[it] >= S.max_position ? S.max_position - 1 : pos[it]);
+        const u32x4 *row = reinterpret_cast<const u32x4 *>(S.cos_sin + p * D + 8 * c);
+        cs4[it][0] = row[0];
+        cs4[it][1] = row[1];
+        sn4[it][0] = row[D / 8];
+        sn4[it][1] = row[D / 8 + 1];
+      }
+      uint16_t *const stage = smem + (1 + 2 * (wave >> 1)) * kTileElems + (wave & 1) * (kTileElems / 2);
+#pragma unroll
+      for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int it = 2 * pass + h, r = 8 * h + r8;
+          float cs[8], sn[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            cs[e] = __uint_as_float(cs4[it][e >> 2][e & 3]);
+            sn[e] = __uint_as_float(sn4[it][e >> 2][e & 3]);
+          }
+          const uint4 x = make_uint4(lo[it].x, lo[it].y, lo[it].z, lo[it].w);
+          const uint4 y = make_uint4(hi[it].x, hi[it].y, hi[it].z, hi[it].w);
+          const uint4 xr = rotate_chunk<T>(x, y, cs, sn, false), yr = rotate_chunk<T>(y, x, cs, sn, true);
+          const u32x4 xo = {xr.x, xr.y, xr.z, xr.w}, yo = {yr.x, yr.y, yr.z, yr.w};
+          *reinterpret_cast<u32x4 *>(qp[it]) = xo;
+          *reinterpret_cast<u32x4 *>(qp[it] + D / 2) = yo;
+          *reinterpret_cast<u32x4 *>(stage + r * D + 8 * (c ^ swz(r))) = xo;
+          *reinterpret_cast<u32x4 *>(stage + r * D + 8 * ((c + 8) ^ swz(r))) = yo;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int r = qcol & 15;
+        const bool take = (qcol >> 4) == pass && my_q < len;
+#pragma unroll
+        for (int f = 0; f < 8; ++f) {
+          const u32x4 x = *reinterpret_cast<const u32x4 *>(stage + r * D + 8 * ((2 * f + half) ^ swz(r)));
+#pragma unroll
+          for (int e = 0; e < 4; ++e) qf[f].u[e] = take ? x[e] : qf[f].u[e];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+  }
+  bool stores_counted = false;             // the previous tile's pool stores: exactly four, behind this tile's loads
   for (int t = 0; t < n_tiles; ++t) {
     const int k0 = t * kBN;
     const int cur = t & 1;
     // This wave's part of tile t has landed; after the barrier all of it has,
     // and everybody is done with the other buffer.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+    if constexpr (STEP) {
+      // (the barrier by itself: __syncthreads() would wait for the stores as well)
+      if (stores_counted) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+    }
 #ifdef MUX_TRACE
     if (t == 0) tr_first = __builtin_amdgcn_s_memrealtime();
 #endif
-    if (t + 1 < n_tiles) dma_tile(cur ^ 1);
-    // Nothing to compute: every key of the tile is in this wave's future, or all
-    // of the wave's rows are past the prompt's end.
-    if (k0 > wq0 + 31 || wq0 >= len) continue;
-    const uint16_t *const Kt = smem + cur * kTileElems;           // this tile's K
-    const uint16_t *const Vr = smem + (2 + cur) * kTileElems;     // this tile's V (row-major)
-
-    // ---- S^T = K . Q^T : kNKB 32-key blocks -----------------------------------------
-    // LDS fragment reads run kDepth steps ahead of the MFMAs that consume them.
-    // In the P.V product consecutive MFMAs go to different accumulators (4 dim
-    // blocks); a single dependent chain, as here with one key block, runs at 3/4
-    // of the rate.
-    constexpr int kDepth = 4;
-    v16f32 sacc[kNKB];
-#pragma unroll
-    for (int kb = 0; kb < kNKB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sacc[kb][i] = 0.f;
-    {
-      // Fragment j: key block j % kNKB, dims 16 (j / kNKB) + 8 half .. +7 of key row qcol.
-      auto read_k = [&](int j) {
-        Frag f;
-        const int row = 32 * (j % kNKB) + qcol, chunk = 2 * (j / kNKB) + half;
-        f.u = *reinterpret_cast<const u32x4 *>(Kt + row * D + 8 * (chunk ^ swz(row)));
-        return f;
-      };
-      Frag ring[kDepth];
-#pragma unroll
-      for (int j = 0; j < kDepth; ++j) ring[j] = read_k(j);
-      __builtin_amdgcn_sched_barrier(0);   // keep the scheduler from sinking the reads to their uses
-      MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
-#pragma unroll
-      for (int j = 0; j < 8 * kNKB; ++j) {
-        sacc[j % kNKB] = mfma<T>(ring[j % kDepth], qf[j / kNKB], sacc[j % kNKB]);
-        if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_k(j + kDepth);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      MUX_PF_PRIO(MUX_PF_PRIO_VALU);
+    // A workgroup's own rows are its last four tiles: their K and V go to the pool
+    // behind the tile's math (the slots' loads hide behind it).
+    const bool to_pool = STEP && writes_pool && k0 >= q0;
+    int64_t slot = -1;                     // of row lane % 32 of the tile
+    if constexpr (STEP) {
+      if (to_pool && k0 + qcol < len) slot = S.slots[static_cast<int64_t>(seq_begin + k0 + qcol) * S.slot_stride + hk];
     }
+    if (t + 1 < n_tiles) dma_tile(cur ^ 1);
+    // (nothing to compute where every key of the tile is in this wave's future, or
+    // all of the wave's rows are past the prompt's end)
+    if (k0 <= wq0 + 31 && wq0 < len) {
+      const uint16_t *const Kt = smem + cur * kTileElems;           // this tile's K
+      const uint16_t *const Vr = smem + (2 + cur) * kTileElems;     // this tile's V (row-major)
 
-    // ---- softmax over keys, per query column --------------------------------------
-    // register i of block kb is key k0 + 32 kb + 8 (i/4) + 4 half + i%4.
-    // Raw scores stay unscaled; scale (> 0) is folded into the exponent:
-    // p = exp2(s * scale_log2 - m * scale_log2).
-    // Exactly one tile per wave straddles the diagonal; only it pays for the mask.
-    if (k0 + kBN - 1 > wq0) {
-      const int rel = my_q - k0 - 4 * half;   // key offset inside the tile, less this lane's share
+      // ---- S^T = K . Q^T : kNKB 32-key blocks -----------------------------------------
+      // LDS fragment reads run kDepth steps ahead of the MFMAs that consume them.
+      // In the P.V product consecutive MFMAs go to different accumulators (4 dim
+      // blocks); a single dependent chain, as here with one key block, runs at 3/4
+      // of the rate.
+      constexpr int kDepth = 4;
+      v16f32 sacc[kNKB];
 #pragma unroll
       for (int kb = 0; kb < kNKB; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * kb + 8 * (i / 4) + (i % 4) > rel) sacc[kb][i] = -INFINITY;
-    }
-    float mx = -INFINITY;
+        for (int i = 0; i < 16; ++i) sacc[kb][i] = 0.f;
+      {
+        // Fragment j: key block j % kNKB, dims 16 (j / kNKB) + 8 half .. +7 of key row qcol.
+        auto read_k = [&](int j) {
+          Frag f;
+          const int row = 32 * (j % kNKB) + qcol, chunk = 2 * (j / kNKB) + half;
+          f.u = *reinterpret_cast<const u32x4 *>(Kt + row * D + 8 * (chunk ^ swz(row)));
+          return f;
+        };
+        Frag ring[kDepth];
 #pragma unroll
-    for (int kb = 0; kb < kNKB; ++kb)
+        for (int j = 0; j < kDepth; ++j) ring[j] = read_k(j);
+        __builtin_amdgcn_sched_barrier(0);   // keep the scheduler from sinking the reads to their uses
+        MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[kb][i]);
-    mx = max_with_lane_xor32(mx);
-    // The reference of the exponents (m_run) only moves when some row's maximum has
-    // risen more than kRescaleStep (in the exponent's units) above it - and on the
-    // wave's first tile, to that tile's maximum: probabilities then reach
-    // 2^kRescaleStep at most, and the 64 accumulators and the running sum are
-    // rescaled rarely instead of whenever a maximum rises at all (with 32 rows per
-    // wave, that is in most tiles of a prompt's first hundreds of keys).
-    constexpr float kRescaleStep = 8.f;
-    const bool move = m_run == -INFINITY ? mx != -INFINITY : (mx - m_run) * I.scale_log2 > kRescaleStep;
-    if (__builtin_amdgcn_ballot_w64(move) != 0) {
-      const float m_new = fmaxf(m_run, mx);
-      // Rows past the prompt may have no valid key at all; keep them finite.
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = fast_exp2((m_run - m_use) * I.scale_log2);
-      l_run *= alpha;
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[mb][i] *= alpha;
-      m_run = m_use;
-    }
-    // (a row that has not seen a valid key yet keeps a finite reference)
-    const float neg_m = m_run == -INFINITY ? 0.f : -m_run * I.scale_log2;
-    float psum = 0.f;
-    Frag pf[2 * kNKB];                          // B fragments: [kb][step] -> index 2 kb + st
-    // bf16 keeps only 8 mantissa bits of a probability, which alone would cost
-    // more than the 2e-3 budget, so bf16 P is carried as hi + lo parts.
-    constexpr bool kSplitP = __is_same(T, BF16);
-    Frag pf_lo[kSplitP ? 2 * kNKB : 1];
-#pragma unroll
-    for (int kb = 0; kb < kNKB; ++kb) {
-      float p[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) p[i] = fast_exp2(__builtin_fmaf(sacc[kb][i], I.scale_log2, neg_m));
-#pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        uint32_t w[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = pack2<T>(p[8 * st + 2 * j], p[8 * st + 2 * j + 1]);
-        pf[2 * kb + st].u = u32x4{w[0], w[1], w[2], w[3]};
-        if constexpr (kSplitP) {
-          // The part of p that its bf16 rounding lost, as a second bf16.
-          uint32_t lo[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            lo[j] = pack2<T>(p[8 * st + 2 * j] - bf16_lo(w[j]), p[8 * st + 2 * j + 1] - bf16_hi(w[j]));
-            psum += p[8 * st + 2 * j] + p[8 * st + 2 * j + 1];
-          }
-          pf_lo[2 * kb + st].u = u32x4{lo[0], lo[1], lo[2], lo[3]};
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) psum += p[8 * st + j];
+        for (int j = 0; j < 8 * kNKB; ++j) {
+          sacc[j % kNKB] = mfma<T>(ring[j % kDepth], qf[j / kNKB], sacc[j % kNKB]);
+          if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_k(j + kDepth);
+          __builtin_amdgcn_sched_barrier(0);
         }
+        MUX_PF_PRIO(MUX_PF_PRIO_VALU);
       }
-    }
-    l_run += psum;
 
-    // ---- O^T += V^T . P^T ---------------------------------------------------------------
-    // k-slot j of lane half h in step (kb, st) is key 32 kb + 16 st + 8 (j/4) + 4 h + j%4
-    {
-      auto read_v = [&](int n) {         // fragment n = 4 ks + mb
-        const int mb = n % 4, ks = n / 4;
-        Frag f;
-        // The transposing read works on groups of 16 lanes: lane 4 j + m of a
-        // group points at dims 4 m .. 4 m + 3 of key row j, and lane i of the
-        // group receives dim i of rows 0..3.  Here a group covers dims
-        // 32 mb + 16 (lane/16 % 2) .. +15 and keys 16 ks + 4 half (+ 8) .. +3.
-        // Address: row = 16 ks + 8 hsel + rl with rl = 4 half + jrow, chunk =
-        // 4 mb + cl, position = chunk ^ swz(row) = (cl ^ swz(rl)) ^ 4 (mb ^ 2 hsel).
-        // The lane part cl ^ rl is below 8, so bit 3 of the constant part adds
-        // and only its bit 2 (mb odd) has to be folded into the lane's base:
-        // two bases per lane, everything else is an immediate offset.
-        typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-        u32x2 part[2];
+      // ---- softmax over keys, per query column --------------------------------------
+      // register i of block kb is key k0 + 32 kb + 8 (i/4) + 4 half + i%4.
+      // Raw scores stay unscaled; scale (> 0) is folded into the exponent:
+      // p = exp2(s * scale_log2 - m * scale_log2).
+      // Exactly one tile per wave straddles the diagonal; only it pays for the mask.
+      if (k0 + kBN - 1 > wq0) {
+        const int rel = my_q - k0 - 4 * half;   // key offset inside the tile, less this lane's share
 #pragma unroll
-        for (int hsel = 0; hsel < 2; ++hsel) {
-          const uint16_t *src = Vr + v_lane_base[mb & 1] + (16 * ks + 8 * hsel) * D + 64 * (((mb >> 1) ^ hsel) & 1);
-          const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)src);
-          union { v4i16 v; u32x2 u; } c;
-          c.v = r;
-          part[hsel] = c.u;
-        }
-        f.u = u32x4{part[0].x, part[0].y, part[1].x, part[1].y};
-        return f;
-      };
-      Frag ring[kDepth];
+        for (int kb = 0; kb < kNKB; ++kb)
 #pragma unroll
-      for (int j = 0; j < kDepth; ++j) ring[j] = read_v(j);
-      __builtin_amdgcn_sched_barrier(0);
-      MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
-#pragma unroll
-      for (int j = 0; j < 8 * kNKB; ++j) {
-        oacc[j % 4] = mfma<T>(ring[j % kDepth], pf[j / 4], oacc[j % 4]);
-        if constexpr (kSplitP) oacc[j % 4] = mfma<T>(ring[j % kDepth], pf_lo[j / 4], oacc[j % 4]);
-        if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_v(j + kDepth);
-        __builtin_amdgcn_sched_barrier(0);
+          for (int i = 0; i < 16; ++i)
+            if (32 * kb + 8 * (i / 4) + (i % 4) > rel) sacc[kb][i] = -INFINITY;
       }
-      MUX_PF_PRIO(MUX_PF_PRIO_VALU);
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < kNKB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[kb][i]);
+      mx = max_with_lane_xor32(mx);
+      // The reference of the exponents (m_run) only moves when some row's maximum has
+      // risen more than kRescaleStep (in the exponent's units) above it - and on the
+      // wave's first tile, to that tile's maximum: probabilities then reach
+      // 2^kRescaleStep at most, and the 64 accumulators and the running sum are
+      // rescaled rarely instead of whenever a maximum rises at all (with 32 rows per
+      // wave, that is in most tiles of a prompt's first hundreds of keys).
+      constexpr float kRescaleStep = 8.f;
+      const bool move = m_run == -INFINITY ? mx != -INFINITY : (mx - m_run) * I.scale_log2 > kRescaleStep;
+      if (__builtin_amdgcn_ballot_w64(move) != 0) {
+        const float m_new = fmaxf(m_run, mx);
+        // Rows past the prompt may have no valid key at all; keep them finite.
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = fast_exp2((m_run - m_use) * I.scale_log2);
+        l_run *= alpha;
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) oacc[mb][i] *= alpha;
+        m_run = m_use;
+      }
+      // (a row that has not seen a valid key yet keeps a finite reference)
+      const float neg_m = m_run == -INFINITY ? 0.f : -m_run * I.scale_log2;
+      float psum = 0.f;
+      Frag pf[2 * kNKB];                          // B fragments: [kb][step] -> index 2 kb + st
+      // bf16 keeps only 8 mantissa bits of a probability, which alone would cost
+      // more than the 2e-3 budget, so bf16 P is carried as hi + lo parts.
+      constexpr bool kSplitP = __is_same(T, BF16);
+      Frag pf_lo[kSplitP ? 2 * kNKB : 1];
+#pragma unroll
+      for (int kb = 0; kb < kNKB; ++kb) {
+        float p[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) p[i] = fast_exp2(__builtin_fmaf(sacc[kb][i], I.scale_log2, neg_m));
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          uint32_t w[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[j] = pack2<T>(p[8 * st + 2 * j], p[8 * st + 2 * j + 1]);
+          pf[2 * kb + st].u = u32x4{w[0], w[1], w[2], w[3]};
+          if constexpr (kSplitP) {
+            // The part of p that its bf16 rounding lost, as a second bf16.
+            uint32_t lo[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              lo[j] = pack2<T>(p[8 * st + 2 * j] - bf16_lo(w[j]), p[8 * st + 2 * j + 1] - bf16_hi(w[j]));
+              psum += p[8 * st + 2 * j] + p[8 * st + 2 * j + 1];
+            }
+            pf_lo[2 * kb + st].u = u32x4{lo[0], lo[1], lo[2], lo[3]};
+          } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) psum += p[8 * st + j];
+          }
+        }
+      }
+      l_run += psum;
+
+      // ---- O^T += V^T . P^T ---------------------------------------------------------------
+      // k-slot j of lane half h in step (kb, st) is key 32 kb + 16 st + 8 (j/4) + 4 h + j%4
+      {
+        auto read_v = [&](int n) {         // fragment n = 4 ks + mb
+          const int mb = n % 4, ks = n / 4;
+          Frag f;
+          // The transposing read works on groups of 16 lanes: lane 4 j + m of a
+          // group points at dims 4 m .. 4 m + 3 of key row j, and lane i of the
+          // group receives dim i of rows 0..3.  Here a group covers dims
+          // 32 mb + 16 (lane/16 % 2) .. +15 and keys 16 ks + 4 half (+ 8) .. +3.
+          // Address: row = 16 ks + 8 hsel + rl with rl = 4 half + jrow, chunk =
+          // 4 mb + cl, position = chunk ^ swz(row) = (cl ^ swz(rl)) ^ 4 (mb ^ 2 hsel).
+          // The lane part cl ^ rl is below 8, so bit 3 of the constant part adds
+          // and only its bit 2 (mb odd) has to be folded into the lane's base:
+          // two bases per lane, everything else is an immediate offset.
+          typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+          u32x2 part[2];
+#pragma unroll
+          for (int hsel = 0; hsel < 2; ++hsel) {
+            const uint16_t *src = Vr + v_lane_base[mb & 1] + (16 * ks + 8 * hsel) * D + 64 * (((mb >> 1) ^ hsel) & 1);
+            const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)src);
+            union { v4i16 v; u32x2 u; } c;
+            c.v = r;
+            part[hsel] = c.u;
+          }
+          f.u = u32x4{part[0].x, part[0].y, part[1].x, part[1].y};
+          return f;
+        };
+        Frag ring[kDepth];
+#pragma unroll
+        for (int j = 0; j < kDepth; ++j) ring[j] = read_v(j);
+        __builtin_amdgcn_sched_barrier(0);
+        MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
+#pragma unroll
+        for (int j = 0; j < 8 * kNKB; ++j) {
+          oacc[j % 4] = mfma<T>(ring[j % kDepth], pf[j / 4], oacc[j % 4]);
+          if constexpr (kSplitP) oacc[j % 4] = mfma<T>(ring[j % kDepth], pf_lo[j / 4], oacc[j % 4]);
+          if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_v(j + kDepth);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        MUX_PF_PRIO(MUX_PF_PRIO_VALU);
+      }
+    }
+    if constexpr (STEP) {
+      stores_counted = false;
+      // (a use on every path: a load left pending would be waited for, and the
+      // next tile's loads with it, where the register is written again)
+      asm volatile("" : "+v"(slot));
+      if (to_pool) {
+        if (slot < 0 || slot >= S.pool_slots) slot = -1;
+        // Rows 0 - 15 (16 - 31) of the tile to all four groups of 16 lanes.
+        const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(slot), static_cast<uint32_t>(slot), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(slot >> 32),
+                                                         static_cast<uint32_t>(slot >> 32), false, false);
+        stores_counted = true;
+#pragma unroll
+        for (int pair = 0; pair < 2; ++pair)
+          stores_counted &= write_tokens_to_pool(
+              smem + cur * kTileElems, smem + (2 + cur) * kTileElems, 16 * pair,
+              static_cast<int64_t>((static_cast<uint64_t>(hi[pair]) << 32) | lo[pair]), wave, lane, S);
+      }
     }
   }
 
@@ -498,6 +715,15 @@ __global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillPar
 #endif
 }
 
+template <typename T>
+__global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillParams P) {
+  prefill_body<T, false>(P, PrefillStep{});
+}
+template <typename T>
+__global__ __launch_bounds__(256, 3) void prefill_step_kernel(const PrefillParams P, const PrefillStep S) {
+  prefill_body<T, true>(P, S);
+}
+
 }  // namespace mux
 
 namespace mux {
@@ -547,16 +773,20 @@ PrefillItemDev device_item(const MuxPrefillItem &it) {
   return d;
 }
 
-hipError_t launch_prefill(const PrefillParams &P, int64_t n_wg, int32_t dtype, hipStream_t st) {
+hipError_t launch_prefill(const PrefillParams &P, const PrefillStep *S, int64_t n_wg, int32_t dtype, hipStream_t st) {
   const dim3 grid(static_cast<uint32_t>(n_wg));
-  if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_causal_kernel<F16>), grid, dim3(256), 0, st, P);
+  if (S != nullptr) {
+    if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_step_kernel<F16>), grid, dim3(256), 0, st, P, *S);
+    else hipLaunchKernelGGL((prefill_step_kernel<BF16>), grid, dim3(256), 0, st, P, *S);
+  } else if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_causal_kernel<F16>), grid, dim3(256), 0, st, P);
   else hipLaunchKernelGGL((prefill_causal_kernel<BF16>), grid, dim3(256), 0, st, P);
   return hipGetLastError();
 }
 
 // One model on the grid sized by its longest prompt (no host-side lengths, or too
 // many query tiles for the kernel argument).
-int32_t launch_dense(const MuxPrefillItem &it, const int32_t *prompt_order, int32_t dtype, hipStream_t st) {
+int32_t launch_dense(const MuxPrefillItem &it, const int32_t *prompt_order, const PrefillStep *S, int32_t dtype,
+                     hipStream_t st) {
   PrefillParams P = {};
   P.it[0] = device_item(it);
   P.prompt_order = prompt_order;
@@ -564,15 +794,16 @@ int32_t launch_dense(const MuxPrefillItem &it, const int32_t *prompt_order, int3
   P.num_groups = it.num_prompts * it.num_kv_heads;
   const int64_t n_wg = static_cast<int64_t>((P.num_groups + 7) / 8) * 8 * P.it[0].ratio * P.q_tiles;
   if (n_wg > 0x7fffffff || P.q_tiles > 0xffff) return MUXA_EUNSUPPORTED;
-  hipError_t e = launch_prefill(P, n_wg, dtype, st);
+  hipError_t e = launch_prefill(P, S, n_wg, dtype, st);
   if (e != hipSuccess) return hip_fail(e);
   return MUXA_OK;
 }
 
 // items[first .. first + n): one launch over the query tiles that exist, the
 // heaviest (most keys) of all models first; false when they do not fit the
-// kernel argument.
-bool launch_compact(const MuxPrefillItem *items, int n, int32_t dtype, hipStream_t st, int32_t *rc) {
+// kernel argument.  S: the step form (one item).
+bool launch_compact(const MuxPrefillItem *items, int n, const PrefillStep *S, int32_t dtype, hipStream_t st,
+                    int32_t *rc) {
   PrefillParams P = {};
   int64_t total = 0;
   int max_tiles = 0, slots = 0, n_dev = 0;
@@ -625,7 +856,7 @@ bool launch_compact(const MuxPrefillItem *items, int n, int32_t dtype, hipStream
     *rc = MUXA_EUNSUPPORTED;
     return true;
   }
-  hipError_t e = launch_prefill(P, n_wg, dtype, st);
+  hipError_t e = launch_prefill(P, S, n_wg, dtype, st);
   if (e != hipSuccess) *rc = hip_fail(e);
   return true;
 }
@@ -644,11 +875,12 @@ extern "C" int32_t mux_multi_prefill_causal(const MuxPrefillItem *items, int32_t
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   int32_t rc = MUXA_OK;
-  if (launch_compact(items, n_items, dtype, st, &rc)) return rc;
+  if (launch_compact(items, n_items, nullptr, dtype, st, &rc)) return rc;
   // Not all in one kernel argument: one launch per model, compact where possible.
   for (int i = 0; i < n_items; ++i) {
     if (items[i].num_prompts == 0 || items[i].max_prompt_len == 0) continue;
-    if (!launch_compact(items + i, 1, dtype, st, &rc)) rc = launch_dense(items[i], nullptr, dtype, st);
+    if (!launch_compact(items + i, 1, nullptr, dtype, st, &rc))
+      rc = launch_dense(items[i], nullptr, nullptr, dtype, st);
     if (rc != MUXA_OK) return rc;
   }
   return MUXA_OK;
@@ -682,8 +914,50 @@ extern "C" int32_t mux_prefill_causal(void *out, int64_t out_row_stride, const v
   if (num_prompts == 0 || max_prompt_len == 0) return MUXA_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
   int32_t rc = MUXA_OK;
-  if (launch_compact(&it, 1, dtype, st, &rc)) return rc;
-  return launch_dense(it, prompt_order, dtype, st);
+  if (launch_compact(&it, 1, nullptr, dtype, st, &rc)) return rc;
+  return launch_dense(it, prompt_order, nullptr, dtype, st);
+}
+
+extern "C" int32_t mux_rope_prefill_and_cache(const MuxPrefillItem *attn, const MuxCacheWriteItem *write, void *k_pool,
+                                              void *v_pool, int64_t num_pool_blocks, int32_t head_size,
+                                              int32_t block_size, int32_t dtype, void *stream) {
+  using namespace mux;
+  if (!attn || !write) return MUXA_EINVAL;
+  if (dtype != MUXA_DTYPE_F16 && dtype != MUXA_DTYPE_BF16) return MUXA_EUNSUPPORTED;
+  const MuxPrefillItem &it = *attn;
+  const MuxCacheWriteItem &w = *write;
+  int32_t rc = check_prefill_item(it, head_size);
+  if (rc != MUXA_OK) return rc;
+  rc = check_cache_write(w.k, w.v, w.kv_row_stride, k_pool, v_pool, num_pool_blocks, w.slot_mapping, w.layer,
+                         w.num_layers, w.num_tokens, w.num_kv_heads, head_size, block_size, dtype);
+  if (rc != MUXA_OK) return rc;
+  // Both items describe the same q, k and v, and every token belongs to a prompt.
+  if (it.q != w.q || it.k != w.k || it.v != w.v || it.q_row_stride != w.q_row_stride ||
+      it.kv_row_stride != w.kv_row_stride || it.num_q_heads != w.num_q_heads || it.num_kv_heads != w.num_kv_heads)
+    return MUXA_EINVAL;
+  if (w.num_tokens > 0 && (!w.positions || !w.cos_sin || !it.prompt_lens_host)) return MUXA_EINVAL;
+  if (w.max_position <= 0) return MUXA_EINVAL;
+  if (w.rotary_dim != kHeadSize) return MUXA_EUNSUPPORTED;
+  int64_t tokens = 0;
+  for (int p = 0; p < it.num_prompts && it.prompt_lens_host; ++p) tokens += it.prompt_lens_host[p];
+  if (tokens != w.num_tokens) return MUXA_EINVAL;
+  if (tokens == 0) return MUXA_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const hipError_t e = launch_rotary_k(w.positions, static_cast<uint16_t *>(w.k), w.kv_row_stride, w.cos_sin,
+                                       w.max_position, w.num_tokens, w.num_kv_heads, dtype, st);
+  if (e != hipSuccess) return hip_fail(e);
+  PrefillStep S = {};
+  S.positions = w.positions;
+  S.cos_sin = w.cos_sin;
+  S.slots = w.slot_mapping + static_cast<int64_t>(w.layer) * w.num_kv_heads;
+  S.slot_stride = static_cast<int64_t>(w.num_layers) * w.num_kv_heads;
+  S.k_pool = static_cast<uint16_t *>(k_pool);
+  S.v_pool = static_cast<uint16_t *>(v_pool);
+  S.pool_slots = num_pool_blocks * block_size;
+  S.max_position = w.max_position;
+  S.block_size = block_size;
+  if (launch_compact(&it, 1, &S, dtype, st, &rc)) return rc;
+  return launch_dense(it, nullptr, &S, dtype, st);
 }
 
 #ifdef MUX_TRACE

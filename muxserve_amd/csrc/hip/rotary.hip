@@ -8,7 +8,7 @@
 // the host; arithmetic is fp32 and each result is rounded once to the storage
 // type.  One workgroup per token; a thread handles two adjacent pair indices
 // (4-byte loads/stores), heads of q first, then heads of k.
-#include "mux_common.h"
+#include "cache_write.h"
 
 namespace mux {
 
@@ -50,6 +50,19 @@ __global__ __launch_bounds__(256) void rotary_neox_kernel(const int64_t *__restr
     *reinterpret_cast<uint32_t *>(row + i) = xo;
     *reinterpret_cast<uint32_t *>(row + half + i) = yo;
   }
+}
+
+hipError_t launch_rotary_k(const int64_t *positions, uint16_t *k, int64_t k_stride, const float *cos_sin,
+                           int32_t max_position, int32_t num_tokens, int32_t num_kv_heads, int32_t dtype,
+                           hipStream_t st) {
+  const dim3 grid(num_tokens);
+  if (dtype == MUXA_DTYPE_F16)
+    hipLaunchKernelGGL(rotary_neox_kernel<F16>, grid, dim3(256), 0, st, positions, nullptr, 0, k, k_stride, cos_sin,
+                       max_position, kHeadSize, 0, num_kv_heads);
+  else
+    hipLaunchKernelGGL(rotary_neox_kernel<BF16>, grid, dim3(256), 0, st, positions, nullptr, 0, k, k_stride, cos_sin,
+                       max_position, kHeadSize, 0, num_kv_heads);
+  return hipGetLastError();
 }
 
 }  // namespace mux

@@ -15,7 +15,7 @@
 #include <algorithm>
 #include <vector>
 
-#include "muxserve_attn.h"
+#include "muxserve_attn_step.h"
 
 namespace {
 
@@ -381,6 +381,75 @@ void prefill_causal(at::Tensor out, const at::Tensor &q, const at::Tensor &k, co
         "mux_prefill_causal");
 }
 
+// A prompt step of one layer: rotary embedding of q and k in place, causal
+// attention, cache write; every token belongs to a prompt.
+void rope_prefill_and_cache(at::Tensor out, const at::Tensor &positions, at::Tensor q, at::Tensor k,
+                            const at::Tensor &v, const at::Tensor &cos_sin, at::Tensor k_pool, at::Tensor v_pool,
+                            const at::Tensor &slot_mapping, int64_t layer, const at::Tensor &cu_seqlens,
+                            at::IntArrayRef prompt_lens, double scale) {
+  need_gpu({&out, &positions, &q, &k, &v, &cos_sin, &k_pool, &v_pool, &slot_mapping, &cu_seqlens});
+  const int64_t bs = check_pools(k_pool, v_pool);
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.dim() == 1 && positions.is_contiguous(),
+              "positions: expected contiguous int64 [T]");
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.dim() == 2 && cos_sin.is_contiguous(),
+              "cos_sin: expected contiguous float32 [max_position, rotary_dim]");
+  TORCH_CHECK(slot_mapping.scalar_type() == at::kLong && slot_mapping.dim() == 3 && slot_mapping.is_contiguous(),
+              "slot_mapping: expected contiguous int64 [T, L, Hkv]");
+  TORCH_CHECK(cu_seqlens.scalar_type() == at::kInt && cu_seqlens.dim() == 1 && cu_seqlens.is_contiguous() &&
+                  cu_seqlens.size(0) == static_cast<int64_t>(prompt_lens.size()) + 1,
+              "cu_seqlens: expected contiguous int32 [P+1], one prompt length per prompt");
+  const std::vector<int32_t> lens(prompt_lens.begin(), prompt_lens.end());
+  int64_t T = 0, longest = 0;
+  for (int64_t n : prompt_lens) {
+    T += n;
+    longest = std::max(longest, n);
+  }
+  const int64_t L = slot_mapping.size(1), H = slot_mapping.size(2);
+  const int64_t stride = rows(k, "k");
+  TORCH_CHECK(rows(v, "v") == stride && k.sizes() == v.sizes() && k.scalar_type() == v.scalar_type() &&
+                  k.scalar_type() == k_pool.scalar_type() && q.scalar_type() == k.scalar_type() &&
+                  out.scalar_type() == q.scalar_type(),
+              "q, k, v, out must share a dtype with the pool; k and v a shape and strides");
+  TORCH_CHECK(q.dim() == 2 && q.size(1) % kHead == 0 && k.size(1) == H * kHead && out.dim() == 2 &&
+                  out.size(1) == q.size(1) &&
+                  std::min({q.size(0), k.size(0), out.size(0), positions.size(0), slot_mapping.size(0)}) >= T,
+              "q/out [>=T, Hq*128], k/v [>=T, Hkv*128], positions [>=T], slot_mapping [>=T, L, Hkv] expected");
+  MuxPrefillItem it = {};
+  it.out = out.data_ptr();
+  it.out_row_stride = rows(out, "out");
+  it.q = q.data_ptr();
+  it.q_row_stride = rows(q, "q");
+  it.k = k.data_ptr();
+  it.v = v.data_ptr();
+  it.kv_row_stride = stride;
+  it.cu_seqlens = cu_seqlens.data_ptr<int32_t>();
+  it.prompt_lens_host = lens.data();
+  it.num_prompts = static_cast<int32_t>(lens.size());
+  it.max_prompt_len = static_cast<int32_t>(longest);
+  it.num_q_heads = static_cast<int32_t>(q.size(1) / kHead);
+  it.num_kv_heads = static_cast<int32_t>(H);
+  it.scale = static_cast<float>(scale);
+  MuxCacheWriteItem w = {};
+  w.positions = positions.data_ptr<int64_t>();
+  w.q = q.data_ptr();
+  w.q_row_stride = it.q_row_stride;
+  w.k = k.data_ptr();
+  w.v = v.data_ptr();
+  w.kv_row_stride = stride;
+  w.cos_sin = cos_sin.data_ptr<float>();
+  w.slot_mapping = slot_mapping.data_ptr<int64_t>();
+  w.max_position = static_cast<int32_t>(cos_sin.size(0));
+  w.rotary_dim = static_cast<int32_t>(cos_sin.size(1));
+  w.layer = static_cast<int32_t>(layer);
+  w.num_layers = static_cast<int32_t>(L);
+  w.num_tokens = static_cast<int32_t>(T);
+  w.num_q_heads = it.num_q_heads;
+  w.num_kv_heads = it.num_kv_heads;
+  check(mux_rope_prefill_and_cache(&it, &w, k_pool.data_ptr(), v_pool.data_ptr(), k_pool.size(0), kHead,
+                                   static_cast<int32_t>(bs), dtype_code(q), stream_of(q)),
+        "mux_rope_prefill_and_cache");
+}
+
 // The prompts of several colocated models in one launch: element i of every
 // list describes model i.  prompt_lens_host: CPU int32 [P_i] per model (the
 // reference holds them on the host, InputMetadata.prompt_lens), or an empty
@@ -477,6 +546,9 @@ TORCH_LIBRARY(muxserve_amd, m) {
         "int total_context_len, Tensor(b!) workspace, Tensor? context_lens_host=None) -> ()");
   m.def("prefill_causal(Tensor(a!) out, Tensor q, Tensor k, Tensor v, Tensor cu_seqlens, int[] prompt_lens, "
         "int max_prompt_len, float scale, int num_kv_heads) -> ()");
+  m.def("rope_prefill_and_cache(Tensor(a!) out, Tensor positions, Tensor(b!) q, Tensor(c!) k, Tensor v, "
+        "Tensor cos_sin, Tensor(d!) k_pool, Tensor(e!) v_pool, Tensor slot_mapping, int layer, Tensor cu_seqlens, "
+        "int[] prompt_lens, float scale) -> ()");
   m.def("multi_prefill_causal(Tensor(a!)[] outs, Tensor[] qs, Tensor[] ks, Tensor[] vs, Tensor[] cu_seqlens, "
         "Tensor[] prompt_lens_host, int[] max_prompt_lens, float[] scales, int[] num_kv_heads) -> ()");
   m.def("multi_decode_workspace_bytes(Tensor[] outs, Tensor[] qs, Tensor[] block_tables, Tensor[] context_lens, "
@@ -499,6 +571,7 @@ TORCH_LIBRARY_IMPL(muxserve_amd, CUDA, m) {
   m.impl("paged_decode_workspace_bytes", &paged_decode_workspace_bytes);
   m.impl("paged_decode", &paged_decode);
   m.impl("prefill_causal", &prefill_causal);
+  m.impl("rope_prefill_and_cache", &rope_prefill_and_cache);
   m.impl("multi_prefill_causal", &multi_prefill_causal);
   m.impl("multi_decode_workspace_bytes", &multi_decode_workspace_bytes);
   m.impl("multi_decode", &multi_decode);

@@ -23,7 +23,7 @@ TORCH_LIB_PATH = os.environ.get("MUXSERVE_TORCH_LIB", os.path.join(_PKG, "libmux
 OPERATORS = ("reshape_and_cache", "rope_reshape_and_cache", "multi_reshape_and_cache", "rotary_neox",
              "paged_decode_workspace_bytes",
              "paged_decode", "multi_decode_workspace_bytes", "multi_decode", "prefill_causal",
-             "multi_prefill_causal", "rms_norm",
+             "rope_prefill_and_cache", "multi_prefill_causal", "rms_norm",
              "silu_and_mul", "greedy_sample_workspace_bytes", "greedy_sample")
 
 _loaded = False
@@ -72,6 +72,12 @@ def prefill_causal(out, q, k, v, cu_seqlens, max_prompt_len: int, scale: float, 
                    prompt_lens=None) -> None:
     load().prefill_causal(out, q, k, v, cu_seqlens, [] if prompt_lens is None else [int(x) for x in prompt_lens],
                           int(max_prompt_len), float(scale), int(num_kv_heads))
+
+
+def rope_prefill_and_cache(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer: int, cu_seqlens,
+                           prompt_lens, scale: float) -> None:
+    load().rope_prefill_and_cache(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,
+                                  prompt_lens, scale)
 
 
 def multi_prefill_causal(calls) -> None:

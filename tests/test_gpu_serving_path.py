@@ -158,6 +158,56 @@ def test_fused_rotary_cache_write_equals_the_two_kernels(dtype, Hq, Hkv, bs):
     assert torch.equal(results[1][0][T:], qkv.cpu().view(torch.int16)[T:]), "padding rows must not be touched"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Hq,Hkv,bs,many", [(3, 3, 16, False), (8, 2, 8, False), (16, 2, 32, False), (2, 1, 16, True)])
+def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many):
+    """rope_prefill_and_cache against rotary, cache write and attention in turn:
+    q, k, both pools and the outputs bitwise equal.  Prompt lengths around the
+    tile and run sizes (or more prompts than the kernel argument lists), tokens
+    without a slot, with a slot outside the pool, and a prompt whose slots are
+    scattered token by token."""
+    print(f"[case] prompt step operator {dtype} Hq={Hq} Hkv={Hkv} bs={bs} many={many}", flush=True)
+    from muxserve_amd import torch_ops, workloads
+    from muxserve_amd.attention import build_cos_sin_cache
+    rng = np.random.Generator(np.random.PCG64(5 + bs))
+    g = torch.Generator().manual_seed(5 + bs)
+    lens = [1] * 400 + [2] * 400 if many else [1, 7, 8, 31, 32, 33, 127, 0, 128, 129, 257, 300]
+    T, L, layer = sum(lens), 2, 1
+    N = sum((n + bs - 1) // bs for n in lens) * Hkv + 5
+    slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), Hkv, bs, rng.permutation(N))
+    first = T - lens[-1]
+    slots[first:, 0, :] = slots[first + rng.permutation(lens[-1]), 0, :]
+    slots[first + 40:first + 56, 0, :] = np.sort(slots[first + 40:first + 56, 0, :], axis=0)
+    slots[T // 2, 0, 0] = -1
+    slots[T - 1, 0, :] = -1
+    slots[T // 3, 0, -1] = N * bs
+    slots = np.concatenate([np.full_like(slots, -1), slots], axis=1)        # layer 1 of 2
+    pad = (T + 7) // 8 * 8
+    qkv = torch.randn((pad, (Hq + 2 * Hkv) * D), generator=g).to(dtype).to(DEV)
+    positions = torch.from_numpy(rng.integers(-3, 2060, size=pad)).to(DEV)   # clamped to the table
+    cos_sin = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    dslots = torch.from_numpy(slots).to(DEV)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
+    results = []
+    for fused in (False, True):
+        x = qkv.clone()
+        q, k, v = x.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+        kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=dtype)
+        kp.fill_(3)
+        vp.fill_(5)
+        out = torch.zeros((pad, Hq * D), dtype=dtype, device=DEV)
+        if fused:
+            torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, dslots, layer, cu, lens, D ** -0.5)
+        else:
+            ops.rotary_neox(positions, q, k, cos_sin, num_tokens=T)
+            ops.reshape_and_cache(k, v, kp, vp, dslots, layer=layer, num_tokens=T)
+            ops.prefill_causal(out[:T], q[:T], k[:T], v[:T], cu, max(lens), D ** -0.5, Hkv, prompt_lens=lens)
+        torch.cuda.synchronize()
+        results.append([t.cpu().view(torch.int16) for t in (x, kp, vp, out)])
+    for a, b, what in zip(*results, ("qkv rows", "k pool", "v pool", "outputs")):
+        assert torch.equal(a, b), f"{what} differ between the step operator and the three kernels"
+
+
 @pytest.mark.parametrize("rope", [True, False])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_multi_model_cache_write_equals_one_launch_per_model(rope, dtype):

@@ -274,8 +274,126 @@ __global__ __launch_bounds__(256) void multi_reshape_and_cache_kernel(const Mult
                               I.num_tokens, P.block_size, I.rope, h, ty * 16);
 }
 
+// What lane 0 (0x00), 1 (0x55), 2 (0xAA) or 3 (0xFF) of the quad holds.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, 0xf, 0xf, true);
+}
+
+// The rotary form for steps of few tokens, where the chain of dependent loads is
+// what counts: 32 lanes per (token, row), a row being a kv head (k rotated in
+// place and scattered, v scattered) or a query head (rotated in place).  A lane
+// holds both halves of its pairs, so nothing meets in LDS or at a barrier, and
+// everything but the cos|sin row is requested at once: two memory latencies
+// against the window kernel's five.  No runs are looked for (a decode step has
+// none); a V store instruction covers 32 neighbouring dims of the block, four
+// lanes to a 128-byte line, where the window kernel's element path spreads 64
+// lanes over 64 lines.
+template <typename T>
+__global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWriteParams P) {
+  constexpr int D = kHeadSize;
+  const int w = blockIdx.x;
+  int ii = 0;
+#pragma unroll
+  for (int i = 1; i < MUXA_MAX_DECODE_ITEMS; ++i)
+    if (i < P.n_items && w >= P.it[i].work_begin) ii = i;
+  const CacheWriteItemDev I = P.it[ii];
+  const RopeArgs R = I.rope;
+  // A kv head is followed by its query heads: all of a token's kv rows first
+  // would put them, and the pool stores, on half of the XCDs where the rows of a
+  // token are a multiple of 64 (32 + 32 heads, 256 tokens: 18.9 us).
+  const int per_kv = R.q != nullptr ? R.ratio + 1 : 1;
+  const int rows = I.num_kv_heads * per_kv;
+  const int unit = (w - I.work_begin) * 8 + (threadIdx.x >> 5);
+  const int l = threadIdx.x & 31;
+  const int t = unit / rows, row = unit - t * rows;
+  if (t >= I.num_tokens) return;
+  const int h = row / per_kv, hq = row - h * per_kv - 1;
+  const bool kv = hq < 0;
+  int64_t pos = R.positions[t];
+  uint32_t *const x = reinterpret_cast<uint32_t *>(
+      kv ? I.k + static_cast<int64_t>(t) * I.row_stride + h * D
+         : R.q + static_cast<int64_t>(t) * R.q_stride + (h * R.ratio + hq) * D);
+  const uint32_t lo = x[l], hi = x[32 + l];
+  int64_t slot = -1;
+  uint16_t ve[4] = {0, 0, 0, 0};
+  if (kv) {
+    slot = I.slots[static_cast<int64_t>(t) * I.slot_stride + h];
+    const uint16_t *vp = I.v + static_cast<int64_t>(t) * I.row_stride + h * D + l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ve[e] = vp[32 * e];
+  }
+  __builtin_amdgcn_sched_barrier(0);       // all of that is requested before the position is waited for
+  pos = pos < 0 ? 0 : (pos >= R.max_position ? R.max_position - 1 : pos);
+  const float2 cs = reinterpret_cast<const float2 *>(R.cos_sin + pos * D)[l];
+  const float2 sn = reinterpret_cast<const float2 *>(R.cos_sin + pos * D + D / 2)[l];
+  float x0, x1, y0, y1;
+  if constexpr (__is_same(T, F16)) {
+    const half2_t a = as_half2(lo), b = as_half2(hi);
+    x0 = static_cast<float>(a.x); x1 = static_cast<float>(a.y);
+    y0 = static_cast<float>(b.x); y1 = static_cast<float>(b.y);
+  } else {
+    x0 = bf16_lo(lo); x1 = bf16_hi(lo);
+    y0 = bf16_lo(hi); y1 = bf16_hi(hi);
+  }
+  const uint32_t xo = static_cast<uint32_t>(to_storage<T>(x0 * cs.x - y0 * sn.x)) |
+                      (static_cast<uint32_t>(to_storage<T>(x1 * cs.y - y1 * sn.y)) << 16);
+  const uint32_t yo = static_cast<uint32_t>(to_storage<T>(y0 * cs.x + x0 * sn.x)) |
+                      (static_cast<uint32_t>(to_storage<T>(y1 * cs.y + x1 * sn.y)) << 16);
+  x[l] = xo;
+  x[32 + l] = yo;
+  // A chunk of the K pool (8 dims) is spread over four lanes: the first of them
+  // stores the lower half's chunk, the second the upper half's (64 dims on).
+  // (both are fetched before the choice: all four lanes take part)
+  const uint32_t ka[4] = {quad_bcast<0x00>(xo), quad_bcast<0x55>(xo), quad_bcast<0xAA>(xo), quad_bcast<0xFF>(xo)};
+  const uint32_t kb[4] = {quad_bcast<0x00>(yo), quad_bcast<0x55>(yo), quad_bcast<0xAA>(yo), quad_bcast<0xFF>(yo)};
+  uint4 kc;
+  kc.x = (l & 1) ? kb[0] : ka[0];
+  kc.y = (l & 1) ? kb[1] : ka[1];
+  kc.z = (l & 1) ? kb[2] : ka[2];
+  kc.w = (l & 1) ? kb[3] : ka[3];
+  if (slot >= 0 && slot < P.num_blocks * P.block_size) {
+    const int bs = P.block_size;
+    const int64_t blk = slot >> __builtin_ctz(static_cast<unsigned>(bs));
+    const int o = static_cast<int>(slot) & (bs - 1);
+    if ((l & 2) == 0) P.k_pool[(blk * (D / 8) + (l >> 2) + 8 * (l & 1)) * bs + o] = kc;
+    uint16_t *const vp = P.v_pool + (blk * D + l) * bs + o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) vp[32 * e * bs] = ve[e];
+  }
+}
+
 }  // namespace mux
 
+namespace mux {
+namespace {
+
+// Up to this many (token, kv head) pairs of all models of a call take
+// rope_scatter_kernel.  us, window kernel -> scatter kernel: decode tokens,
+// 32 heads: 1 token 3.3 -> 2.8, 16 4.7 -> 3.3, 64 6.6 -> 5.0, 256 13.5 -> 11.5;
+// 52 heads: 16 tokens 5.1 -> 3.6; 8 kv heads of 64: 1 token 4.8 -> 2.5, 64
+// 6.5 -> 3.5, 256 8.7 -> 6.4.  The tokens of one prompt, which the window kernel
+// writes as whole chunks: 45 tokens x 32 heads 4.1 -> 3.2, x 52 heads 4.2 -> 5.6,
+// 240 x 8 of 64 8.9 -> 6.1, but 128 x 32 4.5 -> 4.6, 512 x 32 6.9 -> 11.7 and
+// 512 x 8 7.1 -> 9.2: the line lies where the prompts begin to lose.
+constexpr int64_t kScatterPairs = 2560;
+
+hipError_t launch_rope_scatter(MultiCacheWriteParams &P, int32_t dtype, hipStream_t st) {
+  int64_t work = 0;
+  for (int i = 0; i < P.n_items; ++i) {
+    CacheWriteItemDev &d = P.it[i];
+    const int64_t rows = static_cast<int64_t>(d.num_kv_heads) * (d.rope.q != nullptr ? d.rope.ratio + 1 : 1);
+    d.work_begin = static_cast<int32_t>(work);
+    work += (d.num_tokens * rows + 7) / 8;
+  }
+  const dim3 grid(static_cast<unsigned>(work));
+  if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL(rope_scatter_kernel<F16>, grid, dim3(256), 0, st, P);
+  else hipLaunchKernelGGL(rope_scatter_kernel<BF16>, grid, dim3(256), 0, st, P);
+  return hipGetLastError();
+}
+
+}  // namespace
+}  // namespace mux
 
 extern "C" int32_t mux_reshape_and_cache(const void *k, const void *v, int64_t kv_row_stride,
                                          void *k_pool, void *v_pool, int64_t num_pool_blocks,
@@ -328,8 +446,20 @@ extern "C" int32_t mux_rope_reshape_and_cache(const int64_t *positions, void *q,
   R.positions = positions;
   R.cos_sin = cos_sin;
   R.max_position = max_position;
-  dim3 grid(num_kv_heads, (num_tokens + 15) / 16);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (static_cast<int64_t>(num_tokens) * num_kv_heads <= kScatterPairs) {
+    MultiCacheWriteParams P = {};
+    P.it[0] = {static_cast<uint16_t *>(k), static_cast<const uint16_t *>(v), kv_row_stride, slots, slot_stride, R,
+               num_tokens, num_kv_heads, 0};
+    P.k_pool = static_cast<uint4 *>(k_pool);
+    P.v_pool = static_cast<uint16_t *>(v_pool);
+    P.num_blocks = num_pool_blocks;
+    P.n_items = 1;
+    P.block_size = block_size;
+    const hipError_t e = launch_rope_scatter(P, dtype, st);
+    return e == hipSuccess ? MUXA_OK : hip_fail(e);
+  }
+  dim3 grid(num_kv_heads, (num_tokens + 15) / 16);
   if (dtype == MUXA_DTYPE_F16)
     hipLaunchKernelGGL((reshape_and_cache_kernel<F16, true>), grid, dim3(256), 0, st, static_cast<uint16_t *>(k),
                        static_cast<const uint16_t *>(v), kv_row_stride, static_cast<uint4 *>(k_pool),
@@ -400,8 +530,14 @@ extern "C" int32_t mux_multi_rope_reshape_and_cache(const MuxCacheWriteItem *ite
     if (work > 0x7fffffff) return MUXA_EUNSUPPORTED;
   }
   if (P.n_items == 0) return MUXA_OK;
-  const dim3 grid(static_cast<unsigned>(work));
   hipStream_t st = static_cast<hipStream_t>(stream);
+  int64_t pairs = 0;
+  for (int i = 0; i < P.n_items; ++i) pairs += static_cast<int64_t>(P.it[i].num_tokens) * P.it[i].num_kv_heads;
+  if (rope && pairs <= kScatterPairs) {
+    const hipError_t e = launch_rope_scatter(P, dtype, st);
+    return e == hipSuccess ? MUXA_OK : hip_fail(e);
+  }
+  const dim3 grid(static_cast<unsigned>(work));
   if (!rope)
     hipLaunchKernelGGL((multi_reshape_and_cache_kernel<F16, false>), grid, dim3(256), 0, st, P);
   else if (dtype == MUXA_DTYPE_F16)

@@ -159,6 +159,52 @@ def test_fused_rotary_cache_write_equals_the_two_kernels(dtype, Hq, Hkv, bs):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [16, 8, 32])
+@pytest.mark.parametrize("T,Hq,Hkv", [(1, 1, 1), (9, 5, 5), (320, 16, 8), (321, 16, 8)])
+def test_rotary_cache_write_on_both_sides_of_the_scatter_rule(dtype, bs, T, Hq, Hkv):
+    """Steps of few (token, kv head) pairs take a kernel of their own (up to 2560
+    = 320 x 8): one model and two models per call against rotary and cache write in
+    turn, q, k and both pools bitwise equal.  Scattered slots, as decode steps
+    have them, next to runs, missing slots and slots outside the pool."""
+    print(f"[case] rotary + cache write {dtype} T={T} Hq={Hq} Hkv={Hkv} bs={bs}", flush=True)
+    from muxserve_amd.attention import build_cos_sin_cache
+    rng = np.random.Generator(np.random.PCG64(T + bs))
+    g = torch.Generator().manual_seed(T + bs)
+    N = 2 * (2 * T * Hkv // bs + 4)
+    free = rng.permutation(N // 2 * bs)                                # model 0: anywhere in the first half
+    slots = [free[:T * Hkv].reshape(T, 1, Hkv), (N // 2 * bs + np.arange(T * Hkv)).reshape(Hkv, T).T.reshape(T, 1, Hkv)]
+    slots = [np.ascontiguousarray(s.astype(np.int64)) for s in slots]
+    slots[0][T // 2, 0, 0] = -1
+    slots[1][T - 1, 0, -1] = N * bs
+    dslots = [torch.from_numpy(s).to(DEV) for s in slots]
+    rows = [torch.randn((T, (Hq + 2 * Hkv) * D), generator=g).to(dtype).to(DEV) for _ in range(2)]
+    positions = [torch.from_numpy(rng.integers(-2, 2050, size=T)).to(DEV) for _ in range(2)]
+    cos_sin = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    results = []
+    for how in ("kernels", "one", "two"):
+        xs = [x.clone() for x in rows]
+        qkv = [x.split([Hq * D, Hkv * D, Hkv * D], dim=-1) for x in xs]
+        kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=dtype)
+        kp.fill_(3)
+        vp.fill_(5)
+        if how == "two":
+            ops.multi_reshape_and_cache([ops.CacheWriteCall(k, v, s, 0, p, cos_sin, q, T)
+                                         for (q, k, v), s, p in zip(qkv, dslots, positions)], kp, vp)
+        else:
+            for (q, k, v), s, p in zip(qkv, dslots, positions):
+                if how == "one":
+                    ops.rope_reshape_and_cache(p, q, k, v, cos_sin, kp, vp, s)
+                else:
+                    ops.rotary_neox(p, q, k, cos_sin)
+                    ops.reshape_and_cache(k, v, kp, vp, s)
+        torch.cuda.synchronize()
+        results.append([t.cpu().view(torch.int16) for t in (*xs, kp, vp)])
+    for got in results[1:]:
+        for a, b, what in zip(results[0], got, ("rows of model 0", "rows of model 1", "k pool", "v pool")):
+            assert torch.equal(a, b), f"{what} differ from rotary and cache write in turn"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Hq,Hkv,bs,many", [(3, 3, 16, False), (8, 2, 8, False), (16, 2, 32, False), (2, 1, 16, True)])
 def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many):
     """rope_prefill_and_cache against rotary, cache write and attention in turn:

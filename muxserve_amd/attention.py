@@ -201,39 +201,46 @@ class PagedAttentionWithRoPE(PagedAttention):
                 input_metadata: InputMetadata, cache_event: Optional[torch.cuda.Event] = None) -> torch.Tensor:
         md = input_metadata
         n_valid = md.num_valid_tokens
-        fused = False
-        if n_valid > 0:
-            # Rotation and cache write in one launch for small steps (decode: saves a
-            # launch, 12.6 against 20.4 us per layer), when the whole head rotates and
-            # the rows allow 16-byte accesses (q, k, v of one qkv row always do).  Larger
-            # steps that hold generation tokens too keep the two kernels: the fused one
-            # re-reads the cos/sin row of a token once per kv head and is slower there
-            # (101 against 93 us for 4096 tokens x 52 heads).
-            fused = (key_cache is not None and value_cache is not None and self.rotary_dim == self.head_size
-                     and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (query, key, value)))
-            many = md.num_prompts * (self.num_heads // self.num_kv_heads) >= 16
-            if fused and md.num_generation_tokens == 0 and (n_valid > self.fused_rope_max_tokens or many):
-                # A prompt step: the attention kernel rotates q and writes the cache
-                # itself, behind the rotation of k.  A small step with few prompts
-                # is bound by one workgroup's chain of waits, which the rotation
-                # lengthens (32 heads, one prompt of 45 / 400 tokens: 8.9 / 19.9 us
-                # as below, 11.7 / 22.9 us this way; 16 of 30 tokens 15.8 against
-                # 14.4 us; 64 query heads on 8, 4 of 45 tokens 14.6 against 11.8 us;
-                # from 512 tokens on this way is never slower).
-                if cache_event is not None:
-                    cache_event.wait()
-                out = torch.empty((query.shape[0], self.num_heads * self.head_size), dtype=query.dtype,
-                                  device=query.device)
-                T.rope_prefill_and_cache(out, positions, query, key, value, self._cache(query.device), key_cache,
-                                         value_cache, md.slot_mapping, self._layer(md), md.cu_seqlens(query.device),
-                                         md.prompt_lens, self.scale)
-                return out
-            fused = fused and n_valid <= self.fused_rope_max_tokens
-            if fused:
-                if cache_event is not None:
-                    cache_event.wait()
-                T.rope_reshape_and_cache(positions, query, key, value, self._cache(query.device), key_cache,
-                                           value_cache, md.slot_mapping, layer=self._layer(md), num_tokens=n_valid)
-            else:
+        if key_cache is None or value_cache is None or n_valid == 0 or self.rotary_dim != self.head_size:
+            if n_valid > 0:
                 T.rotary_neox(positions, query, key, self._cache(query.device), num_tokens=n_valid)
+            return super().forward(query, key, value, key_cache, value_cache, md, cache_event)
+        # Rotation and cache write in one launch for small steps (decode: saves a
+        # launch, 12.6 against 20.4 us per layer), when the whole head rotates and
+        # the rows allow 16-byte accesses (q, k, v of one qkv row always do).  Larger
+        # steps that hold generation tokens too keep the two kernels: the fused one
+        # re-reads the cos/sin row of a token once per kv head and is slower there
+        # (101 against 93 us for 4096 tokens x 52 heads).
+        cos_sin, layer = self._cache(query.device), self._layer(md)
+        small = n_valid <= self.fused_rope_max_tokens
+        out = None
+        if md.num_prompt_tokens == 0 and small:
+            if cache_event is not None:
+                cache_event.wait()
+            out = T.decode_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping,
+                                 md.block_tables, md.context_lens, md.max_context_len, self.scale, layer,
+                                 self.partition_size, md.total_context_len, md.context_lens_host)
+        elif md.num_generation_tokens == 0:
+            # Prompts only: the attention kernel rotates q and writes the cache
+            # itself, behind the rotation of k.  A small step with few prompts is
+            # bound by one workgroup's chain of waits, which the rotation lengthens
+            # (32 heads, one prompt of 45 / 400 tokens: 8.9 / 19.9 us with rotation
+            # and cache write as a launch of their own, 11.7 / 22.9 us this way; 16
+            # of 30 tokens 15.8 against 14.4 us; 64 query heads on 8, 4 of 45 tokens
+            # 14.6 against 11.8 us; from 512 tokens on this way is never slower).
+            step = not small or md.num_prompts * (self.num_heads // self.num_kv_heads) >= 16
+            if cache_event is not None:
+                cache_event.wait()
+            out = T.prompt_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping, layer,
+                                 md.cu_seqlens(query.device), md.prompt_lens, self.scale, step)
+        if out is not None:
+            return out
+        fused = small and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (query, key, value))
+        if fused:
+            if cache_event is not None:
+                cache_event.wait()
+            T.rope_reshape_and_cache(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping,
+                                     layer=layer, num_tokens=n_valid)
+        else:
+            T.rotary_neox(positions, query, key, cos_sin, num_tokens=n_valid)
         return super().forward(query, key, value, key_cache, value_cache, md, cache_event, _cache_written=fused)

@@ -505,6 +505,62 @@ void multi_prefill_causal(at::TensorList outs, at::TensorList qs, at::TensorList
         "mux_multi_prefill_causal");
 }
 
+// A whole attention layer of a step as one operator: at one short sequence the
+// separate operators' Python and dispatch took twice the time of their kernels
+// (24 against 9 us per layer).  q, k, v rows that 16-byte accesses cannot take are
+// left to the general path, which the caller has for mixed steps as well.
+bool rows_of_16_bytes(const at::Tensor &t) {
+  return t.dim() == 2 && t.stride(0) % 8 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
+// Decode: rotary embedding and cache write of the new tokens, paged attention.
+// Returns (out, 0); or (undefined, bytes) with nothing launched: -1 for rows of
+// another alignment, else the workspace that the call needs.
+std::tuple<at::Tensor, int64_t> decode_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k,
+                                             const at::Tensor &v, const at::Tensor &cos_sin, at::Tensor k_pool,
+                                             at::Tensor v_pool, const at::Tensor &slot_mapping,
+                                             const at::Tensor &block_tables, const at::Tensor &context_lens,
+                                             int64_t max_context_len, double scale, int64_t layer,
+                                             int64_t partition_size, int64_t total_context_len,
+                                             const c10::optional<at::Tensor> &workspace,
+                                             const c10::optional<at::Tensor> &context_lens_host) {
+  if (!rows_of_16_bytes(q) || !rows_of_16_bytes(k) || !rows_of_16_bytes(v)) return {at::Tensor(), -1};
+  at::Tensor out = at::empty(q.sizes(), q.options());
+  const int64_t need =
+      paged_decode_workspace_bytes(out, q, block_tables, context_lens, max_context_len, partition_size);
+  const int64_t have = workspace.has_value() && workspace->defined() ? workspace->numel() : 0;
+  if (need > have) return {at::Tensor(), need};
+  rope_reshape_and_cache(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, context_lens.size(0));
+  paged_decode(out, q, k_pool, v_pool, block_tables, context_lens, max_context_len, scale, layer, partition_size,
+               total_context_len, have > 0 ? *workspace : at::Tensor(), context_lens_host);
+  return {out, 0};
+}
+
+// Prompts: rotary embedding, causal attention, cache write.  step: with the
+// attention kernel doing all but the rotation of k, else rotation and cache write
+// in one launch and the attention behind it.  Undefined with nothing launched: rows
+// of another alignment.
+at::Tensor prompt_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k, const at::Tensor &v,
+                        const at::Tensor &cos_sin, at::Tensor k_pool, at::Tensor v_pool,
+                        const at::Tensor &slot_mapping, int64_t layer, const at::Tensor &cu_seqlens,
+                        at::IntArrayRef prompt_lens, double scale, bool step) {
+  if (!rows_of_16_bytes(q) || !rows_of_16_bytes(k) || !rows_of_16_bytes(v)) return at::Tensor();
+  at::Tensor out = at::empty(q.sizes(), q.options());
+  if (step) {
+    rope_prefill_and_cache(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,
+                           prompt_lens, scale);
+    return out;
+  }
+  int64_t tokens = 0, longest = 0;
+  for (int64_t n : prompt_lens) {
+    tokens += n;
+    longest = std::max(longest, n);
+  }
+  rope_reshape_and_cache(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, tokens);
+  prefill_causal(out, q, k, v, cu_seqlens, prompt_lens, longest, scale, slot_mapping.size(2));
+  return out;
+}
+
 at::Tensor rms_norm(const at::Tensor &x, const at::Tensor &weight, double eps) {
   need_gpu({&x, &weight});
   TORCH_CHECK(x.dim() == 2 && weight.dim() == 1 && weight.size(0) == x.size(1) &&
@@ -560,6 +616,13 @@ TORCH_LIBRARY(muxserve_amd, m) {
   m.def("greedy_sample_workspace_bytes(int vocab_size) -> int", &greedy_sample_workspace_bytes);
   m.def("greedy_sample(Tensor embedding, Tensor hidden_states, int vocab_size, int num_rows, Tensor row_index, "
         "Tensor(a!) workspace) -> Tensor");
+  m.def("decode_layer(Tensor positions, Tensor(a!) q, Tensor(b!) k, Tensor v, Tensor cos_sin, Tensor(c!) k_pool, "
+        "Tensor(d!) v_pool, Tensor slot_mapping, Tensor block_tables, Tensor context_lens, int max_context_len, "
+        "float scale, int layer, int partition_size, int total_context_len, Tensor(e!)? workspace, "
+        "Tensor? context_lens_host) -> (Tensor, int)");
+  m.def("prompt_layer(Tensor positions, Tensor(a!) q, Tensor(b!) k, Tensor v, Tensor cos_sin, Tensor(c!) k_pool, "
+        "Tensor(d!) v_pool, Tensor slot_mapping, int layer, Tensor cu_seqlens, int[] prompt_lens, float scale, "
+        "bool step) -> Tensor");
   m.def("rms_norm(Tensor x, Tensor weight, float eps) -> Tensor");
   m.def("silu_and_mul(Tensor x) -> Tensor");
 }
@@ -577,6 +640,8 @@ TORCH_LIBRARY_IMPL(muxserve_amd, CUDA, m) {
   m.impl("multi_decode", &multi_decode);
   m.impl("rotary_neox", &rotary_neox);
   m.impl("greedy_sample", &greedy_sample);
+  m.impl("decode_layer", &decode_layer);
+  m.impl("prompt_layer", &prompt_layer);
   m.impl("rms_norm", &rms_norm);
   m.impl("silu_and_mul", &silu_and_mul);
 }

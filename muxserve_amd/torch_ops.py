@@ -23,7 +23,7 @@ TORCH_LIB_PATH = os.environ.get("MUXSERVE_TORCH_LIB", os.path.join(_PKG, "libmux
 OPERATORS = ("reshape_and_cache", "rope_reshape_and_cache", "multi_reshape_and_cache", "rotary_neox",
              "paged_decode_workspace_bytes",
              "paged_decode", "multi_decode_workspace_bytes", "multi_decode", "prefill_causal",
-             "rope_prefill_and_cache", "multi_prefill_causal", "rms_norm",
+             "rope_prefill_and_cache", "decode_layer", "prompt_layer", "multi_prefill_causal", "rms_norm",
              "silu_and_mul", "greedy_sample_workspace_bytes", "greedy_sample")
 
 _loaded = False
@@ -101,6 +101,33 @@ def paged_decode(out, q, k_pool, v_pool, block_tables, context_lens, max_context
         ws = torch.empty((0,), dtype=torch.uint8, device=q.device)
     T.paged_decode(out, q, k_pool, v_pool, block_tables, context_lens, int(max_context_len), float(scale), int(layer),
                    int(partition_size), int(total_context_len), ws, context_lens_host)
+
+
+def decode_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, block_tables, context_lens,
+                 max_context_len: int, scale: float, layer: int, partition_size: int, total_context_len: int,
+                 context_lens_host):
+    """The decode step of a layer in one operator: the attention output, or None
+    where the rows of q, k and v do not allow it."""
+    from . import ops
+    op = load().decode_layer
+    device = q.device
+    # (the raw handle: current_stream() builds a Stream object for it)
+    stream = torch._C._cuda_getCurrentRawStream(device.index) if device.index is not None else _current_stream_ptr(device)
+    ws = ops._workspaces.get((device, stream))
+    while True:
+        out, need = op(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, block_tables, context_lens,
+                       max_context_len, scale, layer, partition_size, total_context_len, ws, context_lens_host)
+        if need <= 0:
+            return out if need == 0 else None
+        ws = ops._workspace(need, device, stream)
+
+
+def prompt_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer: int, cu_seqlens, prompt_lens,
+                 scale: float, step: bool):
+    """The prompt step of a layer in one operator: the attention output, or None
+    where the rows of q, k and v do not allow it."""
+    return load().prompt_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,
+                               prompt_lens, scale, step)
 
 
 def rms_norm(x, weight, eps: float):

@@ -335,6 +335,42 @@ def test_multi_model_cache_write_equals_one_launch_per_model(rope, dtype):
         assert torch.equal(results[1][2].view(torch.int16), hv_pool.view(torch.int16))
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_decode_layer_operator_equals_the_general_path(dtype):
+    """One decode step through PagedAttentionWithRoPE as one operator, with the two
+    kernels of large steps (fused_rope_max_tokens 0), and with query rows that
+    16-byte accesses cannot take: rows, pools and outputs bitwise equal."""
+    print(f"[case] decode layer operator {dtype}", flush=True)
+    from muxserve_amd.attention import InputMetadata
+    Hq, Hkv, bs, lens = 8, 2, 16, [1, 17, 700, 33, 1100]
+    B, nb = len(lens), -(-max(lens) // bs)
+    g = torch.Generator().manual_seed(9)
+    N = B * Hkv * nb
+    tables = torch.randperm(N, generator=g).to(torch.int32).reshape(1, B, Hkv, nb)
+    slots = torch.stack([tables[0, i, :, (n - 1) // bs].long() * bs + (n - 1) % bs for i, n in enumerate(lens)])[:, None]
+    ctx = torch.tensor(lens, dtype=torch.int32)
+    md = InputMetadata(prompt_lens=[], slot_mapping=slots.contiguous().to(DEV), context_lens=ctx.to(DEV),
+                       max_context_len=max(lens), block_tables=tables.to(DEV), total_context_len=sum(lens))
+    rows = torch.randn((8, (Hq + 2 * Hkv) * D), generator=g).to(dtype)
+    kp0 = torch.randn((N, D // 8, bs, 8), generator=g).to(dtype)
+    vp0 = torch.randn((N, D, bs), generator=g).to(dtype)
+    positions = torch.tensor([n - 1 for n in lens] + [0] * 3, device=DEV)
+    results = []
+    for fused_max, pad in ((512, 0), (0, 0), (512, 2)):
+        layer = PagedAttentionWithRoPE(Hq, D, D ** -0.5, max_position=2048, rotary_dim=D, num_kv_heads=Hkv, layer_idx=0)
+        layer.fused_rope_max_tokens = fused_max
+        kp, vp = kp0.to(DEV), vp0.to(DEV)
+        _, k, v = rows.to(DEV).split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+        q = torch.zeros((8, Hq * D + pad), dtype=dtype, device=DEV)[:, pad:]
+        q.copy_(rows[:, :Hq * D])
+        out = layer(positions, q, k, v, kp, vp, md, None)
+        torch.cuda.synchronize()
+        results.append([t.cpu().contiguous().view(torch.int16) for t in (out[:B], q, k, kp, vp)])
+    for got in results[1:]:
+        for a, b, what in zip(results[0], got, ("outputs", "q", "k", "k pool", "v pool")):
+            assert torch.equal(a, b), what
+
+
 def test_empty_steps_are_accepted():
     """No tokens, no sequences, no prompts, no sampled rows: every entry point
     returns without launching and without touching its outputs."""

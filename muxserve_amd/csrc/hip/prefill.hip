@@ -336,6 +336,14 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[mb][i] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
+  // Kept beside m_run and changed with it, so that a tile whose reference stays
+  // spends one comparison on it: the score beyond which the reference moves (see
+  // the softmax), and the reference as an exponent.  (Formed in every tile they
+  // were a tenth of its vector instructions: attention of 16 x 2048 tokens f16
+  // 634 -> 619 us, three bf16 prompts of 700 - 4000 tokens 477 -> 469 us.)
+  constexpr float kRescaleStep = 8.f;
+  const float rescale_score = kRescaleStep / I.scale_log2;
+  float m_limit = -INFINITY, neg_m = 0.f;
 
   // Keys needed by this workgroup: positions 0 .. min(len, q0 + 128) - 1.
   const int kv_end = min(len, q0 + kBM);
@@ -547,9 +555,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
       // 2^kRescaleStep at most, and the 64 accumulators and the running sum are
       // rescaled rarely instead of whenever a maximum rises at all (with 32 rows per
       // wave, that is in most tiles of a prompt's first hundreds of keys).
-      constexpr float kRescaleStep = 8.f;
-      const bool move = m_run == -INFINITY ? mx != -INFINITY : (mx - m_run) * I.scale_log2 > kRescaleStep;
-      if (__builtin_amdgcn_ballot_w64(move) != 0) {
+      if (__builtin_amdgcn_ballot_w64(mx > m_limit) != 0) {
         const float m_new = fmaxf(m_run, mx);
         // Rows past the prompt may have no valid key at all; keep them finite.
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -560,9 +566,9 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
           for (int i = 0; i < 16; ++i) oacc[mb][i] *= alpha;
         m_run = m_use;
+        m_limit = m_use + rescale_score;
+        neg_m = -m_use * I.scale_log2;
       }
-      // (a row that has not seen a valid key yet keeps a finite reference)
-      const float neg_m = m_run == -INFINITY ? 0.f : -m_run * I.scale_log2;
       float psum = 0.f;
       Frag pf[2 * kNKB];                          // B fragments: [kb][step] -> index 2 kb + st
       // bf16 keeps only 8 mantissa bits of a probability, which alone would cost

@@ -23,6 +23,14 @@ int32_t mux_rope_prefill_and_cache(const MuxPrefillItem *attn, const MuxCacheWri
                                    void *v_pool, int64_t num_pool_blocks, int32_t head_size, int32_t block_size,
                                    int32_t dtype, void *stream);
 
+/* mux_build_step_inputs and the widening of n_wide int32 (the step's token ids
+ * and positions) to int64, in one launch.  narrow, wide: DEVICE; n_wide may be 0. */
+int32_t mux_build_step(int32_t *mirror, int32_t max_rows, int32_t max_blocks_per_seq, int32_t num_layers,
+                       int32_t num_heads, int32_t block_size, const int32_t *desc, int32_t num_seqs,
+                       const int32_t *block_info, int64_t n_block_info, int32_t max_new_blocks, int32_t num_tokens,
+                       int64_t *slot_mapping, int32_t *block_tables, int32_t max_blocks_out, const int32_t *narrow,
+                       int64_t *wide, int64_t n_wide, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -166,6 +166,8 @@ ATTN_SIGNATURES = {
     "mux_greedy_sample_workspace_init": (c_i32, [c_vp, c_sz, c_vp]),
     "mux_greedy_sample": (c_i32, [c_vp, c_vp, c_i64, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32, c_i32, c_i32, c_i32,
                                   c_vp, c_sz, c_vp]),
+    "mux_build_step": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32,
+                                      c_i32, c_vp, c_vp, c_i32, c_vp, c_vp, c_i64, c_vp]),
     "mux_build_step_inputs": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32,
                                       c_i32, c_vp, c_vp, c_i32, c_vp]),
     "mux_cu_parts_mask": (c_i32, [ctypes.c_uint32, c_i32, c_vp, c_i32]),

@@ -6,16 +6,25 @@
 // of every live request's block-id run in the reference's own order,
 //     mirror[row][token block][layer][head]          (csrc/batch_scheduler.h:19,44-52)
 // and a step uploads only the allocator's reply plus 8 ints per sequence
-// (mux_sched_get_batch_compact).  Three small kernels, all plain coalesced
-// integer copies bound by HBM:
+// (mux_sched_get_batch_compact).  One kernel of four kinds of workgroups, all
+// plain coalesced integer copies; the kinds do not wait for each other, because
+// ids that this step appends are read from the reply rather than from the mirror.
+// (As three kernels and two conversions a decode step of 32 sequences spent 20 us
+// of the GPU and five launches on them; the 17 steps of a batch of 32 requests,
+// host work included, 2145 -> 1893 us.)
 //   append   the reply's new ids are copied behind each request's run
 //   slots    slot_mapping[t][l][h] = id * block_size + offset, read from the
 //            mirror: prompt token k -> block k / bs, offset k % bs; decode token ->
 //            last block, offset (ctx - 1) % bs    (csrc/batch_scheduler.h:42-67)
 //   table    decode steps: mirror rows transposed through LDS into the layout the
 //            attention kernel reads, [L][sequence][H][token block]
+//   widen    token ids and positions, uploaded as int32, to the int64 that the
+//            model takes
 // Results are bit-identical to what mux_sched_get_batch writes.
+#include <algorithm>
+
 #include "mux_common.h"
+#include "muxserve_attn_step.h"
 
 namespace mux {
 
@@ -27,7 +36,13 @@ struct StepParams {
   const int32_t *block_info;     // the allocator's reply, [n_block_info]
   int64_t *slot_mapping;         // [num_tokens][per]
   int32_t *block_tables;         // [L][num_seqs][H][max_blocks_out]
-  int64_t n_block_info;
+  const int32_t *narrow;         // [n_wide]
+  int64_t *wide;                 // [n_wide]
+  int64_t n_block_info, n_wide;
+  // Workgroups: append_chunks per sequence, then slot_rows per token, then
+  // table_x * table_y per sequence, then those of widen.
+  int64_t begin_slots, begin_table, begin_widen, end;
+  int32_t append_chunks, slot_rows, table_x, table_y;
   int32_t num_seqs, per, H, max_rows, max_blocks_per_seq, block_size, max_blocks_out, num_tokens;
 };
 
@@ -38,19 +53,25 @@ __device__ __forceinline__ bool desc_ok(const StepParams &P, const int32_t *d) {
          static_cast<int64_t>(d[2]) + d[3] <= d[1] && d[4] >= 1 && d[4] + count <= P.n_block_info && d[5] >= 0 && d[6] >= 0;
 }
 
-__global__ __launch_bounds__(256) void step_append_kernel(const StepParams P) {
-  const int32_t *d = P.desc + blockIdx.y * kDescInts;
+// Id j (layer and head) of a sequence's token block tb.
+__device__ __forceinline__ const int32_t *block_ids(const StepParams &P, const int32_t *d, int tb) {
+  const int fresh = tb - d[2];
+  if (fresh >= 0 && fresh < d[3]) return P.block_info + d[4] + static_cast<int64_t>(fresh) * P.per;
+  return P.mirror + (static_cast<int64_t>(d[0]) * P.max_blocks_per_seq + tb) * P.per;
+}
+
+__device__ __forceinline__ void step_append(const StepParams &P, int seq, int chunk) {
+  const int32_t *d = P.desc + seq * kDescInts;
   if (!desc_ok(P, d)) return;
   const int64_t count = static_cast<int64_t>(d[3]) * P.per;
-  const int64_t begin = static_cast<int64_t>(blockIdx.x) * 1024;
+  const int64_t begin = static_cast<int64_t>(chunk) * 1024;
   const int64_t end = min(count, begin + 1024);
   int32_t *dst = P.mirror + (static_cast<int64_t>(d[0]) * P.max_blocks_per_seq + d[2]) * P.per;
   const int32_t *src = P.block_info + d[4];
   for (int64_t e = begin + threadIdx.x; e < end; e += 256) dst[e] = src[e];
 }
 
-__global__ __launch_bounds__(256) void step_slots_kernel(const StepParams P) {
-  const int t = blockIdx.x;
+__device__ __forceinline__ void step_slots(const StepParams &P, int t, int part) {
   const int lane = threadIdx.x & 63;
   // The batch entry that owns token t: the last one whose first token is <= t.
   int before = 0;
@@ -74,27 +95,25 @@ __global__ __launch_bounds__(256) void step_slots_kernel(const StepParams P) {
     off = k % P.block_size;
   }
   if (tb < 0 || tb >= d[1]) return;
-  const int32_t *ids = P.mirror + (static_cast<int64_t>(d[0]) * P.max_blocks_per_seq + tb) * P.per;
+  const int32_t *ids = block_ids(P, d, tb);
   int64_t *out = P.slot_mapping + static_cast<int64_t>(t) * P.per;
-  for (int j = blockIdx.y * 1024 + threadIdx.x; j < min(P.per, (static_cast<int>(blockIdx.y) + 1) * 1024); j += 256)
+  for (int j = part * 1024 + threadIdx.x; j < min(P.per, (part + 1) * 1024); j += 256)
     out[j] = static_cast<int64_t>(ids[j]) * P.block_size + off;
 }
 
 // One 64 x 64 tile of a sequence's [token block][layer, head] matrix, transposed.
-__global__ __launch_bounds__(256) void step_table_kernel(const StepParams P) {
+__device__ __forceinline__ void step_table(const StepParams &P, int c, int bx, int by) {
   __shared__ int32_t tile[64][65];
-  const int c = blockIdx.z;
   const int32_t *d = P.desc + c * kDescInts;
   const bool ok = desc_ok(P, d) && d[7];
   const int n_blocks = ok ? d[1] : 0;
-  const int j0 = blockIdx.x * 64, tb0 = blockIdx.y * 64;
+  const int j0 = bx * 64, tb0 = by * 64;
   const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
   if (n_blocks > tb0) {
-    const int32_t *src = P.mirror + static_cast<int64_t>(d[0]) * P.max_blocks_per_seq * P.per;
 #pragma unroll 4
     for (int r = y; r < 64; r += 4) {
       const int tb = tb0 + r, j = j0 + x;
-      tile[r][x] = (tb < n_blocks && j < P.per) ? src[static_cast<int64_t>(tb) * P.per + j] : 0;
+      tile[r][x] = (tb < n_blocks && j < P.per) ? block_ids(P, d, tb)[j] : 0;
     }
   }
   __syncthreads();
@@ -110,6 +129,24 @@ __global__ __launch_bounds__(256) void step_table_kernel(const StepParams P) {
   }
 }
 
+__global__ __launch_bounds__(256) void step_build_kernel(const StepParams P) {
+  const int64_t w = static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x;
+  if (w >= P.end) return;
+  if (w < P.begin_slots) {
+    step_append(P, static_cast<int>(w / P.append_chunks), static_cast<int>(w % P.append_chunks));
+  } else if (w < P.begin_table) {
+    const int64_t u = w - P.begin_slots;
+    step_slots(P, static_cast<int>(u / P.slot_rows), static_cast<int>(u % P.slot_rows));
+  } else if (w < P.begin_widen) {
+    const int64_t u = w - P.begin_table, xy = static_cast<int64_t>(P.table_x) * P.table_y;
+    const int in = static_cast<int>(u % xy);
+    step_table(P, static_cast<int>(u / xy), in % P.table_x, in / P.table_x);
+  } else {
+    const int64_t e = (w - P.begin_widen) * 256 + threadIdx.x;
+    if (e < P.n_wide) P.wide[e] = P.narrow[e];
+  }
+}
+
 }  // namespace mux
 
 extern "C" int32_t mux_build_step_inputs(int32_t *mirror, int32_t max_rows, int32_t max_blocks_per_seq,
@@ -118,12 +155,24 @@ extern "C" int32_t mux_build_step_inputs(int32_t *mirror, int32_t max_rows, int3
                                          int64_t n_block_info, int32_t max_new_blocks, int32_t num_tokens,
                                          int64_t *slot_mapping, int32_t *block_tables, int32_t max_blocks_out,
                                          void *stream) {
+  return mux_build_step(mirror, max_rows, max_blocks_per_seq, num_layers, num_heads, block_size, desc, num_seqs,
+                        block_info, n_block_info, max_new_blocks, num_tokens, slot_mapping, block_tables,
+                        max_blocks_out, nullptr, nullptr, 0, stream);
+}
+
+extern "C" int32_t mux_build_step(int32_t *mirror, int32_t max_rows, int32_t max_blocks_per_seq, int32_t num_layers,
+                                  int32_t num_heads, int32_t block_size, const int32_t *desc, int32_t num_seqs,
+                                  const int32_t *block_info, int64_t n_block_info, int32_t max_new_blocks,
+                                  int32_t num_tokens, int64_t *slot_mapping, int32_t *block_tables,
+                                  int32_t max_blocks_out, const int32_t *narrow, int64_t *wide, int64_t n_wide,
+                                  void *stream) {
   using namespace mux;
   if (!mirror || max_rows <= 0 || max_blocks_per_seq <= 0 || num_layers <= 0 || num_heads <= 0 || block_size <= 0)
     return MUXA_EINVAL;
   if (num_seqs < 0 || num_tokens < 0 || n_block_info < 1 || max_new_blocks < 0 || max_blocks_out < 0) return MUXA_EINVAL;
-  if (num_seqs == 0) return MUXA_OK;
-  if (!desc || !block_info || (num_tokens > 0 && !slot_mapping) || (max_blocks_out > 0 && !block_tables))
+  if (n_wide < 0 || (n_wide > 0 && (!narrow || !wide))) return MUXA_EINVAL;
+  if (num_seqs == 0) num_tokens = max_new_blocks = max_blocks_out = 0;      // nothing but the conversion
+  if (num_seqs > 0 && (!desc || !block_info || (num_tokens > 0 && !slot_mapping) || (max_blocks_out > 0 && !block_tables)))
     return MUXA_EINVAL;
   const int64_t per = static_cast<int64_t>(num_layers) * num_heads;
   // Grid limits: y and z dimensions hold at most 65535 workgroups.
@@ -145,19 +194,25 @@ extern "C" int32_t mux_build_step_inputs(int32_t *mirror, int32_t max_rows, int3
   P.block_size = block_size;
   P.max_blocks_out = max_blocks_out;
   P.num_tokens = num_tokens;
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  if (max_new_blocks > 0) {
-    const int64_t chunks = (static_cast<int64_t>(max_new_blocks) * per + 1023) / 1024;
-    if (chunks > 0x7fffffff) return MUXA_EUNSUPPORTED;
-    hipLaunchKernelGGL(step_append_kernel, dim3(static_cast<uint32_t>(chunks), num_seqs), dim3(256), 0, st, P);
-  }
-  if (num_tokens > 0)
-    hipLaunchKernelGGL(step_slots_kernel, dim3(num_tokens, static_cast<uint32_t>((per + 1023) / 1024)), dim3(256), 0,
-                       st, P);
-  if (max_blocks_out > 0)
-    hipLaunchKernelGGL(step_table_kernel,
-                       dim3(static_cast<uint32_t>((per + 63) / 64), (max_blocks_out + 63) / 64, num_seqs), dim3(256), 0,
-                       st, P);
+  P.narrow = narrow;
+  P.wide = wide;
+  P.n_wide = n_wide;
+  const int64_t chunks = (static_cast<int64_t>(max_new_blocks) * per + 1023) / 1024;
+  if (chunks > 0x7fffffff) return MUXA_EUNSUPPORTED;
+  P.append_chunks = static_cast<int32_t>(chunks);
+  P.slot_rows = static_cast<int32_t>((per + 1023) / 1024);
+  P.table_x = static_cast<int32_t>((per + 63) / 64);
+  P.table_y = (max_blocks_out + 63) / 64;
+  P.begin_slots = chunks * num_seqs;
+  P.begin_table = P.begin_slots + static_cast<int64_t>(num_tokens) * P.slot_rows;
+  P.begin_widen = P.begin_table + static_cast<int64_t>(P.table_x) * P.table_y * num_seqs;
+  P.end = P.begin_widen + (n_wide + 255) / 256;
+  if (P.end == 0) return MUXA_OK;
+  // (a dimension of the grid holds fewer than 2^32 threads)
+  const int64_t gx = std::min<int64_t>(P.end, 1 << 20), gy = (P.end + gx - 1) / gx;
+  if (gy > 65535) return MUXA_EUNSUPPORTED;
+  hipLaunchKernelGGL(step_build_kernel, dim3(static_cast<uint32_t>(gx), static_cast<uint32_t>(gy)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), P);
   MUX_HIP_TRY(hipGetLastError());
   return MUXA_OK;
 }

@@ -51,10 +51,13 @@ class DeviceBlockTables:
         return dev
 
     def build(self, desc: torch.Tensor, block_info: torch.Tensor, num_seqs: int, max_new_blocks: int,
-              num_tokens: int, max_blocks_out: int, stream=None) -> Tuple[torch.Tensor, torch.Tensor]:
+              num_tokens: int, max_blocks_out: int, stream=None, narrow=None, wide=None
+              ) -> Tuple[torch.Tensor, torch.Tensor]:
         """desc int32 [num_seqs, 8] and block_info int32 [n] on the device ->
         (slot_mapping int64 [num_tokens, L, H], block_tables int32
-        [L, num_seqs, H, max_blocks_out] or the reference's empty prefill table)."""
+        [L, num_seqs, H, max_blocks_out] or the reference's empty prefill table).
+        narrow, wide: optionally an int32 tensor that goes to the int64 tensor of as
+        many elements in the same launch."""
         slot_mapping = torch.empty((num_tokens, self.L, self.H), dtype=torch.int64, device=self.device)
         if max_blocks_out > 0:
             block_tables = torch.empty((self.L, num_seqs, self.H, max_blocks_out), dtype=torch.int32,
@@ -64,9 +67,11 @@ class DeviceBlockTables:
             block_tables = torch.empty((0, 0, 0, self.max_blocks_per_seq), dtype=torch.int32, device=self.device)
             bt_ptr = None
         st = torch.cuda.current_stream(self.device).cuda_stream if stream is None else stream
-        rc = _lib.attn().mux_build_step_inputs(
+        rc = _lib.attn().mux_build_step(
             self.mirror.data_ptr(), self.max_rows, self.max_blocks_per_seq, self.L, self.H, self.block_size,
             desc.data_ptr(), int(num_seqs), block_info.data_ptr(), block_info.numel(), int(max_new_blocks),
-            int(num_tokens), slot_mapping.data_ptr() if num_tokens else None, bt_ptr, int(max_blocks_out), st)
-        _lib.check_attn(rc, "mux_build_step_inputs")
+            int(num_tokens), slot_mapping.data_ptr() if num_tokens else None, bt_ptr, int(max_blocks_out),
+            None if narrow is None else narrow.data_ptr(), None if wide is None else wide.data_ptr(),
+            0 if narrow is None else narrow.numel(), st)
+        _lib.check_attn(rc, "mux_build_step")
         return slot_mapping, block_tables

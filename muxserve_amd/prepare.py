@@ -120,12 +120,12 @@ def _prepare_on_device(sched, dt, batch_block_request, block_info, num_tokens, n
     batch_reqs = sched.get_batch_reqs()
 
     dev = dt.upload(total)
-    input_tensor = dev[o_tok:o_pos].long()                                       # llm_runtime.py:324-325
-    input_positions = dev[o_pos:o_ctx].long()
+    tokens_positions = torch.empty((2, padded_len), dtype=torch.int64, device=dt.device)     # llm_runtime.py:324-325
+    input_tensor, input_positions = tokens_positions.unbind(0)
     context_lens = dev[o_ctx:o_ctx + num_contexts]
     decoding = max_context_len > 0
     slot_mapping, block_tables = dt.build(dev[o_desc:o_info], dev[o_info:total], n_entries, max_new, num_tokens,
-                                          max_num_blocks_per_seq if decoding else 0)
+                                          max_num_blocks_per_seq if decoding else 0, narrow=dev[:o_ctx], wide=tokens_positions)
     input_metadata = InputMetadata(prompt_lens=prompt_lens, slot_mapping=slot_mapping, context_lens=context_lens,
                                    max_context_len=max_context_len, block_tables=block_tables,
                                    total_context_len=total_context_len, context_lens_host=context_lens_host)

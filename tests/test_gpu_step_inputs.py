@@ -171,3 +171,43 @@ def test_descriptors_that_do_not_fit_are_skipped():
     assert torch.equal(slots.cpu(), want_slots)
     # no descriptor here is a decode step: every table row is defined and empty
     assert (tables.cpu() == 0).all()
+
+
+@pytest.mark.parametrize("num_seqs,n_wide", [(0, 1), (0, 256), (0, 257), (3, 0), (3, 513)])
+def test_one_launch_appends_reads_the_appended_and_widens(num_seqs, n_wide):
+    """mux_build_step: sequences whose last blocks arrive with this step (slots and
+    tables read them from the reply, the mirror gets them) beside the int32 ->
+    int64 conversion around the size of a workgroup."""
+    print(f"[case] step build num_seqs={num_seqs} n_wide={n_wide}", flush=True)
+    from muxserve_amd import _lib
+    L, H, bs, rows, max_blk = 3, 25, 16, 5, 70
+    per = L * H
+    g = torch.Generator().manual_seed(1)
+    mirror = torch.randint(0, 1 << 20, (rows, max_blk, L, H), generator=g, dtype=torch.int32)
+    reply = torch.randint(0, 1 << 20, (1 + 3 * per,), generator=g, dtype=torch.int32)
+    # row, blocks, first new, new, reply offset, length, first token, decoding
+    desc = torch.tensor([[4, 66, 65, 1, 1, 65 * bs + 3, 0, 1], [0, 2, 0, 2, 1 + per, 2 * bs, 1, 1],
+                         [2, 3, 3, 0, 1, 3 * bs - 2, 2, 1]], dtype=torch.int32)
+    narrow = torch.randint(-5, 1 << 30, (max(n_wide, 1),), generator=g, dtype=torch.int32)
+    d_mirror, d_reply, d_desc, d_narrow = mirror.to(DEV), reply.to(DEV), desc.to(DEV), narrow.to(DEV)
+    wide = torch.full((max(n_wide, 1) + 8,), -3, dtype=torch.int64, device=DEV)
+    slots = torch.full((3, L, H), -1, dtype=torch.int64, device=DEV)
+    tables = torch.full((L, 3, H, max_blk), -9, dtype=torch.int32, device=DEV)
+    rc = _lib.attn().mux_build_step(
+        d_mirror.data_ptr(), rows, max_blk, L, H, bs, d_desc.data_ptr(), num_seqs, d_reply.data_ptr(), reply.numel(),
+        2, 3, slots.data_ptr(), tables.data_ptr(), max_blk, d_narrow.data_ptr(), wide.data_ptr(), n_wide,
+        torch.cuda.current_stream().cuda_stream)
+    _lib.check_attn(rc, "mux_build_step")
+    torch.cuda.synchronize()
+    assert torch.equal(wide.cpu()[:n_wide], narrow.long()[:n_wide]) and (wide.cpu()[n_wide:] == -3).all()
+    if num_seqs == 0:
+        assert (slots.cpu() == -1).all() and (tables.cpu() == -9).all() and torch.equal(d_mirror.cpu(), mirror)
+        return
+    want = mirror.clone()
+    want[4, 65] = reply[1:1 + per].view(L, H)
+    want[0, :2] = reply[1 + per:].view(2, L, H)
+    assert torch.equal(d_mirror.cpu(), want)
+    for c, (row, n, _, _, _, length, tok, _) in enumerate(desc.tolist()):
+        assert torch.equal(slots.cpu()[tok], want[row, n - 1].long() * bs + (length - 1) % bs)
+        got = tables.cpu()[:, c]
+        assert torch.equal(got[:, :, :n], want[row, :n].permute(1, 2, 0)) and (got[:, :, n:] == 0).all()

@@ -214,13 +214,16 @@ class PagedAttentionWithRoPE(PagedAttention):
         cos_sin, layer = self._cache(query.device), self._layer(md)
         small = n_valid <= self.fused_rope_max_tokens
         out = None
-        if md.num_prompt_tokens == 0 and small:
+        # (shapes that do not fit each other keep the general path and its refusals)
+        if query.shape[-1] != self.num_heads * self.head_size:
+            pass
+        elif md.num_prompt_tokens == 0 and small:
             if cache_event is not None:
                 cache_event.wait()
             out = T.decode_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping,
                                  md.block_tables, md.context_lens, md.max_context_len, self.scale, layer,
                                  self.partition_size, md.total_context_len, md.context_lens_host)
-        elif md.num_generation_tokens == 0:
+        elif md.num_generation_tokens == 0 and md.slot_mapping.shape[::2] == (n_valid, self.num_kv_heads):
             # Prompts only: the attention kernel rotates q and writes the cache
             # itself, behind the rotation of k.  A small step with few prompts is
             # bound by one workgroup's chain of waits, which the rotation lengthens

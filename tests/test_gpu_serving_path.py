@@ -371,6 +371,26 @@ def test_decode_layer_operator_equals_the_general_path(dtype):
             assert torch.equal(a, b), what
 
 
+@pytest.mark.parametrize("n", [40, 600])
+def test_prompt_step_with_unaligned_query_rows_is_refused(n):
+    """The attention kernel takes 16-byte accesses to the query rows only; such a
+    step reaches the general path, which refuses it, whatever its size."""
+    from muxserve_amd.attention import InputMetadata
+    H, bs = 2, 16
+    nb = -(-n // bs)
+    kp, vp = allocate_gpu_cache(nb * H, bs, DEV)
+    t = torch.arange(n, device=DEV)
+    slots = torch.stack([(t // bs * H + h) * bs + t % bs for h in range(H)], dim=1)[:, None].contiguous()
+    none = torch.empty((0,), dtype=torch.int32, device=DEV)
+    md = InputMetadata(prompt_lens=[n], slot_mapping=slots, context_lens=none, max_context_len=0,
+                       block_tables=none.view(0, 0, 0, 0))
+    layer = PagedAttentionWithRoPE(H, D, D ** -0.5, max_position=2048, rotary_dim=D, num_kv_heads=H, layer_idx=0)
+    k, v = (torch.randn((n, H * D), device=DEV).half() for _ in range(2))
+    q = torch.zeros((n, H * D + 2), dtype=torch.float16, device=DEV)[:, 2:]
+    with pytest.raises(RuntimeError, match="invalid argument"):
+        layer(t, q, k, v, kp, vp, md, None)
+
+
 def test_empty_steps_are_accepted():
     """No tokens, no sequences, no prompts, no sampled rows: every entry point
     returns without launching and without touching its outputs."""

@@ -42,7 +42,7 @@ constexpr int kSlotWin = 48;             // slots of tokens 16w-16 .. 16w+31 are
 constexpr int kTileRows = 32;            // a window lies inside tokens 16w-16 .. 16w+15
 
 // One workgroup's window: kv head h, tokens around T0 (a multiple of 16).
-template <typename T, bool ROPE>
+template <typename T, bool ROPE, bool EARLY_Q>
 __device__ __forceinline__ void cache_write_window(
     uint16_t *k, const uint16_t *__restrict__ v, int64_t row_stride,
     uint4 *__restrict__ k_pool, uint16_t *__restrict__ v_pool, int64_t num_blocks,
@@ -120,33 +120,32 @@ __device__ __forceinline__ void cache_write_window(
   const bool two_passes = jb - ja > 16;                    // uniform
   const int il = threadIdx.x >> 4, cl = threadIdx.x & 15;
   const int pc = (cl ^ 8) - cl;            // the partner chunk of the rotation, in chunks from this one
-  // Rotating, the positions and the rows of the query head (where a kv head has
-  // one) are requested with k and v, so that only the cos|sin row is a memory
-  // latency of its own: prompts of three models, 1.25 GB, 264 -> 255 us (4.9 TB/s;
-  // more waves per SIMD at fewer registers are slower, 260 - 270 us).
-  uint4 kx2[2], vx2[2], kp2[2], qx2[2], qp2[2];
-  int64_t pos2[2];
+  // EARLY_Q, for one query head per kv head: the positions and the query rows are
+  // requested with k and v, so that only the cos|sin row is a memory latency of
+  // its own.
+  uint4 kx2[2], vx2[2], kp2[2], qx2[EARLY_Q ? 2 : 1], qp2[EARLY_Q ? 2 : 1];
+  int64_t pos2[EARLY_Q ? 2 : 1];
   const int n_q = ROPE && R.q != nullptr ? R.ratio : 0;
   const int64_t q_head0 = static_cast<int64_t>(h) * R.ratio * D + cl * 8;
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
-    kx2[pass] = vx2[pass] = kp2[pass] = qx2[pass] = qp2[pass] = make_uint4(0, 0, 0, 0);
-    pos2[pass] = 0;
+    kx2[pass] = vx2[pass] = kp2[pass] = make_uint4(0, 0, 0, 0);
+    if constexpr (EARLY_Q) {
+      qx2[pass] = qp2[pass] = make_uint4(0, 0, 0, 0);
+      pos2[pass] = 0;
+    }
     if (pass == 1 && !two_passes) break;
     const int j = ja + 16 * pass + il;
     if (j < jb && (ROPE || s_slot[j] >= 0)) {
       const int64_t src = static_cast<int64_t>(T0 - kBack + j) * row_stride + h * D + cl * 8;
       kx2[pass] = *reinterpret_cast<const uint4 *>(k + src);
       vx2[pass] = *reinterpret_cast<const uint4 *>(v + src);
-      if constexpr (ROPE) {
-        const int t = T0 - kBack + j;
-        pos2[pass] = R.positions[t];
-        kp2[pass] = *reinterpret_cast<const uint4 *>(k + src + pc * 8);
-        if (n_q == 1) {
-          const uint16_t *qp = R.q + static_cast<int64_t>(t) * R.q_stride + q_head0;
-          qx2[pass] = *reinterpret_cast<const uint4 *>(qp);
-          qp2[pass] = *reinterpret_cast<const uint4 *>(qp + pc * 8);
-        }
+      if constexpr (EARLY_Q) pos2[pass] = R.positions[T0 - kBack + j];
+      if constexpr (ROPE) kp2[pass] = *reinterpret_cast<const uint4 *>(k + src + pc * 8);
+      if (EARLY_Q && n_q == 1) {
+        const uint16_t *qp = R.q + static_cast<int64_t>(T0 - kBack + j) * R.q_stride + q_head0;
+        qx2[pass] = *reinterpret_cast<const uint4 *>(qp);
+        qp2[pass] = *reinterpret_cast<const uint4 *>(qp + pc * 8);
       }
     }
   }
@@ -165,7 +164,9 @@ __device__ __forceinline__ void cache_write_window(
       const int64_t src = static_cast<int64_t>(t) * row_stride + h * D + cl * 8;
       float cs[8], sn[8];
       if (mine) {
-        int64_t pos = pos2[pass];
+        int64_t pos;
+        if constexpr (EARLY_Q) pos = pos2[pass];
+        else pos = R.positions[t];
         pos = pos < 0 ? 0 : (pos >= R.max_position ? R.max_position - 1 : pos);
         const float *row = R.cos_sin + pos * D + (cl & 7) * 8;
 #pragma unroll
@@ -182,10 +183,11 @@ __device__ __forceinline__ void cache_write_window(
         for (int g = 0; g < 4; ++g)
           if (mine && g0 + g < n_q) {
             const uint16_t *qp = q0 + (g0 + g) * D;
-            const bool here = n_q == 1;                // requested above
-            const uint4 own = here ? qx2[pass] : *reinterpret_cast<const uint4 *>(qp);
-            const uint4 partner = here ? qp2[pass] : *reinterpret_cast<const uint4 *>(qp + pc * 8);
-            qx[g] = rotate_chunk<T>(own, partner, cs, sn, cl >= 8);
+            if (EARLY_Q && n_q == 1)
+              qx[g] = rotate_chunk<T>(qx2[pass], qp2[pass], cs, sn, cl >= 8);
+            else
+              qx[g] = rotate_chunk<T>(*reinterpret_cast<const uint4 *>(qp),
+                                      *reinterpret_cast<const uint4 *>(qp + pc * 8), cs, sn, cl >= 8);
           }
         __syncthreads();
         if (mine && g0 == 0) *reinterpret_cast<uint4 *>(k + src) = kx;
@@ -244,13 +246,13 @@ __device__ __forceinline__ void cache_write_window(
 // Heads vary fastest over the workgroup ids: workgroups that run together read
 // the neighbouring 256-byte head slices of the same k/v rows (one DRAM page)
 // rather than one slice out of each of many rows.
-template <typename T, bool ROPE>
+template <typename T, bool ROPE, bool EARLY_Q>
 __global__ __launch_bounds__(256) void reshape_and_cache_kernel(
     uint16_t *k, const uint16_t *__restrict__ v, int64_t row_stride,
     uint4 *__restrict__ k_pool, uint16_t *__restrict__ v_pool, int64_t num_blocks,
     const int64_t *__restrict__ slots, int64_t slot_stride, int num_tokens, int block_size, const RopeArgs R) {
-  cache_write_window<T, ROPE>(k, v, row_stride, k_pool, v_pool, num_blocks, slots, slot_stride, num_tokens,
-                              block_size, R, blockIdx.x, blockIdx.y * 16);
+  cache_write_window<T, ROPE, EARLY_Q>(k, v, row_stride, k_pool, v_pool, num_blocks, slots, slot_stride, num_tokens,
+                                       block_size, R, blockIdx.x, blockIdx.y * 16);
 }
 
 // Several colocated models' cache writes of one step in one grid: the kernel
@@ -277,7 +279,7 @@ struct MultiCacheWriteParams {
   int32_t block_size;
 };
 
-template <typename T, bool ROPE>
+template <typename T, bool ROPE, bool EARLY_Q>
 __global__ __launch_bounds__(256) void multi_reshape_and_cache_kernel(const MultiCacheWriteParams P) {
   const int w = blockIdx.x;
   int ii = 0;
@@ -288,8 +290,8 @@ __global__ __launch_bounds__(256) void multi_reshape_and_cache_kernel(const Mult
   const int local = w - I.work_begin;
   const int ty = local / I.num_kv_heads;
   const int h = local - ty * I.num_kv_heads;
-  cache_write_window<T, ROPE>(I.k, I.v, I.row_stride, P.k_pool, P.v_pool, P.num_blocks, I.slots, I.slot_stride,
-                              I.num_tokens, P.block_size, I.rope, h, ty * 16);
+  cache_write_window<T, ROPE, EARLY_Q>(I.k, I.v, I.row_stride, P.k_pool, P.v_pool, P.num_blocks, I.slots, I.slot_stride,
+                                       I.num_tokens, P.block_size, I.rope, h, ty * 16);
 }
 
 // What lane 0 (0x00), 1 (0x55), 2 (0xAA) or 3 (0xFF) of the quad holds.
@@ -396,6 +398,16 @@ namespace {
 // 512 x 8 7.1 -> 9.2: the line lies where the prompts begin to lose.
 constexpr int64_t kScatterPairs = 2560;
 
+// From this many pairs on of kv heads with one query head each (and most pairs of
+// the call being such), the window kernel requests the query rows early.  It takes
+// 88 registers instead of 74 for that: five waves per SIMD instead of six.  us,
+// late -> early, f16: prompts of 10 x 300 tokens x 32 heads 42.5 -> 40.2, 3 x 4000
+// x 32 141.3 -> 135.4 and x 52 227.7 -> 218.0, 1024 x 52 25.2 -> 24.4; but 512 x 32
+// 7.9 -> 8.0, 512 x 52 11.5 -> 11.7 and 384 decode tokens x 32 35.6 -> 36.0.  With
+// more query heads the registers are for nothing (64 / 8 heads, three prompts of
+// 700 - 2000 tokens 41.0 -> 42.2; 16 / 4 heads, 2 x 2000 11.5 -> 12.3).
+constexpr int64_t kEarlyQPairs = 40960;
+
 hipError_t launch_rope_scatter(MultiCacheWriteParams &P, int32_t dtype, hipStream_t st) {
   int64_t work = 0;
   for (int i = 0; i < P.n_items; ++i) {
@@ -427,7 +439,7 @@ extern "C" int32_t mux_reshape_and_cache(const void *k, const void *v, int64_t k
   const int64_t *slots = slot_mapping + static_cast<int64_t>(layer) * num_kv_heads;
   dim3 grid(num_kv_heads, (num_tokens + 15) / 16);
   // Without the rotary part the kernel only moves bytes and never writes k.
-  hipLaunchKernelGGL((reshape_and_cache_kernel<F16, false>), grid, dim3(256), 0, static_cast<hipStream_t>(stream),
+  hipLaunchKernelGGL((reshape_and_cache_kernel<F16, false, false>), grid, dim3(256), 0, static_cast<hipStream_t>(stream),
                      const_cast<uint16_t *>(static_cast<const uint16_t *>(k)), static_cast<const uint16_t *>(v),
                      kv_row_stride, static_cast<uint4 *>(k_pool), static_cast<uint16_t *>(v_pool), num_pool_blocks,
                      slots, slot_stride, num_tokens, block_size, RopeArgs{});
@@ -465,7 +477,8 @@ extern "C" int32_t mux_rope_reshape_and_cache(const int64_t *positions, void *q,
   R.cos_sin = cos_sin;
   R.max_position = max_position;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (static_cast<int64_t>(num_tokens) * num_kv_heads <= kScatterPairs) {
+  const int64_t pairs = static_cast<int64_t>(num_tokens) * num_kv_heads;
+  if (pairs <= kScatterPairs) {
     MultiCacheWriteParams P = {};
     P.it[0] = {static_cast<uint16_t *>(k), static_cast<const uint16_t *>(v), kv_row_stride, slots, slot_stride, R,
                num_tokens, num_kv_heads, 0};
@@ -478,14 +491,14 @@ extern "C" int32_t mux_rope_reshape_and_cache(const int64_t *positions, void *q,
     return e == hipSuccess ? MUXA_OK : hip_fail(e);
   }
   dim3 grid(num_kv_heads, (num_tokens + 15) / 16);
-  if (dtype == MUXA_DTYPE_F16)
-    hipLaunchKernelGGL((reshape_and_cache_kernel<F16, true>), grid, dim3(256), 0, st, static_cast<uint16_t *>(k),
-                       static_cast<const uint16_t *>(v), kv_row_stride, static_cast<uint4 *>(k_pool),
-                       static_cast<uint16_t *>(v_pool), num_pool_blocks, slots, slot_stride, num_tokens, block_size, R);
-  else
-    hipLaunchKernelGGL((reshape_and_cache_kernel<BF16, true>), grid, dim3(256), 0, st, static_cast<uint16_t *>(k),
-                       static_cast<const uint16_t *>(v), kv_row_stride, static_cast<uint4 *>(k_pool),
-                       static_cast<uint16_t *>(v_pool), num_pool_blocks, slots, slot_stride, num_tokens, block_size, R);
+  const bool early_q = R.ratio == 1 && pairs >= kEarlyQPairs;
+  const auto kernel =
+      dtype == MUXA_DTYPE_F16
+          ? (early_q ? reshape_and_cache_kernel<F16, true, true> : reshape_and_cache_kernel<F16, true, false>)
+          : (early_q ? reshape_and_cache_kernel<BF16, true, true> : reshape_and_cache_kernel<BF16, true, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, static_cast<uint16_t *>(k), static_cast<const uint16_t *>(v),
+                     kv_row_stride, static_cast<uint4 *>(k_pool), static_cast<uint16_t *>(v_pool), num_pool_blocks, slots,
+                     slot_stride, num_tokens, block_size, R);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e);
   return MUXA_OK;
@@ -549,19 +562,24 @@ extern "C" int32_t mux_multi_rope_reshape_and_cache(const MuxCacheWriteItem *ite
   }
   if (P.n_items == 0) return MUXA_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  int64_t pairs = 0;
-  for (int i = 0; i < P.n_items; ++i) pairs += static_cast<int64_t>(P.it[i].num_tokens) * P.it[i].num_kv_heads;
+  int64_t pairs = 0, one_q_pairs = 0;
+  for (int i = 0; i < P.n_items; ++i) {
+    const int64_t n = static_cast<int64_t>(P.it[i].num_tokens) * P.it[i].num_kv_heads;
+    pairs += n;
+    if (P.it[i].rope.ratio == 1) one_q_pairs += n;
+  }
+  const bool early_q = one_q_pairs >= kEarlyQPairs && one_q_pairs > pairs / 2;
   if (rope && pairs <= kScatterPairs) {
     const hipError_t e = launch_rope_scatter(P, dtype, st);
     return e == hipSuccess ? MUXA_OK : hip_fail(e);
   }
   const dim3 grid(static_cast<unsigned>(work));
-  if (!rope)
-    hipLaunchKernelGGL((multi_reshape_and_cache_kernel<F16, false>), grid, dim3(256), 0, st, P);
-  else if (dtype == MUXA_DTYPE_F16)
-    hipLaunchKernelGGL((multi_reshape_and_cache_kernel<F16, true>), grid, dim3(256), 0, st, P);
-  else
-    hipLaunchKernelGGL((multi_reshape_and_cache_kernel<BF16, true>), grid, dim3(256), 0, st, P);
+  const auto kernel =
+      !rope ? multi_reshape_and_cache_kernel<F16, false, false>
+      : dtype == MUXA_DTYPE_F16
+          ? (early_q ? multi_reshape_and_cache_kernel<F16, true, true> : multi_reshape_and_cache_kernel<F16, true, false>)
+          : (early_q ? multi_reshape_and_cache_kernel<BF16, true, true> : multi_reshape_and_cache_kernel<BF16, true, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, P);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e);
   return MUXA_OK;

@@ -5,6 +5,9 @@ for every layer, exactly as the reference's serving loop drives its attention
 layer (llm_runtime.py:277-339, models/llama.py:149-163).  Checked per layer
 against the oracle; the pool is compared bit-exact at the end.
 """
+import os
+import re
+
 import numpy as np
 import pytest
 import torch
@@ -201,6 +204,66 @@ def test_rotary_cache_write_on_both_sides_of_the_scatter_rule(dtype, bs, T, Hq, 
         results.append([t.cpu().view(torch.int16) for t in (*xs, kp, vp)])
     for got in results[1:]:
         for a, b, what in zip(results[0], got, ("rows of model 0", "rows of model 1", "k pool", "v pool")):
+            assert torch.equal(a, b), f"{what} differ from rotary and cache write in turn"
+
+
+def _cache_write_line(name):
+    """A limit of cache_write.hip's choice of kernels, from its source."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    text = open(os.path.join(root, "muxserve_amd", "csrc", "hip", "cache_write.hip")).read()
+    return int(re.search(rf"constexpr int64_t {name} = (\d+);", text).group(1))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("T,Hq,Hkv,kernel", [(435, 3, 3, "scatter"), (435, 5, 5, "scatter"), (435, 8, 8, "window"),
+                                             (435, 16, 8, "window"), (5119, 8, 8, "window"), (5120, 8, 8, "early"),
+                                             (1030, 40, 40, "early"), (5121, 16, 8, "window")])
+def test_rotary_cache_write_of_packed_prompts_in_each_kernel(dtype, bs, T, Hq, Hkv, kernel):
+    """Packed ragged prompts (windows of up to 31 tokens, runs at every phase) in
+    every form of the rotary cache write, as one call of one model and as one call
+    of two models that hold the two halves of the tokens: rows and pools bitwise
+    those of rotary and cache write in turn."""
+    print(f"[case] packed prompts {dtype} bs={bs} T={T} Hq={Hq} Hkv={Hkv} {kernel}", flush=True)
+    from muxserve_amd import workloads
+    from muxserve_amd.attention import build_cos_sin_cache
+    pairs, small, early = T * Hkv, _cache_write_line("kScatterPairs"), _cache_write_line("kEarlyQPairs")
+    assert kernel == ("scatter" if pairs <= small else "early" if Hq == Hkv and pairs >= early else "window")
+    rng = np.random.Generator(np.random.PCG64(T + bs))
+    g = torch.Generator().manual_seed(T + bs)
+    lens = []
+    while sum(lens) < T:
+        lens.append(min(int(rng.integers(1, 60)), T - sum(lens)))
+    half = len(lens) // 2
+    N = sum((n + bs - 1) // bs for n in lens) * Hkv + 5
+    slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), Hkv, bs, rng.permutation(N))
+    slots[7, 0, 0] = -1
+    slots[T - 1, 0, :] = -1
+    slots[T // 2, 0, -1] = N * bs
+    dslots = torch.from_numpy(slots).to(DEV)
+    qkv = torch.randn((T, (Hq + 2 * Hkv) * D), generator=g).to(dtype).to(DEV)
+    positions = torch.from_numpy(rng.integers(-2, 2050, size=T)).to(DEV)
+    cos_sin = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    results = []
+    for how in ("kernels", "one", "two"):
+        x = qkv.clone()
+        q, k, v = x.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+        kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=dtype)
+        kp.fill_(3)
+        vp.fill_(5)
+        if how == "kernels":
+            ops.rotary_neox(positions, q, k, cos_sin)
+            ops.reshape_and_cache(k, v, kp, vp, dslots)
+        elif how == "one":
+            ops.rope_reshape_and_cache(positions, q, k, v, cos_sin, kp, vp, dslots)
+        else:
+            cut = sum(lens[:half])
+            ops.multi_reshape_and_cache([ops.CacheWriteCall(k[a:b], v[a:b], dslots[a:b], 0, positions[a:b], cos_sin, q[a:b],
+                                                            b - a) for a, b in ((0, cut), (cut, T))], kp, vp)
+        torch.cuda.synchronize()
+        results.append([t.cpu().view(torch.int16) for t in (x, kp, vp)])
+    for got in results[1:]:
+        for a, b, what in zip(results[0], got, ("qkv rows", "k pool", "v pool")):
             assert torch.equal(a, b), f"{what} differ from rotary and cache write in turn"
 
 

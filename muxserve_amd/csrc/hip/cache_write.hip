@@ -269,6 +269,7 @@ struct CacheWriteItemDev {
   int32_t num_tokens;
   int32_t num_kv_heads;
   int32_t work_begin;            // first workgroup of this model
+  int32_t per_xcd;               // rope_scatter_kernel: workgroups of this model per XCD; 0: rows packed token after token
 };
 struct MultiCacheWriteParams {
   CacheWriteItemDev it[MUXA_MAX_DECODE_ITEMS];
@@ -324,10 +325,21 @@ __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWrite
   // token are a multiple of 64 (32 + 32 heads, 256 tokens: 18.9 us).
   const int per_kv = R.q != nullptr ? R.ratio + 1 : 1;
   const int rows = I.num_kv_heads * per_kv;
-  const int unit = (w - I.work_begin) * 8 + (threadIdx.x >> 5);
   const int l = threadIdx.x & 31;
-  const int t = unit / rows, row = unit - t * rows;
-  if (t >= I.num_tokens) return;
+  int t, row;
+  if (I.per_xcd == 0) {
+    const int unit = (w - I.work_begin) * 8 + (threadIdx.x >> 5);
+    t = unit / rows;
+    row = unit - t * rows;
+    if (t >= I.num_tokens) return;
+  } else {
+    const int local = w - I.work_begin;
+    const int u = (local & 7) * I.per_xcd + (local >> 3);
+    const int rows8 = u / I.num_tokens;
+    t = u - rows8 * I.num_tokens;
+    row = 8 * rows8 + (threadIdx.x >> 5);
+    if (row >= rows) return;
+  }
   const int h = row / per_kv, hq = row - h * per_kv - 1;
   const bool kv = hq < 0;
   int64_t pos = R.positions[t];
@@ -389,13 +401,13 @@ namespace mux {
 namespace {
 
 // Up to this many (token, kv head) pairs of all models of a call take
-// rope_scatter_kernel.  us, window kernel -> scatter kernel: decode tokens,
-// 32 heads: 1 token 3.3 -> 2.8, 16 4.7 -> 3.3, 64 6.6 -> 5.0, 256 13.5 -> 11.5;
-// 52 heads: 16 tokens 5.1 -> 3.6; 8 kv heads of 64: 1 token 4.8 -> 2.5, 64
-// 6.5 -> 3.5, 256 8.7 -> 6.4.  The tokens of one prompt, which the window kernel
-// writes as whole chunks: 45 tokens x 32 heads 4.1 -> 3.2, x 52 heads 4.2 -> 5.6,
-// 240 x 8 of 64 8.9 -> 6.1, but 128 x 32 4.5 -> 4.6, 512 x 32 6.9 -> 11.7 and
-// 512 x 8 7.1 -> 9.2: the line lies where the prompts begin to lose.
+// rope_scatter_kernel.  us, window kernel -> scatter kernel, decode: 32 heads, 1
+// token 3.3 -> 2.8, 16 4.7 -> 3.2, 80 7.9 -> 6.3; 52 heads, 48 tokens 7.7 -> 6.1; 64
+// query heads on 8, 1 token 4.8 -> 2.5, 64 6.8 -> 3.5.  One prompt, whose V the
+// window kernel writes as whole chunks: 45 tokens x 32 heads 4.1 -> 3.2, 80 x 32
+// 4.2 -> 4.0, 64 x 40 4.2 -> 4.0, 45 x 52 4.3 -> 4.0, 320 x 8 4.2 -> 4.0, 320 x 8 of
+// 64 8.8 -> 7.4; beyond the line prompts lose (128 x 32 4.7 -> 4.8, 512 x 32 8.0 ->
+// 12.0), though decode goes on winning (256 x 32 23.0 -> 21.7).
 constexpr int64_t kScatterPairs = 2560;
 
 // From this many pairs on of kv heads with one query head each (and most pairs of
@@ -412,9 +424,20 @@ hipError_t launch_rope_scatter(MultiCacheWriteParams &P, int32_t dtype, hipStrea
   int64_t work = 0;
   for (int i = 0; i < P.n_items; ++i) {
     CacheWriteItemDev &d = P.it[i];
-    const int64_t rows = static_cast<int64_t>(d.num_kv_heads) * (d.rope.q != nullptr ? d.rope.ratio + 1 : 1);
+    const int per_kv = d.rope.q != nullptr ? d.rope.ratio + 1 : 1;
+    const int64_t rows = static_cast<int64_t>(d.num_kv_heads) * per_kv;
+    // Eight rows to a workgroup (w runs on XCD w % 8: a model takes multiples of 8).
+    // Packed token after token, a head's tokens come to one XCD where a token's rows
+    // are a multiple of 64 and wander over the XCDs otherwise; the tokens of a prompt
+    // then write their two bytes of a V line in different L2s (45 tokens x 52 heads
+    // 5.4 us, the window kernel 4.3), unless query rows thin out the stores (64 query
+    // heads on 8, where packed decode is 3 % faster).  Else eight rows of one token
+    // per workgroup, and the workgroups of the same eight rows on one XCD or on two
+    // neighbouring ones: 45 x 52 4.0 us, 64 tokens x 40 heads 4.9 -> 4.0.
+    const bool packed = per_kv > 2 || rows % 64 == 0;
+    d.per_xcd = packed ? 0 : static_cast<int32_t>(((rows + 7) / 8 * d.num_tokens + 7) / 8);
     d.work_begin = static_cast<int32_t>(work);
-    work += (d.num_tokens * rows + 7) / 8;
+    work += 8 * (packed ? (d.num_tokens * rows + 63) / 64 : static_cast<int64_t>(d.per_xcd));
   }
   const dim3 grid(static_cast<unsigned>(work));
   if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL(rope_scatter_kernel<F16>, grid, dim3(256), 0, st, P);
@@ -481,7 +504,7 @@ extern "C" int32_t mux_rope_reshape_and_cache(const int64_t *positions, void *q,
   if (pairs <= kScatterPairs) {
     MultiCacheWriteParams P = {};
     P.it[0] = {static_cast<uint16_t *>(k), static_cast<const uint16_t *>(v), kv_row_stride, slots, slot_stride, R,
-               num_tokens, num_kv_heads, 0};
+               num_tokens, num_kv_heads, 0, 0};
     P.k_pool = static_cast<uint4 *>(k_pool);
     P.v_pool = static_cast<uint16_t *>(v_pool);
     P.num_blocks = num_pool_blocks;

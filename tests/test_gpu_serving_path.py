@@ -216,7 +216,9 @@ def _cache_write_line(name):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("bs", [8, 16, 32])
-@pytest.mark.parametrize("T,Hq,Hkv,kernel", [(435, 3, 3, "scatter"), (435, 5, 5, "scatter"), (435, 8, 8, "window"),
+@pytest.mark.parametrize("T,Hq,Hkv,kernel", [(435, 3, 3, "scatter"), (435, 5, 5, "scatter"), (2, 1, 1, "scatter"),
+                                             (49, 52, 52, "scatter"), (64, 40, 40, "scatter"), (320, 32, 8, "scatter"),
+                                             (65, 40, 40, "window"), (435, 8, 8, "window"),
                                              (435, 16, 8, "window"), (5119, 8, 8, "window"), (5120, 8, 8, "early"),
                                              (1030, 40, 40, "early"), (5121, 16, 8, "window")])
 def test_rotary_cache_write_of_packed_prompts_in_each_kernel(dtype, bs, T, Hq, Hkv, kernel):
@@ -233,11 +235,11 @@ def test_rotary_cache_write_of_packed_prompts_in_each_kernel(dtype, bs, T, Hq, H
     g = torch.Generator().manual_seed(T + bs)
     lens = []
     while sum(lens) < T:
-        lens.append(min(int(rng.integers(1, 60)), T - sum(lens)))
+        lens.append(min(int(rng.integers(1, min(60, T))), T - sum(lens)))
     half = len(lens) // 2
     N = sum((n + bs - 1) // bs for n in lens) * Hkv + 5
     slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), Hkv, bs, rng.permutation(N))
-    slots[7, 0, 0] = -1
+    slots[min(7, T - 1), 0, 0] = -1
     slots[T - 1, 0, :] = -1
     slots[T // 2, 0, -1] = N * bs
     dslots = torch.from_numpy(slots).to(DEV)

@@ -343,7 +343,8 @@ int32_t mux_silu_and_mul(void *out, int64_t out_row_stride, const void *x, int64
  *     h = hidden_states[row_index ? row_index[r] : r]     (entries clamped to num_hidden_rows - 1)
  *     next_tokens[r] = argmax_{v < vocab_size} T(h . embedding[v,:])
  * (fp32 accumulation, each logit rounded to T before the comparison as the
- * reference's fp16 logits are; ties go to the lowest id).  On a prompt step
+ * reference's fp16 logits are; ties go to the lowest id; a logit's products are
+ * added up in the same order in every batch size).  On a prompt step
  * row_index holds cumsum(prompt_lens) - 1 (sampler.py:18-24), on a decode step
  * it is NULL.  embedding: [embedding_rows >= vocab_size, hidden_size], the
  * lm_head weight (models/llama.py:317-323); hidden_size a multiple of 256.

@@ -45,9 +45,11 @@ union SmFrag {
 constexpr int kSmTile = 256;              // the hidden size must be a multiple of this
 constexpr int kSmMaxRowsPerPass = 256;
 // Up to 32 sampled rows the narrow kernel, beyond them the wide one (32000 rows of
-// 4096, us, narrow / wide: 8 rows 46.8 / 48.0, 32 rows 47.7 / 47.1, 33 rows
-// 54.3 / 47.1, 64 rows 55.7 / 47.4; with 128 and 256 rows 112 / 57 and 221 / 84,
-// the narrow one passing over the matrix once per 64 rows).
+// 4096, us, narrow / wide: 8 rows 46.8 / 48.0, 32 rows 46.0 / 48.6, 33 rows
+// 52.3 / 48.7, 64 rows 53.5 / 48.7; with 128 and 256 rows 107 / 58 and 214 / 82,
+// the narrow one passing over the matrix once per 64 rows).  Small vocabularies
+// too, though the wide kernel keeps its 128 rows per workgroup there: 16000 rows,
+// 33 rows 46.6 / 35.1, 64 rows 48.0 / 38.5; 4000 rows 37.0 / 30.9 and 38.3 / 33.8.
 constexpr int kSmNarrowRows = 32;
 #ifndef MUX_SM_PREFETCH_TILES
 #define MUX_SM_PREFETCH_TILES 2
@@ -167,8 +169,11 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
   // Workgroups start their walk over the hidden dimension at different tiles
   // (a dot product does not care about the order): with a row pitch that is a
   // power of two - 8 KiB at hidden size 4096 - workgroups walking in step would
-  // all be reading the same few memory channels at any moment.
-  const int t_start = blockIdx.x % n_tiles;
+  // all be reading the same few memory channels at any moment.  The tile depends on the
+  // vocabulary row alone (128 rows start together, in both kernels and at both
+  // workgroup sizes), so that a logit, rounding included, is the same whatever
+  // batch its row is sampled in.
+  const int t_start = blockIdx.x / (8 / (NW * RB)) % n_tiles;
   auto tile_of = [&](int t) {
     const int x = t + t_start;
     return x >= n_tiles ? x - n_tiles : x;
@@ -364,7 +369,11 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
   const int wm = wave >> 2, wn = wave & 3;
   const int r16 = lane & 15, g = lane >> 4;
   const int n_tiles = P.hidden_size / KT;
-  const int t_start = blockIdx.x % n_tiles;            // (see the kernel above)
+  // The same element as in the kernel above.  (Starts at odd tiles as well would
+  // spread a power-of-two pitch better - 32000 x 4096, 33 - 64 rows 46.6 us against
+  // 48.7, 256 rows 80.8 against 81.6 - but a near tie could then go another way in
+  // a batch of 33 rows than in one of 32.)
+  const int t_start = 2 * (blockIdx.x % (n_tiles / 2));
   const int vrow0 = blockIdx.x * VR;
 
   // Staging: thread -> row tid / 8 (+ 64 j), chunk tid % 8.  Every load is

@@ -185,6 +185,28 @@ def test_greedy_sample_many_rows_planted_winners(dtype, R, V, Hd, gathered):
     assert toks.cpu().tolist() == ids.tolist()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("V,Hd", [(1000, 256), (5003, 768), (24448, 1024), (24577, 512)])
+def test_greedy_sample_does_not_depend_on_the_batch(dtype, V, Hd):
+    """A row's token is the same whatever batch it is sampled in: the kernels for
+    few and for many rows add up a logit's products in one order, on both sides of
+    the vocabulary's line (24449 rows).  The second half of every dot product
+    cancels the first exactly, so that logits are nothing but rounding errors and
+    any other order would give other tokens."""
+    print(f"[case] greedy_sample batches {dtype} V={V} hidden={Hd}", flush=True)
+    g = torch.Generator().manual_seed(V + Hd)
+    R = 300
+    emb = (torch.randn((V, Hd), generator=g) * 30).to(dtype).to(DEV)
+    hid = torch.randn((R, Hd), generator=g).to(dtype).to(DEV)
+    emb[:, Hd // 2:] = -emb[:, :Hd // 2]
+    hid[:, Hd // 2:] = hid[:, :Hd // 2]
+    want = torch.cat([ops.greedy_sample(emb, hid[r:r + 1], V, 1) for r in range(R)])
+    assert want.unique().numel() > R // 4                       # rounding errors do decide
+    for batch in (16, 17, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257, 300):
+        got = torch.cat([ops.greedy_sample(emb, hid[r:r + batch], V, min(batch, R - r)) for r in range(0, R, batch)])
+        assert torch.equal(got, want), f"batches of {batch}"
+
+
 def test_greedy_sampler_module_prompt_and_decode_steps():
     print("[case] GreedySampler module", flush=True)
     g = torch.Generator().manual_seed(11)

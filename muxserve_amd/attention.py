@@ -112,6 +112,33 @@ def build_cos_sin_cache(rotary_dim: int, max_position: int, base: float, device)
     return torch.cat([freqs.cos(), freqs.sin()], dim=-1).float().to(device)
 
 
+def prompt_step_pays(prompts: int, tokens: int, heads: int, kv_heads: int) -> bool:
+    """Whether a step of prompts is faster with the attention kernel rotating q and
+    writing the cache itself, behind the rotation of k, than with rotation and cache
+    write in one launch and the attention behind it.  us, two launches / attention
+    kernel doing it, where the lines lie:
+
+    * few query rows are bound by one workgroup's chain of waits, which the rotation
+      lengthens: 32 heads, one prompt of 45 tokens 9.0 / 12.4; 16 on 2 heads, 2 of
+      256 16.9 / 18.9, 4 of 300 22.7 / 21.7;
+    * a workgroup holds 128 query rows and writes the cache in groups of 16: prompts
+      of 6 tokens fill neither (128 of them, 32 heads 33 / 47; 64 of 16 tokens, 52
+      heads 37.4 / 41.6; 256 of 19, 32 heads 104 / 92), and with several query heads
+      per kv head one of them does all the writing (32 on 8 heads, 128 of 45 tokens
+      59.8 / 65.6, 128 of 128 148 / 140);
+    * up to 512 tokens: the workgroups have to fill the chip (64 on 8 heads, 2
+      prompts of 100 tokens 13.5 / 15.9, 4 of 100 19.2 / 17.0), in one round where
+      each has a cache part to write (32 heads, 16 of 30 tokens 16.0 / 14.9; 52
+      heads 22.6 / 24.0)."""
+    ratio = heads // kv_heads
+    if tokens * heads < 12288 or (ratio > 1 and tokens < 48 * prompts and tokens * kv_heads > 16384):
+        return False
+    if tokens > 512:
+        return tokens >= 18 * prompts
+    return (prompts * ratio >= 16 and tokens >= 24 * prompts and (prompts + tokens // 128) * heads > 256
+            and (ratio > 1 or prompts * heads <= 768))
+
+
 class PagedAttention(torch.nn.Module):
     """Cache write + causal prefill attention + paged decode attention for one
     layer of one model over the unified pool."""
@@ -224,14 +251,7 @@ class PagedAttentionWithRoPE(PagedAttention):
                                  md.block_tables, md.context_lens, md.max_context_len, self.scale, layer,
                                  self.partition_size, md.total_context_len, md.context_lens_host)
         elif md.num_generation_tokens == 0 and md.slot_mapping.shape[::2] == (n_valid, self.num_kv_heads):
-            # Prompts only: the attention kernel rotates q and writes the cache
-            # itself, behind the rotation of k.  A small step with few prompts is
-            # bound by one workgroup's chain of waits, which the rotation lengthens
-            # (32 heads, one prompt of 45 / 400 tokens: 8.9 / 19.9 us with rotation
-            # and cache write as a launch of their own, 11.7 / 22.9 us this way; 16
-            # of 30 tokens 15.8 against 14.4 us; 64 query heads on 8, 4 of 45 tokens
-            # 14.6 against 11.8 us; from 512 tokens on this way is never slower).
-            step = not small or md.num_prompts * (self.num_heads // self.num_kv_heads) >= 16
+            step = prompt_step_pays(md.num_prompts, n_valid, self.num_heads, self.num_kv_heads)
             if cache_event is not None:
                 cache_event.wait()
             out = T.prompt_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping, layer,

@@ -412,13 +412,16 @@ constexpr int64_t kScatterPairs = 2560;
 
 // From this many pairs on of kv heads with one query head each (and most pairs of
 // the call being such), the window kernel requests the query rows early.  It takes
-// 88 registers instead of 74 for that: five waves per SIMD instead of six.  us,
-// late -> early, f16: prompts of 10 x 300 tokens x 32 heads 42.5 -> 40.2, 3 x 4000
-// x 32 141.3 -> 135.4 and x 52 227.7 -> 218.0, 1024 x 52 25.2 -> 24.4; but 512 x 32
-// 7.9 -> 8.0, 512 x 52 11.5 -> 11.7 and 384 decode tokens x 32 35.6 -> 36.0.  With
-// more query heads the registers are for nothing (64 / 8 heads, three prompts of
-// 700 - 2000 tokens 41.0 -> 42.2; 16 / 4 heads, 2 x 2000 11.5 -> 12.3).
-constexpr int64_t kEarlyQPairs = 40960;
+// 88 registers instead of 74 for that: five waves per SIMD instead of six, which
+// pays where the rows come from memory.  Below the line they are what the projection
+// has just left in the last-level cache (256 MB; q, k, v and pool lines of 262144
+// pairs are 336 MB).  us, late -> early, f16, rows in that cache | in memory, prompts
+// of two and three models: 83808 pairs 27.9 -> 29.7 | 39.5 -> 37.3, 226780 64.7 ->
+// 65.3 | 90.5 -> 88.3, 340376 129.8 -> 128.5 | 131.1 -> 127.1, 829392 300.8 -> 290.2.
+// With more query heads per kv head the registers are for nothing (64 / 8 heads,
+// three prompts of 700 - 2000 tokens 41.0 -> 42.2; 16 / 4 heads, 2 x 2000 11.5 ->
+// 12.3).
+constexpr int64_t kEarlyQPairs = 262144;
 
 hipError_t launch_rope_scatter(MultiCacheWriteParams &P, int32_t dtype, hipStream_t st) {
   int64_t work = 0;

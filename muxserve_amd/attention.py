@@ -252,10 +252,15 @@ class PagedAttentionWithRoPE(PagedAttention):
                                  self.partition_size, md.total_context_len, md.context_lens_host)
         elif md.num_generation_tokens == 0 and md.slot_mapping.shape[::2] == (n_valid, self.num_kv_heads):
             step = prompt_step_pays(md.num_prompts, n_valid, self.num_heads, self.num_kv_heads)
-            if cache_event is not None:
-                cache_event.wait()
-            out = T.prompt_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping, layer,
-                                 md.cu_seqlens(query.device), md.prompt_lens, self.scale, step)
+            # (Large steps of short prompts: rotation and cache write in one launch
+            # are 2 - 13 % faster than in two, but with several query heads per kv
+            # head up to 9 % slower: 40 prompts of 13 tokens, 64 on 8 heads, 33.5
+            # against 30.7 us.)
+            if step or small or self.num_heads == self.num_kv_heads:
+                if cache_event is not None:
+                    cache_event.wait()
+                out = T.prompt_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping,
+                                     layer, md.cu_seqlens(query.device), md.prompt_lens, self.scale, step)
         if out is not None:
             return out
         fused = small and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (query, key, value))

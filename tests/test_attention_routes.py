@@ -13,10 +13,13 @@ def _prompt_route(monkeypatch, lens, heads, kv_heads):
     calls = []
 
     def prompt_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slots, layer, cu_seqlens, prompt_lens, scale, step):
-        calls.append(step)
+        calls.append("step" if step else "one launch")
         return torch.empty_like(q)
 
     monkeypatch.setattr(attention.T, "prompt_layer", prompt_layer)
+    monkeypatch.setattr(attention.T, "rotary_neox", lambda *a, **kw: calls.append("two launches"))
+    for name in ("reshape_and_cache", "prefill_causal"):
+        monkeypatch.setattr(attention.T, name, lambda *a, **kw: None)
     n = sum(lens)
     none = torch.empty((0,), dtype=torch.int32)
     md = InputMetadata(prompt_lens=lens, slot_mapping=torch.zeros((n, 1, kv_heads), dtype=torch.int64), context_lens=none,
@@ -29,13 +32,13 @@ def _prompt_route(monkeypatch, lens, heads, kv_heads):
     return calls[0]
 
 
-@pytest.mark.parametrize("lens,heads,kv_heads,step", [
-    ([6] * 100, 32, 32, False), ([6] * 100, 64, 8, False), ([16] * 64, 52, 52, False), ([20] * 16, 52, 52, False),
-    ([45] * 128, 32, 8, False), ([100] * 2, 64, 8, False), ([45], 32, 32, False), ([400], 32, 32, False),
-    ([30] * 16, 32, 32, True), ([45] * 16, 32, 32, True), ([100] * 4, 64, 8, True), ([128] * 128, 32, 8, True),
-    ([600], 32, 32, True), ([2048] * 4, 52, 52, True)])
-def test_prompt_steps_take_the_faster_of_the_two_forms(monkeypatch, lens, heads, kv_heads, step):
-    """Many short prompts keep rotation and cache write in a launch of their own
-    (as part of the attention kernel they took up to 1.5 times as long), long ones
-    and grouped queries do not."""
-    assert _prompt_route(monkeypatch, lens, heads, kv_heads) is step
+@pytest.mark.parametrize("lens,heads,kv_heads,route", [
+    ([6] * 100, 32, 32, "one launch"), ([6] * 100, 64, 8, "two launches"), ([13] * 40, 64, 8, "two launches"),
+    ([16] * 64, 52, 52, "one launch"), ([20] * 16, 52, 52, "one launch"), ([45] * 128, 32, 8, "two launches"),
+    ([100] * 2, 64, 8, "one launch"), ([45], 32, 32, "one launch"), ([400], 32, 32, "one launch"),
+    ([30] * 16, 32, 32, "step"), ([45] * 16, 32, 32, "step"), ([100] * 4, 64, 8, "step"), ([128] * 128, 32, 8, "step"),
+    ([600], 32, 32, "step"), ([2048] * 4, 52, 52, "step")])
+def test_prompt_steps_take_the_faster_form(monkeypatch, lens, heads, kv_heads, route):
+    """Many short prompts keep rotation and cache write out of the attention kernel
+    (as part of it they took up to 1.5 times as long), long ones do not."""
+    assert _prompt_route(monkeypatch, lens, heads, kv_heads) == route

@@ -54,6 +54,11 @@ def _current_stream_ptr(device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+# The handle without the Stream object that current_stream() builds for it; not a
+# public function of torch, so a torch without it takes the other way.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def reshape_and_cache(k, v, k_pool, v_pool, slot_mapping, layer: int = 0, num_tokens=None) -> None:
     load().reshape_and_cache(k, v, k_pool, v_pool, slot_mapping, int(layer), -1 if num_tokens is None else int(num_tokens))
 
@@ -111,8 +116,7 @@ def decode_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, bloc
     from . import ops
     op = load().decode_layer
     device = q.device
-    # (the raw handle: current_stream() builds a Stream object for it)
-    stream = torch._C._cuda_getCurrentRawStream(device.index) if device.index is not None else _current_stream_ptr(device)
+    stream = _raw_stream(device.index) if _raw_stream is not None else _current_stream_ptr(device)
     ws = ops._workspaces.get((device, stream))
     while True:
         out, need = op(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, block_tables, context_lens,

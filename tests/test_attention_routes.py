@@ -42,3 +42,24 @@ def test_prompt_steps_take_the_faster_form(monkeypatch, lens, heads, kv_heads, r
     """Many short prompts keep rotation and cache write out of the attention kernel
     (as part of it they took up to 1.5 times as long), long ones do not."""
     assert _prompt_route(monkeypatch, lens, heads, kv_heads) == route
+
+
+def test_decode_layer_does_without_torchs_private_stream_handle(monkeypatch):
+    """The workspace of the decode operator is looked up under the current stream's
+    handle, with or without torch's private function for it."""
+    from types import SimpleNamespace
+    from muxserve_amd import ops, torch_ops
+    device, ws, seen = torch.device("cuda", 0), object(), []
+
+    def op(*args):
+        seen.append(args[-2])
+        return "out", 0
+
+    monkeypatch.setattr(torch_ops, "load", lambda: SimpleNamespace(decode_layer=op))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(cuda_stream=7))
+    monkeypatch.setitem(ops._workspaces, (device, 7), ws)
+    q = SimpleNamespace(device=device)
+    for raw in (None, lambda index: 7):
+        monkeypatch.setattr(torch_ops, "_raw_stream", raw, raising=False)
+        assert torch_ops.decode_layer(None, q, *[None] * 15) == "out"
+    assert seen == [ws, ws]

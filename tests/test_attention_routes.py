@@ -61,5 +61,5 @@ def test_decode_layer_does_without_torchs_private_stream_handle(monkeypatch):
     q = SimpleNamespace(device=device)
     for raw in (None, lambda index: 7):
         monkeypatch.setattr(torch_ops, "_raw_stream", raw, raising=False)
-        assert torch_ops.decode_layer(None, q, *[None] * 15) == "out"
+        assert torch_ops.decode_layer(None, q, *[None] * 14) == "out"
     assert seen == [ws, ws]

@@ -94,7 +94,7 @@ def check_host(rc, what):
 
 
 # ---------------------------------------------------------------------------
-# libmuxattn.so (include/muxserve_attn.h)
+# libmuxattn.so (include/muxserve_attn.h, include/muxserve_attn_step.h)
 # ---------------------------------------------------------------------------
 c_f32 = ctypes.c_float
 c_sz = ctypes.c_size_t
@@ -166,8 +166,9 @@ ATTN_SIGNATURES = {
     "mux_greedy_sample_workspace_init": (c_i32, [c_vp, c_sz, c_vp]),
     "mux_greedy_sample": (c_i32, [c_vp, c_vp, c_i64, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32, c_i32, c_i32, c_i32,
                                   c_vp, c_sz, c_vp]),
+    "mux_rope_prefill_and_cache": (c_i32, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i32, c_i32, c_i32, c_vp]),
     "mux_build_step": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32,
-                                      c_i32, c_vp, c_vp, c_i32, c_vp, c_vp, c_i64, c_vp]),
+                               c_i32, c_vp, c_vp, c_i32, c_vp, c_vp, c_i64, c_vp]),
     "mux_build_step_inputs": (c_i32, [c_vp, c_i32, c_i32, c_i32, c_i32, c_i32, c_vp, c_i32, c_vp, c_i64, c_i32,
                                       c_i32, c_vp, c_vp, c_i32, c_vp]),
     "mux_cu_parts_mask": (c_i32, [ctypes.c_uint32, c_i32, c_vp, c_i32]),

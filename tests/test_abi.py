@@ -21,16 +21,17 @@ def _declared(header):
 @pytest.mark.parametrize("header,loader,path", [
     ("muxserve_host.h", _lib.host, _lib.HOST_LIB_PATH),
     ("muxserve_attn.h", _lib.attn, _lib.ATTN_LIB_PATH),
+    ("muxserve_attn_step.h", _lib.attn, _lib.ATTN_LIB_PATH),
 ])
 def test_library_exports_every_declared_symbol(header, loader, path):
     names = _declared(header)
-    assert len(names) >= 10, names
+    assert len(names) >= (2 if header == "muxserve_attn_step.h" else 10), names
     lib = loader()
     raw = ctypes.CDLL(path)
     for n in names:
         assert hasattr(raw, n), f"{n} declared in include/{header} but not exported by {os.path.basename(path)}"
     # every declared symbol also has a typed binding
-    typed = set(_lib.ATTN_SIGNATURES) if header == "muxserve_attn.h" else None
+    typed = set(_lib.ATTN_SIGNATURES) if loader is _lib.attn else None
     if typed is not None:
         assert set(names) <= typed, sorted(set(names) - typed)
     assert lib is loader()      # cached handle
@@ -208,7 +209,7 @@ def test_library_chosen_partition_follows_the_size_of_the_launch():
 
 
 # ---------------------------------------------------------------------------
-# Every entry point of include/muxserve_attn.h called once with well-formed
+# Every entry point of include/muxserve_attn.h and muxserve_attn_step.h called once with well-formed
 # arguments.  No device is present where this runs, so nothing can be launched:
 # each call has to come back with a return code - MUXA_EHIP where it got as far
 # as the HIP runtime, MUXA_OK where the host side had nothing to launch, a byte
@@ -218,6 +219,17 @@ def test_library_chosen_partition_follows_the_size_of_the_launch():
 # dereference them.  Host arrays (context_lens_host, prompt_lens_host, the
 # descriptor arrays, output words) are real.
 # ---------------------------------------------------------------------------
+def _rope_write_item(attn):
+    """The cache-write item that goes with a prefill item of 49 tokens."""
+    w = _lib.MuxCacheWriteItem()
+    w.positions, w.q, w.q_row_stride = 0x7F0000A00000, attn.q, attn.q_row_stride
+    w.k, w.v, w.kv_row_stride = attn.k, attn.v, attn.kv_row_stride
+    w.cos_sin, w.slot_mapping, w.max_position, w.rotary_dim = 0x7F0000B00000, 0x7F0000C00000, 4096, 128
+    w.layer, w.num_layers, w.num_tokens = 0, 1, 49
+    w.num_q_heads, w.num_kv_heads = attn.num_q_heads, attn.num_kv_heads
+    return w
+
+
 def _call_table():
     import numpy as np
     P = lambda k: 0x7F0000000000 + 0x100000 * k          # noqa: E731  fake, 1 MiB apart, 16-byte aligned
@@ -245,11 +257,12 @@ def _call_table():
     cw = (_lib.MuxCacheWriteItem * 1)()
     cw[0].k, cw[0].v, cw[0].kv_row_stride, cw[0].slot_mapping = P(3), P(4), 512, P(6)
     cw[0].layer, cw[0].num_layers, cw[0].num_tokens, cw[0].num_kv_heads = 0, 1, 8, 4
+    rcw = _rope_write_item(pit[0])
     words = (ctypes.c_uint32 * 8)()
     info = (ctypes.c_int32 * 2)()
     sout = ctypes.c_void_p()
     ncu = ctypes.c_int32()
-    keep += [lens, pit, cw, words, info, sout, ncu]
+    keep += [lens, pit, cw, rcw, words, info, sout, ncu]
     ws = 1 << 22
     table = {
         "mux_attn_version": lambda f: f(),
@@ -277,6 +290,9 @@ def _call_table():
         "mux_greedy_sample": lambda f: f(P(1), P(2), 4096, 8, None, 8, P(3), 4096, 32000, 32000, 4096, 0, P(9), ws,
                                          None),
         "mux_build_step_inputs": lambda f: f(P(1), 8, 16, 2, 4, 16, P(2), 4, P(3), 40, 1, 4, P(4), P(5), 16, None),
+        "mux_build_step": lambda f: f(P(1), 8, 16, 2, 4, 16, P(2), 4, P(3), 40, 1, 4, P(4), P(5), 16, P(6), P(7), 24, None),
+        "mux_rope_prefill_and_cache": lambda f: f(ctypes.addressof(pit), ctypes.addressof(rcw), P(7), P(8), 64, 128, 16,
+                                                  0, None),
         "mux_cu_parts_mask": lambda f: f(0b1001, 256, ctypes.addressof(words), 8),
         "mux_stream_create_cu_parts": lambda f: f(ctypes.byref(sout), 0b11, ctypes.byref(ncu)),
         "mux_stream_create_cu_range": lambda f: f(ctypes.byref(sout), 0, 40, ctypes.byref(ncu)),
@@ -292,7 +308,8 @@ def test_every_attn_entry_point_returns_a_code_when_called_without_a_device():
         pytest.skip("a device is present: the made-up device pointers of this test must not reach a kernel")
     lib = _lib.attn()
     table, keep = _call_table()
-    assert set(table) == set(_declared("muxserve_attn.h")), sorted(set(table) ^ set(_declared("muxserve_attn.h")))
+    declared = set(_declared("muxserve_attn.h")) | set(_declared("muxserve_attn_step.h"))
+    assert set(table) == declared, sorted(set(table) ^ declared)
     sizes = {"mux_paged_decode_workspace_bytes", "mux_multi_decode_noalloc_max_bytes",
              "mux_greedy_sample_workspace_bytes"}
     got = {}
@@ -323,3 +340,49 @@ def test_single_model_decode_wrapper_equals_the_fused_entry_point_on_its_argumen
         rc = lib.mux_paged_decode(P, 512, P + 4096, 512, P + 8192, P + 16384, 64, P + 32768, P + 65536, 0, 1, 4, 4, 4,
                                   128, 16, max_blocks, max_ctx, 0.088, 0, 0, P + (1 << 20), 1 << 22, None)
         assert rc == want, (max_ctx, max_blocks, rc)
+
+
+@pytest.mark.parametrize("change,want", [
+    ({}, -4), ({"write.q": 0x7F0000D00000}, -1), ({"write.k": 0x7F0000D00000}, -1), ({"write.v": 0x7F0000D00000}, -1),
+    ({"write.q_row_stride": 1024}, -1), ({"write.kv_row_stride": 1024}, -1), ({"write.num_q_heads": 8}, -1),
+    ({"write.num_kv_heads": 2}, -1), ({"write.num_tokens": 48}, -1), ({"write.num_tokens": 50}, -1),
+    ({"attn.prompt_lens_host": None}, -1), ({"write.positions": None}, -1), ({"write.cos_sin": None}, -1),
+    ({"write.slot_mapping": None}, -1), ({"write.max_position": 0}, -1), ({"write.rotary_dim": 64}, -2),
+    ({"write.layer": 1}, -1), ({"attn.q_row_stride": 516, "write.q_row_stride": 516}, -1),
+    ({"head_size": 64}, -2), ({"block_size": 4}, -2), ({"dtype": 2}, -2), ({"k_pool": None}, -1), ({"blocks": 0}, -1)])
+def test_prompt_step_entry_point_refuses_on_the_host_side(change, want):
+    """mux_rope_prefill_and_cache: items that do not describe the same rows, missing
+    pointers, other sizes - and, unchanged, a call that gets as far as the launch."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("made-up device pointers")
+    lens = (ctypes.c_int32 * 2)(40, 9)
+    it = _lib.MuxPrefillItem()
+    it.out, it.out_row_stride, it.q, it.q_row_stride = 0x7F0000100000, 512, 0x7F0000200000, 512
+    it.k, it.v, it.kv_row_stride, it.cu_seqlens = 0x7F0000300000, 0x7F0000400000, 512, 0x7F0000500000
+    it.prompt_lens_host, it.num_prompts, it.max_prompt_len = ctypes.addressof(lens), 2, 40
+    it.num_q_heads, it.num_kv_heads, it.scale = 4, 4, 0.088
+    w = _rope_write_item(it)
+    args = {"k_pool": 0x7F0000700000, "blocks": 64, "head_size": 128, "block_size": 16, "dtype": 0}
+    for name, value in change.items():
+        where, _, field = name.partition(".")
+        if field:
+            setattr(it if where == "attn" else w, field, value)
+        else:
+            args[name] = value
+    assert _lib.attn().mux_rope_prefill_and_cache(ctypes.addressof(it), ctypes.addressof(w), args["k_pool"], 0x7F0000800000,
+                                                  args["blocks"], args["head_size"], args["block_size"], args["dtype"],
+                                                  None) == want
+
+
+@pytest.mark.parametrize("change,want", [({}, -4), ({"narrow": None}, -1), ({"wide": None}, -1), ({"n_wide": -1}, -1),
+                                         ({"num_seqs": 0, "n_wide": 0}, 0), ({"num_seqs": 0, "desc": None}, -4),
+                                         ({"desc": None}, -1), ({"num_seqs": 1 << 17}, -2)])
+def test_step_input_entry_point_refuses_on_the_host_side(change, want):
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("made-up device pointers")
+    a = {"desc": 0x7F0000200000, "num_seqs": 4, "narrow": 0x7F0000600000, "wide": 0x7F0000700000, "n_wide": 24, **change}
+    assert _lib.attn().mux_build_step(0x7F0000100000, 8, 16, 2, 4, 16, a["desc"], a["num_seqs"], 0x7F0000300000, 40, 1, 4,
+                                      0x7F0000400000, 0x7F0000500000, 16, a["narrow"], a["wide"], a["n_wide"],
+                                      None) == want

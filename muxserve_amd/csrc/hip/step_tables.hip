@@ -43,7 +43,7 @@ struct StepParams {
   // table_x * table_y per sequence, then those of widen.
   int64_t begin_slots, begin_table, begin_widen, end;
   int32_t append_chunks, slot_rows, table_x, table_y;
-  int32_t num_seqs, per, H, max_rows, max_blocks_per_seq, block_size, max_blocks_out, num_tokens;
+  int32_t num_seqs, per, H, max_rows, max_blocks_per_seq, block_size, max_blocks_out;
 };
 
 // A descriptor that does not fit the mirror or the reply is skipped, never followed.
@@ -175,7 +175,7 @@ extern "C" int32_t mux_build_step(int32_t *mirror, int32_t max_rows, int32_t max
   if (num_seqs > 0 && (!desc || !block_info || (num_tokens > 0 && !slot_mapping) || (max_blocks_out > 0 && !block_tables)))
     return MUXA_EINVAL;
   const int64_t per = static_cast<int64_t>(num_layers) * num_heads;
-  // Grid limits: y and z dimensions hold at most 65535 workgroups.
+  // Sizes that no step has (the workgroup count below stays far from 64 bits).
   if (per > 65535 * 1024 || num_seqs > 65535 || max_blocks_out > 65535 * 64 ||
       static_cast<int64_t>(max_new_blocks) * per > (int64_t{1} << 40))
     return MUXA_EUNSUPPORTED;
@@ -193,7 +193,6 @@ extern "C" int32_t mux_build_step(int32_t *mirror, int32_t max_rows, int32_t max
   P.max_blocks_per_seq = max_blocks_per_seq;
   P.block_size = block_size;
   P.max_blocks_out = max_blocks_out;
-  P.num_tokens = num_tokens;
   P.narrow = narrow;
   P.wide = wide;
   P.n_wide = n_wide;

@@ -6,8 +6,8 @@ head) on the host every step and uploads them
 (csrc/batch_scheduler.cpp:131-169, muxserve/flexserver/llm_runtime.py:301-327).
 With a DeviceBlockTables attached to a BatchScheduler a step uploads only the
 token ids, positions, context lengths, the allocator's reply and 8 ints per
-sequence - in one copy - and `mux_build_step_inputs` derives slot_mapping and
-the step's block table on the device, bit-identical to the reference path's.
+sequence - in one copy - and `mux_build_step` derives slot_mapping and the
+step's block table on the device, bit-identical to the reference path's.
 """
 from typing import Tuple
 

@@ -186,6 +186,55 @@ def test_greedy_sample_many_rows_planted_winners(dtype, R, V, Hd, gathered):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("R", [32, 33, 100, 150, 256])
+def test_greedy_sample_many_rows_ties_nan_inf_and_strides(dtype, R):
+    """Exact by construction at every row count: equal winning logits 64 rows apart
+    (the two halves of a tile), in neighbouring and in far workgroups go to the
+    lowest id; rows of NaN give token 0 and rows whose logits are all -inf theirs;
+    +inf wins; NaN logits beside numbers are passed over.  Hidden states and
+    embedding are columns of wider tensors."""
+    print(f"[case] greedy_sample ties, nan, inf {dtype} R={R}", flush=True)
+    V, Hd = 1500, 256
+    g = torch.Generator().manual_seed(R)
+    wide_e, wide_h = torch.full((V, Hd + 24), 7.0).to(dtype), torch.full((R, Hd + 8), 7.0).to(dtype)
+    emb, hid = wide_e[:, 8:8 + Hd], wide_h[:, :Hd]
+    emb.copy_(torch.randn((V, Hd), generator=g) * 0.01)
+    emb[:, :8] = 0
+    hid.copy_(torch.randn((R, Hd), generator=g))
+    hid[:, :8] = 0
+    # column c < 4 is read by the rows r with r % 6 == c alone: its winners, of equal logits
+    winners = [[70, 6, 134], [127, 128, 1499], [900, 1300], [1499]]
+    want = []
+    for c, ids in enumerate(winners):
+        emb[ids, c] = 30.0
+    for r in range(R):
+        c = r % 6
+        if c < 4:
+            hid[r, c] = 2.0
+            hid[r, 8:] = 0                                     # every other logit is 0
+            want.append(min(winners[c]))
+        elif c == 4:
+            hid[r, 9] = float("nan")                           # every logit NaN
+            want.append(0)
+        else:
+            hid[r] = 0                                         # two ids of +inf (elsewhere: NaN), the others 0
+            hid[r, 5] = 1.0
+            want.append(733)
+    emb[733, 5] = float("inf")
+    emb[734, 5] = float("inf")
+    out = ops.greedy_sample(wide_e.to(DEV)[:, 8:8 + Hd], wide_h.to(DEV)[:, :Hd], V, R)
+    assert out.cpu().tolist() == want
+    # all logits -inf: the first id; any number beats them
+    low = torch.zeros((V, Hd), dtype=dtype)
+    low[:, 3] = float("-inf")
+    one = torch.zeros((R, Hd), dtype=dtype)
+    one[:, 3] = 1.0
+    assert ops.greedy_sample(low.to(DEV), one.to(DEV), V, R).cpu().tolist() == [0] * R
+    low[1234, 3] = -60000.0 if dtype == torch.float16 else -3e38
+    assert ops.greedy_sample(low.to(DEV), one.to(DEV), V, R).cpu().tolist() == [1234] * R
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("V,Hd", [(1000, 256), (5003, 768), (24448, 1024), (24577, 512)])
 def test_greedy_sample_does_not_depend_on_the_batch(dtype, V, Hd):
     """A row's token is the same whatever batch it is sampled in: the kernels for

@@ -44,12 +44,13 @@ union SmFrag {
 
 constexpr int kSmTile = 256;              // the hidden size must be a multiple of this
 constexpr int kSmMaxRowsPerPass = 256;
-// Up to 32 sampled rows the narrow kernel, beyond them the wide one (32000 rows of
-// 4096, us, narrow / wide: 8 rows 46.8 / 48.0, 32 rows 46.0 / 48.6, 33 rows
-// 52.3 / 48.7, 64 rows 53.5 / 48.7; with 128 and 256 rows 107 / 58 and 214 / 82,
-// the narrow one passing over the matrix once per 64 rows).  Small vocabularies
-// too, though the wide kernel keeps its 128 rows per workgroup there: 16000 rows,
-// 33 rows 46.6 / 35.1, 64 rows 48.0 / 38.5; 4000 rows 37.0 / 30.9 and 38.3 / 33.8.
+// Up to 32 sampled rows the narrow kernel, beyond them the wide one.  32000 rows of
+// 4096, us: the narrow one with 32 rows 43.5, the wide one with 33 to 64 rows 46.5
+// (the narrow one with four row blocks per wave took 52.3 to 53.5 there, and 107 and
+// 214 with 128 and 256 rows, passing over the matrix once per 64; the wide one 56
+// and 82).  Small vocabularies too, though the wide kernel keeps its 128 rows per
+// workgroup there: 16000 rows, 33 sampled 46.6 / 34.9, 64 48.0 / 38.1; 4000 rows
+// 37.0 / 30.8 and 38.3 / 33.8.
 constexpr int kSmNarrowRows = 32;
 #ifndef MUX_SM_PREFETCH_TILES
 #define MUX_SM_PREFETCH_TILES 2
@@ -63,6 +64,7 @@ struct LmHeadParams {
   int64_t weight_stride;
   int32_t hidden_size, vocab, num_rows;
   int32_t hidden_rows;                    // rows of `hidden`: row_index entries are clamped to it
+  int32_t half_tiles;                     // the wide kernel: a large vocabulary, which the narrow one gives 8 waves
   uint32_t *counter;                      // workgroups arrived, zero between launches
   unsigned long long *table;              // [workgroups][16 NB] keys, written before they are read
   int64_t *next_tokens;
@@ -166,17 +168,27 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, g = lane >> 4;
   const int n_tiles = P.hidden_size / KT;
-  // Workgroups start their walk over the hidden dimension at different tiles
-  // (a dot product does not care about the order): with a row pitch that is a
-  // power of two - 8 KiB at hidden size 4096 - workgroups walking in step would
-  // all be reading the same few memory channels at any moment.  The tile depends on the
-  // vocabulary row alone (128 rows start together, in both kernels and at both
-  // workgroup sizes), so that a logit, rounding included, is the same whatever
-  // batch its row is sampled in.
-  const int t_start = blockIdx.x / (8 / NW) % n_tiles;
-  auto tile_of = [&](int t) {
-    const int x = t + t_start;
-    return x >= n_tiles ? x - n_tiles : x;
+  // Workgroups start their walk over the hidden dimension at different tiles (a dot
+  // product does not care about the order): with a row pitch that is a power of two
+  // - 8 KiB at hidden size 4096 - workgroups walking in step would all be reading
+  // the same few memory channels at any moment.  Large vocabularies (8 waves) start
+  // at half tiles too, which spreads such a pitch better; one tile then consists of
+  // the end and of the beginning of the hidden dimension, and a lane's column offset
+  // is that of its half of the tile.  (32000 x 4096, one row 47.0 -> 43.0 us, 32 rows
+  // 46.7 -> 43.5; small vocabularies wait for latencies and lose, 4000 x 5120 29.1 ->
+  // 30.8.)
+  // The start depends on the vocabulary and the vocabulary row alone (128 rows start
+  // together, in both kernels and at both workgroup sizes), so that a logit, rounding
+  // included, is the same whatever batch its row is sampled in.
+  constexpr bool kHalfTiles = NW == 8;
+  const int start = (kHalfTiles ? blockIdx.x % (2 * n_tiles) : 2 * (blockIdx.x / 2 % n_tiles)) * (KT / 2);
+  const bool upper = r16 & 8;              // (of the chunks whose position in the row is r16)
+  auto offset_of = [&](int t, bool upper_half) {
+    int x = start + t * KT;
+    if (x >= P.hidden_size) x -= P.hidden_size;
+    if constexpr (!kHalfTiles) return x;
+    const int wrapped = x + KT > P.hidden_size ? x - P.hidden_size : x;
+    return upper_half ? wrapped : x;
   };
 
   // Embedding rows of this wave (rows past the vocabulary re-read its last row
@@ -207,7 +219,7 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
   auto stage_load = [&](sm_u32x4 (&st)[SJ], int t) {
 #pragma unroll
     for (int j = 0; j < SJ; ++j)
-      st[j] = hvalid[j] ? *reinterpret_cast<const sm_u32x4 *>(hsrc[j] + tile_of(t) * KT) : sm_u32x4{0, 0, 0, 0};
+      st[j] = hvalid[j] ? *reinterpret_cast<const sm_u32x4 *>(hsrc[j] + offset_of(t, upper)) : sm_u32x4{0, 0, 0, 0};
   };
   auto stage_store = [&](const sm_u32x4 (&st)[SJ], int buf) {
 #pragma unroll
@@ -215,9 +227,9 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
       if (hstore[j]) *reinterpret_cast<sm_u32x4 *>(&htile[buf][hoff + RPP * j * kHRow]) = st[j];
   };
   auto load_w = [&](sm_u32x4 (&w)[4], int t) {
-    const int off = tile_of(t) * KT;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) w[j] = __builtin_nontemporal_load(reinterpret_cast<const sm_u32x4 *>(wsrc[j] + off));
+    for (int j = 0; j < 4; ++j)            // (row 4 j + g holds chunk r16 ^ row there)
+      w[j] = __builtin_nontemporal_load(reinterpret_cast<const sm_u32x4 *>(wsrc[j] + offset_of(t, upper != (j >= 2))));
   };
 
   sm_v4f32 acc[NB];
@@ -352,11 +364,8 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
   const int wm = wave >> 2, wn = wave & 3;
   const int r16 = lane & 15, g = lane >> 4;
   const int n_tiles = P.hidden_size / KT;
-  // The same element as in the kernel above.  (Starts at odd tiles as well would
-  // spread a power-of-two pitch better - 32000 x 4096, 33 - 64 rows 46.6 us against
-  // 48.7, 256 rows 80.8 against 81.6 - but a near tie could then go another way in
-  // a batch of 33 rows than in one of 32.)
-  const int t_start = 2 * (blockIdx.x % (n_tiles / 2));
+  // The same element as in the kernel above.
+  const int t_start = P.half_tiles ? blockIdx.x % n_tiles : 2 * (blockIdx.x % (n_tiles / 2));
   const int vrow0 = blockIdx.x * VR;
 
   // Staging: thread -> row tid / 8 (+ 64 j), chunk tid % 8.  Every load is
@@ -590,6 +599,7 @@ extern "C" int32_t mux_greedy_sample(int64_t *next_tokens, const void *hidden_st
     P.hidden_size = hidden_size;
     P.vocab = vocab_size;
     P.num_rows = rows;
+    P.half_tiles = wide;
     P.hidden_rows = row_index ? num_hidden_rows : num_hidden_rows - r0;
     P.counter = static_cast<uint32_t *>(workspace);
     P.table = reinterpret_cast<unsigned long long *>(static_cast<char *>(workspace) + kSmCounterBytes);

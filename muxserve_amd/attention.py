@@ -232,12 +232,13 @@ class PagedAttentionWithRoPE(PagedAttention):
             if n_valid > 0:
                 T.rotary_neox(positions, query, key, self._cache(query.device), num_tokens=n_valid)
             return super().forward(query, key, value, key_cache, value_cache, md, cache_event)
-        # Rotation and cache write in one launch for small steps (decode: saves a
-        # launch, 12.6 against 20.4 us per layer), when the whole head rotates and
-        # the rows allow 16-byte accesses (q, k, v of one qkv row always do).  Larger
-        # steps that hold generation tokens too keep the two kernels: the fused one
-        # re-reads the cos/sin row of a token once per kv head and is slower there
-        # (101 against 93 us for 4096 tokens x 52 heads).
+        # Rotation and cache write in one launch for small steps, when the whole head
+        # rotates and the rows allow 16-byte accesses (q, k, v of one qkv row always
+        # do): decode of 56 tokens x 32 heads 4.9 against 10.8 us in two launches, 512
+        # x 32 39.9 against 46.8.  Larger steps that hold generation tokens take the
+        # two launches, which are at most 3 % faster (2000 prompt tokens, 64 on 8 heads,
+        # 26.5 against 27.2 us) and mostly slower (1024 decode tokens x 32 heads 86.2
+        # against 82.1, 4096 prompt tokens x 52 heads 86.1 against 76.2).
         cos_sin, layer = self._cache(query.device), self._layer(md)
         small = n_valid <= self.fused_rope_max_tokens
         out = None
@@ -254,9 +255,10 @@ class PagedAttentionWithRoPE(PagedAttention):
             step = prompt_step_pays(md.num_prompts, n_valid, self.num_heads, self.num_kv_heads)
             # (Large steps of short prompts: rotation and cache write in one launch
             # are 2 - 13 % faster than in two, but with several query heads per kv
-            # head up to 9 % slower: 40 prompts of 13 tokens, 64 on 8 heads, 33.5
-            # against 30.7 us.)
-            if step or small or self.num_heads == self.num_kv_heads:
+            # head up to 9 % slower where they are many: 40 prompts of 13 tokens, 64
+            # on 8 heads, 33.5 against 30.7 us; 16 of 45, 16 on 2 heads, 12.6 against
+            # 15.4.)
+            if step or small or self.num_heads == self.num_kv_heads or n_valid * self.num_kv_heads <= 2560:
                 if cache_event is not None:
                     cache_event.wait()
                 out = T.prompt_layer(positions, query, key, value, cos_sin, key_cache, value_cache, md.slot_mapping,

@@ -34,6 +34,7 @@ def _prompt_route(monkeypatch, lens, heads, kv_heads):
 
 @pytest.mark.parametrize("lens,heads,kv_heads,route", [
     ([6] * 100, 32, 32, "one launch"), ([6] * 100, 64, 8, "two launches"), ([13] * 40, 64, 8, "two launches"),
+    ([45] * 16, 16, 2, "one launch"),
     ([16] * 64, 52, 52, "one launch"), ([20] * 16, 52, 52, "one launch"), ([45] * 128, 32, 8, "two launches"),
     ([100] * 2, 64, 8, "one launch"), ([45], 32, 32, "one launch"), ([400], 32, 32, "one launch"),
     ([30] * 16, 32, 32, "step"), ([45] * 16, 32, 32, "step"), ([100] * 4, 64, 8, "step"), ([128] * 128, 32, 8, "step"),

@@ -31,10 +31,12 @@
 // are loaded into (one workgroup reads each of them once; a lane holds both
 // halves of a pair), and a workgroup scatters the 128 rows of K and V that its
 // last four tiles bring into LDS anyway, so k and v are not read again and the
-// stores go out under the matrix work.  Measured, whole step: 16 x 2048 tokens
-// f16 1031 -> 845 us (the kernel 740 us of it: attention alone 620, pool stores
-// 75, rotation of q 35), three bf16 prompts of 700 - 4000 tokens on 64 / 8 heads
-// 528 -> 506 us.
+// stores go out under the matrix work.  Measured, whole step, both sides in turn
+// on one machine: 16 x 2048 tokens f16 1052 -> 863 us (rotation of k 100, attention
+// by itself 620, pool stores 75, rotation of q 35), three bf16 prompts of 700 - 4000
+// tokens on 64 / 8 heads 548 -> 517 us.  Prompts of a few tokens lose in this form:
+// 128 of 6 tokens, 32 heads, 47 us against 33 with rotation and cache write in a
+// launch of their own.
 #include "cache_write.h"
 
 #include <algorithm>

@@ -10,8 +10,9 @@
 // plain coalesced integer copies; the kinds do not wait for each other, because
 // ids that this step appends are read from the reply rather than from the mirror.
 // (As three kernels and two conversions a decode step of 32 sequences spent 20 us
-// of the GPU and five launches on them; the 17 steps of a batch of 32 requests,
-// host work included, 2145 -> 1893 us.)
+// of the GPU and five launches on them, now 11.3 and one.  The 17 steps of a batch
+// of 32 requests are mostly host work: 2070 - 2110 -> 1860 - 1900 us in four runs of
+// both in turn on one machine; two runs of one side have differed by 13 % on another.)
 //   append   the reply's new ids are copied behind each request's run
 //   slots    slot_mapping[t][l][h] = id * block_size + offset, read from the
 //            mirror: prompt token k -> block k / bs, offset k % bs; decode token ->

@@ -318,6 +318,43 @@ def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many)
         assert torch.equal(a, b), f"{what} differ between the step operator and the three kernels"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rotary_table_at_any_float_offset(dtype):
+    """The cos|sin table is taken at any 4-byte boundary, as the rotary kernel takes
+    it, by the small-step cache write and by the prompt step: rows, pools and
+    outputs bitwise those of an aligned table."""
+    print(f"[case] rotary table offset {dtype}", flush=True)
+    from muxserve_amd import torch_ops, workloads
+    from muxserve_amd.attention import build_cos_sin_cache
+    rng = np.random.Generator(np.random.PCG64(3))
+    Hq, Hkv, bs, lens = 4, 2, 16, [5, 150, 33]
+    T = sum(lens)
+    N = sum((n + bs - 1) // bs for n in lens) * Hkv
+    slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), Hkv, bs, rng.permutation(N))
+    dslots, positions = torch.from_numpy(slots).to(DEV), torch.from_numpy(rng.integers(0, 2048, size=T)).to(DEV)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
+    table = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    qkv = torch.randn((T, (Hq + 2 * Hkv) * D), device=DEV).to(dtype)
+    results = []
+    for offset in (0, 1):
+        cos_sin = torch.zeros(table.numel() + 4, device=DEV)[offset:offset + table.numel()].view_as(table).copy_(table)
+        got = []
+        for step in (False, True):
+            x = qkv.clone()
+            q, k, v = x.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+            kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=dtype)
+            kp.zero_()
+            vp.zero_()
+            out = torch.zeros((T, Hq * D), dtype=dtype, device=DEV)
+            if step:
+                torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, dslots, 0, cu, lens, D ** -0.5)
+            else:
+                ops.rope_reshape_and_cache(positions, q, k, v, cos_sin, kp, vp, dslots)
+            got += [t.view(torch.int16) for t in (x, kp, vp, out)]
+        results.append(got)
+    assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
 @pytest.mark.parametrize("rope", [True, False])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_multi_model_cache_write_equals_one_launch_per_model(rope, dtype):

@@ -257,7 +257,8 @@ class PagedAttentionWithRoPE(PagedAttention):
             # are 2 - 13 % faster than in two, but with several query heads per kv
             # head up to 9 % slower where they are many: 40 prompts of 13 tokens, 64
             # on 8 heads, 33.5 against 30.7 us; 16 of 45, 16 on 2 heads, 12.6 against
-            # 15.4.)
+            # 15.4.  Up to 2560 (token, kv head) pairs the one launch is the kernel for
+            # small steps.)
             if step or small or self.num_heads == self.num_kv_heads or n_valid * self.num_kv_heads <= 2560:
                 if cache_event is not None:
                     cache_event.wait()

@@ -22,6 +22,16 @@
 // read from LDS anyway.
 // The next tile's global loads are issued before the current tile's math.
 //
+// What bounds it: power.  With every CU busy the clock settles at 1.6 GHz; on half
+// of the CUs 16 x 2048 tokens take 0.67 of the whole chip's CU time, on a quarter
+// 0.63.  So what counts is work per score, in any unit: no maximum where the sum
+// tells as much (attention of that shape 604 -> 588 us), fragment addresses that
+// are registers or immediates (the tile loop is unrolled over its two buffers),
+// waits for exactly the loads that are needed, two stores and no address
+// arithmetic per 16 tokens for the pool (the step form 813 -> 793 us).  Fragments of
+// V^T requested before the softmax, a third tile buffer, two chains of sums: no
+// difference.
+//
 // The step form (STEP = true, mux_rope_prefill_and_cache) is a whole prompt step
 // of the attention layer behind the rotation of k: it also rotates q and writes
 // k and v to the pool.  As kernels of their own these passes are bound by
@@ -32,14 +42,15 @@
 // halves of a pair), and a workgroup scatters the 128 rows of K and V that its
 // last four tiles bring into LDS anyway, so k and v are not read again and the
 // stores go out under the matrix work.  Measured, whole step, both sides in turn
-// on one machine: 16 x 2048 tokens f16 1052 -> 863 us (rotation of k 100, attention
-// by itself 620, pool stores 75, rotation of q 35), three bf16 prompts of 700 - 4000
-// tokens on 64 / 8 heads 548 -> 517 us.  Prompts of a few tokens lose in this form:
+// on one machine: 16 x 2048 tokens f16 1052 -> 800 us (rotation of k 100, attention
+// by itself 600, pool stores 55, rotation of q 45), three bf16 prompts of 700 - 4000
+// tokens on 64 / 8 heads 548 -> 490 us.  Prompts of a few tokens lose in this form:
 // 128 of 6 tokens, 32 heads, 47 us against 33 with rotation and cache write in a
 // launch of their own.
 #include "cache_write.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace mux {
@@ -51,8 +62,7 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBM = 128;                 // query rows per workgroup
-constexpr int kBN = 32;                  // keys per tile
-constexpr int kNKB = kBN / 32;           // 32-key blocks (one MFMA row block) per tile
+constexpr int kBN = 32;                  // keys per tile (one MFMA row block)
 
 // Query tiles listed in the kernel argument (its size limit is 4 KiB).
 constexpr int kMaxPairs = 768;
@@ -157,21 +167,21 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 #define MUX_PF_PRIO_VALU 0
 constexpr int kTileElems = kBN * kHeadSize;          // one unpadded row-major tile
 // The swizzle: the 16-byte chunk c of tile row r sits at chunk position
-// c ^ swz(r), swz(r) = the low three bits of r rotated left by one, bit 3 kept.
-// LDS has 32 banks of 4 bytes: a 256-byte row covers them twice, so only the low
-// three bits of a chunk position choose the banks.  The K fragments are read 8
-// rows at a time (one chunk each, ds_read_b128): the rotated low bits of 8
-// consecutive rows are all different.  The V^T fragments are read 16 lanes at a
-// time (ds_read_b64_tr_b16) over 4 consecutive rows x 2 neighbouring chunks x
-// the two halves of a chunk: the rows' two low bits land in position bits 1-2
-// and the chunk pair in bit 0 - again all different.  (With the plain c ^ r the
-// four rows and the chunk pair shared two position bits: a two-way conflict on
-// every V^T read.)
-__device__ __forceinline__ int swz(int row) { return ((row & 3) << 1) | ((row >> 2) & 1) | (row & 8); }
+// c ^ swz(r), swz(r) = the low three bits of r rotated left by one.  LDS has 32
+// banks of 4 bytes: a 256-byte row covers them twice, so only the low three bits
+// of a chunk position choose the banks, and bit 3 of a chunk is left alone, an
+// immediate offset of the reads.  The K fragments are read 8 rows at a time (one
+// chunk each, ds_read_b128): the rotated bits of 8 consecutive rows are all
+// different.  The V^T fragments are read 16 lanes at a time (ds_read_b64_tr_b16)
+// over 4 consecutive rows x 2 neighbouring chunks x the two halves of a chunk: the
+// rows' two low bits land in position bits 1-2 and the chunk pair in bit 0 - again
+// all different.  (With the plain c ^ r the four rows and the chunk pair shared two
+// position bits: a two-way conflict on every V^T read.)
+__device__ __forceinline__ int swz(int row) { return ((row & 3) << 1) | ((row >> 2) & 1); }
 
 // 16 tokens (rows row0 .. row0 + 15 of the K and V tile in LDS) to the pool, by
-// the four waves of a workgroup together.  slot: lane's token row0 + lane % 16,
-// -1 for none.  K: a thread stores one token's chunk, the 16 tokens of a chunk
+// the four waves of a workgroup together.  slot_at: LDS address of row0's slot, -1
+// for none.  K: a thread stores one token's chunk, the 16 tokens of a chunk
 // side by side, so a wave fills 1 KiB of a 16-token block.  V: the transposing
 // read hands a lane 8 consecutive tokens of one dim, which is a chunk of the pool
 // where those tokens are a run (consecutive slots from a multiple of 8: every
@@ -181,7 +191,7 @@ __device__ __forceinline__ int swz(int row) { return ((row & 3) << 1) | ((row >>
 // tile's among them.
 // True if exactly two vector-memory instructions were issued (both 8-token
 // halves are runs): the caller's wait for older loads can then leave them.
-__device__ __forceinline__ bool write_tokens_to_pool(const uint16_t *Kt, const uint16_t *Vr, int row0, int64_t slot,
+__device__ __forceinline__ bool write_tokens_to_pool(const uint16_t *Kt, const uint16_t *Vr, int row0, uint32_t slot_at,
                                                      int wave, int lane, const PrefillStep &S) {
   constexpr int D = kHeadSize;
   // (kept from the tile loop's registers: the compiler would hoist the addresses
@@ -201,9 +211,11 @@ __device__ __forceinline__ bool write_tokens_to_pool(const uint16_t *Kt, const u
   const uint32_t va1 = (uint32_t)(uintptr_t)(lds_u16 *)(Vr + r1 * D + 8 * (c ^ swz(r1)) + 4 * (m & 1));
   u32x4 kx;
   u32x2 v0, v1;
-  asm volatile("ds_read_b128 %0, %3\n\tds_read_b64_tr_b16 %1, %4\n\tds_read_b64_tr_b16 %2, %5\n\ts_waitcnt lgkmcnt(0)"
-               : "=&v"(kx), "=&v"(v0), "=&v"(v1)
-               : "v"(ka), "v"(va0), "v"(va1)
+  int64_t slot;
+  asm volatile("ds_read_b64 %3, %7\n\tds_read_b128 %0, %4\n\tds_read_b64_tr_b16 %1, %5\n\t"
+               "ds_read_b64_tr_b16 %2, %6\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(kx), "=&v"(v0), "=&v"(v1), "=&v"(slot)
+               : "v"(ka), "v"(va0), "v"(va1), "v"(slot_at + 8u * i)
                : "memory");
   // Runs: the previous lane's slot plus one, from a multiple of 8.
   const uint32_t slot_lo = static_cast<uint32_t>(slot), slot_hi = static_cast<uint32_t>(slot >> 32);
@@ -246,6 +258,45 @@ __device__ __forceinline__ bool write_tokens_to_pool(const uint16_t *Kt, const u
     }
   }
   return false;
+}
+
+// What a lane keeps for writing 16 tokens that fill (part of) one pool block in
+// order, chunk c = 4 wave + lane / 16: LDS offsets of its K chunk and of its two V
+// reads (see write_tokens_to_pool) in a tile, and its places in a K and V block.
+struct BlockWriter {
+  uint32_t k_lds, v_lds0, v_lds1, k_off, v_off;
+  __device__ __forceinline__ BlockWriter(int wave, int lane, int bs) {
+    constexpr int D = kHeadSize;
+    const int i = lane & 15, c = 4 * wave + (lane >> 4), j = i >> 2, m = i & 3;
+    const int r0 = 8 * (m >> 1) + j, r1 = r0 + 4;
+    k_lds = 2 * (i * D + 8 * (c ^ swz(i)));
+    v_lds0 = 2 * (r0 * D + 8 * (c ^ swz(r0)) + 4 * (m & 1));
+    v_lds1 = 2 * (r1 * D + 8 * (c ^ swz(r1)) + 4 * (m & 1));
+    k_off = 16 * (c * bs + i);
+    v_off = 2 * ((8 * c + (lane & 7)) * bs + 8 * (i >> 3));
+  }
+};
+
+// Rows row0 .. row0 + 15 of the tile (K at kt, V at vt, LDS addresses) to the 16
+// slots from `base`, a multiple of 16, of one block: two stores.
+__device__ __forceinline__ void write_block_to_pool(uint32_t kt, uint32_t vt, const BlockWriter &w, int64_t base,
+                                                    const PrefillStep &S) {
+  constexpr int D = kHeadSize;
+  u32x4 kx;
+  u32x2 v0, v1;
+  asm volatile("ds_read_b128 %0, %3\n\tds_read_b64_tr_b16 %1, %4\n\tds_read_b64_tr_b16 %2, %5\n\ts_waitcnt lgkmcnt(0)"
+               : "=&v"(kx), "=&v"(v0), "=&v"(v1)
+               : "v"(kt + w.k_lds), "v"(vt + w.v_lds0), "v"(vt + w.v_lds1)
+               : "memory");
+  const u32x4 vx = {v0.x, v0.y, v1.x, v1.y};
+  const int bs_shift = __builtin_ctz(static_cast<unsigned>(S.block_size));
+  const int64_t first = (base >> bs_shift) * (D << bs_shift);           // the block's first element
+  const int64_t in_block = base & (S.block_size - 1);
+  const uint16_t *const kp = S.k_pool + first + 8 * in_block, *const vp = S.v_pool + first + in_block;
+  // (as in write_tokens_to_pool: whole lines stream past the L2)
+  asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.k_off), "v"(kx), "s"(kp) : "memory");
+  if (S.block_size == 16) asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
+  else asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
 }
 
 template <typename T, bool STEP>
@@ -338,14 +389,9 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[mb][i] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-  // Kept beside m_run and changed with it, so that a tile whose reference stays
-  // spends one comparison on it: the score beyond which the reference moves (see
-  // the softmax), and the reference as an exponent.  (Formed in every tile they
-  // were a tenth of its vector instructions: attention of 16 x 2048 tokens f16
-  // 634 -> 619 us, three bf16 prompts of 700 - 4000 tokens 477 -> 469 us.)
-  constexpr float kRescaleStep = 8.f;
-  const float rescale_score = kRescaleStep / I.scale_log2;
-  float m_limit = -INFINITY, neg_m = 0.f;
+  // The reference as an exponent, kept beside m_run and changed with it; infinite
+  // until the wave's first tile has set it.
+  float neg_m = INFINITY;
 
   // Keys needed by this workgroup: positions 0 .. min(len, q0 + 128) - 1.
   const int kv_end = min(len, q0 + kBM);
@@ -369,32 +415,60 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
   const int chunk0 = (lane & 15) ^ swz(row0);
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) koff[i] = static_cast<uint32_t>(row0 + 16 * i) * row_bytes + 16u * chunk0;
-  const uint32_t kmax = last_row + 16u * chunk0;
-  auto dma_tile = [&](int buf) {           // the next tile in sequence into buffer buf
-    typedef __attribute__((address_space(3))) void lds_void;
-    typedef const __attribute__((address_space(1))) void global_void;
+  typedef const __attribute__((address_space(3))) uint16_t lds_u16;
+  const uint32_t smem_at = (uint32_t)(uintptr_t)(lds_u16 *)smem;
+  // The loads are written out (they have no destination registers), with the waits
+  // for them in the loop: after a load to LDS of its own the compiler takes every
+  // LDS access to be out of order, so that it waits for all fragments before the
+  // first MFMA and for the next tile's loads before the V^T fragments (the step of
+  // 16 x 2048 tokens 4 %, three bf16 prompts 3 % slower).
+  auto dma_tile = [&](int t, int buf) {    // tile t into buffer buf
+    const char *const kt = kbase + static_cast<uint64_t>(t) * tile_bytes, *const vt = vbase + static_cast<uint64_t>(t) * tile_bytes;
+    const bool whole = (t + 1) * kBN <= len;
+    const uint32_t omax = last_row - static_cast<uint32_t>(t) * tile_bytes + 16u * chunk0;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-      const uint32_t o = min(koff[i], kmax);
-      uint16_t *kd = smem + buf * kTileElems + (4 * i + wave) * 512;
-      uint16_t *vd = smem + (2 + buf) * kTileElems + (4 * i + wave) * 512;
-      // (address-space casts need the C form)
-      __builtin_amdgcn_global_load_lds((global_void *)(kbase + o), (lds_void *)kd, 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((global_void *)(vbase + o), (lds_void *)vd, 16, 0, 0);
-      koff[i] += tile_bytes;
+      const uint32_t o = whole ? koff[i] : min(koff[i], omax);
+      const uint32_t kd = smem_at + 2 * (buf * kTileElems + (4 * i + wave) * 512);
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd), "v"(o), "s"(kt) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd + 4 * kTileElems), "v"(o), "s"(vt)
+                   : "memory", "m0");
     }
   };
 
   // Lane-dependent part of the V^T fragment addresses (see read_v), in elements.
-  int v_lane_base[2];
+  int v_lane_base[2], k_lane_base[4];
   {
     const int jrow = (lane & 15) >> 2, m = lane & 3;
     const int rl = 4 * half + jrow, cl = 2 * ((lane >> 4) & 1) + (m >> 1);
     // rl < 8, cl < 4: the lane's part of the position is cl ^ swz(rl), below 8.
     v_lane_base[0] = rl * D + 8 * (cl ^ swz(rl)) + 4 * (m & 1);
     v_lane_base[1] = rl * D + 8 * (cl ^ swz(rl) ^ 4) + 4 * (m & 1);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) k_lane_base[f] = qcol * D + 8 * ((2 * f + half) ^ swz(qcol));
   }
-  dma_tile(0);
+  dma_tile(0, 0);
+  // The slots of the workgroup's own rows, -1 for none, in LDS behind the tile
+  // buffers (where only the epilogue's staging reaches): a load of them in the tile
+  // loop would be waited for behind the previous tile's pool stores.
+  // Behind them, for every 16 rows, the first one's slot where they are 16 slots in
+  // order from a multiple of 16 inside one block (every prompt behind a block table
+  // of 16 or more tokens, up to its last few), else -1.
+  int64_t *const own_slots = reinterpret_cast<int64_t *>(smem + 4 * kTileElems);
+  static_assert(8 * kTileElems + 8 * (kBM + kBM / 16) <= 2 * kSmemElems, "the slots fit behind the tile buffers");
+  const BlockWriter writer(wave, lane, STEP ? S.block_size : 0);
+  if constexpr (STEP) {
+    if (writes_pool && tid < kBM) {
+      int64_t slot = -1;
+      if (q0 + tid < len) slot = S.slots[static_cast<int64_t>(seq_begin + q0 + tid) * S.slot_stride + hk];
+      if (slot >= S.pool_slots) slot = -1;
+      own_slots[tid] = slot;
+      const int64_t first = __shfl(slot, lane & 48);
+      const uint64_t in_order = __builtin_amdgcn_ballot_w64(first >= 0 && (first & 15) == 0 && slot == first + (lane & 15) &&
+                                                            S.block_size >= 16);
+      if ((lane & 15) == 0) own_slots[kBM + tid / 16] = ((in_order >> (lane & 48)) & 0xffff) == 0xffff ? first : -1;
+    }
+  }
   if constexpr (STEP) {
     // Rotation of the wave's 32 query rows: a lane takes the chunks c and c + 8
     // (the two halves of the same pairs) of one row, 8 rows at a time, so that
@@ -454,11 +528,10 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const int r = qcol & 15;
         const bool take = (qcol >> 4) == pass && my_q < len;
+        if (take) {
 #pragma unroll
-        for (int f = 0; f < 8; ++f) {
-          const u32x4 x = *reinterpret_cast<const u32x4 *>(stage + r * D + 8 * ((2 * f + half) ^ swz(r)));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) qf[f].u[e] = take ? x[e] : qf[f].u[e];
+          for (int f = 0; f < 8; ++f)
+            qf[f].u = *reinterpret_cast<const u32x4 *>(stage + r * D + 8 * ((2 * f + half) ^ swz(r)));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -467,55 +540,44 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
     }
   }
   bool stores_counted = false;             // the previous tile's pool stores: exactly four, behind this tile's loads
-  for (int t = 0; t < n_tiles; ++t) {
+  // (the compiler's own loads are behind it: a wait for them would be one for the tiles)
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  auto tile = [&](int t, auto buffer) {
+    constexpr int cur = decltype(buffer)::value;
     const int k0 = t * kBN;
-    const int cur = t & 1;
     // This wave's part of tile t has landed; after the barrier all of it has,
-    // and everybody is done with the other buffer.
-    if constexpr (STEP) {
-      // (the barrier by itself: __syncthreads() would wait for the stores as well)
-      if (stores_counted) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-    }
+    // and everybody is done with the other buffer.  (The barrier by itself:
+    // __syncthreads() would wait for the pool stores as well.)
+    if (STEP && stores_counted) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
 #ifdef MUX_TRACE
     if (t == 0) tr_first = __builtin_amdgcn_s_memrealtime();
 #endif
     // A workgroup's own rows are its last four tiles: their K and V go to the pool
-    // behind the tile's math (the slots' loads hide behind it).
+    // behind the tile's math.
     const bool to_pool = STEP && writes_pool && k0 >= q0;
-    int64_t slot = -1;                     // of row lane % 32 of the tile
-    if constexpr (STEP) {
-      if (to_pool && k0 + qcol < len) slot = S.slots[static_cast<int64_t>(seq_begin + k0 + qcol) * S.slot_stride + hk];
-    }
-    if (t + 1 < n_tiles) dma_tile(cur ^ 1);
+    if (t + 1 < n_tiles) dma_tile(t + 1, cur ^ 1);
+    const uint16_t *const Kt = smem + cur * kTileElems;           // this tile's K
+    const uint16_t *const Vr = smem + (2 + cur) * kTileElems;     // this tile's V (row-major)
     // (nothing to compute where every key of the tile is in this wave's future, or
     // all of the wave's rows are past the prompt's end)
     if (k0 <= wq0 + 31 && wq0 < len) {
-      const uint16_t *const Kt = smem + cur * kTileElems;           // this tile's K
-      const uint16_t *const Vr = smem + (2 + cur) * kTileElems;     // this tile's V (row-major)
-
-      // ---- S^T = K . Q^T : kNKB 32-key blocks -----------------------------------------
+      // ---- S^T = K . Q^T ------------------------------------------------------------------
       // LDS fragment reads run kDepth steps ahead of the MFMAs that consume them.
       // In the P.V product consecutive MFMAs go to different accumulators (4 dim
-      // blocks); a single dependent chain, as here with one key block, runs at 3/4
+      // blocks); a single dependent chain, as here, runs at 3/4
       // of the rate.
       constexpr int kDepth = 4;
-      v16f32 sacc[kNKB];
+      v16f32 sacc;
 #pragma unroll
-      for (int kb = 0; kb < kNKB; ++kb)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[kb][i] = 0.f;
+      for (int i = 0; i < 16; ++i) sacc[i] = 0.f;
       {
-        // Fragment j: key block j % kNKB, dims 16 (j / kNKB) + 8 half .. +7 of key row qcol.
+        // Fragment j: dims 16 j + 8 half .. +7 of key row qcol.
         auto read_k = [&](int j) {
           Frag f;
-          const int row = 32 * (j % kNKB) + qcol, chunk = 2 * (j / kNKB) + half;
-          f.u = *reinterpret_cast<const u32x4 *>(Kt + row * D + 8 * (chunk ^ swz(row)));
+          f.u = *reinterpret_cast<const u32x4 *>(Kt + k_lane_base[j & 3] + 64 * (j >> 2));
           return f;
         };
         Frag ring[kDepth];
@@ -524,41 +586,50 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
         __builtin_amdgcn_sched_barrier(0);   // keep the scheduler from sinking the reads to their uses
         MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
 #pragma unroll
-        for (int j = 0; j < 8 * kNKB; ++j) {
-          sacc[j % kNKB] = mfma<T>(ring[j % kDepth], qf[j / kNKB], sacc[j % kNKB]);
-          if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_k(j + kDepth);
+        for (int j = 0; j < 8; ++j) {
+          sacc = mfma<T>(ring[j % kDepth], qf[j], sacc);
+          if (j + kDepth < 8) ring[j % kDepth] = read_k(j + kDepth);
           __builtin_amdgcn_sched_barrier(0);
         }
         MUX_PF_PRIO(MUX_PF_PRIO_VALU);
       }
 
       // ---- softmax over keys, per query column --------------------------------------
-      // register i of block kb is key k0 + 32 kb + 8 (i/4) + 4 half + i%4.
+      // register i is key k0 + 8 (i/4) + 4 half + i%4.
       // Raw scores stay unscaled; scale (> 0) is folded into the exponent:
       // p = exp2(s * scale_log2 - m * scale_log2).
       // Exactly one tile per wave straddles the diagonal; only it pays for the mask.
       if (k0 + kBN - 1 > wq0) {
         const int rel = my_q - k0 - 4 * half;   // key offset inside the tile, less this lane's share
 #pragma unroll
-        for (int kb = 0; kb < kNKB; ++kb)
-#pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if (32 * kb + 8 * (i / 4) + (i % 4) > rel) sacc[kb][i] = -INFINITY;
+        for (int i = 0; i < 16; ++i)
+          if (8 * (i / 4) + (i % 4) > rel) sacc[i] = -INFINITY;
       }
-      float mx = -INFINITY;
+      // The exponents' reference (m_run) stays where it is until a lane's
+      // probabilities of a tile add up to more than kRescaleSum: a probability is then
+      // kRescaleSum at most, well inside fp16 and fp32, and the 64 accumulators and the
+      // running sum are rescaled rarely instead of whenever a maximum rises at all (with
+      // 32 rows per wave, that is in most tiles of a prompt's first hundreds of keys).
+      // Not further: the key that dominates a row is exact where it is the reference
+      // itself, and rounded to 11 bits where the reference lags behind it.
+      // The sum is needed anyway; the maxima are taken only where the reference moves,
+      // which the infinite reference before a wave's first tile (and anything that is
+      // not a number) makes it do.
+      constexpr float kRescaleSum = 256.f;
+      float p[16], psum;
+      auto exponentials = [&] {
 #pragma unroll
-      for (int kb = 0; kb < kNKB; ++kb)
+        for (int i = 0; i < 16; ++i) p[i] = fast_exp2(__builtin_fmaf(sacc[i], I.scale_log2, neg_m));
+        psum = p[0];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[kb][i]);
-      mx = max_with_lane_xor32(mx);
-      // The reference of the exponents (m_run) only moves when some row's maximum has
-      // risen more than kRescaleStep (in the exponent's units) above it - and on the
-      // wave's first tile, to that tile's maximum: probabilities then reach
-      // 2^kRescaleStep at most, and the 64 accumulators and the running sum are
-      // rescaled rarely instead of whenever a maximum rises at all (with 32 rows per
-      // wave, that is in most tiles of a prompt's first hundreds of keys).
-      if (__builtin_amdgcn_ballot_w64(mx > m_limit) != 0) {
-        const float m_new = fmaxf(m_run, mx);
+        for (int i = 1; i < 16; ++i) psum += p[i];
+      };
+      exponentials();
+      if (__builtin_amdgcn_ballot_w64(!(psum <= kRescaleSum)) != 0) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[i]);
+        const float m_new = fmaxf(m_run, max_with_lane_xor32(mx));
         // Rows past the prompt may have no valid key at all; keep them finite.
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
         const float alpha = fast_exp2((m_run - m_use) * I.scale_log2);
@@ -568,45 +639,33 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
           for (int i = 0; i < 16; ++i) oacc[mb][i] *= alpha;
         m_run = m_use;
-        m_limit = m_use + rescale_score;
         neg_m = -m_use * I.scale_log2;
+        exponentials();
       }
-      float psum = 0.f;
-      Frag pf[2 * kNKB];                          // B fragments: [kb][step] -> index 2 kb + st
+      l_run += psum;
+      Frag pf[2];                                 // B fragments, 16 keys each
       // bf16 keeps only 8 mantissa bits of a probability, which alone would cost
       // more than the 2e-3 budget, so bf16 P is carried as hi + lo parts.
       constexpr bool kSplitP = __is_same(T, BF16);
-      Frag pf_lo[kSplitP ? 2 * kNKB : 1];
+      Frag pf_lo[kSplitP ? 2 : 1];
 #pragma unroll
-      for (int kb = 0; kb < kNKB; ++kb) {
-        float p[16];
+      for (int st = 0; st < 2; ++st) {
+        uint32_t w[4];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) p[i] = fast_exp2(__builtin_fmaf(sacc[kb][i], I.scale_log2, neg_m));
+        for (int j = 0; j < 4; ++j) w[j] = pack2<T>(p[8 * st + 2 * j], p[8 * st + 2 * j + 1]);
+        pf[st].u = u32x4{w[0], w[1], w[2], w[3]};
+        if constexpr (kSplitP) {
+          // The part of p that its bf16 rounding lost, as a second bf16.
+          uint32_t lo[4];
 #pragma unroll
-        for (int st = 0; st < 2; ++st) {
-          uint32_t w[4];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) w[j] = pack2<T>(p[8 * st + 2 * j], p[8 * st + 2 * j + 1]);
-          pf[2 * kb + st].u = u32x4{w[0], w[1], w[2], w[3]};
-          if constexpr (kSplitP) {
-            // The part of p that its bf16 rounding lost, as a second bf16.
-            uint32_t lo[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              lo[j] = pack2<T>(p[8 * st + 2 * j] - bf16_lo(w[j]), p[8 * st + 2 * j + 1] - bf16_hi(w[j]));
-              psum += p[8 * st + 2 * j] + p[8 * st + 2 * j + 1];
-            }
-            pf_lo[2 * kb + st].u = u32x4{lo[0], lo[1], lo[2], lo[3]};
-          } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) psum += p[8 * st + j];
-          }
+          for (int j = 0; j < 4; ++j)
+            lo[j] = pack2<T>(p[8 * st + 2 * j] - bf16_lo(w[j]), p[8 * st + 2 * j + 1] - bf16_hi(w[j]));
+          pf_lo[st].u = u32x4{lo[0], lo[1], lo[2], lo[3]};
         }
       }
-      l_run += psum;
 
       // ---- O^T += V^T . P^T ---------------------------------------------------------------
-      // k-slot j of lane half h in step (kb, st) is key 32 kb + 16 st + 8 (j/4) + 4 h + j%4
+      // k-slot j of lane half h in step st is key 16 st + 8 (j/4) + 4 h + j%4
       {
         auto read_v = [&](int n) {         // fragment n = 4 ks + mb
           const int mb = n % 4, ks = n / 4;
@@ -616,15 +675,14 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
           // group receives dim i of rows 0..3.  Here a group covers dims
           // 32 mb + 16 (lane/16 % 2) .. +15 and keys 16 ks + 4 half (+ 8) .. +3.
           // Address: row = 16 ks + 8 hsel + rl with rl = 4 half + jrow, chunk =
-          // 4 mb + cl, position = chunk ^ swz(row) = (cl ^ swz(rl)) ^ 4 (mb ^ 2 hsel).
-          // The lane part cl ^ rl is below 8, so bit 3 of the constant part adds
-          // and only its bit 2 (mb odd) has to be folded into the lane's base:
+          // 4 mb + cl, position = chunk ^ swz(rl): cl ^ swz(rl) is below 8, so only
+          // bit 2 of the constant part (mb odd) has to be folded into the lane's base:
           // two bases per lane, everything else is an immediate offset.
           typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
           u32x2 part[2];
 #pragma unroll
           for (int hsel = 0; hsel < 2; ++hsel) {
-            const uint16_t *src = Vr + v_lane_base[mb & 1] + (16 * ks + 8 * hsel) * D + 64 * (((mb >> 1) ^ hsel) & 1);
+            const uint16_t *src = Vr + v_lane_base[mb & 1] + (16 * ks + 8 * hsel) * D + 64 * (mb >> 1);
             const v4i16 r = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)src);
             union { v4i16 v; u32x2 u; } c;
             c.v = r;
@@ -639,34 +697,41 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
         __builtin_amdgcn_sched_barrier(0);
         MUX_PF_PRIO(MUX_PF_PRIO_MFMA);
 #pragma unroll
-        for (int j = 0; j < 8 * kNKB; ++j) {
+        for (int j = 0; j < 8; ++j) {
           oacc[j % 4] = mfma<T>(ring[j % kDepth], pf[j / 4], oacc[j % 4]);
           if constexpr (kSplitP) oacc[j % 4] = mfma<T>(ring[j % kDepth], pf_lo[j / 4], oacc[j % 4]);
-          if (j + kDepth < 8 * kNKB) ring[j % kDepth] = read_v(j + kDepth);
+          if (j + kDepth < 8) ring[j % kDepth] = read_v(j + kDepth);
           __builtin_amdgcn_sched_barrier(0);
         }
         MUX_PF_PRIO(MUX_PF_PRIO_VALU);
       }
     }
     if constexpr (STEP) {
-      stores_counted = false;
-      // (a use on every path: a load left pending would be waited for, and the
-      // next tile's loads with it, where the register is written again)
-      asm volatile("" : "+v"(slot));
+      stores_counted = to_pool;
       if (to_pool) {
-        if (slot < 0 || slot >= S.pool_slots) slot = -1;
-        // Rows 0 - 15 (16 - 31) of the tile to all four groups of 16 lanes.
-        const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(slot), static_cast<uint32_t>(slot), false, false);
-        const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(slot >> 32),
-                                                         static_cast<uint32_t>(slot >> 32), false, false);
-        stores_counted = true;
-#pragma unroll
-        for (int pair = 0; pair < 2; ++pair)
-          stores_counted &= write_tokens_to_pool(
-              smem + cur * kTileElems, smem + (2 + cur) * kTileElems, 16 * pair,
-              static_cast<int64_t>((static_cast<uint64_t>(hi[pair]) << 32) | lo[pair]), wave, lane, S);
+#pragma unroll 1
+        for (int r = 0; r < kBN; r += 16) {
+          const uint32_t slots_at = smem_at + 8 * kTileElems + 8 * (k0 - q0 + r);
+          int64_t base;
+          asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)"
+                       : "=&v"(base)
+                       : "v"(smem_at + 8 * kTileElems + 8 * (kBM + (k0 - q0 + r) / 16))
+                       : "memory");
+          const uint32_t base_lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
+          const uint32_t base_hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32));
+          base = static_cast<int64_t>((static_cast<uint64_t>(base_hi) << 32) | base_lo);
+          if (base >= 0)
+            write_block_to_pool(smem_at + 2 * (cur * kTileElems + r * D), smem_at + 2 * ((2 + cur) * kTileElems + r * D), writer,
+                                base, S);
+          else
+            stores_counted &= write_tokens_to_pool(Kt, Vr, r, slots_at, wave, lane, S);
+        }
       }
     }
+  };
+  for (int t = 0; t < n_tiles; t += 2) {
+    tile(t, std::integral_constant<int, 0>{});
+    if (t + 1 < n_tiles) tile(t + 1, std::integral_constant<int, 1>{});
   }
 
 #ifdef MUX_TRACE

@@ -348,6 +348,36 @@ def test_prefill_row_maxima_that_jump_far_above_the_softmax_reference(dtype):
     assert excess <= 0, f"max-abs error {(got - want).abs().max().item():.3e}"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lift", [2.0, 4.5, 7.5, 12.0])
+def test_prefill_probabilities_on_both_sides_of_the_reference_rule(dtype, lift):
+    """The reference of the exponents moves when a lane's 16 probabilities of a tile
+    add up to more than 256 times it: all keys from the 40th on score `lift` (in the
+    exponent) above those before them, so that 16 of them add up to 64, 362, 2896 or
+    65536 - one above the rule by its sum although none is by itself, and two
+    (7.5 and 12) that 16-bit probabilities would lose or overflow further on."""
+    _announce(f"prefill sums around the reference rule {dtype} {lift}")
+    Hq = Hkv = 2
+    lens = [33, 260]
+    g = torch.Generator().manual_seed(78)
+    T = sum(lens)
+    pad = (T + 7) // 8 * 8
+    u = torch.randn((Hq, D), generator=g)
+    u = u / u.norm(dim=-1, keepdim=True)
+    q = 0.05 * torch.randn((pad, Hq, D), generator=g) + 8.0 * u
+    k = 0.05 * torch.randn((pad, Hkv, D), generator=g)
+    v = torch.randn((pad, Hkv, D), generator=g)
+    k[33 + 40:] += lift / 1.4427 * D ** 0.5 / 8.0 * u
+    q, k, v = (x.reshape(pad, -1).to(dtype) for x in (q, k, v))
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
+    out = torch.zeros((pad, Hq * D), dtype=dtype, device=DEV)
+    ops.prefill_causal(out, q.to(DEV), k.to(DEV), v.to(DEV), cu, max(lens), D ** -0.5, Hkv, prompt_lens=lens)
+    torch.cuda.synchronize()
+    got = out.float().cpu()[:T]
+    want = orc.prefill_causal(q, k, v, lens, D ** -0.5, Hkv)
+    assert ((got - want).abs() - _bound(want, dtype)).max().item() <= 0
+
+
 def test_prefill_rejects_bad_arguments():
     q = torch.zeros((8, 256), dtype=torch.float16, device=DEV)
     cu = torch.tensor([0, 8], dtype=torch.int32, device=DEV)

@@ -318,6 +318,45 @@ def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many)
         assert torch.equal(a, b), f"{what} differ between the step operator and the three kernels"
 
 
+@pytest.mark.parametrize("bs,off", [(16, 0), (16, 8), (16, 5), (32, 0), (32, 16), (32, 8), (8, 0)])
+def test_prompt_step_pool_writes_of_runs_that_start_anywhere_in_a_block(bs, off):
+    """The step operator writes 16 tokens with two stores where they are 16 slots in
+    order from a multiple of 16 inside one block: runs that start at, before and
+    behind such a multiple, up to the pool's last slot, against the cache write."""
+    print(f"[case] prompt step runs bs={bs} off={off}", flush=True)
+    from muxserve_amd import torch_ops
+    from muxserve_amd.attention import build_cos_sin_cache
+    Hq = Hkv = 2
+    lens = [160, 48]
+    T = sum(lens)
+    N = Hkv * ((T + off + bs - 1) // bs)
+    slots = torch.empty((T, 1, Hkv), dtype=torch.int64)
+    for h in range(Hkv):
+        slots[:, 0, h] = h * (N // Hkv) * bs + off + torch.arange(T)
+    slots[-16:, 0, 1] = N * bs - 16 + torch.arange(16)                    # the pool's last slots
+    qkv = torch.randn((T + (-T) % 8, (Hq + 2 * Hkv) * D), generator=torch.Generator().manual_seed(bs + off)).half().to(DEV)
+    positions = torch.arange(T + (-T) % 8, device=DEV)
+    cos_sin = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    cu = torch.tensor([0, lens[0], T], dtype=torch.int32, device=DEV)
+    results = []
+    for fused in (False, True):
+        x = qkv.clone()
+        q, k, v = x.split([Hq * D, Hkv * D, Hkv * D], dim=-1)
+        kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=torch.float16)
+        kp.fill_(3)
+        vp.fill_(5)
+        if fused:
+            out = torch.zeros((x.shape[0], Hq * D), dtype=x.dtype, device=DEV)
+            torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, slots.to(DEV), 0, cu, lens, D ** -0.5)
+        else:
+            ops.rotary_neox(positions, q, k, cos_sin, num_tokens=T)
+            ops.reshape_and_cache(k, v, kp, vp, slots.to(DEV), layer=0, num_tokens=T)
+        torch.cuda.synchronize()
+        results.append([t.cpu().view(torch.int16) for t in (x, kp, vp)])
+    for a, b, what in zip(*results, ("qkv rows", "k pool", "v pool")):
+        assert torch.equal(a, b), f"{what} differ from the rotation and the cache write"
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_rotary_table_at_any_float_offset(dtype):
     """The cos|sin table is taken at any 4-byte boundary, as the rotary kernel takes

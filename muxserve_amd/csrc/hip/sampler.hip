@@ -45,10 +45,10 @@ union SmFrag {
 constexpr int kSmTile = 256;              // the hidden size must be a multiple of this
 constexpr int kSmMaxRowsPerPass = 256;
 // Up to 32 sampled rows the narrow kernel, beyond them the wide one.  32000 rows of
-// 4096, us: the narrow one with 32 rows 43.5, the wide one with 33 to 64 rows 46.5
+// 4096, us: the narrow one with 32 rows 43.5, the wide one with 33 to 64 rows 45
 // (the narrow one with four row blocks per wave took 52.3 to 53.5 there, and 107 and
-// 214 with 128 and 256 rows, passing over the matrix once per 64; the wide one 56
-// and 82).  Small vocabularies too, though the wide kernel keeps its 128 rows per
+// 214 with 128 and 256 rows, passing over the matrix once per 64; the wide one 53
+// and 73).  Small vocabularies too, though the wide kernel keeps its 128 rows per
 // workgroup there: 16000 rows, 33 sampled 46.6 / 34.9, 64 48.0 / 38.1; 4000 rows
 // 37.0 / 30.8 and 38.3 / 33.8.
 constexpr int kSmNarrowRows = 32;
@@ -65,7 +65,7 @@ struct LmHeadParams {
   int32_t hidden_size, vocab, num_rows;
   int32_t hidden_rows;                    // rows of `hidden`: row_index entries are clamped to it
   int32_t half_tiles;                     // the wide kernel: a large vocabulary, which the narrow one gives 8 waves
-  uint32_t *counter;                      // workgroups arrived, zero between launches
+  uint32_t *counter;                      // workgroups arrived (and, behind it, per group of them), zero between launches
   unsigned long long *table;              // [workgroups][16 NB] keys, written before they are read
   int64_t *next_tokens;
 };
@@ -99,56 +99,72 @@ __device__ __forceinline__ void store_key(const LmHeadParams &P, int64_t at, flo
   __hip_atomic_store(&P.table[at], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Announces this workgroup's line of the table; true in the workgroup that came
-// last.  The table is written and read with device-coherent accesses (they
+// Announces this workgroup's line of the table to the `expected` workgroups of a
+// counter; true in the one that came last.  The table is written and read with device-coherent accesses (they
 // bypass the per-XCD L2), so ordering them against the counter takes only a wait
 // for this wave's table stores to be acknowledged before the workgroup meets
 // and bumps the counter.  A device-scope fence would also write back and
 // invalidate this XCD's L2, which holds the hidden states every other
 // workgroup is still reading (measured: +30 us per launch).
-__device__ __forceinline__ bool last_to_arrive(const LmHeadParams &P, int *s_last) {
+__device__ __forceinline__ bool last_to_arrive(uint32_t *counter, uint32_t expected, int *s_last) {
   wait_own_vector_memory();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __syncthreads();
   if (threadIdx.x == 0)
-    *s_last = __hip_atomic_fetch_add(P.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    *s_last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expected - 1;
   __syncthreads();
   if (!*s_last) return false;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
   return true;
 }
 
-// Last workgroup to arrive: thread -> (sampled row tid % ROWS, slice tid / ROWS
-// of the workgroups), sixteen loads in flight.  fin: THREADS keys of LDS.
+// Maximum over n lines of the table from `first`, `step` lines apart, per sampled
+// row: thread -> (row tid % ROWS, slice tid / ROWS of the lines), sixteen loads in
+// flight.  The result is whole in the threads below ROWS.  fin: THREADS keys of LDS.
 template <int ROWS, int THREADS>
-__device__ __forceinline__ void reduce_table(const LmHeadParams &P, unsigned long long *fin) {
+__device__ __forceinline__ unsigned long long reduce_lines(const LmHeadParams &P, int first, int n, int step,
+                                                           unsigned long long *fin) {
   constexpr int SLICES = THREADS / ROWS;
   const int tid = threadIdx.x;
   const int row = tid % ROWS, slice = tid / ROWS;
   unsigned long long best = 0;
-  const int n_wg = gridDim.x;
-  for (int b0 = slice; b0 < n_wg && slice < SLICES; b0 += 16 * SLICES) {
+  for (int b0 = slice; b0 < n && slice < SLICES; b0 += 16 * SLICES) {
     unsigned long long v[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       const int b = b0 + j * SLICES;
-      v[j] = b < n_wg ? __hip_atomic_load(&P.table[static_cast<int64_t>(b) * ROWS + row], __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT)
-                      : 0ull;
+      v[j] = b < n ? __hip_atomic_load(&P.table[static_cast<int64_t>(first + b * step) * ROWS + row], __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT)
+                   : 0ull;
     }
 #pragma unroll
     for (int j = 0; j < 16; ++j) best = v[j] > best ? v[j] : best;
   }
   fin[tid] = best;
   __syncthreads();
-  if (tid < P.num_rows) {
-    unsigned long long k = fin[tid];
+  if (tid < ROWS) {
 #pragma unroll
-    for (int sl = 1; sl < SLICES; ++sl) k = fin[sl * ROWS + tid] > k ? fin[sl * ROWS + tid] : k;
-    const uint32_t idx = 0xffffffffu - static_cast<uint32_t>(k);
-    P.next_tokens[tid] = idx < static_cast<uint32_t>(P.vocab) ? idx : 0;   // every logit NaN: token 0
+    for (int sl = 1; sl < SLICES; ++sl) best = fin[sl * ROWS + tid] > best ? fin[sl * ROWS + tid] : best;
   }
-  if (tid == 0) __hip_atomic_store(P.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return best;
+}
+
+__device__ __forceinline__ void store_token(const LmHeadParams &P, int row, unsigned long long key) {
+  const uint32_t idx = 0xffffffffu - static_cast<uint32_t>(key);
+  P.next_tokens[row] = idx < static_cast<uint32_t>(P.vocab) ? idx : 0;   // every logit NaN: token 0
+}
+
+__device__ __forceinline__ void clear_counter(uint32_t *counter) {
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The last workgroup to arrive reduces the table.
+template <int ROWS, int THREADS>
+__device__ __forceinline__ void reduce_table(const LmHeadParams &P, unsigned long long *fin, int *s_last) {
+  if (!last_to_arrive(P.counter, gridDim.x, s_last)) return;
+  const unsigned long long key = reduce_lines<ROWS, THREADS>(P, 0, gridDim.x, 1, fin);
+  if (static_cast<int>(threadIdx.x) < P.num_rows) store_token(P, threadIdx.x, key);
+  clear_counter(P.counter);
 }
 
 template <typename T, int NB, int NW>
@@ -322,9 +338,8 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
     for (int w = 1; w < NW; ++w) take_better(bv, bi, red_v[w][tid], red_i[w][tid]);
     store_key(P, static_cast<int64_t>(blockIdx.x) * ROWS + tid, bv, bi);
   }
-  if (!last_to_arrive(P, &s_last)) return;
   __shared__ unsigned long long fin[64 * NW];
-  reduce_table<ROWS, 64 * NW>(P, fin);
+  reduce_table<ROWS, 64 * NW>(P, fin, &s_last);
 }
 
 // ---------------------------------------------------------------------------
@@ -338,24 +353,34 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
 //   * 128 rows per workgroup: a 32000-row vocabulary is 250 workgroups, one per
 //     compute unit, one round.
 //   * The hidden dimension is walked in tiles of 64 (a 128-byte line per row).  A
-//     tile goes global -> registers -> LDS (two LDS buffers, one barrier per tile;
-//     16-byte chunk c of a row at position c ^ (row % 8): no bank conflicts), and
-//     PD further tiles are in flight in registers.
-// Up to 64 rows it is bound by HBM (262 MB of a 32000 x 4096 matrix in 47 us =
-// 5.6 TB/s).  With 256 rows (84 us: 3.1 TB/s, 0.8 PFLOP/s) the clock is 1.66 GHz,
-// the matrix cores are busy half and the LDS 44 % of the time; the memory is not
-// what it waits for (every tile from the L1: 77 us), and a third LDS buffer with
-// a barrier that waits for the writes only changes nothing.
-// The reduction is the one above with 64 NB columns per table line.
-template <typename T, int NB, int PD>
+//     tile goes from global memory straight into LDS, NBUF - 1 tiles ahead, one
+//     barrier per tile, 16-byte chunk c of a row at position c ^ (row % 8): no bank
+//     conflicts.  NBUF is what 160 KB hold (at most 5).
+// 32000 x 4096, us (tiles staged through registers / straight into LDS, the
+// two-level reduction in both): 64 rows 46.3 / 44.8, 128 rows 54.3 / 53.1, 256 rows
+// 79 / 73; 128256 x 4096 bf16, 256 rows 304 / 295.  Up to 64 rows it is bound by HBM
+// (5.8 TB/s).  With 256 rows the clock is 1.66 GHz and LDS is the busiest unit: 128 KB
+// of fragments and 48 KB of tiles in per 1024 cycles of MFMA and compute unit, at 128
+// bytes a cycle.  Fewer fragment reads cost more than they save: four waves of 64 x
+// 32 NB (a quarter less) 80, four waves of 128 x 16 NB with the hidden states straight
+// from global memory in registers (half of it) 100 before the reduction, one wave per
+// SIMD hides neither the barrier nor the latencies.
+// The reduction is the one above with 64 NB columns per table line.  One workgroup
+// reads 250 lines of 256 keys in 8 rounds of loads, so beyond 64 workgroups (4 rounds
+// in two slices) it takes two levels: groups of 16, or 32 groups (one level / two:
+// 32000 x 4096, 256 rows 84.5 / 79, 128 rows 56.2 / 54.3; 128256 x 4096, 256 rows
+// 331 / 304; 9000 rows, 71 workgroups, 62.5 / 61.8).
+constexpr size_t kSmCounterBytes = 256;    // the arrival counters, in front of the table
+constexpr int kSmOneLevelWgs = 64, kSmGroupWgs = 16, kSmMaxGroups = 32;
+template <typename T, int NB, int NBUF>
 __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHeadParams P) {
   constexpr int KT = 64;                   // hidden elements per tile
   constexpr int ROWS = 64 * NB;            // sampled rows
   constexpr int VR = 128;                  // vocabulary rows
   constexpr int NW = 8;
-  constexpr int kMfma = 0x8, kVmemRead = 0x20, kDsRead = 0x100, kDsWrite = 0x200;   // instruction classes of the scheduler
+  constexpr int kMfma = 0x8, kDsRead = 0x100;   // instruction classes of the scheduler
   constexpr int TILE = (VR + ROWS) * KT;   // elements of one LDS buffer: embedding rows, then hidden rows
-  __shared__ __attribute__((aligned(16))) uint16_t tile[2][TILE];
+  __shared__ __attribute__((aligned(16))) uint16_t tile[NBUF][TILE];
   __shared__ float red_v[2][ROWS];
   __shared__ int red_i[2][ROWS];
   __shared__ int s_last;
@@ -368,39 +393,35 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
   const int t_start = P.half_tiles ? blockIdx.x % n_tiles : 2 * (blockIdx.x % (n_tiles / 2));
   const int vrow0 = blockIdx.x * VR;
 
-  // Staging: thread -> row tid / 8 (+ 64 j), chunk tid % 8.  Every load is
-  // unconditional - behind a branch the compiler waits for all loads in flight
-  // instead of the oldest: rows past the vocabulary re-read its last row (masked
+  // Staging, global memory to LDS: instruction j of wave w fills 8 rows of a tile
+  // (lane l's 16 bytes land at base + 16 l: row l / 8, position l % 8, which holds
+  // chunk (l % 8) ^ (l / 8)).  Rows past the vocabulary re-read its last row (masked
   // at the end), sampled rows past the last re-read a valid one (not stored).
-  const int srow = tid >> 3, schunk = tid & 7;
-  const uint16_t *wsrc[2], *hsrc[NB];
+  const int srow = 8 * wave + (lane >> 3), schunk = (lane & 7) ^ (lane >> 3);
+  const uint16_t *src[2 + NB];
 #pragma unroll
   for (int j = 0; j < 2; ++j)
-    wsrc[j] = P.weight + static_cast<int64_t>(min(vrow0 + srow + 64 * j, P.vocab - 1)) * P.weight_stride + 8 * schunk;
+    src[j] = P.weight + static_cast<int64_t>(min(vrow0 + srow + 64 * j, P.vocab - 1)) * P.weight_stride + 8 * schunk;
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
     const int row = min(srow + 64 * j, P.num_rows - 1);
-    const int src = P.row_index ? min(max(P.row_index[row], 0), P.hidden_rows - 1) : row;
-    hsrc[j] = P.hidden + static_cast<int64_t>(src) * P.hidden_stride + 8 * schunk;
+    const int r = P.row_index ? min(max(P.row_index[row], 0), P.hidden_rows - 1) : row;
+    src[2 + j] = P.hidden + static_cast<int64_t>(r) * P.hidden_stride + 8 * schunk;
   }
-  const int soff = srow * KT + 8 * (schunk ^ (srow & 7));     // (rows 64 apart swizzle alike)
-  struct Staged {
-    sm_u32x4 w[2], h[NB];
-  };
-  auto load = [&](Staged &r, int t) {
+  typedef const __attribute__((address_space(3))) uint16_t lds_u16;
+  const uint32_t tile_at = (uint32_t)(uintptr_t)(lds_u16 *)&tile[0][0];
+  auto load = [&](int t, int buf) {
     int x = t + t_start;
     x = (x >= n_tiles ? x - n_tiles : x) * KT;
+    const uint32_t at = tile_at + 2 * (buf * TILE + 8 * wave * KT);
 #pragma unroll
-    for (int j = 0; j < NB; ++j) r.h[j] = *reinterpret_cast<const sm_u32x4 *>(hsrc[j] + x);
+    for (int j = 2; j < 2 + NB; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at + 2 * 64 * j * KT), "v"(src[j] + x)
+                   : "memory", "m0");
 #pragma unroll
-    for (int j = 0; j < 2; ++j) r.w[j] = __builtin_nontemporal_load(reinterpret_cast<const sm_u32x4 *>(wsrc[j] + x));
-  };
-  auto store = [&](const Staged &r, int buf) {
-    uint16_t *const dst = &tile[buf][soff];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) *reinterpret_cast<sm_u32x4 *>(dst + (VR + 64 * j) * KT) = r.h[j];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) *reinterpret_cast<sm_u32x4 *>(dst + 64 * j * KT) = r.w[j];
+    for (int j = 0; j < 2; ++j)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(at + 2 * 64 * j * KT), "v"(src[j] + x)
+                   : "memory", "m0");
   };
 
   sm_v4f32 acc[4][NB];
@@ -433,44 +454,33 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
       }
   };
 
-  // Register set s holds the tile t with t % PD == s that comes next.
-  Staged st[PD];
-  load(st[0], 0);
-  store(st[0], 0);
 #pragma unroll
-  for (int s = 1; s <= PD; ++s) load(st[s % PD], min(s, n_tiles - 1));
+  for (int t = 0; t < NBUF - 1; ++t)
+    if (t < n_tiles) load(t, t);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  int buf = 0;
-  // One tile.  Each half's fragments are on their way while the half before it is
-  // being multiplied: the second half's behind the first, the next tile's first
-  // half behind the second (which is therefore multiplied after the barrier that
-  // completes the next tile); LDS accesses and MFMAs are dealt one by one, since a
-  // wave that issues its reads in a row waits for the LDS queue with the matrix
-  // cores idle (256 rows: 88 -> 83 us).
   Half f0, f1;
   read_half(f0, 0, 0);
-  auto step = [&](Staged &next, int t, bool store_next, bool load_next) {
+  int buf = 0;
+  for (int t = 0; t < n_tiles; ++t) {
+    const int next = buf + 1 == NBUF ? 0 : buf + 1;
+    const bool more = t + NBUF - 1 < n_tiles;
+    if (more) load(t + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
     read_half(f1, buf, 1);
     multiply(f0);
-    if (store_next) store(next, buf ^ 1);
-    if (load_next) load(next, t + 1 + PD);
 #pragma unroll
     for (int i = 0; i < 4 + NB; ++i) {
       __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
       __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
     }
-#pragma unroll
-    for (int i = 0; i < 2 + NB; ++i) {
-      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(kDsWrite, 1, 0);
-    }
     __builtin_amdgcn_sched_group_barrier(kMfma, 4 * NB, 0);
-    __builtin_amdgcn_sched_group_barrier(kVmemRead, 2 + NB, 0);
     __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
+    if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * (2 + NB)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    buf ^= 1;
-    if (store_next) read_half(f0, buf, 0);
+    read_half(f0, next, 0);              // (behind the last tile: some buffer, not used)
     multiply(f1);
 #pragma unroll
     for (int i = 0; i < 4 + NB; ++i) {
@@ -479,19 +489,9 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
     }
     __builtin_amdgcn_sched_group_barrier(kMfma, 4 * NB, 0);
     __builtin_amdgcn_sched_barrier(0);
-  };
-  int t0 = 0;
-  for (; t0 + 2 * PD < n_tiles; t0 += PD) {
-#pragma unroll
-    for (int s = 0; s < PD; ++s) step(st[(s + 1) % PD], t0 + s, true, true);
+    buf = next;
   }
-  for (; t0 < n_tiles; t0 += PD) {
-#pragma unroll
-    for (int s = 0; s < PD; ++s) {
-      const int t = t0 + s;
-      if (t < n_tiles) step(st[(s + 1) % PD], t, t + 1 < n_tiles, t + 1 + PD < n_tiles);
-    }
-  }
+  __syncthreads();
 
   // Lane holds logits[vocab row vrow0 + 64 wm + 16 mb + 4 g + i][sampled row 16 (NB wn + nb) + r16].
 #pragma unroll
@@ -524,8 +524,28 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
     take_better(bv, bi, red_v[1][tid], red_i[1][tid]);
     store_key(P, static_cast<int64_t>(blockIdx.x) * ROWS + tid, bv, bi);
   }
-  if (!last_to_arrive(P, &s_last)) return;
-  reduce_table<ROWS, 64 * NW>(P, reinterpret_cast<unsigned long long *>(&tile[0][0]));
+  unsigned long long *const fin = reinterpret_cast<unsigned long long *>(&tile[0][0]);
+  const int n_wg = gridDim.x;
+  if (n_wg <= kSmOneLevelWgs) {
+    reduce_table<ROWS, 64 * NW>(P, fin, &s_last);
+    return;
+  }
+  // Two levels: the last workgroup of a group leaves the group's maxima in the
+  // group's first line (each thread in the column it has read itself), the last of
+  // these reduces the groups' lines.
+  const int per_group = max(kSmGroupWgs, (n_wg + kSmMaxGroups - 1) / kSmMaxGroups);
+  const int group = blockIdx.x / per_group, first = group * per_group, groups = (n_wg + per_group - 1) / per_group;
+  const int members = min(per_group, n_wg - first);
+  uint32_t *const group_counter = P.counter + 1 + group;
+  if (!last_to_arrive(group_counter, members, &s_last)) return;
+  unsigned long long key = reduce_lines<ROWS, 64 * NW>(P, first, members, 1, fin);
+  if (tid < ROWS)
+    __hip_atomic_store(&P.table[static_cast<int64_t>(first) * ROWS + tid], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  clear_counter(group_counter);
+  if (!last_to_arrive(P.counter, groups, &s_last)) return;
+  key = reduce_lines<ROWS, 64 * NW>(P, 0, groups, per_group, fin);
+  if (tid < P.num_rows) store_token(P, tid, key);
+  clear_counter(P.counter);
 }
 
 __global__ void sampler_zero_kernel(uint32_t *p, int n) {
@@ -533,7 +553,7 @@ __global__ void sampler_zero_kernel(uint32_t *p, int n) {
   if (i < n) p[i] = 0;
 }
 
-constexpr size_t kSmCounterBytes = 256;        // the arrival counter, then the table
+static_assert(4 * (1 + kSmMaxGroups) <= kSmCounterBytes, "the counters fit in front of the table");
 #ifndef MUX_SM_EIGHT_WAVE_MIN_WGS
 #define MUX_SM_EIGHT_WAVE_MIN_WGS 192
 #endif
@@ -609,10 +629,10 @@ extern "C" int32_t mux_greedy_sample(int64_t *next_tokens, const void *hidden_st
       const dim3 wide_grid((vocab_size + 127) / 128);
 #define MUX_LM_WIDE(TT)                                                                                            \
   do {                                                                                                            \
-    if (rows <= 64) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 1, 4>), wide_grid, dim3(512), 0, st, P);   \
-    else if (rows <= 128) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 2, 3>), wide_grid, dim3(512), 0, st, P); \
-    else if (rows <= 192) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 3, 2>), wide_grid, dim3(512), 0, st, P); \
-    else hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 4, 2>), wide_grid, dim3(512), 0, st, P);              \
+    if (rows <= 64) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 1, 5>), wide_grid, dim3(512), 0, st, P);   \
+    else if (rows <= 128) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 2, 4>), wide_grid, dim3(512), 0, st, P); \
+    else if (rows <= 192) hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 3, 3>), wide_grid, dim3(512), 0, st, P); \
+    else hipLaunchKernelGGL((lm_head_argmax_wide_kernel<TT, 4, 3>), wide_grid, dim3(512), 0, st, P);              \
   } while (0)
       if (dtype == MUXA_DTYPE_F16) MUX_LM_WIDE(F16);
       else MUX_LM_WIDE(BF16);

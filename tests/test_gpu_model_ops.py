@@ -282,6 +282,42 @@ def test_greedy_sampler_module_prompt_and_decode_steps():
     _check_tokens(toks, emb, hid[:13], V, torch.float16, "decode step")
 
 
+@pytest.mark.parametrize("V,R", [(8192, 256), (8193, 256), (8321, 33), (65536, 65), (65537, 193), (65537, 256), (70000, 129)])
+def test_greedy_sample_two_level_reduction(V, R):
+    """From 65 workgroups of 128 vocabulary rows on, groups of 16 (or 32 groups: 513
+    workgroups are 30 of 17 and one of 3) reduce their lines of the table first.  Planted
+    winners in the first and last rows of workgroups and groups, each with an equal
+    logit further up, go to the lower id; twice on one workspace, whose counters are
+    left at zero."""
+    print(f"[case] greedy_sample two levels V={V} R={R}", flush=True)
+    from muxserve_amd import _lib
+    g = torch.Generator().manual_seed(V + R)
+    wgs = (V + 127) // 128
+    size = max(16, (wgs + 31) // 32)
+    edges = sorted({min(128 * w + o, V - 1) for w in list(range(0, wgs, size)) + list(range(size - 1, wgs, size)) + [wgs - 1]
+                    for o in (0, 127)})
+    emb = (torch.randn((V, 256), generator=g) * 0.01).half()
+    hid = torch.randn((R, 256), generator=g).half()
+    emb[:, :64] = 0
+    want = []
+    for r in range(R):                                         # rows r and r + 64 share column r % 64
+        c = r % 64
+        hid[r, :64] = 0
+        hid[r, c] = 4.0
+    for c in range(64):
+        first = edges[c * len(edges) // 64]
+        emb[first, c] = 30.0
+        emb[min(first + 128 * (1 + c % (2 * size)), V - 1), c] = 30.0
+        want.append(first)
+        emb[first, 64:] = 0
+        emb[min(first + 128 * (1 + c % (2 * size)), V - 1), 64:] = 0
+    ws = torch.zeros((_lib.attn().mux_greedy_sample_workspace_bytes(V),), dtype=torch.uint8, device=DEV)
+    for _ in range(2):
+        toks = ops.greedy_sample(emb.to(DEV), hid.to(DEV), V, R, workspace=ws)
+        assert toks.cpu().tolist() == [want[r % 64] for r in range(R)]
+        assert int(ws[:256].count_nonzero()) == 0
+
+
 def test_greedy_sample_leaves_its_counter_zeroed_and_the_workspace_reusable():
     """One caller-owned workspace serves calls of different vocabulary sizes,
     batch sizes and workgroup shapes one after the other."""

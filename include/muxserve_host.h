@@ -157,6 +157,22 @@ int64_t mux_sched_get_batch_compact(MuxBatchScheduler *s, const int32_t *req, in
                                     int32_t *context_lens, int64_t context_lens_cap,
                                     int32_t *desc, int64_t desc_cap);
 
+/* The host side of a compact step in one call: mux_sched_get_batch_info and
+ * mux_sched_get_batch_compact in turn, with all that the step uploads packed into
+ * `host`:
+ *   [tokens | positions | context lens, padded to 4 | descriptors | block_info]
+ * tokens and positions padded to the next multiple of 8 with zeros.  `info` (at
+ * least MUX_STEP_INFO_INTS + 4 * (n_req / 3) ints):
+ *   { numTokens, numContexts, maxContextLen, maxNumBlocksPerSeq, ints used of host,
+ *     most token blocks that one entry received, sum of the context lens (low, high
+ *     32 bits), number of prompts, of preempted requests, of batch entries },
+ * then the prompt lens, the preempted ids and (id, maxTokens) per entry.  On failure
+ * info[0] says where: 0 host is too small (MUX_ENOSPC with the ints it needs in
+ * info[4], nothing has changed), 1 get_batch_info, 2 get_batch_compact. */
+#define MUX_STEP_INFO_INTS 11
+int32_t mux_sched_step(MuxBatchScheduler *s, const int32_t *req, int32_t n_req, const int32_t *block_info,
+                       int64_t n_block_info, int32_t *host, int64_t host_cap, int32_t *info, int32_t info_cap);
+
 /* BatchScheduler::releaseRequests, csrc/batch_scheduler.cpp:195-199. */
 int32_t mux_sched_release_requests(MuxBatchScheduler *s, const int32_t *request_ids, int32_t n);
 

@@ -63,6 +63,7 @@ def host():
         "mux_sched_enable_device_rows": (c_i32, [c_vp, c_i32]),
         "mux_sched_get_batch_compact": (c_i64, [c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_vp, c_i64,
                                                 c_vp, c_i64, c_vp, c_i64]),
+        "mux_sched_step": (c_i32, [c_vp, c_vp, c_i32, c_vp, c_i64, c_vp, c_i64, c_vp, c_i32]),
         "mux_sched_release_requests": (c_i32, [c_vp, c_vp, c_i32]),
         "mux_sched_get_preempt_requests": (c_i32, [c_vp, c_vp, c_i32]),
         "mux_sched_get_prompt_info": (c_i32, [c_vp, c_vp, c_i32]),

@@ -16,6 +16,8 @@ from . import _lib
 
 
 def _i32(a):
+    if type(a) is np.ndarray and a.dtype == np.int32 and a.ndim == 1 and a.flags.c_contiguous:
+        return a
     return np.ascontiguousarray(np.asarray(a, dtype=np.int32).reshape(-1))
 
 
@@ -41,6 +43,7 @@ class BatchScheduler:
                                              int(max_seq_len), int(block_size))
         if not self._h:
             raise ValueError("BatchScheduler: all four arguments must be positive")
+        self._step_info = None
         self.num_layers, self.num_heads = int(num_layers), int(num_heads)
         self.max_seq_len, self.block_size = int(max_seq_len), int(block_size)
         self.max_blocks_per_seq = (self.max_seq_len + self.block_size - 1) // self.block_size
@@ -72,7 +75,7 @@ class BatchScheduler:
                                                                blk.ctypes.data, blk.size,
                                                                out.ctypes.data, out.size),
                             "BatchScheduler.get_batch_info")
-        return [int(x) for x in out[:n]]
+        return out[:n].tolist()
 
     def get_batch(self, batch_info, block_info, token_tensor, token_position_tensor,
                   context_len_tensor, block_table_tensor, slot_mapping_tensor) -> None:
@@ -137,6 +140,37 @@ class BatchScheduler:
                                                               tok, pos, n_tok, ctx, n_ctx, desc, n_desc),
                         "BatchScheduler.get_batch_compact")
 
+    STEP_INFO_INTS = 11
+
+    def step(self, batch_info, block_info, staging):
+        """Not in the reference: get_batch_info, get_batch_compact, get_preempt_requests
+        and get_batch_reqs in one call (a decode step of 32 requests spends as much in
+        their four round trips as in everything else).  staging(n): a contiguous CPU int32
+        tensor of at least n elements, into which all that the step uploads is packed (see
+        mux_sched_step in include/muxserve_host.h).  Returns (staging tensor, the
+        STEP_INFO_INTS sizes, prompt lens, preempted ids, [id, max tokens] per entry)."""
+        req, blk = _i32(batch_info), _i32(block_info)
+        cap = self.STEP_INFO_INTS + 4 * (req.size // 3)
+        if self._step_info is None or len(self._step_info) < cap:
+            self._step_info = (_lib.c_i32 * (2 * cap))()
+        info = self._step_info
+        host = staging(0)
+        while True:
+            addr, cap = _buf(host, np.int32, "staging")
+            rc = self._lib.mux_sched_step(self._h, req.ctypes.data, req.size, blk.ctypes.data, blk.size, addr, cap,
+                                          info, len(info))
+            if rc != -2 or info[0] != 0:
+                break
+            host = staging(info[4])
+        if rc < 0:
+            _lib.check_host(rc, ("BatchScheduler.step", "BatchScheduler.get_batch_info",
+                                 "BatchScheduler.get_batch_compact")[info[0]])
+        head = info[:self.STEP_INFO_INTS]
+        a = self.STEP_INFO_INTS + head[8]
+        b = a + head[9]
+        flat = info[b:b + 2 * head[10]]
+        return host, head, info[self.STEP_INFO_INTS:a], info[a:b], [[x, y] for x, y in zip(flat[::2], flat[1::2])]
+
     def release_requests(self, request_ids) -> None:
         ids = _i32(list(request_ids))
         _lib.check_host(self._lib.mux_sched_release_requests(self._h, ids.ctypes.data, ids.size),
@@ -146,7 +180,7 @@ class BatchScheduler:
         n = fn(self._h, None, 0)
         out = np.empty(max(n, 1), dtype=np.int32)
         fn(self._h, out.ctypes.data, n)
-        return [int(x) for x in out[:n]]
+        return out[:n].tolist()
 
     def get_preempt_requests(self):
         return self._vec(self._lib.mux_sched_get_preempt_requests)

@@ -13,6 +13,7 @@
 #include "muxserve_host.h"
 
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 #include <memory>
 #include <unordered_map>
@@ -441,6 +442,60 @@ int64_t mux_sched_get_batch_compact(MuxBatchScheduler *s, const int32_t *req, in
     positions[k] = 0;
   }
   return n_tokens;
+}
+
+int32_t mux_sched_step(MuxBatchScheduler *s, const int32_t *req, int32_t n_req, const int32_t *block_info,
+                       int64_t n_block_info, int32_t *host, int64_t host_cap, int32_t *info, int32_t info_cap) {
+  if (!s || !req || !block_info || (!host && host_cap > 0) || !info || n_req < 0 || n_block_info < 1 ||
+      n_block_info > INT32_MAX)
+    return MUX_EINVAL;
+  const int32_t rows = n_req / 3;
+  if (info_cap < MUX_STEP_INFO_INTS + 4 * static_cast<int64_t>(rows)) return MUX_EINVAL;
+
+  // Sizes first: nothing has changed when the buffer is too small.  (Unknown ids and
+  // replies that are too short are left to the two calls.)
+  const int32_t entries = std::min(std::max(block_info[0], 0), rows);
+  int64_t tokens = 0, contexts = 0;
+  for (int32_t i = 0; i < entries; ++i) {
+    const Sequence *q = s->find(req[3 * i]);
+    if (!q) continue;
+    tokens += q->decoding() ? 1 : static_cast<int64_t>(q->prompt.size());
+    contexts += q->decoding() ? 1 : 0;
+  }
+  const int64_t padded = (tokens + 7) / 8 * 8;
+  const int64_t at_ctx = 2 * padded, at_desc = at_ctx + (contexts + 3) / 4 * 4;
+  const int64_t at_reply = at_desc + static_cast<int64_t>(entries) * MUX_STEP_DESC_INTS;
+  const int64_t total = at_reply + n_block_info;
+  info[0] = 0;
+  if (total > INT32_MAX) return MUX_EINVAL;
+  info[4] = static_cast<int32_t>(total);
+  if (total > host_cap) return MUX_ENOSPC;
+
+  info[0] = 1;
+  // (its six sizes where the head's last ones go, the prompt lens behind the head)
+  int32_t *const sizes = info + MUX_STEP_INFO_INTS - 6;
+  const int32_t n = mux_sched_get_batch_info(s, req, n_req, block_info, n_block_info, sizes,
+                                             info_cap - (MUX_STEP_INFO_INTS - 6));
+  if (n < 0) return n;
+  info[0] = 2;
+  const int64_t rc = mux_sched_get_batch_compact(s, req, n_req, block_info, n_block_info, host, host + padded, padded,
+                                                 host + at_ctx, contexts, host + at_desc,
+                                                 static_cast<int64_t>(entries) * MUX_STEP_DESC_INTS);
+  if (rc < 0) return static_cast<int32_t>(rc);
+  std::memcpy(host + at_reply, block_info, sizeof(int32_t) * static_cast<size_t>(n_block_info));
+
+  int32_t most = 0;
+  for (int32_t i = 0; i < entries; ++i) most = std::max(most, host[at_desc + i * MUX_STEP_DESC_INTS + 3]);
+  int64_t context_sum = 0;
+  for (int64_t c = 0; c < contexts; ++c) context_sum += host[at_ctx + c];
+  const int32_t prompts = n - 6, preempted = static_cast<int32_t>(s->preempted.size());
+  const int32_t head[MUX_STEP_INFO_INTS] = {
+      sizes[0], sizes[1], sizes[2], sizes[3], static_cast<int32_t>(total), most,
+      static_cast<int32_t>(context_sum & 0xffffffff), static_cast<int32_t>(context_sum >> 32), prompts, preempted, entries};
+  std::copy(head, head + MUX_STEP_INFO_INTS, info);
+  int32_t *at = std::copy(s->preempted.begin(), s->preempted.end(), info + MUX_STEP_INFO_INTS + prompts);
+  std::copy(s->batch_reqs.begin(), s->batch_reqs.end(), at);
+  return MUX_OK;
 }
 
 int32_t mux_sched_release_requests(MuxBatchScheduler *s, const int32_t *request_ids, int32_t n) {

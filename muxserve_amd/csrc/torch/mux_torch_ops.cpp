@@ -9,6 +9,7 @@
 //     torch.ops.muxserve_amd.paged_decode(out, q, k_pool, v_pool, block_tables,
 //                                         context_lens, max_ctx, scale, layer, 0, 0, workspace)
 #include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
@@ -561,6 +562,44 @@ at::Tensor prompt_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k,
   return out;
 }
 
+// The tensors of a step from its packed form (mux_sched_step in muxserve_host.h:
+// host, and the head of its info in `sizes`): one asynchronous copy, one launch.
+std::vector<at::Tensor> step_inputs(at::Tensor mirror, const at::Tensor &host, at::IntArrayRef sizes, int64_t block_size) {
+  need_gpu({&mirror});
+  TORCH_CHECK(mirror.scalar_type() == at::kInt && mirror.dim() == 4 && mirror.is_contiguous(),
+              "mirror: expected contiguous int32 [rows, blocks, L, H]");
+  TORCH_CHECK(sizes.size() >= 11, "sizes: the head of a step's info");
+  const int64_t tokens = sizes[0], contexts = sizes[1], longest = sizes[2], max_blocks = sizes[3], total = sizes[4];
+  const int64_t most = sizes[5], entries = sizes[10];
+  const int64_t padded = (tokens + 7) / 8 * 8, at_ctx = 2 * padded, at_desc = at_ctx + (contexts + 3) / 4 * 4;
+  const int64_t at_reply = at_desc + 8 * entries, L = mirror.size(2), H = mirror.size(3);
+  TORCH_CHECK(tokens >= 0 && contexts >= 0 && entries >= 0 && max_blocks >= 0 && at_reply < total,
+              "sizes do not describe a step");
+  TORCH_CHECK(host.device().is_cpu() && host.scalar_type() == at::kInt && host.dim() == 1 && host.is_contiguous() &&
+                  host.numel() >= total,
+              "host: expected the packed step, contiguous CPU int32");
+  const c10::DeviceGuard guard(mirror.device());
+  const at::TensorOptions i32 = mirror.options(), i64 = i32.dtype(at::kLong);
+  at::Tensor dev = at::empty({total}, i32);
+  dev.copy_(host.narrow(0, 0, total), /*non_blocking=*/true);
+  const at::Tensor wide = at::empty({2, padded}, i64);
+  const at::Tensor slots = at::empty({tokens, L, H}, i64);
+  const bool decoding = longest > 0 && max_blocks > 0;
+  const at::Tensor tables = decoding ? at::empty({L, entries, H, max_blocks}, i32) : at::empty({0, 0, 0, mirror.size(1)}, i32);
+  const at::Tensor lens = at::empty({contexts}, at::TensorOptions().dtype(at::kInt));
+  if (contexts > 0) std::copy_n(host.data_ptr<int32_t>() + at_ctx, contexts, lens.data_ptr<int32_t>());
+  const int32_t *const d = dev.data_ptr<int32_t>();
+  check(mux_build_step(mirror.data_ptr<int32_t>(), static_cast<int32_t>(mirror.size(0)),
+                       static_cast<int32_t>(mirror.size(1)), static_cast<int32_t>(L), static_cast<int32_t>(H),
+                       static_cast<int32_t>(block_size), d + at_desc, static_cast<int32_t>(entries), d + at_reply,
+                       total - at_reply, static_cast<int32_t>(most), static_cast<int32_t>(tokens),
+                       tokens > 0 ? slots.data_ptr<int64_t>() : nullptr, decoding ? tables.data_ptr<int32_t>() : nullptr,
+                       static_cast<int32_t>(decoding ? max_blocks : 0), d, wide.data_ptr<int64_t>(), at_ctx,
+                       stream_of(mirror)),
+        "mux_build_step");
+  return {wide.select(0, 0), wide.select(0, 1), dev.narrow(0, at_ctx, contexts), lens, slots, tables};
+}
+
 at::Tensor rms_norm(const at::Tensor &x, const at::Tensor &weight, double eps) {
   need_gpu({&x, &weight});
   TORCH_CHECK(x.dim() == 2 && weight.dim() == 1 && weight.size(0) == x.size(1) &&
@@ -616,6 +655,7 @@ TORCH_LIBRARY(muxserve_amd, m) {
   m.def("greedy_sample_workspace_bytes(int vocab_size) -> int", &greedy_sample_workspace_bytes);
   m.def("greedy_sample(Tensor embedding, Tensor hidden_states, int vocab_size, int num_rows, Tensor row_index, "
         "Tensor(a!) workspace) -> Tensor");
+  m.def("step_inputs(Tensor(a!) mirror, Tensor host, int[] sizes, int block_size) -> Tensor[]");
   m.def("decode_layer(Tensor positions, Tensor(a!) q, Tensor(b!) k, Tensor v, Tensor cos_sin, Tensor(c!) k_pool, "
         "Tensor(d!) v_pool, Tensor slot_mapping, Tensor block_tables, Tensor context_lens, int max_context_len, "
         "float scale, int layer, int partition_size, int total_context_len, Tensor(e!)? workspace, "
@@ -640,6 +680,7 @@ TORCH_LIBRARY_IMPL(muxserve_amd, CUDA, m) {
   m.impl("multi_decode", &multi_decode);
   m.impl("rotary_neox", &rotary_neox);
   m.impl("greedy_sample", &greedy_sample);
+  m.impl("step_inputs", &step_inputs);
   m.impl("decode_layer", &decode_layer);
   m.impl("prompt_layer", &prompt_layer);
   m.impl("rms_norm", &rms_norm);

@@ -14,6 +14,7 @@ from typing import Tuple
 import torch
 
 from . import _lib
+from . import torch_ops as T
 from .batch_scheduler import BatchScheduler
 
 
@@ -25,7 +26,7 @@ class DeviceBlockTables:
         self.L, self.H = scheduler.num_layers, scheduler.num_heads
         self.block_size = scheduler.block_size
         self.max_blocks_per_seq = scheduler.max_blocks_per_seq
-        # int32 [row][token block][layer][head]; written only by build().
+        # int32 [row][token block][layer][head]; written only by step_inputs() and build().
         self.mirror = torch.zeros((self.max_rows, self.max_blocks_per_seq, self.L, self.H), dtype=torch.int32,
                                   device=self.device)
         self._staging = None
@@ -41,6 +42,19 @@ class DeviceBlockTables:
             self._staging = torch.empty((max(n_ints, 1 << 16),), dtype=torch.int32,
                                         pin_memory=torch.cuda.is_available())
         return self._staging
+
+    def step_inputs(self, host: torch.Tensor, head) -> Tuple[torch.Tensor, ...]:
+        """host, head: the packed step and its sizes from BatchScheduler.step.  One
+        asynchronous copy and one launch; returns token ids and positions int64
+        [padded], context lens int32 on the device and on the host (a tensor of its own:
+        the staging buffer is reused by the next step), slot_mapping int64 [tokens, L, H]
+        and block_tables int32 [L, sequences, H, max blocks], or the reference's empty
+        prefill table."""
+        tensors = T.load().step_inputs(self.mirror, host, head, self.block_size)
+        if self._uploaded is None:
+            self._uploaded = torch.cuda.Event()
+        self._uploaded.record(torch.cuda.current_stream(self.device))
+        return tensors
 
     def upload(self, n_ints: int) -> torch.Tensor:
         """One asynchronous copy of the first n_ints of the staging buffer."""

@@ -15,6 +15,8 @@ from . import _lib
 
 
 def _i32(a):
+    if type(a) is np.ndarray and a.dtype == np.int32 and a.ndim == 1 and a.flags.c_contiguous:
+        return a
     return np.ascontiguousarray(np.asarray(a, dtype=np.int32).reshape(-1))
 
 

@@ -45,14 +45,13 @@ def prepare_inputs(batch_scheduler: BatchScheduler, cache_alloc: Callable[[np.nd
     else:
         block_info = np.array([len(batch_request_ids)], dtype=np.int32)        # llm_runtime.py:287-288
 
+    if device_tables is not None:
+        return _prepare_on_device(batch_scheduler, device_tables, batch_block_request, block_info)
     batch_info = batch_scheduler.get_batch_info(batch_block_request, block_info)
     num_tokens, num_contexts, max_context_len, max_num_blocks_per_seq, num_layers, num_heads = batch_info[:6]
     prompt_lens = batch_info[6:]
 
     padded_len = (num_tokens + 7) // 8 * 8                                      # llm_runtime.py:300
-    if device_tables is not None:
-        return _prepare_on_device(batch_scheduler, device_tables, batch_block_request, block_info, num_tokens,
-                                  num_contexts, max_context_len, max_num_blocks_per_seq, prompt_lens, padded_len)
     pin = torch.cuda.is_available()
     slot_mapping = torch.empty((num_tokens, num_layers, num_heads), dtype=torch.int64, pin_memory=pin)
     input_tensor = torch.empty((padded_len,), dtype=torch.int32, pin_memory=pin)
@@ -93,40 +92,18 @@ def prepare_inputs(batch_scheduler: BatchScheduler, cache_alloc: Callable[[np.nd
     return input_tensor, input_positions, input_metadata, batch_reqs, preempted_reqs
 
 
-def _prepare_on_device(sched, dt, batch_block_request, block_info, num_tokens, num_contexts, max_context_len,
-                       max_num_blocks_per_seq, prompt_lens, padded_len):
+def _prepare_on_device(sched, dt, batch_block_request, block_info):
     """The device_tables path of prepare_inputs: everything the step uploads is
     packed into one pinned int32 buffer
         [tokens | positions | context_lens | descriptors | allocator reply]
-    and copied once."""
-    n_entries = max(int(block_info[0]), 0)
-    D = sched.STEP_DESC_INTS
-    n_info = int(block_info.size)
-    o_tok, o_pos = 0, padded_len
-    o_ctx = 2 * padded_len
-    o_desc = o_ctx + (num_contexts + 3) // 4 * 4
-    o_info = o_desc + n_entries * D
-    total = o_info + n_info
-    host = dt.staging(total)
-    sched.get_batch_compact(batch_block_request, block_info, host[o_tok:o_pos], host[o_pos:o_ctx],
-                            host[o_ctx:o_ctx + num_contexts], host[o_desc:o_info])
-    host[o_info:total] = torch.from_numpy(block_info)
-    desc_host = host[o_desc:o_info].view(n_entries, D)
-    max_new = int(desc_host[:, 3].max()) if n_entries else 0
-    total_context_len = int(host[o_ctx:o_ctx + num_contexts].sum()) if num_contexts else 0
-    # (the staging buffer is reused by the next step: the host copy is its own tensor)
-    context_lens_host = host[o_ctx:o_ctx + num_contexts].clone() if num_contexts else None
-    preempted_reqs = sched.get_preempt_requests()
-    batch_reqs = sched.get_batch_reqs()
-
-    dev = dt.upload(total)
-    tokens_positions = torch.empty((2, padded_len), dtype=torch.int64, device=dt.device)     # llm_runtime.py:324-325
-    input_tensor, input_positions = tokens_positions.unbind(0)
-    context_lens = dev[o_ctx:o_ctx + num_contexts]
-    decoding = max_context_len > 0
-    slot_mapping, block_tables = dt.build(dev[o_desc:o_info], dev[o_info:total], n_entries, max_new, num_tokens,
-                                          max_num_blocks_per_seq if decoding else 0, narrow=dev[:o_ctx], wide=tokens_positions)
+    and copied once; one operator copies it, allocates the step's tensors and launches
+    the kernel that fills them."""
+    host, head, prompt_lens, preempted_reqs, batch_reqs = sched.step(batch_block_request, block_info, dt.staging)
+    max_context_len = head[2]
+    input_tensor, input_positions, context_lens, context_lens_host, slot_mapping, block_tables = dt.step_inputs(host, head)
+    total_context_len = (head[6] & 0xffffffff) + (head[7] << 32)
     input_metadata = InputMetadata(prompt_lens=prompt_lens, slot_mapping=slot_mapping, context_lens=context_lens,
                                    max_context_len=max_context_len, block_tables=block_tables,
-                                   total_context_len=total_context_len, context_lens_host=context_lens_host)
+                                   total_context_len=total_context_len,
+                                   context_lens_host=context_lens_host if head[1] else None)
     return input_tensor, input_positions, input_metadata, batch_reqs, preempted_reqs

@@ -24,7 +24,7 @@ OPERATORS = ("reshape_and_cache", "rope_reshape_and_cache", "multi_reshape_and_c
              "paged_decode_workspace_bytes",
              "paged_decode", "multi_decode_workspace_bytes", "multi_decode", "prefill_causal",
              "rope_prefill_and_cache", "decode_layer", "prompt_layer", "multi_prefill_causal", "rms_norm",
-             "silu_and_mul", "greedy_sample_workspace_bytes", "greedy_sample")
+             "silu_and_mul", "greedy_sample_workspace_bytes", "greedy_sample", "step_inputs")
 
 _loaded = False
 

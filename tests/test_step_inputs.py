@@ -161,3 +161,54 @@ def test_compact_step_needs_rows_enabled():
     with pytest.raises(ValueError):
         sched.get_batch_compact(req, blk, torch.zeros(8, dtype=torch.int32), torch.zeros(8, dtype=torch.int32),
                                 torch.zeros(0, dtype=torch.int32), torch.zeros((1, D), dtype=torch.int32))
+
+
+@pytest.mark.parametrize("blocks,cap", [(40, 0), (40, 3), (9, 0), (9, 1 << 12)])
+def test_step_in_one_call_equals_its_four(blocks, cap):
+    """BatchScheduler.step against get_batch_info, get_batch_compact,
+    get_preempt_requests and get_batch_reqs on a second scheduler: prompts, decode steps
+    across block boundaries, preemption (9 token blocks), a staging buffer that has to
+    grow (which must not move the step on) and what an unknown request raises."""
+    L, H, bs = 2, 3, 16
+    pair = []
+    for _ in range(2):
+        store, sched = KVStorage(blocks * L * H), BatchScheduler(L, H, 256, bs)
+        sched.enable_device_rows(4)
+        for i, p in enumerate([3 * bs, 2 * bs + 1, bs, 3]):
+            sched.add_request(np.arange(p, dtype=np.int32) + i, i, 20 + i)
+        pair.append((store, sched))
+    buffers = [torch.full((cap,), -5, dtype=torch.int32)]
+
+    def staging(n):
+        if buffers[-1].numel() < n:
+            buffers.append(torch.full((n,), -5, dtype=torch.int32))
+        return buffers[-1]
+
+    alive, last = [0, 1, 2, 3], []
+    for step in range(2 * bs + 2):
+        got = []
+        for store, sched in pair:
+            info = sched.try_batch(alive, last)
+            req = np.ascontiguousarray(info[:-1])
+            reply = store.allocate_batch(req, L, H) if int(info[-1]) > 0 else np.array([len(alive)], dtype=np.int32)
+            got.append((sched, req, reply))
+        (sched, req, reply), (one, req1, reply1) = got
+        assert np.array_equal(req, req1) and np.array_equal(reply, reply1)
+        bi = sched.get_batch_info(req, reply)
+        n, pad = max(int(reply[0]), 0), (bi[0] + 7) // 8 * 8
+        tok, pos, ctx, desc = (torch.full((k,), -7, dtype=torch.int32) for k in (pad, pad, bi[1], n * D))
+        sched.get_batch_compact(req, reply, tok, pos, ctx, desc)
+        host, head, lens, preempted, reqs = one.step(req1, reply1, staging)
+        at = 2 * pad + (bi[1] + 3) // 4 * 4
+        assert head[:4] == bi[:4] and head[4] == at + n * D + reply.size and head[10] == n
+        assert lens == bi[6:] and preempted == sched.get_preempt_requests() and reqs == sched.get_batch_reqs()
+        assert head[5] == (int(desc.view(n, D)[:, 3].max()) if n else 0) and head[6] == int(ctx.sum()) and head[7] == 0
+        assert torch.equal(host[:2 * pad], torch.cat([tok, pos])) and torch.equal(host[2 * pad:2 * pad + bi[1]], ctx)
+        assert torch.equal(host[at:at + n * D], desc) and np.array_equal(host[at + n * D:head[4]].numpy(), reply)
+        alive = [r for r in alive if r not in preempted]
+        last = [step] * len(alive)
+        if not alive:
+            break
+    assert (blocks > 9) == (len(alive) == 4)
+    with pytest.raises(KeyError):
+        pair[1][1].step(np.array([77, 1, 0], dtype=np.int32), np.arange(1 + L * H, dtype=np.int32) * 0 + 1, staging)

@@ -13,7 +13,8 @@ extern "C" {
 /* A whole prompt step of the attention layer (models/llama.py:159-161): rotary
  * embedding of q and k in place, causal attention, and the cache write of the
  * rotated k and of v.  Two launches: k is rotated by itself, the attention
- * kernel rotates q and scatters the K and V tiles that it reads anyway.  `attn`
+ * kernel rotates q and scatters the K and V tiles that it reads anyway; one launch
+ * for short prompts with as many kv heads as query heads (csrc/prompt_step.h).  `attn`
  * and `write` describe the same q, k and v (equal pointers, strides and head
  * counts); attn->prompt_lens_host is required, adds up to write->num_tokens and
  * agrees with cu_seqlens, so that every token belongs to a prompt; the head

@@ -113,9 +113,10 @@ def build_cos_sin_cache(rotary_dim: int, max_position: int, base: float, device)
 
 
 def prompt_step_pays(prompts: int, tokens: int, heads: int, kv_heads: int) -> bool:
-    """Whether a step of prompts is faster with the attention kernel rotating q and
-    writing the cache itself, behind the rotation of k, than with rotation and cache
-    write in one launch and the attention behind it.  us, two launches / attention
+    """Whether a step of prompts that the one launch for short prompts does not take
+    (csrc/prompt_step.h) is faster with the attention kernel rotating q and writing
+    the cache itself, behind the rotation of k, than with rotation and cache write in
+    one launch and the attention behind it.  us, two launches / attention
     kernel doing it, where the lines lie:
 
     * few query rows are bound by one workgroup's chain of waits, which the rotation

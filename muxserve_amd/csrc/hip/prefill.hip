@@ -45,8 +45,11 @@
 // on one machine: 16 x 2048 tokens f16 1052 -> 800 us (rotation of k 100, attention
 // by itself 600, pool stores 55, rotation of q 45), three bf16 prompts of 700 - 4000
 // tokens on 64 / 8 heads 548 -> 490 us.  Prompts of a few tokens lose in this form:
-// 128 of 6 tokens, 32 heads, 47 us against 33 with rotation and cache write in a
-// launch of their own.
+// 128 of 6 tokens, 32 heads, 47 us against 34 with rotation and cache write in a
+// launch of their own, and 29.5 in the short form (SHORT, below), which one launch
+// is: it waits for one chain of loads instead of two and reads k once; 16 prompts
+// of 100 tokens, 32 heads, 30 -> 21 us, 64 of 128 101 -> 90.
+#include "../prompt_step.h"
 #include "cache_write.h"
 
 #include <algorithm>
@@ -147,6 +150,7 @@ struct PrefillStep {
   int64_t pool_slots;
   int32_t max_position;
   int32_t block_size;
+  int32_t short_waves;           // the host's choice of kernel: W of the short form, or 0
 };
 static_assert(sizeof(PrefillParams) + sizeof(PrefillStep) <= 4096, "kernel argument segment");
 constexpr int kPairTileBits = 12;       // tile in bits 0-11, prompt in bits 12-27, model in bits 28-30
@@ -277,10 +281,10 @@ struct BlockWriter {
   }
 };
 
-// Rows row0 .. row0 + 15 of the tile (K at kt, V at vt, LDS addresses) to the 16
-// slots from `base`, a multiple of 16, of one block: two stores.
-__device__ __forceinline__ void write_block_to_pool(uint32_t kt, uint32_t vt, const BlockWriter &w, int64_t base,
-                                                    const PrefillStep &S) {
+// The first n of 16 rows of the tile (K at kt, V at vt, LDS addresses) to the n slots
+// from `base`, a multiple of 16, of one block.  True if that took exactly two stores.
+__device__ __forceinline__ bool write_block_to_pool(uint32_t kt, uint32_t vt, const BlockWriter &w, int64_t base, int n,
+                                                    int lane, const PrefillStep &S) {
   constexpr int D = kHeadSize;
   u32x4 kx;
   u32x2 v0, v1;
@@ -292,19 +296,46 @@ __device__ __forceinline__ void write_block_to_pool(uint32_t kt, uint32_t vt, co
   const int bs_shift = __builtin_ctz(static_cast<unsigned>(S.block_size));
   const int64_t first = (base >> bs_shift) * (D << bs_shift);           // the block's first element
   const int64_t in_block = base & (S.block_size - 1);
-  const uint16_t *const kp = S.k_pool + first + 8 * in_block, *const vp = S.v_pool + first + in_block;
-  // (as in write_tokens_to_pool: whole lines stream past the L2)
-  asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.k_off), "v"(kx), "s"(kp) : "memory");
-  if (S.block_size == 16) asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
-  else asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
+  uint16_t *const kp = S.k_pool + first + 8 * in_block, *const vp = S.v_pool + first + in_block;
+  if (n == 16) {
+    // (as in write_tokens_to_pool: whole lines stream past the L2)
+    asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.k_off), "v"(kx), "s"(kp) : "memory");
+    if (S.block_size == 16) asm volatile("global_store_dwordx4 %0, %1, %2 nt\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
+    else asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 4" ::"v"(w.v_off), "v"(vx), "s"(vp) : "memory");
+    return true;
+  }
+  if ((lane & 15) < n) *reinterpret_cast<u32x4 *>(reinterpret_cast<char *>(kp) + w.k_off) = kx;
+  // V: this lane's 8 tokens of a dim, as many as there are, in pieces of 8, 4, 2 and 1.
+  const int mine = n - (lane & 8);
+  uint16_t *const v = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(vp) + w.v_off);
+  if (mine >= 8) {
+    *reinterpret_cast<u32x4 *>(v) = vx;
+  } else if (mine > 0) {
+    const bool four = mine & 4;
+    if (four) *reinterpret_cast<u32x2 *>(v) = u32x2{vx[0], vx[1]};
+    const uint32_t next = four ? vx[2] : vx[0], last = four ? vx[3] : vx[1];
+    uint16_t *const rest = v + (four ? 4 : 0);
+    if (mine & 2) *reinterpret_cast<uint32_t *>(rest) = next;
+    if (mine & 1) rest[mine & 2] = static_cast<uint16_t>((mine & 2) ? last : next);
+  }
+  return false;
 }
 
-template <typename T, bool STEP>
+// SHORT = W > 0: the step of prompts of at most 32 W tokens (W = 1, 2, 4) with as
+// many kv heads as query heads, by workgroups of W waves.  A workgroup then holds all
+// of a (prompt, head): it rotates k as well, in the registers its waves load their 32
+// rows into, and the whole of K and V (W tiles each) sits in LDS, so that one launch
+// does the step and its tile loop has one barrier in front of it.
+template <typename T, bool STEP, int SHORT = 0>
 __device__ __forceinline__ void prefill_body(const PrefillParams &P, const PrefillStep &S) {
   constexpr int D = kHeadSize;
-  // K[2], V[2] tile buffers.  The epilogue reuses the memory for the output rows
-  // (4 waves x 32 rows of 272 bytes), which is the larger of the two.
-  constexpr int kSmemElems = 4 * kTileElems > 4 * 32 * (D + 8) ? 4 * kTileElems : 4 * 32 * (D + 8);
+  constexpr int W = SHORT > 0 ? SHORT : 4;     // waves
+  constexpr int kRows = 32 * W;                // query rows
+  // K[2], V[2] tile buffers (SHORT: W of each).  The epilogue reuses the memory for
+  // the output rows (W waves x 32 rows of 272 bytes).
+  constexpr int NBUF = SHORT > 0 ? W : 2;
+  constexpr int kSmemElems =
+      SHORT > 0 ? 2 * W * kTileElems + 4 * (kRows + kRows / 16) : std::max(4 * kTileElems, 4 * 32 * (D + 8));
   __shared__ __attribute__((aligned(16))) uint16_t smem[kSmemElems];
 
 #ifdef MUX_TRACE
@@ -394,7 +425,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
   float neg_m = INFINITY;
 
   // Keys needed by this workgroup: positions 0 .. min(len, q0 + 128) - 1.
-  const int kv_end = min(len, q0 + kBM);
+  const int kv_end = min(len, q0 + kRows);
   const int n_tiles = (kv_end + kBN - 1) / kBN;
 
   // ---- tile staging -------------------------------------------------------------------
@@ -406,15 +437,15 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
   // Rows past the prompt re-read its last row: finite data whose probability is
   // exactly 0 (such a key is in the future of every valid query).
 
-  // Instruction i of wave w fills KiB 4 i + w of a tile = rows 16 i + 4 w .. +3;
-  // lane l sits at row 16 i + 4 w + l/16, position l%16, and fetches chunk
-  // position ^ swz(row) - the same chunk for every i (rows 16 apart swizzle alike).
-  constexpr int kLoads = kBN / 16;         // such instructions per wave, tile and operand
+  // Instruction i of wave w fills KiB W i + w of a tile = rows 4 (W i + w) .. +3;
+  // lane l sits at row 4 (W i + w) + l/16, position l%16, and fetches chunk
+  // position ^ swz(row) - with W > 1 the same for every i (rows 8 apart swizzle alike).
+  constexpr int kLoads = kBN / (4 * W);    // such instructions per wave, tile and operand
   uint32_t koff[kLoads];
   const int row0 = 4 * wave + (lane >> 4);
-  const int chunk0 = (lane & 15) ^ swz(row0);
+  auto chunk_of = [&](int i) { return static_cast<uint32_t>((lane & 15) ^ swz(row0 + 4 * W * i)); };
 #pragma unroll
-  for (int i = 0; i < kLoads; ++i) koff[i] = static_cast<uint32_t>(row0 + 16 * i) * row_bytes + 16u * chunk0;
+  for (int i = 0; i < kLoads; ++i) koff[i] = static_cast<uint32_t>(row0 + 4 * W * i) * row_bytes + 16u * chunk_of(i);
   typedef const __attribute__((address_space(3))) uint16_t lds_u16;
   const uint32_t smem_at = (uint32_t)(uintptr_t)(lds_u16 *)smem;
   // The loads are written out (they have no destination registers), with the waits
@@ -425,13 +456,15 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
   auto dma_tile = [&](int t, int buf) {    // tile t into buffer buf
     const char *const kt = kbase + static_cast<uint64_t>(t) * tile_bytes, *const vt = vbase + static_cast<uint64_t>(t) * tile_bytes;
     const bool whole = (t + 1) * kBN <= len;
-    const uint32_t omax = last_row - static_cast<uint32_t>(t) * tile_bytes + 16u * chunk0;
+    const uint32_t omax = last_row - static_cast<uint32_t>(t) * tile_bytes;
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
-      const uint32_t o = whole ? koff[i] : min(koff[i], omax);
-      const uint32_t kd = smem_at + 2 * (buf * kTileElems + (4 * i + wave) * 512);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd), "v"(o), "s"(kt) : "memory", "m0");
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd + 4 * kTileElems), "v"(o), "s"(vt)
+      const uint32_t o = whole ? koff[i] : min(koff[i], omax + 16u * chunk_of(i));
+      const uint32_t kd = smem_at + 2 * (buf * kTileElems + (W * i + wave) * 512);
+      if constexpr (SHORT == 0)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd), "v"(o), "s"(kt) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(kd + 2 * NBUF * kTileElems), "v"(o),
+                   "s"(vt)
                    : "memory", "m0");
     }
   };
@@ -447,29 +480,114 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
     for (int f = 0; f < 4; ++f) k_lane_base[f] = qcol * D + 8 * ((2 * f + half) ^ swz(qcol));
   }
-  dma_tile(0, 0);
+  if constexpr (SHORT > 0) {
+    for (int t = 0; t < n_tiles; ++t) dma_tile(t, t);
+  } else {
+    dma_tile(0, 0);
+  }
   // The slots of the workgroup's own rows, -1 for none, in LDS behind the tile
   // buffers (where only the epilogue's staging reaches): a load of them in the tile
   // loop would be waited for behind the previous tile's pool stores.
-  // Behind them, for every 16 rows, the first one's slot where they are 16 slots in
-  // order from a multiple of 16 inside one block (every prompt behind a block table
-  // of 16 or more tokens, up to its last few), else -1.
-  int64_t *const own_slots = reinterpret_cast<int64_t *>(smem + 4 * kTileElems);
-  static_assert(8 * kTileElems + 8 * (kBM + kBM / 16) <= 2 * kSmemElems, "the slots fit behind the tile buffers");
-  const BlockWriter writer(wave, lane, STEP ? S.block_size : 0);
+  // Behind them, for every 16 rows, (first slot << 5 | n) where the first n rows have
+  // slots in order from a multiple of 16 inside one block and the others none (every
+  // prompt behind a block table of 16 or more tokens), else -1.
+  int64_t *const own_slots = reinterpret_cast<int64_t *>(smem + 2 * NBUF * kTileElems);
+  static_assert(4 * NBUF * kTileElems + 8 * (kRows + kRows / 16) <= 2 * kSmemElems, "the slots fit behind the tile buffers");
+  const BlockWriter writer(wave, lane, STEP && SHORT == 0 ? S.block_size : 0);
   if constexpr (STEP) {
-    if (writes_pool && tid < kBM) {
+    if (writes_pool && tid < kRows) {
       int64_t slot = -1;
       if (q0 + tid < len) slot = S.slots[static_cast<int64_t>(seq_begin + q0 + tid) * S.slot_stride + hk];
       if (slot >= S.pool_slots) slot = -1;
       own_slots[tid] = slot;
       const int64_t first = __shfl(slot, lane & 48);
-      const uint64_t in_order = __builtin_amdgcn_ballot_w64(first >= 0 && (first & 15) == 0 && slot == first + (lane & 15) &&
-                                                            S.block_size >= 16);
-      if ((lane & 15) == 0) own_slots[kBM + tid / 16] = ((in_order >> (lane & 48)) & 0xffff) == 0xffff ? first : -1;
+      const uint32_t some = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(slot >= 0) >> (lane & 48)) & 0xffffu;
+      const uint32_t fits = static_cast<uint32_t>(__builtin_amdgcn_ballot_w64(slot < 0 || slot == first + (lane & 15)) >> (lane & 48)) & 0xffffu;
+      const bool in_order = fits == 0xffffu && (some & 1) && (some & (some + 1)) == 0 && (first & 15) == 0 && S.block_size >= 16;
+      if ((lane & 15) == 0) own_slots[kRows + tid / 16] = in_order ? (first << 5 | __builtin_popcount(some)) : -1;
     }
   }
-  if constexpr (STEP) {
+  if constexpr (SHORT > 0) {
+    // The wave's 32 rows of q and of k, as below but 32 at a time: the rows of q pass
+    // through the wave's own K tile, which then takes those of k.
+#pragma unroll
+    for (int f = 0; f < 8; ++f) qf[f].u = u32x4{0, 0, 0, 0};
+    if (wq0 < len) {
+      const int c = lane & 7, r8 = lane >> 3;
+      u32x4 qlo[4], qhi[4], klo[4], khi[4];
+      uint16_t *qp[4], *kp[4];
+      int64_t pos[4];
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int64_t row = seq_begin + min(wq0 + 8 * it + r8, len - 1);
+        pos[it] = S.positions[row];
+        qp[it] = const_cast<uint16_t *>(I.q) + row * I.q_stride + hq * D + 8 * c;
+        kp[it] = const_cast<uint16_t *>(I.k) + row * I.kv_stride + hk * D + 8 * c;
+        qlo[it] = *reinterpret_cast<const u32x4 *>(qp[it]);
+        qhi[it] = *reinterpret_cast<const u32x4 *>(qp[it] + D / 2);
+        klo[it] = *reinterpret_cast<const u32x4 *>(kp[it]);
+        khi[it] = *reinterpret_cast<const u32x4 *>(kp[it] + D / 2);
+      }
+      uint16_t *const stage = smem + wave * kTileElems;
+      auto rotate = [&](u32x4 &lo, u32x4 &hi, const float (&cs)[8], const float (&sn)[8], int r) {
+        const uint4 x = make_uint4(lo.x, lo.y, lo.z, lo.w), y = make_uint4(hi.x, hi.y, hi.z, hi.w);
+        const uint4 xr = rotate_chunk<T>(x, y, cs, sn, false), yr = rotate_chunk<T>(y, x, cs, sn, true);
+        lo = u32x4{xr.x, xr.y, xr.z, xr.w};
+        hi = u32x4{yr.x, yr.y, yr.z, yr.w};
+      };
+      auto to_stage = [&](const u32x4 (&lo)[4], const u32x4 (&hi)[4]) {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const int r = 8 * it + r8;
+          *reinterpret_cast<u32x4 *>(stage + r * D + 8 * (c ^ swz(r))) = lo[it];
+          *reinterpret_cast<u32x4 *>(stage + r * D + 8 * ((c + 8) ^ swz(r))) = hi[it];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      };
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int64_t p = pos[it] < 0 ? 0 : (pos[it] >= S.max_position ? S.max_position - 1 : pos[it]);
+        const u32x4 *row = reinterpret_cast<const u32x4 *>(S.cos_sin + p * D + 8 * c);
+        const u32x4 c0 = row[0], c1 = row[1], s0 = row[D / 8], s1 = row[D / 8 + 1];
+        float cs[8], sn[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          cs[e] = __uint_as_float(e < 4 ? c0[e] : c1[e & 3]);
+          sn[e] = __uint_as_float(e < 4 ? s0[e] : s1[e & 3]);
+        }
+        rotate(qlo[it], qhi[it], cs, sn, 8 * it + r8);
+        rotate(klo[it], khi[it], cs, sn, 8 * it + r8);
+      }
+      to_stage(qlo, qhi);
+      if (my_q < len) {
+#pragma unroll
+        for (int f = 0; f < 8; ++f)
+          qf[f].u = *reinterpret_cast<const u32x4 *>(stage + qcol * D + 8 * ((2 * f + half) ^ swz(qcol)));
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      to_stage(klo, khi);
+      // (every load of this wave has landed before its stores go out: nothing waits
+      // for the stores)
+      __builtin_amdgcn_s_waitcnt(0x0070);
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        *reinterpret_cast<u32x4 *>(qp[it]) = qlo[it];
+        *reinterpret_cast<u32x4 *>(qp[it] + D / 2) = qhi[it];
+        *reinterpret_cast<u32x4 *>(kp[it]) = klo[it];
+        *reinterpret_cast<u32x4 *>(kp[it] + D / 2) = khi[it];
+      }
+    } else {
+      __builtin_amdgcn_s_waitcnt(0x0070);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  if constexpr (STEP && SHORT == 0) {
     // Rotation of the wave's 32 query rows: a lane takes the chunks c and c + 8
     // (the two halves of the same pairs) of one row, 8 rows at a time, so that
     // rows, table and the write-back go as whole lines, and the fragments come
@@ -541,26 +659,28 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
   }
   bool stores_counted = false;             // the previous tile's pool stores: exactly four, behind this tile's loads
   // (the compiler's own loads are behind it: a wait for them would be one for the tiles)
-  __builtin_amdgcn_s_waitcnt(0x0070);
+  if constexpr (SHORT == 0) __builtin_amdgcn_s_waitcnt(0x0070);
   auto tile = [&](int t, auto buffer) {
     constexpr int cur = decltype(buffer)::value;
     const int k0 = t * kBN;
-    // This wave's part of tile t has landed; after the barrier all of it has,
-    // and everybody is done with the other buffer.  (The barrier by itself:
-    // __syncthreads() would wait for the pool stores as well.)
-    if (STEP && stores_counted) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    if constexpr (SHORT == 0) {
+      // This wave's part of tile t has landed; after the barrier all of it has,
+      // and everybody is done with the other buffer.  (The barrier by itself:
+      // __syncthreads() would wait for the pool stores as well.)
+      if (STEP && stores_counted) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
 #ifdef MUX_TRACE
     if (t == 0) tr_first = __builtin_amdgcn_s_memrealtime();
 #endif
     // A workgroup's own rows are its last four tiles: their K and V go to the pool
     // behind the tile's math.
     const bool to_pool = STEP && writes_pool && k0 >= q0;
-    if (t + 1 < n_tiles) dma_tile(t + 1, cur ^ 1);
+    if (SHORT == 0 && t + 1 < n_tiles) dma_tile(t + 1, cur ^ 1);
     const uint16_t *const Kt = smem + cur * kTileElems;           // this tile's K
-    const uint16_t *const Vr = smem + (2 + cur) * kTileElems;     // this tile's V (row-major)
+    const uint16_t *const Vr = smem + (NBUF + cur) * kTileElems;     // this tile's V (row-major)
     // (nothing to compute where every key of the tile is in this wave's future, or
     // all of the wave's rows are past the prompt's end)
     if (k0 <= wq0 + 31 && wq0 < len) {
@@ -711,27 +831,43 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
       if (to_pool) {
 #pragma unroll 1
         for (int r = 0; r < kBN; r += 16) {
-          const uint32_t slots_at = smem_at + 8 * kTileElems + 8 * (k0 - q0 + r);
-          int64_t base;
+          const uint32_t slots_at = smem_at + 4 * NBUF * kTileElems + 8 * (k0 - q0 + r);
+          int64_t run;
           asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)"
-                       : "=&v"(base)
-                       : "v"(smem_at + 8 * kTileElems + 8 * (kBM + (k0 - q0 + r) / 16))
+                       : "=&v"(run)
+                       : "v"(smem_at + 4 * NBUF * kTileElems + 8 * (kRows + (k0 - q0 + r) / 16))
                        : "memory");
-          const uint32_t base_lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base));
-          const uint32_t base_hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(base >> 32));
-          base = static_cast<int64_t>((static_cast<uint64_t>(base_hi) << 32) | base_lo);
-          if (base >= 0)
-            write_block_to_pool(smem_at + 2 * (cur * kTileElems + r * D), smem_at + 2 * ((2 + cur) * kTileElems + r * D), writer,
-                                base, S);
-          else
-            stores_counted &= write_tokens_to_pool(Kt, Vr, r, slots_at, wave, lane, S);
+          const uint32_t run_lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(run));
+          const uint32_t run_hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(run >> 32));
+          run = static_cast<int64_t>((static_cast<uint64_t>(run_hi) << 32) | run_lo);
+          const uint32_t kt = smem_at + 2 * (cur * kTileElems + r * D), vt = kt + 2 * NBUF * kTileElems;
+          if constexpr (SHORT == 0) {
+            if (run >= 0) stores_counted &= write_block_to_pool(kt, vt, writer, run >> 5, static_cast<int>(run & 31), lane, S);
+            else stores_counted &= write_tokens_to_pool(Kt, Vr, r, slots_at, wave, lane, S);
+          } else {
+            for (int part = wave; part < 4; part += W) {      // (what the four waves of the other forms do)
+              if (run >= 0)
+                write_block_to_pool(kt, vt, BlockWriter(part, lane, S.block_size), run >> 5, static_cast<int>(run & 31), lane, S);
+              else write_tokens_to_pool(Kt, Vr, r, slots_at, part, lane, S);
+            }
+          }
         }
       }
     }
   };
-  for (int t = 0; t < n_tiles; t += 2) {
-    tile(t, std::integral_constant<int, 0>{});
-    if (t + 1 < n_tiles) tile(t + 1, std::integral_constant<int, 1>{});
+  if constexpr (SHORT > 0) {
+    tile(0, std::integral_constant<int, 0>{});
+    if constexpr (W > 1)
+      if (n_tiles > 1) tile(1, std::integral_constant<int, 1>{});
+    if constexpr (W > 2) {
+      if (n_tiles > 2) tile(2, std::integral_constant<int, 2>{});
+      if (n_tiles > 3) tile(3, std::integral_constant<int, 3>{});
+    }
+  } else {
+    for (int t = 0; t < n_tiles; t += 2) {
+      tile(t, std::integral_constant<int, 0>{});
+      if (t + 1 < n_tiles) tile(t + 1, std::integral_constant<int, 1>{});
+    }
   }
 
 #ifdef MUX_TRACE
@@ -745,8 +881,11 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
     // lane, four rows per instruction) instead of 8-byte pieces of 32 rows: the
     // tile buffers are free once every wave has left the loop.
     constexpr int kORow = D + 8;         // 272-byte rows
-    static_assert(4 * 32 * kORow <= kSmemElems, "output staging fits the tile buffers");
-    __syncthreads();
+    static_assert(W * 32 * kORow <= kSmemElems, "output staging fits the tile buffers");
+    // (the barrier by itself, as in the loop: nothing waits for the pool stores)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     uint16_t *stage = smem + wave * 32 * kORow;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
@@ -795,6 +934,10 @@ __global__ __launch_bounds__(256, 3) void prefill_causal_kernel(const PrefillPar
 template <typename T>
 __global__ __launch_bounds__(256, 3) void prefill_step_kernel(const PrefillParams P, const PrefillStep S) {
   prefill_body<T, true>(P, S);
+}
+template <typename T, int W>
+__global__ __launch_bounds__(64 * W, 2) void prefill_short_step_kernel(const PrefillParams P, const PrefillStep S) {
+  prefill_body<T, true, W>(P, S);
 }
 
 }  // namespace mux
@@ -848,7 +991,17 @@ PrefillItemDev device_item(const MuxPrefillItem &it) {
 
 hipError_t launch_prefill(const PrefillParams &P, const PrefillStep *S, int64_t n_wg, int32_t dtype, hipStream_t st) {
   const dim3 grid(static_cast<uint32_t>(n_wg));
-  if (S != nullptr) {
+  if (S != nullptr && S->short_waves > 0) {
+#define MUX_PF_SHORT(W)                                                                                                  \
+  do {                                                                                                                   \
+    if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_short_step_kernel<F16, W>), grid, dim3(64 * W), 0, st, P, *S); \
+    else hipLaunchKernelGGL((prefill_short_step_kernel<BF16, W>), grid, dim3(64 * W), 0, st, P, *S);                     \
+  } while (0)
+    if (S->short_waves == 1) MUX_PF_SHORT(1);
+    else if (S->short_waves == 2) MUX_PF_SHORT(2);
+    else MUX_PF_SHORT(4);
+#undef MUX_PF_SHORT
+  } else if (S != nullptr) {
     if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_step_kernel<F16>), grid, dim3(256), 0, st, P, *S);
     else hipLaunchKernelGGL((prefill_step_kernel<BF16>), grid, dim3(256), 0, st, P, *S);
   } else if (dtype == MUXA_DTYPE_F16) hipLaunchKernelGGL((prefill_causal_kernel<F16>), grid, dim3(256), 0, st, P);
@@ -1016,9 +1169,6 @@ extern "C" int32_t mux_rope_prefill_and_cache(const MuxPrefillItem *attn, const 
   if (tokens != w.num_tokens) return MUXA_EINVAL;
   if (tokens == 0) return MUXA_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const hipError_t e = launch_rotary_k(w.positions, static_cast<uint16_t *>(w.k), w.kv_row_stride, w.cos_sin,
-                                       w.max_position, w.num_tokens, w.num_kv_heads, dtype, st);
-  if (e != hipSuccess) return hip_fail(e);
   PrefillStep S = {};
   S.positions = w.positions;
   S.cos_sin = w.cos_sin;
@@ -1029,6 +1179,12 @@ extern "C" int32_t mux_rope_prefill_and_cache(const MuxPrefillItem *attn, const 
   S.pool_slots = num_pool_blocks * block_size;
   S.max_position = w.max_position;
   S.block_size = block_size;
+  S.short_waves = prompt_step_short_waves(it.prompt_lens_host, it.num_prompts, it.num_q_heads, it.num_kv_heads);
+  if (S.short_waves == 0) {
+    const hipError_t e = launch_rotary_k(w.positions, static_cast<uint16_t *>(w.k), w.kv_row_stride, w.cos_sin,
+                                         w.max_position, w.num_tokens, w.num_kv_heads, dtype, st);
+    if (e != hipSuccess) return hip_fail(e);
+  }
   if (launch_compact(&it, 1, &S, dtype, st, &rc)) return rc;
   return launch_dense(it, nullptr, &S, dtype, st);
 }

@@ -1,0 +1,40 @@
+// Which prompt steps are one launch (prefill.hip's short form): the rule, for the
+// library that launches it and for the operator that chooses between the forms.
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace mux {
+
+// The waves per workgroup of the launch (one per 32 tokens of the longest prompt), or
+// 0 where k is rotated in a launch of its own.
+// The short form needs a (prompt, head) to fit one workgroup.  Four waves per
+// workgroup where the launch does not fill the chip (two such workgroups per compute
+// unit), else as many as the longest prompt needs - unless most prompts would leave
+// most of them idle.  f16, us, two launches (rotation and cache write, attention) /
+// rotation of k and the step form / the short form with 1, 2 or 4 waves:
+//   32 heads, one prompt of 45 tokens 8.9 / 12.0 / - 10.3 9.0, 16 of 30 16.2 / 14.7 /
+//   10.5 - 10.0, 16 of 100 32.0 / 29.9 / - - 21.0, 8 of 128 (40 heads) 26 / 26.7 / - - 18.5;
+//   1 wave: 64 of 16 (52 heads) 37.8 / 41.1 / 29.9, 128 of 6 34.5 / 46.3 / 29.5, 200 of 30 110 /
+//   99 / 75, 2000 of 1 462 / 540 / 352;
+//   2 waves: 64 of 45 51.3 / 48.3 / 41.4, 64 of 64 61.8 / 54.5 / 47.5; 60 and 127 of 6 36.9 / 47.7 /
+//   41.6, 32 of 60 and 96 of 6 54.6 / 58.2 / 49.0;
+//   4 waves: 64 of 128 131 / 101 / 90, 200 of 100 376 / 317 / 285; 128 and 127 of 20 54.6 / 52.1 /
+//   58.0, 128 and 127 of 40 82.8 / 77 / 79.4, 32 of 100 and 32 of 30 (40 heads) 80 / 69 / 64.
+inline int32_t prompt_step_short_waves(const int32_t *prompt_lens_host, int32_t num_prompts, int32_t num_q_heads,
+                                       int32_t num_kv_heads) {
+  if (!prompt_lens_host || num_prompts <= 0 || num_q_heads != num_kv_heads) return 0;
+  int32_t longest = 0;
+  int64_t tokens = 0;
+  for (int32_t p = 0; p < num_prompts; ++p) {
+    longest = std::max(longest, prompt_lens_host[p]);
+    tokens += prompt_lens_host[p];
+  }
+  if (longest > 128) return 0;
+  if (static_cast<int64_t>(num_prompts) * num_kv_heads <= 512) return 4;
+  if (longest <= 32) return 1;
+  if (longest <= 64) return tokens >= int64_t{16} * num_prompts ? 2 : 0;
+  return tokens >= int64_t{45} * num_prompts ? 4 : 0;
+}
+
+}  // namespace mux

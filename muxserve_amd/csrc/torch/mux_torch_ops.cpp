@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "../prompt_step.h"
 #include "muxserve_attn_step.h"
 
 namespace {
@@ -537,9 +538,10 @@ std::tuple<at::Tensor, int64_t> decode_layer(const at::Tensor &positions, at::Te
   return {out, 0};
 }
 
-// Prompts: rotary embedding, causal attention, cache write.  step: with the
-// attention kernel doing all but the rotation of k, else rotation and cache write
-// in one launch and the attention behind it.  Undefined with nothing launched: rows
+// Prompts: rotary embedding, causal attention, cache write.  step, or prompts short
+// enough for the one launch that does it all: with the attention kernel doing all but
+// the rotation of k, else rotation and cache write in one launch and the attention
+// behind it.  Undefined with nothing launched: rows
 // of another alignment.
 at::Tensor prompt_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k, const at::Tensor &v,
                         const at::Tensor &cos_sin, at::Tensor k_pool, at::Tensor v_pool,
@@ -547,6 +549,11 @@ at::Tensor prompt_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k,
                         at::IntArrayRef prompt_lens, double scale, bool step) {
   if (!rows_of_16_bytes(q) || !rows_of_16_bytes(k) || !rows_of_16_bytes(v)) return at::Tensor();
   at::Tensor out = at::empty(q.sizes(), q.options());
+  if (!step && q.size(1) == k.size(1)) {
+    std::vector<int32_t> lens(prompt_lens.begin(), prompt_lens.end());
+    const int32_t heads = static_cast<int32_t>(q.size(1) / kHead);
+    step = mux::prompt_step_short_waves(lens.data(), static_cast<int32_t>(lens.size()), heads, heads) > 0;
+  }
   if (step) {
     rope_prefill_and_cache(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,
                            prompt_lens, scale);

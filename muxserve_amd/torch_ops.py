@@ -129,7 +129,8 @@ def decode_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, bloc
 def prompt_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer: int, cu_seqlens, prompt_lens,
                  scale: float, step: bool):
     """The prompt step of a layer in one operator: the attention output, or None
-    where the rows of q, k and v do not allow it."""
+    where the rows of q, k and v do not allow it.  step: see attention.prompt_step_pays;
+    prompts that fit one launch (csrc/prompt_step.h) take it either way."""
     return load().prompt_layer(positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,
                                prompt_lens, scale, step)
 

@@ -318,6 +318,54 @@ def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many)
         assert torch.equal(a, b), f"{what} differ between the step operator and the three kernels"
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lens,H,bs", [
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16), ([45], 2, 8),                          # few: four waves
+    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16), ([1] * 520 + [9] * 7, 1, 32),           # one wave
+    ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16), ([64, 17, 47] * 30, 7, 8),                # two
+    ([128, 65, 100, 97, 31, 127] * 12, 8, 32), ([96, 113, 128] * 30, 6, 16)])            # four, many
+def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs):
+    """Steps of prompts of at most 128 tokens (one launch, workgroups of 1, 2 or 4
+    waves): q, k, both pools and the outputs bitwise as from rotary, cache write and
+    attention in turn; with tokens without a slot, one outside the pool and a prompt
+    whose slots are scattered token by token."""
+    print(f"[case] short prompts {dtype} {len(lens)} prompts up to {max(lens)} H={H} bs={bs}", flush=True)
+    from muxserve_amd import torch_ops, workloads
+    from muxserve_amd.attention import build_cos_sin_cache
+    rng = np.random.Generator(np.random.PCG64(len(lens) + bs))
+    T = sum(lens)
+    N = sum((n + bs - 1) // bs for n in lens) * H + 3
+    slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), H, bs, rng.permutation(N))
+    first = T - lens[-1]
+    slots[first:, 0, 0] = slots[first + rng.permutation(lens[-1]), 0, 0]
+    slots[T // 2, 0, 0] = -1
+    slots[T // 3, 0, -1] = N * bs
+    dslots = torch.from_numpy(slots).to(DEV)
+    pad = (T + 7) // 8 * 8
+    qkv = torch.randn((pad, 3 * H * D), generator=torch.Generator().manual_seed(T)).to(dtype).to(DEV)
+    positions = torch.from_numpy(rng.integers(-3, 2060, size=pad)).to(DEV)
+    cos_sin = build_cos_sin_cache(D, 2048, 10000.0, DEV)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=DEV)
+    results = []
+    for fused in (False, True):
+        x = qkv.clone()
+        q, k, v = x.split([H * D] * 3, dim=-1)
+        kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=dtype)
+        kp.fill_(3)
+        vp.fill_(5)
+        out = torch.zeros((pad, H * D), dtype=dtype, device=DEV)
+        if fused:
+            torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, dslots, 0, cu, lens, D ** -0.5)
+        else:
+            ops.rotary_neox(positions, q, k, cos_sin, num_tokens=T)
+            ops.reshape_and_cache(k, v, kp, vp, dslots, layer=0, num_tokens=T)
+            ops.prefill_causal(out[:T], q[:T], k[:T], v[:T], cu, max(lens), D ** -0.5, H, prompt_lens=lens)
+        torch.cuda.synchronize()
+        results.append([t.cpu().view(torch.int16) for t in (x, kp, vp, out)])
+    for a, b, what in zip(*results, ("qkv rows", "k pool", "v pool", "outputs")):
+        assert torch.equal(a, b), f"{what} differ between the one launch and the three kernels"
+
+
 @pytest.mark.parametrize("bs,off", [(16, 0), (16, 8), (16, 5), (32, 0), (32, 16), (32, 8), (8, 0)])
 def test_prompt_step_pool_writes_of_runs_that_start_anywhere_in_a_block(bs, off):
     """The step operator writes 16 tokens with two stores where they are 16 slots in

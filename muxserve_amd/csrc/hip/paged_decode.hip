@@ -32,7 +32,8 @@
 // Several models (different head counts, tables, q/out tensors) are covered by
 // one grid: the kernel argument carries up to MUXA_MAX_DECODE_ITEMS item
 // descriptors.
-#include "mux_common.h"
+#include "../decode_step.h"
+#include "cache_write.h"
 
 #include <algorithm>
 #include <mutex>
@@ -1196,6 +1197,144 @@ __global__ __launch_bounds__(64 * NW, 3) void paged_decode_gqa_sweep_kernel(cons
 
 // Zero-fills the arrival counters (a kernel rather than a memset node so the
 // call can be captured into a graph).
+// ---------------------------------------------------------------------------
+// A decode step of ONE sequence with as many kv heads as query heads and a short
+// context, in one launch: rotation of its q and k rows in place, the new token's K and
+// V to the pool, attention.  Bound by latencies and launches.  us, two launches / one,
+// in a graph: 32 heads, 1 token 8.1 / 5.5, 97 8.4 / 5.8, 256 9.2 / 5.7, 512 (eight waves)
+// 11.5 / 7.5; 64 heads, 512 12.1 / 8.8; whole call at 97 tokens, bound by the host, 14.1 /
+// 10.2.
+//
+// One workgroup per head.  Nobody waits for the pool writes: every wave rotates the
+// head's rows itself and puts the new token into the tile it loaded, wherever its
+// table names the block of the head's slot (as the block belongs to this head alone:
+// the step writes to it, so another one's writes would collide there).  The rows go
+// out behind the workgroup's barrier, when all its waves have read them.
+// Several sequences may share blocks (rows that are successive tokens of one
+// sequence), and a longer context needs several workgroups: those keep two launches.
+struct SingleStepParams {
+  DecodeItemDev it;
+  uint16_t *q, *k;
+  const uint16_t *v;
+  const int64_t *positions;
+  const float *cos_sin;
+  const int64_t *slots;            // [Hkv] of the layer
+  uint16_t *k_pool, *v_pool;
+  int64_t pool_slots;
+  int32_t max_position, last_block;
+};
+
+template <typename T, int BS, int NW>
+__global__ __launch_bounds__(64 * NW) void decode_single_step_kernel(const SingleStepParams S) {
+  using Geo = Geometry<BS>;
+  constexpr int D = kHeadSize;
+  __shared__ DecodeSmem<1, NW> sm;
+  __shared__ __attribute__((aligned(16))) uint16_t row_lds[NW][2][D];       // rotated k row, v row
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x;
+  const DecodeItemDev I = S.it;
+  const int ctx = min(max(I.ctx[0], 0), I.max_ctx);
+  const int tb0 = wave * 64;
+  if (wave > 0 && tb0 >= ctx) return;
+  const int n_active = max(1, min(NW, (ctx + 63) / 64));
+
+  const int64_t pos = S.positions[0];
+  int64_t slot = S.slots[h];
+  if (slot < 0 || slot >= S.pool_slots) slot = -1;
+  const int slot_block = slot < 0 ? -1 : static_cast<int>(slot / BS), slot_off = static_cast<int>(slot & (BS - 1));
+  const int32_t *trow = I.tables + static_cast<int64_t>(h) * I.max_blocks;
+  const int id = load_block_id<BS>(trow, tb0, ctx, lane, S.last_block);
+
+  // Rows: lane c of every eight takes chunks c and c + 8 (the halves of the same pairs).
+  const int c = lane & 7;
+  uint4 *const qrow = reinterpret_cast<uint4 *>(S.q + h * D) + c, *const krow = reinterpret_cast<uint4 *>(S.k + h * D) + c;
+  const uint4 q0 = qrow[0], q1 = qrow[8], k0 = krow[0], k1 = krow[8];
+  const uint32_t vpair = reinterpret_cast<const uint32_t *>(S.v + h * D)[lane];
+  const int64_t p = pos < 0 ? 0 : (pos >= S.max_position ? S.max_position - 1 : pos);
+  const float4 *const table = reinterpret_cast<const float4 *>(S.cos_sin + p * D + 8 * c);
+  float cs[8], sn[8];
+  {
+    const float4 a = table[0], b = table[1], e = table[D / 8], f = table[D / 8 + 1];
+    cs[0] = a.x, cs[1] = a.y, cs[2] = a.z, cs[3] = a.w, cs[4] = b.x, cs[5] = b.y, cs[6] = b.z, cs[7] = b.w;
+    sn[0] = e.x, sn[1] = e.y, sn[2] = e.z, sn[3] = e.w, sn[4] = f.x, sn[5] = f.y, sn[6] = f.z, sn[7] = f.w;
+  }
+  const uint4 *kpool = reinterpret_cast<const uint4 *>(S.k_pool);
+  const uint4 *vpool = reinterpret_cast<const uint4 *>(S.v_pool);
+  uint4 kreg[16];
+  uint4 vreg[Geo::BPT][Geo::VI];
+  issue_tile_loads<BS>(kreg, vreg, kpool, vpool, id, tb0, ctx, lane);
+
+  const uint4 qx = rotate_chunk<T>(q0, q1, cs, sn, false), qy = rotate_chunk<T>(q1, q0, cs, sn, true);
+  const uint4 kx = rotate_chunk<T>(k0, k1, cs, sn, false), ky = rotate_chunk<T>(k1, k0, cs, sn, true);
+  uint16_t(*const rows)[D] = row_lds[wave];
+  if (lane < 8) {
+    reinterpret_cast<uint4 *>(rows[0])[c] = kx;
+    reinterpret_cast<uint4 *>(rows[0])[c + 8] = ky;
+  }
+  reinterpret_cast<uint32_t *>(rows[1])[lane] = vpair;
+  wave_lds_sync();
+  uint32_t q_s[64];
+#pragma unroll
+  for (int i = 0; i < 64; ++i) {
+    const uint4 &x = i < 32 ? qx : qy;
+    const uint32_t w = (i & 3) == 0 ? x.x : (i & 3) == 1 ? x.y : (i & 3) == 2 ? x.z : x.w;
+    q_s[i] = __builtin_amdgcn_readlane(w, (i >> 2) & 7);
+  }
+
+  float m[1] = {-INFINITY}, l[1] = {0.f}, acc[1][Geo::VI];
+#pragma unroll
+  for (int j = 0; j < Geo::VI; ++j) acc[0][j] = 0.f;
+  if (tb0 < ctx) {
+    // The new token where its block is: a lane's token of K, one element of V.
+    if (slot_block >= 0) {
+      const int tok = tb0 + lane;
+      if (tok < ctx && id == slot_block && (lane & (BS - 1)) == slot_off) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) kreg[j] = reinterpret_cast<const uint4 *>(rows[0])[j];
+      }
+      const int part = lane % Geo::PARTS;
+#pragma unroll
+      for (int b = 0; b < Geo::BPT; ++b) {
+        if (tb0 + b * BS >= ctx || __builtin_amdgcn_readlane(id, b * BS) != slot_block) continue;
+        if (part != slot_off / 8) continue;
+        const int e = slot_off & 7;
+#pragma unroll
+        for (int j = 0; j < Geo::VI; ++j) {
+          const uint32_t x = rows[1][j * (64 / Geo::PARTS) + lane / Geo::PARTS];
+          uint32_t *const w = reinterpret_cast<uint32_t *>(&vreg[b][j]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (i == (e >> 1)) w[i] = (e & 1) ? (w[i] & 0x0000ffffu) | (x << 16) : (w[i] & 0xffff0000u) | x;
+        }
+      }
+    }
+    consume_tile<T, BS, 1>(kreg, vreg, q_s, sm.q[wave], sm.p[wave], m, l, acc, I.scale_log2, tb0, ctx, lane);
+  }
+  stash_wave_partial<BS, 1>(m, l, acc, sm.x_acc[wave], sm.x_ml[wave], lane);
+  __syncthreads();
+  if (wave != 0) return;
+  if (lane < 8) {
+    qrow[0] = qx, qrow[8] = qy;
+    krow[0] = kx, krow[8] = ky;
+    if (slot >= 0) {
+      uint4 *const kp = reinterpret_cast<uint4 *>(S.k_pool) + static_cast<int64_t>(slot_block) * Geo::BLOCK_CHUNKS + slot_off;
+      kp[c * BS] = kx;
+      kp[(c + 8) * BS] = ky;
+    }
+  }
+  if (slot >= 0) {
+    uint16_t *const vp = S.v_pool + static_cast<int64_t>(slot_block) * (D * BS) + slot_off;
+    vp[(2 * lane) * BS] = static_cast<uint16_t>(vpair);
+    vp[(2 * lane + 1) * BS] = static_cast<uint16_t>(vpair >> 16);
+  }
+  if (ctx == 0) return;
+  Unit u = {};
+  u.wh = h;
+  u.n_splits = 1;
+  merge_and_write<T, 1, NW>(I, u, 0, sm.x_acc, sm.x_ml, n_active, lane);
+}
+
 __global__ void fill_zero_kernel(int32_t *p, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
@@ -1435,6 +1574,67 @@ int32_t validate_item(const MuxDecodeItem &it, int block_size) {
 
 }  // namespace
 }  // namespace mux
+
+// The step of one short sequence in one launch; 0: not one (the caller takes the two
+// launches, with their refusals).  Up to 512 tokens, one round of the workgroup's waves.
+int32_t mux::single_row_step(const MuxDecodeItem &d, const MuxCacheWriteItem &w, void *k_pool, void *v_pool,
+                             int64_t num_pool_blocks, int32_t block_size, int32_t dtype, void *stream, int32_t *taken) {
+  using namespace mux;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  *taken = 0;
+  if (d.num_seqs != 1 || w.num_tokens != 1 || d.num_q_heads != d.num_kv_heads || d.max_context_len < 1 ||
+      d.max_context_len > 512 || d.max_blocks < 1 || w.rotary_dim != kHeadSize || w.max_position <= 0)
+    return MUXA_OK;
+  if (validate_item(d, block_size) != MUXA_OK || !w.positions || !w.cos_sin || !w.q || w.q != d.q ||
+      check_cache_write(w.k, w.v, w.kv_row_stride, k_pool, v_pool, num_pool_blocks, w.slot_mapping, w.layer, w.num_layers, 1,
+                        w.num_kv_heads, kHeadSize, block_size, dtype) != MUXA_OK ||
+      w.num_q_heads != d.num_q_heads || w.num_kv_heads != d.num_kv_heads || num_pool_blocks > 0x7fffffff ||
+      (reinterpret_cast<uintptr_t>(w.q) & 15u) || (reinterpret_cast<uintptr_t>(w.cos_sin) & 15u))
+    return MUXA_OK;
+  SingleStepParams S = {};
+  S.it.out = d.out;
+  S.it.out_stride = d.out_row_stride;
+  S.it.tables = d.block_tables + static_cast<int64_t>(d.layer) * d.num_kv_heads * d.max_blocks;
+  S.it.ctx = d.context_lens;
+  S.it.B = 1;
+  S.it.Hq = S.it.Hkv = d.num_q_heads;
+  S.it.ratio = 1;
+  S.it.max_blocks = d.max_blocks;
+  S.it.max_splits = 1;
+  S.it.max_ctx = d.max_context_len;
+  S.it.scale_log2 = d.scale * 1.4426950408889634f;
+  S.q = static_cast<uint16_t *>(w.q);
+  S.k = static_cast<uint16_t *>(w.k);
+  S.v = static_cast<const uint16_t *>(w.v);
+  S.positions = w.positions;
+  S.cos_sin = w.cos_sin;
+  S.slots = w.slot_mapping + static_cast<int64_t>(w.layer) * w.num_kv_heads;
+  S.k_pool = static_cast<uint16_t *>(k_pool);
+  S.v_pool = static_cast<uint16_t *>(v_pool);
+  S.pool_slots = num_pool_blocks * block_size;
+  S.max_position = w.max_position;
+  S.last_block = static_cast<int32_t>(num_pool_blocks - 1);
+  const dim3 grid(static_cast<uint32_t>(d.num_q_heads));
+#define MUX_SINGLE(TT, BS)                                                                                      \
+  do {                                                                                                          \
+    if (d.max_context_len <= 256)                                                                               \
+      hipLaunchKernelGGL((decode_single_step_kernel<TT, BS, 4>), grid, dim3(256), 0, st, S);                    \
+    else hipLaunchKernelGGL((decode_single_step_kernel<TT, BS, 8>), grid, dim3(512), 0, st, S);                 \
+  } while (0)
+#define MUX_SINGLE_T(TT)                   \
+  do {                                     \
+    if (block_size == 8) MUX_SINGLE(TT, 8); \
+    else if (block_size == 16) MUX_SINGLE(TT, 16); \
+    else MUX_SINGLE(TT, 32);               \
+  } while (0)
+  if (dtype == MUXA_DTYPE_F16) MUX_SINGLE_T(F16);
+  else MUX_SINGLE_T(BF16);
+#undef MUX_SINGLE_T
+#undef MUX_SINGLE
+  MUX_HIP_TRY(hipGetLastError());
+  *taken = 1;
+  return MUXA_OK;
+}
 
 extern "C" {
 

@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "../decode_step.h"
 #include "../prompt_step.h"
 #include "muxserve_attn_step.h"
 
@@ -515,6 +516,48 @@ bool rows_of_16_bytes(const at::Tensor &t) {
   return t.dim() == 2 && t.stride(0) % 8 == 0 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
 }
 
+// One sequence with a short context, as one launch; false where it is not that or the
+// tensors are not what the general path takes (which then says so).
+bool single_row_step(const at::Tensor &out, const at::Tensor &positions, const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
+                     const at::Tensor &cos_sin, const at::Tensor &k_pool, const at::Tensor &v_pool, const at::Tensor &slots,
+                     const at::Tensor &block_tables, const at::Tensor &context_lens, int64_t max_context_len, double scale,
+                     int64_t layer, const c10::optional<at::Tensor> &context_lens_host) {
+  if (context_lens.dim() != 1 || context_lens.size(0) != 1 || q.dim() != 2 || k.dim() != 2 || q.size(1) != k.size(1))
+    return false;
+  for (const at::Tensor *t : {&positions, &q, &k, &v, &cos_sin, &k_pool, &v_pool, &slots, &block_tables, &context_lens})
+    if (!t->is_cuda()) return false;
+  if (positions.scalar_type() != at::kLong || positions.dim() != 1 || !positions.is_contiguous() || positions.size(0) < 1 ||
+      cos_sin.scalar_type() != at::kFloat || cos_sin.dim() != 2 || !cos_sin.is_contiguous() ||
+      slots.scalar_type() != at::kLong || slots.dim() != 3 || !slots.is_contiguous() || slots.size(0) < 1 ||
+      k.sizes() != v.sizes() || q.size(0) < 1 || k.size(0) < 1 || k.size(1) != slots.size(2) * kHead ||
+      k.scalar_type() != v.scalar_type() || k.scalar_type() != k_pool.scalar_type() || q.scalar_type() != k.scalar_type())
+    return false;
+  const int64_t bs = check_pools(k_pool, v_pool);
+  const MuxDecodeItem d = decode_item(out, q, block_tables, context_lens, max_context_len, scale, layer, 0, context_lens_host);
+  MuxCacheWriteItem w = {};
+  w.positions = positions.data_ptr<int64_t>();
+  w.q = q.data_ptr();
+  w.q_row_stride = rows(q, "q");
+  w.k = k.data_ptr();
+  w.v = v.data_ptr();
+  w.kv_row_stride = rows(k, "k");
+  if (rows(v, "v") != w.kv_row_stride) return false;
+  w.cos_sin = cos_sin.data_ptr<float>();
+  w.slot_mapping = slots.data_ptr<int64_t>();
+  w.max_position = static_cast<int32_t>(cos_sin.size(0));
+  w.rotary_dim = static_cast<int32_t>(cos_sin.size(1));
+  w.layer = static_cast<int32_t>(layer);
+  w.num_layers = static_cast<int32_t>(slots.size(1));
+  w.num_tokens = 1;
+  w.num_q_heads = static_cast<int32_t>(q.size(1) / kHead);
+  w.num_kv_heads = static_cast<int32_t>(slots.size(2));
+  int32_t taken = 0;
+  check(mux::single_row_step(d, w, k_pool.data_ptr(), v_pool.data_ptr(), k_pool.size(0), static_cast<int32_t>(bs),
+                             dtype_code(q), stream_of(q), &taken),
+        "single_row_step");
+  return taken != 0;
+}
+
 // Decode: rotary embedding and cache write of the new tokens, paged attention.
 // Returns (out, 0); or (undefined, bytes) with nothing launched: -1 for rows of
 // another alignment, else the workspace that the call needs.
@@ -528,6 +571,9 @@ std::tuple<at::Tensor, int64_t> decode_layer(const at::Tensor &positions, at::Te
                                              const c10::optional<at::Tensor> &context_lens_host) {
   if (!rows_of_16_bytes(q) || !rows_of_16_bytes(k) || !rows_of_16_bytes(v)) return {at::Tensor(), -1};
   at::Tensor out = at::empty(q.sizes(), q.options());
+  if (partition_size == 0 && single_row_step(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, block_tables,
+                                             context_lens, max_context_len, scale, layer, context_lens_host))
+    return {out, 0};
   const int64_t need =
       paged_decode_workspace_bytes(out, q, block_tables, context_lens, max_context_len, partition_size);
   const int64_t have = workspace.has_value() && workspace->defined() ? workspace->numel() : 0;

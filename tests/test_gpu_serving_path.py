@@ -559,6 +559,62 @@ def test_decode_layer_operator_equals_the_general_path(dtype):
             assert torch.equal(a, b), what
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("n", [1, 8, 17, 63, 64, 65, 97, 256, 257, 400, 512, 513])
+def test_decode_of_one_sequence_in_one_launch_equals_the_general_path(dtype, bs, n):
+    """One sequence with as many kv heads as query heads (one launch up to 512 tokens)
+    against rotation, cache write and attention in turn: q, k and the pools bitwise, the
+    output bitwise while the general path has one workgroup per head (256 tokens) and
+    within the rounding of the stored value beyond.  The new token in its place; no slot;
+    a slot outside the pool, in an earlier block of the table, in a block that the table
+    names twice, and in none of its blocks."""
+    print(f"[case] decode of one sequence {dtype} bs={bs} n={n}", flush=True)
+    from muxserve_amd.attention import InputMetadata
+    H, nb = 8, -(-n // bs)
+    g = torch.Generator().manual_seed(n + bs)
+    N = H * (nb + 2)
+    tables = torch.randperm(N, generator=g).to(torch.int32)
+    spare = tables[H * nb:]
+    tables = tables[:H * nb].reshape(1, 1, H, nb).clone()
+    slots = tables[0, 0, :, nb - 1].long() * bs + (n - 1) % bs
+    slots[1] = -1
+    slots[2] = N * bs
+    slots[3] = tables[0, 0, 3, 0].long() * bs + min(bs - 1, n - 1) // 2
+    tables[0, 0, 4, nb // 2] = tables[0, 0, 4, nb - 1]
+    slots[5] = spare[0].long() * bs + bs - 1
+    ctx = torch.tensor([n], dtype=torch.int32)
+    md = InputMetadata(prompt_lens=[], slot_mapping=slots[None, None].contiguous().to(DEV), context_lens=ctx.to(DEV),
+                       max_context_len=n, block_tables=tables.to(DEV), total_context_len=n, context_lens_host=ctx)
+    rows = torch.randn((8, 3 * H * D), generator=g).to(dtype)
+    kp0 = torch.randn((N, D // 8, bs, 8), generator=g).to(dtype)
+    vp0 = torch.randn((N, D, bs), generator=g).to(dtype)
+    positions = torch.tensor([n - 1] + [0] * 7, device=DEV)
+    results = []
+    for fused_max in (512, 0):
+        layer = PagedAttentionWithRoPE(H, D, D ** -0.5, max_position=2048, rotary_dim=D, num_kv_heads=H, layer_idx=0)
+        layer.fused_rope_max_tokens = fused_max
+        kp, vp, x = kp0.to(DEV), vp0.to(DEV), rows.to(DEV)
+        q, k, v = x.split([H * D] * 3, dim=-1)
+        out = layer(positions, q, k, v, kp, vp, md, None)
+        torch.cuda.synchronize()
+        results.append([t.cpu() for t in (x, kp, vp, out[:1])])
+    for a, b, what in zip(*results, ("q, k, v", "k pool", "v pool")):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), what
+    got, want = (r[3].float() for r in results)
+    # Beyond 256 tokens the waves hold other tokens, so their maxima differ, and f16
+    # probabilities, relative to them, round differently: 2^-11 of each weight on either
+    # side, at most 2^-10 max |v| in their mean.  bf16 keeps them in 32 bits (sums in
+    # another order).  Then the rounding of the stored value.
+    if n <= 256:
+        bound = torch.zeros_like(want)
+    elif dtype == torch.float16:
+        bound = want.abs() * 2.0 ** -10 + 2.0 ** -10 * float(vp0.abs().max())
+    else:
+        bound = want.abs() * 2.0 ** -7 + 1e-5
+    assert ((got - want).abs() <= bound).all(), (got - want).abs().max()
+
+
 @pytest.mark.parametrize("n", [40, 600])
 def test_prompt_step_with_unaligned_query_rows_is_refused(n):
     """The attention kernel takes 16-byte accesses to the query rows only; such a

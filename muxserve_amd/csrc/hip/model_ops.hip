@@ -3,10 +3,9 @@
 // 200-232).  Both are bound by HBM: every input element is read once and every
 // output element written once, in 16-byte pieces.
 //
-//   rms_norm      one wave per token row at a time: the row stays in registers
+//   rms_norm      one workgroup per token row at a time: the row stays in registers
 //                 between the sum of squares and the scaling, so x is read once
-//                 (with non-temporal loads: 19.5 instead of 26 us for 4096 rows
-//                 of 6656); the wave sum is a DPP reduction, no LDS, no barrier.
+//                 (with non-temporal loads), the weight once per workgroup.
 //                 out = T(x * rsqrt(mean(x^2) + eps)) * w, the product in T.
 //   silu_and_mul  one thread per 8 outputs: out = T(a / (1 + exp(-a))) * b for
 //                 x = [a | b], the product in T.
@@ -18,11 +17,10 @@ namespace mux {
 
 typedef uint32_t mo_u32x4 __attribute__((ext_vector_type(4)));
 
-#ifndef MUX_RMS_WAVES_PER_CU
-#define MUX_RMS_WAVES_PER_CU 8
-#endif
-constexpr int kRmsWavesPerCu = MUX_RMS_WAVES_PER_CU;
-
+// Workgroups per compute unit of rms_norm.  4096 rows of 6656 f16: 2, 3, 4, 6, 8 of them
+// 22.2, 20.8, 21.4, 21.6, 21.8 us, one workgroup per row 22.4; 2048 of 8192 14.2, 13.3, 14.2,
+// 14.6, 14.7, 14.7.
+constexpr int kRmsWgsPerCu = 3;
 
 template <typename T>
 __device__ __forceinline__ void unpack8(const mo_u32x4 v, float (&f)[8]) {
@@ -55,87 +53,98 @@ __device__ __forceinline__ mo_u32x4 pack8(const float (&f)[8]) {
   return mo_u32x4{w[0], w[1], w[2], w[3]};
 }
 
-// CPL = 16-byte chunks a lane keeps (a row has hidden / 8 chunks, lane l takes
-// chunks l, l + 64, ...).  A wave walks rows wave, wave + W, wave + 2 W, ... (W
-// waves in the grid) with the next row's loads issued before the current row is
-// reduced and stored, so that across the chip reads and writes overlap instead
-// of coming as one burst of each.  CPL = 0: rows of any length, x read twice.
-template <typename T, int CPL>
+// CPT = 16-byte chunks of a row that a thread keeps (thread t takes chunks t, t + 256,
+// ...).  A workgroup walks rows blockIdx, blockIdx + gridDim, ... with the next row's
+// loads issued before the current row is reduced and stored, so that across the chip
+// reads and writes overlap instead of coming as one burst of each.  CPT = 0: rows of any
+// length, x read twice.
+// us, a wave per row (2048 of them, otherwise the same) / a workgroup per row: 64 rows of
+// 8192 6.2 / 3.6, 1024 of 4096 6.6 / 5.9, 2048 of 5120 10.5 / 9.3, 16384 of 4096 53.5 / 49.7,
+// 4096 of 6656 20.4 / 20.8 by themselves, 85.1 / 84.0 with silu_and_mul behind them.  Non-
+// temporal stores make this kernel 6 - 19 % faster and the one that reads its output
+// slower by more (4096 of 6656 and a read 37 / 40 us).
+template <typename T, int CPT>
 __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t *__restrict__ out, int64_t out_stride,
                                                        const uint16_t *__restrict__ x, int64_t x_stride,
                                                        const uint16_t *__restrict__ weight, float eps, int hidden,
                                                        int num_rows) {
-  const int lane = threadIdx.x & 63;
-  const int first = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int step = gridDim.x * 4;
-  if (first >= num_rows) return;
-  const int nchunks = hidden >> 3;
+  __shared__ float part[2][4];             // the waves' sums, two rows
+  const int tid = threadIdx.x, nchunks = hidden >> 3;
+  const int step = gridDim.x;
   const mo_u32x4 *wr = reinterpret_cast<const mo_u32x4 *>(weight);
   const float inv_n = 1.0f / static_cast<float>(hidden);
-  if constexpr (CPL > 0) {
-    auto load_row = [&](mo_u32x4 (&v)[CPL], int row) {
+  // rsqrt(mean + eps) of a row from a thread's part of its sum of squares.  (The barrier
+  // by itself: __syncthreads() would wait for the previous row's stores.)
+  auto scale_of = [&](float ss, int buf) {
+    ss = wave_sum(ss);
+    if ((tid & 63) == 0) part[buf][tid >> 6] = ss;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    return rsqrtf((part[buf][0] + part[buf][1] + part[buf][2] + part[buf][3]) * inv_n + eps);
+  };
+  auto scaled = [&](const mo_u32x4 v, const mo_u32x4 w, float s) {
+    float f[8], g[8];
+    unpack8<T>(v, f);
+    unpack8<T>(w, g);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = round_to<T>(f[j] * s) * g[j];
+    return pack8<T>(f);
+  };
+  auto add_squares = [](const mo_u32x4 v, float ss) {
+    float f[8];
+    unpack8<T>(v, f);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(f[j], f[j], ss);
+    return ss;
+  };
+  if constexpr (CPT > 0) {
+    const mo_u32x4 zero = {0, 0, 0, 0};
+    auto load_row = [&](mo_u32x4 (&v)[CPT], int row) {
       const mo_u32x4 *xr = reinterpret_cast<const mo_u32x4 *>(x + row * x_stride);
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) {
-        const int c = lane + 64 * i;
-        v[i] = c < nchunks ? __builtin_nontemporal_load(&xr[c]) : mo_u32x4{0, 0, 0, 0};
+      for (int i = 0; i < CPT; ++i) {
+        const int c = tid + 256 * i;
+        v[i] = c < nchunks ? __builtin_nontemporal_load(&xr[c]) : zero;
       }
     };
-    auto finish_row = [&](const mo_u32x4 (&v)[CPL], int row) {
+    mo_u32x4 w[CPT];
+    auto finish_row = [&](const mo_u32x4 (&v)[CPT], int row, int buf) {
       float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) {
-        float f[8];
-        unpack8<T>(v[i], f);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(f[j], f[j], ss);
-      }
-      ss = wave_sum(ss);
-      const float s = rsqrtf(ss * inv_n + eps);
+      for (int i = 0; i < CPT; ++i) ss = add_squares(v[i], ss);
+      const float s = scale_of(ss, buf);
       mo_u32x4 *outr = reinterpret_cast<mo_u32x4 *>(out + row * out_stride);
 #pragma unroll
-      for (int i = 0; i < CPL; ++i) {
-        const int c = lane + 64 * i;
-        if (c < nchunks) {
-          float f[8], w[8];
-          unpack8<T>(v[i], f);
-          unpack8<T>(wr[c], w);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) f[j] = round_to<T>(f[j] * s) * w[j];
-          outr[c] = pack8<T>(f);
-        }
+      for (int i = 0; i < CPT; ++i) {
+        const int c = tid + 256 * i;
+        if (c < nchunks) outr[c] = scaled(v[i], w[i], s);
       }
     };
-    mo_u32x4 a[CPL], b[CPL];
-    load_row(a, first);
-    for (int row = first; row < num_rows; row += 2 * step) {
+    mo_u32x4 a[CPT], b[CPT];
+    int row = blockIdx.x;
+    load_row(a, row);
+#pragma unroll
+    for (int i = 0; i < CPT; ++i) {
+      const int c = tid + 256 * i;
+      w[i] = c < nchunks ? wr[c] : zero;
+    }
+    for (; row < num_rows; row += 2 * step) {
       if (row + step < num_rows) load_row(b, row + step);
-      finish_row(a, row);
+      finish_row(a, row, 0);
       if (row + step >= num_rows) break;
       if (row + 2 * step < num_rows) load_row(a, row + 2 * step);
-      finish_row(b, row + step);
+      finish_row(b, row + step, 1);
     }
   } else {
-    for (int row = first; row < num_rows; row += step) {
+    int buf = 0;
+    for (int row = blockIdx.x; row < num_rows; row += step, buf ^= 1) {
       const mo_u32x4 *xr = reinterpret_cast<const mo_u32x4 *>(x + row * x_stride);
       mo_u32x4 *outr = reinterpret_cast<mo_u32x4 *>(out + row * out_stride);
       float ss = 0.f;
-      for (int c = lane; c < nchunks; c += 64) {
-        float f[8];
-        unpack8<T>(xr[c], f);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(f[j], f[j], ss);
-      }
-      ss = wave_sum(ss);
-      const float s = rsqrtf(ss * inv_n + eps);
-      for (int c = lane; c < nchunks; c += 64) {
-        float f[8], w[8];
-        unpack8<T>(xr[c], f);
-        unpack8<T>(wr[c], w);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = round_to<T>(f[j] * s) * w[j];
-        outr[c] = pack8<T>(f);
-      }
+      for (int c = tid; c < nchunks; c += 256) ss = add_squares(xr[c], ss);
+      const float s = scale_of(ss, buf);
+      for (int c = tid; c < nchunks; c += 256) outr[c] = scaled(xr[c], wr[c], s);
     }
   }
 }
@@ -178,7 +187,7 @@ extern "C" int32_t mux_rms_norm(void *out, int64_t out_row_stride, const void *x
     return MUXA_EINVAL;
   if (num_tokens == 0) return MUXA_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // At most kRmsWavesPerCu waves per CU; rows beyond that are walked in sequence.
+  // At most kRmsWgsPerCu workgroups per CU; rows beyond that are walked in sequence.
   static const int cus = [] {                      // compute units of the current device, asked once
     int dev = 0, v = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
@@ -186,19 +195,19 @@ extern "C" int32_t mux_rms_norm(void *out, int64_t out_row_stride, const void *x
       return v;
     return 256;
   }();
-  const int max_wgs = cus * kRmsWavesPerCu / 4;
-  const dim3 grid(std::min((num_tokens + 3) / 4, max_wgs)), block(256);
+  const dim3 grid(std::min(num_tokens, cus * kRmsWgsPerCu)), block(256);
   uint16_t *o = static_cast<uint16_t *>(out);
   const uint16_t *xi = static_cast<const uint16_t *>(x), *w = static_cast<const uint16_t *>(weight);
   const int nchunks = hidden_size / 8;
-#define MUX_RMS_LAUNCH(TT, CPL)                                                                              \
-  hipLaunchKernelGGL((rms_norm_kernel<TT, CPL>), grid, block, 0, st, o, out_row_stride, xi, x_row_stride, w, \
+#define MUX_RMS_LAUNCH(TT, CPT)                                                                              \
+  hipLaunchKernelGGL((rms_norm_kernel<TT, CPT>), grid, block, 0, st, o, out_row_stride, xi, x_row_stride, w, \
                      eps, hidden_size, num_tokens)
 #define MUX_RMS_PICK(TT)                              \
   do {                                                \
-    if (nchunks <= 64 * 4) MUX_RMS_LAUNCH(TT, 4);     \
-    else if (nchunks <= 64 * 8) MUX_RMS_LAUNCH(TT, 8); \
-    else if (nchunks <= 64 * 16) MUX_RMS_LAUNCH(TT, 16); \
+    if (nchunks <= 256 * 1) MUX_RMS_LAUNCH(TT, 1);      \
+    else if (nchunks <= 256 * 2) MUX_RMS_LAUNCH(TT, 2); \
+    else if (nchunks <= 256 * 3) MUX_RMS_LAUNCH(TT, 3); \
+    else if (nchunks <= 256 * 4) MUX_RMS_LAUNCH(TT, 4); \
     else MUX_RMS_LAUNCH(TT, 0);                       \
   } while (0)
   if (dtype == MUXA_DTYPE_F16) MUX_RMS_PICK(F16);

@@ -65,6 +65,21 @@ def test_rms_norm(dtype, T, hidden):
     _close_in_ulps(got.cpu(), lo.rms_norm(x, w, 1e-5), dtype, "rms_norm", _normalised(x, 1e-5), w)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("T,hidden", [(768, 2048), (769, 2056), (1536, 4104), (1537, 6144), (2305, 6152), (3100, 8200)])
+def test_rms_norm_rows_beyond_the_grid(dtype, T, hidden):
+    """Three workgroups per compute unit walk the rows: as many rows as workgroups (256
+    compute units), one more, an odd and an even number of rounds, at the edges of the
+    chunks per thread."""
+    print(f"[case] rms_norm {dtype} T={T} hidden={hidden}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    x = (torch.randn((T, hidden), generator=g) * torch.rand((T, 1), generator=g) * 3).to(dtype)
+    w = (1 + 0.3 * torch.randn((hidden,), generator=g)).to(dtype)
+    got = ops.rms_norm(x.to(DEV), w.to(DEV), 1e-5)
+    torch.cuda.synchronize()
+    _close_in_ulps(got.cpu(), lo.rms_norm(x, w, 1e-5), dtype, "rms_norm", _normalised(x, 1e-5), w)
+
+
 def test_rms_norm_strided_rows_padding_rows_and_module():
     print("[case] rms_norm strided", flush=True)
     g = torch.Generator().manual_seed(5)

@@ -202,6 +202,10 @@ __device__ __forceinline__ void cache_write_window(
     }
   }
   __syncthreads();
+  // Token by itself (bit position j): no neighbour in the batch goes to the slot beside
+  // its own, as in a decode step (see the comment at rope_scatter_kernel).
+  auto alone = [&](int j) { return s_slot[j - 1] != s_slot[j] - 1 && s_slot[j + 1] != s_slot[j] + 1; };
+  static_assert(kBack >= 16, "a window's tokens have a neighbour on either side in s_slot");
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
     if (pass == 1 && !two_passes) break;
@@ -213,8 +217,8 @@ __device__ __forceinline__ void cache_write_window(
       // Element path for tokens that no run covers (a run starts at most 7 tokens back).
       const unsigned long long cover = in_win & (0xffull << (j > 7 ? j - 7 : 0)) & ~(~0ull << (j + 1));
       store16(&k_pool[(blk * (D / 8) + c) * block_size + o], *reinterpret_cast<const uint4 *>(&kt[j][c * 8]),
-              rows_complete);
-      if (cover == 0) {
+              rows_complete || (cover == 0 && alone(j)));
+      if (cover == 0 && !alone(j)) {
         uint16_t *vp = v_pool + (blk * D + c * 8) * block_size + o;
         const uint4 vx = *reinterpret_cast<const uint4 *>(&vt[j][c * 8]);
         const uint32_t w[4] = {vx.x, vx.y, vx.z, vx.w};
@@ -224,6 +228,19 @@ __device__ __forceinline__ void cache_write_window(
           vp[(2 * e + 1) * block_size] = static_cast<uint16_t>(w[e] >> 16);
         }
       }
+    }
+  }
+  // V of tokens by themselves: 32 threads per token, 32 neighbouring dims of the block
+  // per instruction, so that four lanes share a line.
+  if (n_runs == 0 || jb - ja > 8 * n_runs) {
+    for (int j = ja + static_cast<int>(threadIdx.x >> 5); j < jb; j += 8) {
+      const int64_t slot = s_slot[j];
+      const unsigned long long cover = in_win & (0xffull << (j > 7 ? j - 7 : 0)) & ~(~0ull << (j + 1));
+      if (slot < 0 || cover != 0 || !alone(j)) continue;
+      const int l = threadIdx.x & 31;
+      uint16_t *const vp = v_pool + ((slot >> bs_shift) * D + l) * block_size + (static_cast<int>(slot) & (block_size - 1));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) __builtin_nontemporal_store(vt[j][l + 32 * e], &vp[32 * e * block_size]);
     }
   }
   // Up to three runs per window; thread (c, i) stores dim 8c + i%8 of runs i/8, i/8 + 2.
@@ -308,8 +325,16 @@ __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
 // everything but the cos|sin row is requested at once: two memory latencies
 // against the window kernel's five.  No runs are looked for (a decode step has
 // none); a V store instruction covers 32 neighbouring dims of the block, four
-// lanes to a 128-byte line, where the window kernel's element path spreads 64
-// lanes over 64 lines.
+// lanes to a 128-byte line.
+//
+// A token by itself - no neighbour in the batch goes to the slot beside its own, as in
+// a decode step - is stored past the L2, here and in the window kernel: it leaves a few
+// bytes in each of 32 lines of V and 16 of K, and the attention behind it reads those
+// lines whole, from another XCD.  Left in the L2 they cost that launch more than the
+// write: us, write alone and with the attention, kept / past the L2: 56 tokens of three
+// models 6.1, 89.7 / 8.5, 82.7; 16 x 40 heads bf16 4.5, 34.4 / 4.9, 32.5; 256 x 32 heads (window
+// kernel) 14.3, 333 / 25, 299; 64 x 8 heads on 64 bf16 4.3, 239.5 / 4.8, 236.5.  Tokens in a run
+// (prompts) write the same lines again and keep the L2.
 template <typename T>
 __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWriteParams P) {
   constexpr int D = kHeadSize;
@@ -347,10 +372,13 @@ __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWrite
       kv ? I.k + static_cast<int64_t>(t) * I.row_stride + h * D
          : R.q + static_cast<int64_t>(t) * R.q_stride + (h * R.ratio + hq) * D);
   const uint32_t lo = x[l], hi = x[32 + l];
-  int64_t slot = -1;
+  int64_t slot = -1, before = -2, after = -2;
   uint16_t ve[4] = {0, 0, 0, 0};
   if (kv) {
-    slot = I.slots[static_cast<int64_t>(t) * I.slot_stride + h];
+    const int64_t *const sp = I.slots + static_cast<int64_t>(t) * I.slot_stride + h;
+    slot = *sp;
+    if (t > 0) before = *(sp - I.slot_stride);
+    if (t + 1 < I.num_tokens) after = sp[I.slot_stride];
     const uint16_t *vp = I.v + static_cast<int64_t>(t) * I.row_stride + h * D + l;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ve[e] = vp[32 * e];
@@ -388,10 +416,18 @@ __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWrite
     const int bs = P.block_size;
     const int64_t blk = slot >> __builtin_ctz(static_cast<unsigned>(bs));
     const int o = static_cast<int>(slot) & (bs - 1);
-    if ((l & 2) == 0) P.k_pool[(blk * (D / 8) + (l >> 2) + 8 * (l & 1)) * bs + o] = kc;
+    const bool alone = before != slot - 1 && after != slot + 1;
+    if ((l & 2) == 0) store16(&P.k_pool[(blk * (D / 8) + (l >> 2) + 8 * (l & 1)) * bs + o], kc, alone);
     uint16_t *const vp = P.v_pool + (blk * D + l) * bs + o;
+    if (alone) {
+      // (written as an instruction, as in store16: the branches would be folded)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) vp[32 * e * bs] = ve[e];
+      for (int e = 0; e < 4; ++e)
+        asm volatile("global_store_short %0, %1, off nt" ::"v"(&vp[32 * e * bs]), "v"(static_cast<uint32_t>(ve[e])) : "memory");
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) vp[32 * e * bs] = ve[e];
+    }
   }
 }
 

@@ -268,6 +268,50 @@ def test_rotary_cache_write_of_packed_prompts_in_each_kernel(dtype, bs, T, Hq, H
             assert torch.equal(a, b), f"{what} differ from rotary and cache write in turn"
 
 
+@pytest.mark.parametrize("bs", [8, 16, 32])
+@pytest.mark.parametrize("T,H,rope", [(37, 3, True), (37, 3, False), (1100, 3, True), (1100, 3, False)])
+def test_cache_write_of_tokens_by_themselves_and_in_runs(bs, T, H, rope):
+    """Tokens without a neighbour in the slots beside theirs go past the L2, in both
+    rotary kernels (2560 pairs apart) and the plain one: single tokens, pairs, runs of 3, 7,
+    8, 9 and 16 from any offset, skipped tokens between them and slot 0, against a scatter
+    in torch; slots that nobody writes keep their contents."""
+    print(f"[case] cache write alone and in runs bs={bs} T={T} rope={rope}", flush=True)
+    from muxserve_amd.attention import build_cos_sin_cache
+    rng = np.random.Generator(np.random.PCG64(T + bs))
+    N = 4 * T * H // bs + 8
+    slots = np.full((T, 1, H), -1, dtype=np.int64)
+    for h in range(H):
+        lo, t = h * (N * bs // H), 0
+        while t < T:
+            n = min(int(rng.choice([1, 1, 1, 2, 3, 7, 8, 9, 16])), T - t)
+            slots[t:t + n, 0, h] = lo + np.arange(n)
+            lo += n + int(rng.integers(1, 4))
+            t += n + int(rng.random() < 0.2)
+    pad = (T + 7) // 8 * 8
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn((pad, 3 * H * D), generator=g).half().to(DEV)
+    q, k, v = x.split([H * D] * 3, dim=-1)
+    positions = torch.arange(pad, device=DEV)
+    kp, vp = allocate_gpu_cache(N, bs, DEV, dtype=torch.float16)
+    kp.fill_(3)
+    vp.fill_(5)
+    dslots = torch.from_numpy(slots).to(DEV)
+    if rope:
+        ops.rope_reshape_and_cache(positions, q, k, v, build_cos_sin_cache(D, 2048, 10000.0, DEV), kp, vp, dslots, layer=0,
+                                   num_tokens=T)
+    else:
+        ops.reshape_and_cache(k, v, kp, vp, dslots, layer=0, num_tokens=T)
+    torch.cuda.synchronize()
+    wk, wv = torch.full_like(kp, 3), torch.full_like(vp, 5)
+    for h in range(H):
+        sl = dslots[:, 0, h]
+        ok = sl >= 0
+        blk, off = sl[ok] // bs, sl[ok] % bs
+        wk[blk, :, off, :] = k[:T, h * D:(h + 1) * D][ok].reshape(-1, D // 8, 8)       # (k as rotated in place)
+        wv[blk, :, off] = v[:T, h * D:(h + 1) * D][ok]
+    assert torch.equal(kp.view(torch.int16), wk.view(torch.int16)) and torch.equal(vp.view(torch.int16), wv.view(torch.int16))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("Hq,Hkv,bs,many", [(3, 3, 16, False), (8, 2, 8, False), (16, 2, 32, False), (2, 1, 16, True)])
 def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many):

@@ -365,6 +365,7 @@ def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("lens,H,bs", [
     ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16), ([45], 2, 8),                          # few: four waves
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16),
     ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16), ([1] * 520 + [9] * 7, 1, 32),           # one wave
     ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16), ([64, 17, 47] * 30, 7, 8),                # two
     ([128, 65, 100, 97, 31, 127] * 12, 8, 32), ([96, 113, 128] * 30, 6, 16)])            # four, many

@@ -45,10 +45,10 @@ union SmFrag {
 constexpr int kSmTile = 256;              // the hidden size must be a multiple of this
 constexpr int kSmMaxRowsPerPass = 256;
 // Up to 32 sampled rows the narrow kernel, beyond them the wide one.  32000 rows of
-// 4096, us: the narrow one with 32 rows 43.5, the wide one with 33 to 64 rows 45
-// (the narrow one with four row blocks per wave took 52.3 to 53.5 there, and 107 and
-// 214 with 128 and 256 rows, passing over the matrix once per 64; the wide one 53
-// and 73).  Small vocabularies too, though the wide kernel keeps its 128 rows per
+// 4096, us: the narrow one with 32 rows 43.5, the wide one with 33 to 64 rows 46 to
+// 47.5 (the narrow one with four row blocks per wave took 52.3 to 53.5 there, and 107
+// and 214 with 128 and 256 rows, passing over the matrix once per 64; the wide one 55
+// and 76).  Small vocabularies too, though the wide kernel keeps its 128 rows per
 // workgroup there: 16000 rows, 33 sampled 46.6 / 34.9, 64 48.0 / 38.1; 4000 rows
 // 37.0 / 30.8 and 38.3 / 33.8.
 constexpr int kSmNarrowRows = 32;
@@ -356,10 +356,10 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
 //     tile goes from global memory straight into LDS, NBUF - 1 tiles ahead, one
 //     barrier per tile, 16-byte chunk c of a row at position c ^ (row % 8): no bank
 //     conflicts.  NBUF is what 160 KB hold (at most 5).
-// 32000 x 4096, us (tiles staged through registers / straight into LDS, the
-// two-level reduction in both): 64 rows 46.3 / 44.8, 128 rows 54.3 / 53.1, 256 rows
-// 79 / 73; 128256 x 4096 bf16, 256 rows 304 / 295.  Up to 64 rows it is bound by HBM
-// (5.8 TB/s).  With 256 rows the clock is 1.66 GHz and LDS is the busiest unit: 128 KB
+// 32000 x 4096, us (tiles staged through registers and the reduction in one level / as
+// here, both in turn on one machine): 33 rows 47.2 / 46.0, 64 rows 48.4 / 47.5, 128 rows
+// 57.7 / 54.6, 192 rows 70 / 64, 256 rows 85.4 / 76.1; 16000 x 4096, 64 rows 37.7 / 37.9;
+// 128256 x 4096 bf16, 256 rows 334 / 298.  Up to 64 rows it is bound by HBM (5.5 TB/s).  With 256 rows the clock is 1.66 GHz and LDS is the busiest unit: 128 KB
 // of fragments and 48 KB of tiles in per 1024 cycles of MFMA and compute unit, at 128
 // bytes a cycle.  Fewer fragment reads cost more than they save: four waves of 64 x
 // 32 NB (a quarter less) 80, four waves of 128 x 16 NB with the hidden states straight
@@ -475,8 +475,11 @@ __global__ __launch_bounds__(512, 2) void lm_head_argmax_wide_kernel(const LmHea
     }
     __builtin_amdgcn_sched_group_barrier(kMfma, 4 * NB, 0);
     __builtin_amdgcn_sched_barrier(0);
+    // This wave's part of the next tile has landed, and f1 has been read: behind the
+    // barrier the other waves load into its buffer.
     if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * (2 + NB)) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);

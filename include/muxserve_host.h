@@ -167,8 +167,8 @@ int64_t mux_sched_get_batch_compact(MuxBatchScheduler *s, const int32_t *req, in
  *     most token blocks that one entry received, sum of the context lens (low, high
  *     32 bits), number of prompts, of preempted requests, of batch entries },
  * then the prompt lens, the preempted ids and (id, maxTokens) per entry.  On failure
- * info[0] says where: 0 host is too small (MUX_ENOSPC with the ints it needs in
- * info[4], nothing has changed), 1 get_batch_info, 2 get_batch_compact. */
+ * info[0] says where: 0 the arguments, or host is too small (MUX_ENOSPC with the ints
+ * it needs in info[4]), and nothing has changed; 1 get_batch_info, 2 get_batch_compact. */
 #define MUX_STEP_INFO_INTS 11
 int32_t mux_sched_step(MuxBatchScheduler *s, const int32_t *req, int32_t n_req, const int32_t *block_info,
                        int64_t n_block_info, int32_t *host, int64_t host_cap, int32_t *info, int32_t info_cap);

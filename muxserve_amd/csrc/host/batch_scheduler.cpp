@@ -446,6 +446,7 @@ int64_t mux_sched_get_batch_compact(MuxBatchScheduler *s, const int32_t *req, in
 
 int32_t mux_sched_step(MuxBatchScheduler *s, const int32_t *req, int32_t n_req, const int32_t *block_info,
                        int64_t n_block_info, int32_t *host, int64_t host_cap, int32_t *info, int32_t info_cap) {
+  if (info && info_cap > 0) info[0] = 0;     // (where the step fails, from here on)
   if (!s || !req || !block_info || (!host && host_cap > 0) || !info || n_req < 0 || n_block_info < 1 ||
       n_block_info > INT32_MAX)
     return MUX_EINVAL;
@@ -466,7 +467,6 @@ int32_t mux_sched_step(MuxBatchScheduler *s, const int32_t *req, int32_t n_req, 
   const int64_t at_ctx = 2 * padded, at_desc = at_ctx + (contexts + 3) / 4 * 4;
   const int64_t at_reply = at_desc + static_cast<int64_t>(entries) * MUX_STEP_DESC_INTS;
   const int64_t total = at_reply + n_block_info;
-  info[0] = 0;
   if (total > INT32_MAX) return MUX_EINVAL;
   info[4] = static_cast<int32_t>(total);
   if (total > host_cap) return MUX_ENOSPC;

@@ -212,3 +212,23 @@ def test_step_in_one_call_equals_its_four(blocks, cap):
     assert (blocks > 9) == (len(alive) == 4)
     with pytest.raises(KeyError):
         pair[1][1].step(np.array([77, 1, 0], dtype=np.int32), np.arange(1 + L * H, dtype=np.int32) * 0 + 1, staging)
+
+
+def test_step_says_what_an_empty_reply_is():
+    """An allocator reply without its first word is refused as get_batch_info refuses it,
+    also behind a step of more than two tokens (whose count the refusal used to be looked
+    up by)."""
+    L, H, bs = 2, 2, 16
+    store, sched = KVStorage(64 * L * H), BatchScheduler(L, H, 128, bs)
+    sched.enable_device_rows(2)
+    sched.add_request(np.arange(20, dtype=np.int32), 0, 8)
+    buf = torch.zeros((4096,), dtype=torch.int32)
+    info = sched.try_batch([0], [])
+    req = np.ascontiguousarray(info[:-1])
+    sched.step(req, store.allocate_batch(req, L, H), lambda n: buf)
+    req = np.ascontiguousarray(sched.try_batch([0], [7])[:-1])
+    with pytest.raises(ValueError):
+        sched.get_batch_info(req, np.empty((0,), dtype=np.int32))
+    with pytest.raises(ValueError):
+        sched.step(req, np.empty((0,), dtype=np.int32), lambda n: buf)
+    assert sched.step(req, np.array([1], dtype=np.int32), lambda n: buf)[1][:2] == [1, 1]

@@ -50,11 +50,13 @@ class DeviceBlockTables:
         the staging buffer is reused by the next step), slot_mapping int64 [tokens, L, H]
         and block_tables int32 [L, sequences, H, max blocks], or the reference's empty
         prefill table."""
-        tensors = T.load().step_inputs(self.mirror, host, head, self.block_size)
-        if self._uploaded is None:
-            self._uploaded = torch.cuda.Event()
-        self._uploaded.record(torch.cuda.current_stream(self.device))
-        return tensors
+        try:
+            return T.load().step_inputs(self.mirror, host, head, self.block_size)
+        finally:
+            # (also of a step that was refused: its copy may have been queued before that)
+            if self._uploaded is None:
+                self._uploaded = torch.cuda.Event()
+            self._uploaded.record(torch.cuda.current_stream(self.device))
 
     def upload(self, n_ints: int) -> torch.Tensor:
         """One asynchronous copy of the first n_ints of the staging buffer."""

@@ -232,3 +232,33 @@ def test_step_says_what_an_empty_reply_is():
     with pytest.raises(ValueError):
         sched.step(req, np.empty((0,), dtype=np.int32), lambda n: buf)
     assert sched.step(req, np.array([1], dtype=np.int32), lambda n: buf)[1][:2] == [1, 1]
+
+
+def test_staging_waits_for_the_copy_of_a_step_that_was_refused(monkeypatch):
+    """The operator queues the copy out of the staging buffer before its launch can be
+    refused; the next step must still wait for that copy before it packs over it."""
+    from muxserve_amd import device_tables
+    calls = []
+
+    class Event:
+        def record(self, stream):
+            calls.append(("record", stream))
+
+        def synchronize(self):
+            calls.append(("synchronize",))
+
+    class Operators:
+        @staticmethod
+        def step_inputs(*args):
+            calls.append(("copy",))
+            raise RuntimeError("mux_build_step: refused")
+
+    monkeypatch.setattr(device_tables.T, "load", lambda: Operators)
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: "stream")
+    tables = device_tables.DeviceBlockTables(BatchScheduler(2, 2, 128, 16), 2, "cpu")
+    host = tables.staging(0)
+    with pytest.raises(RuntimeError):
+        tables.step_inputs(host, [1, 1, 1, 1, 20, 1, 1, 0, 0, 0, 1])
+    tables.staging(0)
+    assert calls == [("copy",), ("record", "stream"), ("synchronize",)]

@@ -13,7 +13,6 @@ from typing import Tuple
 
 import torch
 
-from . import _lib
 from . import torch_ops as T
 from .batch_scheduler import BatchScheduler
 
@@ -26,7 +25,7 @@ class DeviceBlockTables:
         self.L, self.H = scheduler.num_layers, scheduler.num_heads
         self.block_size = scheduler.block_size
         self.max_blocks_per_seq = scheduler.max_blocks_per_seq
-        # int32 [row][token block][layer][head]; written only by step_inputs() and build().
+        # int32 [row][token block][layer][head]; written only by step_inputs().
         self.mirror = torch.zeros((self.max_rows, self.max_blocks_per_seq, self.L, self.H), dtype=torch.int32,
                                   device=self.device)
         self._staging = None
@@ -50,44 +49,11 @@ class DeviceBlockTables:
         the staging buffer is reused by the next step), slot_mapping int64 [tokens, L, H]
         and block_tables int32 [L, sequences, H, max blocks], or the reference's empty
         prefill table."""
+        operator = T.load().step_inputs
         try:
-            return T.load().step_inputs(self.mirror, host, head, self.block_size)
+            return operator(self.mirror, host, head, self.block_size)
         finally:
             # (also of a step that was refused: its copy may have been queued before that)
             if self._uploaded is None:
                 self._uploaded = torch.cuda.Event()
             self._uploaded.record(torch.cuda.current_stream(self.device))
-
-    def upload(self, n_ints: int) -> torch.Tensor:
-        """One asynchronous copy of the first n_ints of the staging buffer."""
-        dev = self._staging[:n_ints].to(self.device, non_blocking=True)
-        if self._uploaded is None:
-            self._uploaded = torch.cuda.Event()
-        self._uploaded.record(torch.cuda.current_stream(self.device))
-        return dev
-
-    def build(self, desc: torch.Tensor, block_info: torch.Tensor, num_seqs: int, max_new_blocks: int,
-              num_tokens: int, max_blocks_out: int, stream=None, narrow=None, wide=None
-              ) -> Tuple[torch.Tensor, torch.Tensor]:
-        """desc int32 [num_seqs, 8] and block_info int32 [n] on the device ->
-        (slot_mapping int64 [num_tokens, L, H], block_tables int32
-        [L, num_seqs, H, max_blocks_out] or the reference's empty prefill table).
-        narrow, wide: optionally an int32 tensor that goes to the int64 tensor of as
-        many elements in the same launch."""
-        slot_mapping = torch.empty((num_tokens, self.L, self.H), dtype=torch.int64, device=self.device)
-        if max_blocks_out > 0:
-            block_tables = torch.empty((self.L, num_seqs, self.H, max_blocks_out), dtype=torch.int32,
-                                       device=self.device)
-            bt_ptr = block_tables.data_ptr()
-        else:
-            block_tables = torch.empty((0, 0, 0, self.max_blocks_per_seq), dtype=torch.int32, device=self.device)
-            bt_ptr = None
-        st = torch.cuda.current_stream(self.device).cuda_stream if stream is None else stream
-        rc = _lib.attn().mux_build_step(
-            self.mirror.data_ptr(), self.max_rows, self.max_blocks_per_seq, self.L, self.H, self.block_size,
-            desc.data_ptr(), int(num_seqs), block_info.data_ptr(), block_info.numel(), int(max_new_blocks),
-            int(num_tokens), slot_mapping.data_ptr() if num_tokens else None, bt_ptr, int(max_blocks_out),
-            None if narrow is None else narrow.data_ptr(), None if wide is None else wide.data_ptr(),
-            0 if narrow is None else narrow.numel(), st)
-        _lib.check_attn(rc, "mux_build_step")
-        return slot_mapping, block_tables

@@ -5,6 +5,7 @@ for every layer, exactly as the reference's serving loop drives its attention
 layer (llm_runtime.py:277-339, models/llama.py:149-163).  Checked per layer
 against the oracle; the pool is compared bit-exact at the end.
 """
+import ctypes
 import os
 import re
 
@@ -362,18 +363,48 @@ def test_prompt_step_operator_equals_the_three_kernels(dtype, Hq, Hkv, bs, many)
         assert torch.equal(a, b), f"{what} differ between the step operator and the three kernels"
 
 
+def _captured_launches(fn):
+    """Threads per workgroup of every kernel that fn launches, in order, from a graph of it
+    (which is not run; fn runs once before, for its workspaces on that stream)."""
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+
+    class Params(ctypes.Structure):                  # hipKernelNodeParams
+        _fields_ = [("block", ctypes.c_uint32 * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p),
+                    ("grid", ctypes.c_uint32 * 3), ("params", ctypes.c_void_p), ("shared", ctypes.c_uint32)]
+
+    stream, captured = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        fn()
+    stream.synchronize()
+    with torch.cuda.graph(captured, stream=stream):
+        fn()
+    graph, n = ctypes.c_void_p(captured.raw_cuda_graph()), ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, ctypes.byref(n)) == 0
+    threads = []
+    for node in nodes:
+        kind, params = ctypes.c_int(), Params()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node), ctypes.byref(kind)) == 0 and kind.value == 0
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0
+        threads.append(params.block[0])
+    return threads
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("lens,H,bs", [
-    ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16), ([45], 2, 8),                          # few: four waves
-    ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16),
-    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16), ([1] * 520 + [9] * 7, 1, 32),           # one wave
-    ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16), ([64, 17, 47] * 30, 7, 8),                # two
-    ([128, 65, 100, 97, 31, 127] * 12, 8, 32), ([96, 113, 128] * 30, 6, 16)])            # four, many
-def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs):
-    """Steps of prompts of at most 128 tokens (one launch, workgroups of 1, 2 or 4
-    waves): q, k, both pools and the outputs bitwise as from rotary, cache write and
-    attention in turn; with tokens without a slot, one outside the pool and a prompt
-    whose slots are scattered token by token."""
+@pytest.mark.parametrize("lens,H,bs,waves,waves_bf16", [
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16, 4, 0), ([45], 2, 8, 4, 0), ([30, 5], 4, 16, 4, 4),      # few
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16, 4, 4), ([128, 65, 100, 97, 31, 127] * 7, 8, 32, 4, 4),
+    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16, 1, 1), ([1] * 520 + [9] * 7, 1, 32, 1, 1),               # many
+    ([1, 3, 17, 32] * 200, 1, 16, 1, 1),                               # (more than a launch lists one by one)
+    ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16, 2, 2), ([64, 17, 47] * 30, 7, 8, 2, 2),
+    ([128, 65, 100, 97, 31, 127] * 12, 8, 32, 4, 0), ([96, 113, 128] * 30, 6, 16, 4, 0)])
+def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs, waves, waves_bf16):
+    """Steps of prompts of at most 128 tokens (one launch of workgroups of 1, 2 or 4
+    waves, as stated; 0: two launches): q, k, both pools and the outputs bitwise as from
+    rotary, cache write and attention in turn; with tokens without a slot, one outside the
+    pool and a prompt whose slots are scattered token by token."""
     print(f"[case] short prompts {dtype} {len(lens)} prompts up to {max(lens)} H={H} bs={bs}", flush=True)
     from muxserve_amd import torch_ops, workloads
     from muxserve_amd.attention import build_cos_sin_cache
@@ -400,7 +431,9 @@ def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs)
         vp.fill_(5)
         out = torch.zeros((pad, H * D), dtype=dtype, device=DEV)
         if fused:
-            torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, dslots, 0, cu, lens, D ** -0.5)
+            def step():
+                torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, dslots, 0, cu, lens, D ** -0.5)
+            step()
         else:
             ops.rotary_neox(positions, q, k, cos_sin, num_tokens=T)
             ops.reshape_and_cache(k, v, kp, vp, dslots, layer=0, num_tokens=T)
@@ -409,6 +442,9 @@ def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs)
         results.append([t.cpu().view(torch.int16) for t in (x, kp, vp, out)])
     for a, b, what in zip(*results, ("qkv rows", "k pool", "v pool", "outputs")):
         assert torch.equal(a, b), f"{what} differ between the one launch and the three kernels"
+    launched = _captured_launches(step)
+    expected = waves_bf16 if dtype == torch.bfloat16 else waves
+    assert launched == [64 * expected] if expected else len(launched) == 2
 
 
 @pytest.mark.parametrize("bs,off", [(16, 0), (16, 8), (16, 5), (32, 0), (32, 16), (32, 8), (8, 0)])
@@ -451,16 +487,17 @@ def test_prompt_step_pool_writes_of_runs_that_start_anywhere_in_a_block(bs, off)
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_rotary_table_at_any_float_offset(dtype):
+@pytest.mark.parametrize("Hq,Hkv,lens", [(4, 2, [5, 150, 33]), (8, 8, [5, 30, 17] * 12), (20, 20, [128, 33] * 8),
+                                         (8, 8, [60, 33] * 40)])
+def test_rotary_table_at_any_float_offset(dtype, Hq, Hkv, lens):
     """The cos|sin table is taken at any 4-byte boundary, as the rotary kernel takes
-    it, by the small-step cache write and by the prompt step: rows, pools and
-    outputs bitwise those of an aligned table."""
-    print(f"[case] rotary table offset {dtype}", flush=True)
+    it, by the small-step cache write and by the prompt step (the last three in one
+    launch): rows, pools and outputs bitwise those of an aligned table."""
+    print(f"[case] rotary table offset {dtype} {Hq} {Hkv} {len(lens)}", flush=True)
     from muxserve_amd import torch_ops, workloads
     from muxserve_amd.attention import build_cos_sin_cache
     rng = np.random.Generator(np.random.PCG64(3))
-    Hq, Hkv, bs, lens = 4, 2, 16, [5, 150, 33]
-    T = sum(lens)
+    bs, T = 16, sum(lens)
     N = sum((n + bs - 1) // bs for n in lens) * Hkv
     slots, _ = workloads.prefill_slot_mapping(np.array(lens, dtype=np.int32), Hkv, bs, rng.permutation(N))
     dslots, positions = torch.from_numpy(slots).to(DEV), torch.from_numpy(rng.integers(0, 2048, size=T)).to(DEV)
@@ -644,6 +681,9 @@ def test_decode_of_one_sequence_in_one_launch_equals_the_general_path(dtype, bs,
         out = layer(positions, q, k, v, kp, vp, md, None)
         torch.cuda.synchronize()
         results.append([t.cpu() for t in (x, kp, vp, out[:1])])
+        if fused_max:
+            launched = _captured_launches(lambda: layer(positions, q, k, v, kp, vp, md, None))
+            assert launched == [256 if n <= 256 else 512] if n <= 512 else len(launched) > 1
     for a, b, what in zip(*results, ("q, k, v", "k pool", "v pool")):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), what
     got, want = (r[3].float() for r in results)

@@ -37,7 +37,7 @@ __device__ __forceinline__ uint4 rotate_chunk(const uint4 own, const uint4 partn
     // x' = x c - y s for the low half of a head, y' = y c + x s for the high half.
     const float r0 = is_y ? a0 * cs[2 * e] + b0 * sn[2 * e] : a0 * cs[2 * e] - b0 * sn[2 * e];
     const float r1 = is_y ? a1 * cs[2 * e + 1] + b1 * sn[2 * e + 1] : a1 * cs[2 * e + 1] - b1 * sn[2 * e + 1];
-    o[e] = static_cast<uint32_t>(to_storage<T>(r0)) | (static_cast<uint32_t>(to_storage<T>(r1)) << 16);
+    o[e] = to_storage2<T>(r0, r1);
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
 }

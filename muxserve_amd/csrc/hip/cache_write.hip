@@ -396,10 +396,8 @@ __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWrite
     x0 = bf16_lo(lo); x1 = bf16_hi(lo);
     y0 = bf16_lo(hi); y1 = bf16_hi(hi);
   }
-  const uint32_t xo = static_cast<uint32_t>(to_storage<T>(x0 * cs.x - y0 * sn.x)) |
-                      (static_cast<uint32_t>(to_storage<T>(x1 * cs.y - y1 * sn.y)) << 16);
-  const uint32_t yo = static_cast<uint32_t>(to_storage<T>(y0 * cs.x + x0 * sn.x)) |
-                      (static_cast<uint32_t>(to_storage<T>(y1 * cs.y + x1 * sn.y)) << 16);
+  const uint32_t xo = to_storage2<T>(x0 * cs.x - y0 * sn.x, x1 * cs.y - y1 * sn.y);
+  const uint32_t yo = to_storage2<T>(y0 * cs.x + x0 * sn.x, y1 * cs.y + x1 * sn.y);
   x[l] = xo;
   x[32 + l] = yo;
   // A chunk of the K pool (8 dims) is spread over four lanes: the first of them

@@ -49,7 +49,7 @@ __device__ __forceinline__ mo_u32x4 pack8(const float (&f)[8]) {
   uint32_t w[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    w[i] = static_cast<uint32_t>(to_storage<T>(f[2 * i])) | (static_cast<uint32_t>(to_storage<T>(f[2 * i + 1])) << 16);
+    w[i] = to_storage2<T>(f[2 * i], f[2 * i + 1]);
   return mo_u32x4{w[0], w[1], w[2], w[3]};
 }
 

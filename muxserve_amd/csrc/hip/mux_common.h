@@ -48,12 +48,13 @@ __device__ __forceinline__ bf162_t as_bf162(uint32_t u) {
   return c.h;
 }
 
-// fp32 -> bf16 bits, round to nearest even (NaN kept quiet).
+// fp32 -> bf16 bits, round to nearest even (NaN kept quiet): v_cvt_pk_bf16_f32, equal to
+// the integer arithmetic for all 2^32 inputs.  That arithmetic is six instructions per
+// value, and short launches wait for every line of code they run for the first time.
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x0040u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  union { __bf16 h; uint16_t u; } c;
+  c.h = static_cast<__bf16>(f);
+  return c.u;
 }
 
 __device__ __forceinline__ uint16_t f32_to_f16_bits(float f) {
@@ -66,6 +67,20 @@ template <typename T>
 __device__ __forceinline__ uint16_t to_storage(float f) {
   if constexpr (__is_same(T, F16)) return f32_to_f16_bits(f);
   else return f32_to_bf16_bits(f);
+}
+
+// A packed pair.  (f16 one by one: the compiler folds a conversion into the fma in front
+// of it, which rounds once.)
+template <typename T>
+__device__ __forceinline__ uint32_t to_storage2(float lo, float hi) {
+  if constexpr (__is_same(T, F16)) {
+    return static_cast<uint32_t>(to_storage<T>(lo)) | (static_cast<uint32_t>(to_storage<T>(hi)) << 16);
+  } else {
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    union { bf162_t h; uint32_t u; } c;
+    c.h = __builtin_convertvector((float2_t{lo, hi}), bf162_t);
+    return c.u;
+  }
 }
 
 // acc + a.x*b.x + a.y*b.y with a, b packed pairs in storage type T, fp32 accumulate.

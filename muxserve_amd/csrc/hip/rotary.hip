@@ -43,10 +43,8 @@ __global__ __launch_bounds__(256) void rotary_neox_kernel(const int64_t *__restr
       y0 = bf16_lo(yv); y1 = bf16_hi(yv);
     }
     const float c0 = cs[i], c1 = cs[i + 1], s0 = cs[half + i], s1 = cs[half + i + 1];
-    const uint32_t xo = static_cast<uint32_t>(to_storage<T>(x0 * c0 - y0 * s0)) |
-                        (static_cast<uint32_t>(to_storage<T>(x1 * c1 - y1 * s1)) << 16);
-    const uint32_t yo = static_cast<uint32_t>(to_storage<T>(y0 * c0 + x0 * s0)) |
-                        (static_cast<uint32_t>(to_storage<T>(y1 * c1 + x1 * s1)) << 16);
+    const uint32_t xo = to_storage2<T>(x0 * c0 - y0 * s0, x1 * c1 - y1 * s1);
+    const uint32_t yo = to_storage2<T>(y0 * c0 + x0 * s0, y1 * c1 + x1 * s1);
     *reinterpret_cast<uint32_t *>(row + i) = xo;
     *reinterpret_cast<uint32_t *>(row + half + i) = yo;
   }

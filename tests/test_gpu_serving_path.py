@@ -524,6 +524,53 @@ def test_rotary_table_at_any_float_offset(dtype, Hq, Hkv, lens):
     assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
+@pytest.mark.parametrize("form", ["rotary", "cache write of few", "cache write of many", "short prompts"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_rotation_rounds_to_nearest_even(dtype, form):
+    """Rows that the rotation turns into the table's own floats, so that the stored value is
+    one rounding of a chosen float: ties and their neighbours in the last stored bit, the
+    largest finite values and past them, subnormals, infinities, NaN, random bits.  x = (1,
+    0): x' = cos, y' = sin, bitwise as torch rounds them (any NaN for a NaN)."""
+    print(f"[case] rounding {dtype} {form}", flush=True)
+    from muxserve_amd import torch_ops
+    H, bs = 8, 16
+    T = {"rotary": 300, "cache write of few": 300, "cache write of many": 700, "short prompts": 300}[form]
+    rng = np.random.Generator(np.random.PCG64(T))
+    bits = rng.integers(0, 2 ** 32, size=(T, D // 2), dtype=np.uint64).astype(np.uint32)
+    step = 16 if dtype == torch.bfloat16 else 13
+    low = np.array([0, 1, (1 << step - 1) - 1, 1 << step - 1, (1 << step - 1) + 1, (1 << step) - 1], dtype=np.uint32)
+    bits[1::2] = (bits[1::2] >> step << step) | low[rng.integers(0, len(low), size=bits[1::2].shape)]
+    bits[2::6] = (bits[2::6] & 0x807fffff) | (rng.integers(0x67, 0x92, size=bits[2::6].shape).astype(np.uint32) << 23)
+    special = np.array([0x7f800000, 0xff800000, 0x7fc00000, 0xffc12345, 0x7f7fffff, 0x7f7f7fff, 0x7f7f8000, 1, 0x80000001,
+                        0x00007fff, 0x00008000, 0x00018000, 0x477fefff, 0x477ff000, 0x33000000, 0x33000001], dtype=np.uint32)
+    bits[0, :16] = special
+    values = torch.from_numpy(bits.view(np.float32))
+    zero = torch.zeros_like(values)
+    positions = torch.arange(T, device=DEV)
+    slots = torch.randperm(T * H, generator=torch.Generator().manual_seed(1)).reshape(T, 1, H).to(DEV)
+    one = torch.zeros((T, 3 * H * D), dtype=dtype)
+    one.view(T, -1, 2, D // 2)[:, :, 0] = 1
+    for half, table in ((0, torch.cat([values, zero], 1)), (1, torch.cat([zero, values], 1))):
+        q, k, v = one.to(DEV).split([H * D] * 3, dim=-1)
+        cos_sin = table.to(DEV).contiguous()
+        kp, vp = allocate_gpu_cache(T * H // bs + 1, bs, DEV, dtype=dtype)
+        if form == "rotary":
+            ops.rotary_neox(positions, q, k, cos_sin)
+        elif form == "short prompts":
+            cu = torch.arange(0, T + 1, 30, dtype=torch.int32, device=DEV)
+            out = torch.zeros((T, H * D), dtype=dtype, device=DEV)
+            torch_ops.rope_prefill_and_cache(out, positions, q, k, v, cos_sin, kp, vp, slots, 0, cu, [30] * 10, 1.0)
+        else:
+            ops.rope_reshape_and_cache(positions, q, k, v, cos_sin, kp, vp, slots)
+        want = values.to(dtype)
+        for x in (q, k):
+            got = x.cpu().reshape(T, H, 2, D // 2)[:, :, half]
+            nan = want.isnan()[:, None].expand_as(got)
+            assert torch.equal(got.isnan(), nan)
+            same = got.contiguous().view(torch.int16) == want.view(torch.int16)[:, None]
+            assert (same | nan).all(), (half, int((~(same | nan)).sum()))
+
+
 @pytest.mark.parametrize("rope", [True, False])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_multi_model_cache_write_equals_one_launch_per_model(rope, dtype):

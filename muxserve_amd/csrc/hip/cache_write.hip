@@ -70,14 +70,22 @@ __device__ __forceinline__ void cache_write_window(
   }
   __syncthreads();
   // Bit j of `starts`: token j begins a run (8 consecutive slots from a multiple of 8).
-  bool is_start = false;
+  // Bit j of `chained`: the next token goes to the slot behind token j's.
+  bool is_start = false, is_valid = false, is_chained = false;
   if (lane < 40) {
     const int64_t s0 = s_slot[lane];
-    is_start = s0 >= 0 && (s0 & 7) == 0;
+    is_valid = s0 >= 0;
+    is_chained = is_valid && s_slot[lane + 1] == s0 + 1;
+    is_start = is_chained && (s0 & 7) == 0;
 #pragma unroll
-    for (int e = 1; e < 8; ++e) is_start = is_start && s_slot[lane + e] == s0 + e;
+    for (int e = 2; e < 8; ++e) is_start = is_start && s_slot[lane + e] == s0 + e;
   }
   const unsigned long long starts = __builtin_amdgcn_ballot_w64(is_start);
+  // Tokens by themselves, as in a decode step (see the comment at rope_scatter_kernel): no
+  // neighbour in the batch goes to the slot beside theirs.  Not the last token of a prompt
+  // that has a block to itself: the token in front of it is in a run.
+  const unsigned long long chained = __builtin_amdgcn_ballot_w64(is_chained), in_chain = chained | chained << 1;
+  const unsigned long long lone = __builtin_amdgcn_ballot_w64(is_valid) & ~in_chain & ~(in_chain << 1);
   // The boundary next to nominal bit n: the start of the run that contains
   // token n, moved on to the start of that run's pool block when the run is the
   // block's second half and the first half sits right before it - so that
@@ -95,6 +103,7 @@ __device__ __forceinline__ void cache_write_window(
   const int ja = boundary(kBack);
   const int jb = min(boundary(kBack + 16), num_tokens - T0 + kBack);
   const unsigned long long in_win = starts & (~0ull << ja) & ~(~0ull << jb);   // runs that start inside the window
+  const unsigned long long lone_win = lone & (~0ull << ja) & ~(~0ull << jb);   // (prompts: none)
   // Does this window write whole pool rows and nothing else?  K rows of a run are
   // 128 bytes; a V row is block_size * 2 bytes: one run fills it at block size 8,
   // the two runs of a block at 16, never at 32.  Such a window streams its stores
@@ -202,9 +211,6 @@ __device__ __forceinline__ void cache_write_window(
     }
   }
   __syncthreads();
-  // Token by itself (bit position j): no neighbour in the batch goes to the slot beside
-  // its own, as in a decode step (see the comment at rope_scatter_kernel).
-  auto alone = [&](int j) { return s_slot[j - 1] != s_slot[j] - 1 && s_slot[j + 1] != s_slot[j] + 1; };
   static_assert(kBack >= 16, "a window's tokens have a neighbour on either side in s_slot");
 #pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
@@ -217,8 +223,8 @@ __device__ __forceinline__ void cache_write_window(
       // Element path for tokens that no run covers (a run starts at most 7 tokens back).
       const unsigned long long cover = in_win & (0xffull << (j > 7 ? j - 7 : 0)) & ~(~0ull << (j + 1));
       store16(&k_pool[(blk * (D / 8) + c) * block_size + o], *reinterpret_cast<const uint4 *>(&kt[j][c * 8]),
-              rows_complete || (cover == 0 && alone(j)));
-      if (cover == 0 && !alone(j)) {
+              rows_complete || ((lone_win >> j) & 1) != 0);
+      if (cover == 0 && ((lone_win >> j) & 1) == 0) {
         uint16_t *vp = v_pool + (blk * D + c * 8) * block_size + o;
         const uint4 vx = *reinterpret_cast<const uint4 *>(&vt[j][c * 8]);
         const uint32_t w[4] = {vx.x, vx.y, vx.z, vx.w};
@@ -232,11 +238,10 @@ __device__ __forceinline__ void cache_write_window(
   }
   // V of tokens by themselves: 32 threads per token, 32 neighbouring dims of the block
   // per instruction, so that four lanes share a line.
-  if (n_runs == 0 || jb - ja > 8 * n_runs) {
+  if (lone_win != 0) {
     for (int j = ja + static_cast<int>(threadIdx.x >> 5); j < jb; j += 8) {
       const int64_t slot = s_slot[j];
-      const unsigned long long cover = in_win & (0xffull << (j > 7 ? j - 7 : 0)) & ~(~0ull << (j + 1));
-      if (slot < 0 || cover != 0 || !alone(j)) continue;
+      if (((lone_win >> j) & 1) == 0) continue;
       const int l = threadIdx.x & 31;
       uint16_t *const vp = v_pool + ((slot >> bs_shift) * D + l) * block_size + (static_cast<int>(slot) & (block_size - 1));
 #pragma unroll

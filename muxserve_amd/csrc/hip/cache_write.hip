@@ -377,13 +377,13 @@ __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWrite
       kv ? I.k + static_cast<int64_t>(t) * I.row_stride + h * D
          : R.q + static_cast<int64_t>(t) * R.q_stride + (h * R.ratio + hq) * D);
   const uint32_t lo = x[l], hi = x[32 + l];
-  int64_t slot = -1, before = -2, after = -2;
+  int64_t slot = -1, before = -1, after = -1;
   uint16_t ve[4] = {0, 0, 0, 0};
   if (kv) {
     const int64_t *const sp = I.slots + static_cast<int64_t>(t) * I.slot_stride + h;
     slot = *sp;
-    if (t > 0) before = *(sp - I.slot_stride);
-    if (t + 1 < I.num_tokens) after = sp[I.slot_stride];
+    before = sp[t > 0 ? -I.slot_stride : 0];            // (its own slot where there is no neighbour)
+    after = sp[t + 1 < I.num_tokens ? I.slot_stride : 0];
     const uint16_t *vp = I.v + static_cast<int64_t>(t) * I.row_stride + h * D + l;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ve[e] = vp[32 * e];

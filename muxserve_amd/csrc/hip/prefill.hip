@@ -420,9 +420,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[mb][i] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-  // The reference as an exponent, kept beside m_run and changed with it; infinite
-  // until the wave's first tile has set it.
-  float neg_m = INFINITY;
+  float neg_m = 0.f;                     // the reference as an exponent, kept beside m_run and changed with it
 
   // Keys needed by this workgroup: positions 0 .. min(len, q0 + 128) - 1.
   const int kv_end = min(len, q0 + kRows);
@@ -732,9 +730,8 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
       // 32 rows per wave, that is in most tiles of a prompt's first hundreds of keys).
       // Not further: the key that dominates a row is exact where it is the reference
       // itself, and rounded to 11 bits where the reference lags behind it.
-      // The sum is needed anyway; the maxima are taken only where the reference moves,
-      // which the infinite reference before a wave's first tile (and anything that is
-      // not a number) makes it do.
+      // The sum is needed anyway; the maxima are taken only where the reference moves:
+      // there, in a wave's first tile, and wherever the sum is not a number.
       constexpr float kRescaleSum = 256.f;
       float p[16], psum;
       auto exponentials = [&] {
@@ -744,8 +741,12 @@ __device__ __forceinline__ void prefill_body(const PrefillParams &P, const Prefi
 #pragma unroll
         for (int i = 1; i < 16; ++i) psum += p[i];
       };
-      exponentials();
-      if (__builtin_amdgcn_ballot_w64(!(psum <= kRescaleSum)) != 0) {
+      bool moves = t == 0;                 // (no reference yet)
+      if (!moves) {
+        exponentials();
+        moves = __builtin_amdgcn_ballot_w64(!(psum <= kRescaleSum)) != 0;
+      }
+      if (moves) {
         float mx = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[i]);

@@ -1180,8 +1180,7 @@ extern "C" int32_t mux_rope_prefill_and_cache(const MuxPrefillItem *attn, const 
   S.pool_slots = num_pool_blocks * block_size;
   S.max_position = w.max_position;
   S.block_size = block_size;
-  S.short_waves = prompt_step_short_waves(it.prompt_lens_host, it.num_prompts, it.num_q_heads, it.num_kv_heads,
-                                          dtype == MUXA_DTYPE_BF16);
+  S.short_waves = prompt_step_short_waves(it.prompt_lens_host, it.num_prompts, it.num_q_heads, it.num_kv_heads);
   if (S.short_waves == 0) {
     const hipError_t e = launch_rotary_k(w.positions, static_cast<uint16_t *>(w.k), w.kv_row_stride, w.cos_sin,
                                          w.max_position, w.num_tokens, w.num_kv_heads, dtype, st);

@@ -21,12 +21,12 @@ namespace mux {
 //   41.6, 32 of 60 and 96 of 6 54.6 / 58.2 / 49.0;
 //   4 waves: 64 of 128 131 / 101 / 90, 200 of 100 376 / 317 / 285; 128 and 127 of 20 54.6 / 52.1 /
 //   58.0, 128 and 127 of 40 82.8 / 77 / 79.4, 32 of 100 and 32 of 30 (40 heads) 80 / 69 / 64.
-// bf16 multiplies the split weights twice with V, a chain that few workgroups do not
-// hide.  us per call, two launches / the short form: 32 heads, one prompt of 20 tokens 12.6 /
-// 11.2, of 45 12.9 / 13.3, of 128 12.9 / 15.7, 2 of 91 13.2 / 14.9; 40 heads, 8 of 45 17.8 / 16.4, of 128
-// 29.9 / 22.7; 32 heads, 64 of 20 37.5 / 21.0, of 64 59.6 / 57.5, of 91 78.5 / 83.9, of 128 105.0 / 105.7.
+// bf16, us, two launches / the short form: 32 heads, one prompt of 20 tokens 8.2 / 7.4, of 45
+// 9.7 / 9.4, of 128 12.9 / 12.0, 2 of 91 13.1 / 11.1, 16 of 91 25.8 / 19.3; 52 heads, 8 of 128
+// 29.1 / 21.8; 32 heads, 64 of 20 30.7 / 18.0, of 64 55.8 / 48.3, of 91 76.8 / 71.8, of 128 101 /
+// 92: the products with the split weights are hidden.
 inline int32_t prompt_step_short_waves(const int32_t *prompt_lens_host, int32_t num_prompts, int32_t num_q_heads,
-                                       int32_t num_kv_heads, bool bf16) {
+                                       int32_t num_kv_heads) {
   if (!prompt_lens_host || num_prompts <= 0 || num_q_heads != num_kv_heads) return 0;
   int32_t longest = 0;
   int64_t tokens = 0;
@@ -36,7 +36,6 @@ inline int32_t prompt_step_short_waves(const int32_t *prompt_lens_host, int32_t 
   }
   if (longest > 128) return 0;
   const int64_t groups = static_cast<int64_t>(num_prompts) * num_kv_heads;
-  if (bf16 && longest > 32 && (groups < 256 || (groups > 512 && longest > 64))) return 0;
   if (groups <= 512) return 4;
   if (longest <= 32) return 1;
   if (longest <= 64) return tokens >= int64_t{16} * num_prompts ? 2 : 0;

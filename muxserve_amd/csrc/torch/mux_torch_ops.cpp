@@ -598,8 +598,7 @@ at::Tensor prompt_layer(const at::Tensor &positions, at::Tensor q, at::Tensor k,
   if (!step && q.size(1) == k.size(1)) {
     std::vector<int32_t> lens(prompt_lens.begin(), prompt_lens.end());
     const int32_t heads = static_cast<int32_t>(q.size(1) / kHead);
-    step = mux::prompt_step_short_waves(lens.data(), static_cast<int32_t>(lens.size()), heads, heads,
-                                        q.scalar_type() == at::kBFloat16) > 0;
+    step = mux::prompt_step_short_waves(lens.data(), static_cast<int32_t>(lens.size()), heads, heads) > 0;
   }
   if (step) {
     rope_prefill_and_cache(out, positions, q, k, v, cos_sin, k_pool, v_pool, slot_mapping, layer, cu_seqlens,

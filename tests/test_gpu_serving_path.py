@@ -393,14 +393,14 @@ def _captured_launches(fn):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("lens,H,bs,waves,waves_bf16", [
-    ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16, 4, 0), ([45], 2, 8, 4, 0), ([30, 5], 4, 16, 4, 4),      # few
-    ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16, 4, 4), ([128, 65, 100, 97, 31, 127] * 7, 8, 32, 4, 4),
-    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16, 1, 1), ([1] * 520 + [9] * 7, 1, 32, 1, 1),               # many
-    ([1, 3, 17, 32] * 200, 1, 16, 1, 1),                               # (more than a launch lists one by one)
-    ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16, 2, 2), ([64, 17, 47] * 30, 7, 8, 2, 2),
-    ([128, 65, 100, 97, 31, 127] * 12, 8, 32, 4, 0), ([96, 113, 128] * 30, 6, 16, 4, 0)])
-def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs, waves, waves_bf16):
+@pytest.mark.parametrize("lens,H,bs,waves", [
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16, 4), ([45], 2, 8, 4), ([30, 5], 4, 16, 4),                 # few
+    ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16, 4), ([128, 65, 100, 97, 31, 127] * 7, 8, 32, 4),
+    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16, 1), ([1] * 520 + [9] * 7, 1, 32, 1),                       # many
+    ([1, 3, 17, 32] * 200, 1, 16, 1),                                  # (more than a launch lists one by one)
+    ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16, 2), ([64, 17, 47] * 30, 7, 8, 2), ([64, 1, 1, 1, 1] * 12, 10, 16, 0),
+    ([128, 65, 100, 97, 31, 127] * 12, 8, 32, 4), ([96, 113, 128] * 30, 6, 16, 4), ([128, 3, 1] * 30, 6, 16, 0)])
+def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs, waves):
     """Steps of prompts of at most 128 tokens (one launch of workgroups of 1, 2 or 4
     waves, as stated; 0: two launches): q, k, both pools and the outputs bitwise as from
     rotary, cache write and attention in turn; with tokens without a slot, one outside the
@@ -443,8 +443,7 @@ def test_short_prompts_in_one_launch_equal_the_three_kernels(dtype, lens, H, bs,
     for a, b, what in zip(*results, ("qkv rows", "k pool", "v pool", "outputs")):
         assert torch.equal(a, b), f"{what} differ between the one launch and the three kernels"
     launched = _captured_launches(step)
-    expected = waves_bf16 if dtype == torch.bfloat16 else waves
-    assert launched == [64 * expected] if expected else len(launched) == 2
+    assert launched == [64 * waves] if waves else len(launched) == 2
 
 
 @pytest.mark.parametrize("bs,off", [(16, 0), (16, 8), (16, 5), (32, 0), (32, 16), (32, 8), (8, 0)])

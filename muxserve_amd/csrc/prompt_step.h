@@ -11,7 +11,10 @@ namespace mux {
 // The short form needs a (prompt, head) to fit one workgroup.  Four waves per
 // workgroup where the launch does not fill the chip (two such workgroups per compute
 // unit), else as many as the longest prompt needs - unless most prompts would leave
-// most of them idle.  f16, us, two launches (rotation and cache write, attention) /
+// most of them idle, or hold so few tokens that one row of a wave's 32 is at work (up to
+// 1500 (prompt, head)s; two launches / short form: 24 of 4 tokens, 32 heads, 10.6 / 12.4, 40
+// of 4 14.5 / 15.6, 24 of 4, 52 heads, 14.4 / 16.0, 16 of 6 14.2 / 12.9; 64 of 2, 32 heads, 18.0 /
+// 17.2).  f16, us, two launches (rotation and cache write, attention) /
 // rotation of k and the step form / the short form with 1, 2 or 4 waves:
 //   32 heads, one prompt of 45 tokens 8.9 / 12.0 / - 10.3 9.0, 16 of 30 16.2 / 14.7 /
 //   10.5 - 10.0, 16 of 100 32.0 / 29.9 / - - 21.0, 8 of 128 (40 heads) 26 / 26.7 / - - 18.5;
@@ -37,7 +40,7 @@ inline int32_t prompt_step_short_waves(const int32_t *prompt_lens_host, int32_t 
   if (longest > 128) return 0;
   const int64_t groups = static_cast<int64_t>(num_prompts) * num_kv_heads;
   if (groups <= 512) return 4;
-  if (longest <= 32) return 1;
+  if (longest <= 32) return tokens >= int64_t{6} * num_prompts || groups > 1500 ? 1 : 0;
   if (longest <= 64) return tokens >= int64_t{16} * num_prompts ? 2 : 0;
   return tokens >= int64_t{45} * num_prompts ? 4 : 0;
 }

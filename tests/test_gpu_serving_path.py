@@ -396,7 +396,7 @@ def _captured_launches(fn):
 @pytest.mark.parametrize("lens,H,bs,waves", [
     ([1, 7, 16, 17, 32, 33, 0, 127, 128], 3, 16, 4), ([45], 2, 8, 4), ([30, 5], 4, 16, 4),                 # few
     ([1, 7, 16, 17, 32, 33, 0, 127, 128] * 4, 8, 16, 4), ([128, 65, 100, 97, 31, 127] * 7, 8, 32, 4),
-    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16, 1), ([1] * 520 + [9] * 7, 1, 32, 1),                       # many
+    ([1, 2, 15, 16, 17, 31, 32, 0] * 12, 8, 16, 1), ([1] * 220 + [9] * 7, 7, 32, 1), ([1] * 520 + [9] * 7, 1, 32, 0),  # many
     ([1, 3, 17, 32] * 200, 1, 16, 1),                                  # (more than a launch lists one by one)
     ([33, 64, 48, 63, 16, 1, 40] * 10, 8, 16, 2), ([64, 17, 47] * 30, 7, 8, 2), ([64, 1, 1, 1, 1] * 12, 10, 16, 0),
     ([128, 65, 100, 97, 31, 127] * 12, 8, 32, 4), ([96, 113, 128] * 30, 6, 16, 4), ([128, 3, 1] * 30, 6, 16, 0)])

@@ -3,9 +3,9 @@
 // 200-232).  Both are bound by HBM: every input element is read once and every
 // output element written once, in 16-byte pieces.
 //
-//   rms_norm      one workgroup per token row at a time: the row stays in registers
-//                 between the sum of squares and the scaling, so x is read once
-//                 (with non-temporal loads), the weight once per workgroup.
+//   rms_norm      one workgroup (a wave for short rows) per token row at a time: the row
+//                 stays in registers between the sum of squares and the scaling, so x
+//                 is read once (with non-temporal loads), the weight once per workgroup.
 //                 out = T(x * rsqrt(mean(x^2) + eps)) * w, the product in T.
 //   silu_and_mul  one thread per 8 outputs: out = T(a / (1 + exp(-a))) * b for
 //                 x = [a | b], the product in T.
@@ -21,6 +21,12 @@ typedef uint32_t mo_u32x4 __attribute__((ext_vector_type(4)));
 // 22.2, 20.8, 21.4, 21.6, 21.8 us, one workgroup per row 22.4; 2048 of 8192 14.2, 13.3, 14.2,
 // 14.6, 14.7, 14.7.
 constexpr int kRmsWgsPerCu = 3;
+// A wave per row up to this row length, and up to twice that beyond 1024 rows; such
+// workgroups per compute unit (2, 4, 8 of them, 8192 rows of 512 f16: 4.71, 4.44, 4.27 us).
+// us, f16, a workgroup / a wave per row: 8192 rows of 512 7.5 / 4.3, of 1024 9.6 / 6.6, of 1536
+// 12.0 / 10.0, of 2048 13.8 / 13.9; 4096 of 1032 6.0 / 4.7, of 2048 7.4 / 6.7; 256 of 1536 2.60 /
+// 2.76, of 512 2.52 / 2.49.
+constexpr int kRmsWaveHidden = 1024, kRmsWaveWgsPerCu = 8;
 
 template <typename T>
 __device__ __forceinline__ void unpack8(const mo_u32x4 v, float (&f)[8]) {
@@ -63,20 +69,25 @@ __device__ __forceinline__ mo_u32x4 pack8(const float (&f)[8]) {
 // 4096 of 6656 20.4 / 20.8 by themselves, 85.1 / 84.0 with silu_and_mul behind them.  Non-
 // temporal stores make this kernel 6 - 19 % faster and the one that reads its output
 // slower by more (4096 of 6656 and a read 37 / 40 us).
-template <typename T, int CPT>
+// WAVES per row: 4, the workgroup, or 1 for short rows, which leave most of a workgroup idle.
+template <typename T, int CPT, int WAVES = 4>
 __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t *__restrict__ out, int64_t out_stride,
                                                        const uint16_t *__restrict__ x, int64_t x_stride,
                                                        const uint16_t *__restrict__ weight, float eps, int hidden,
                                                        int num_rows) {
   __shared__ float part[2][4];             // the waves' sums, two rows
-  const int tid = threadIdx.x, nchunks = hidden >> 3;
-  const int step = gridDim.x;
+  constexpr int TPR = 64 * WAVES, RPW = 4 / WAVES;       // threads per row, rows per workgroup at a time
+  const int tid = WAVES == 4 ? threadIdx.x : threadIdx.x & 63, nchunks = hidden >> 3;
+  const int step = gridDim.x * RPW;
+  const int first = WAVES == 4 ? blockIdx.x : blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (WAVES == 1 && first >= num_rows) return;
   const mo_u32x4 *wr = reinterpret_cast<const mo_u32x4 *>(weight);
   const float inv_n = 1.0f / static_cast<float>(hidden);
   // rsqrt(mean + eps) of a row from a thread's part of its sum of squares.  (The barrier
   // by itself: __syncthreads() would wait for the previous row's stores.)
   auto scale_of = [&](float ss, int buf) {
     ss = wave_sum(ss);
+    if constexpr (WAVES == 1) return rsqrtf(ss * inv_n + eps);
     if ((tid & 63) == 0) part[buf][tid >> 6] = ss;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -104,7 +115,7 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t *__restrict__ ou
       const mo_u32x4 *xr = reinterpret_cast<const mo_u32x4 *>(x + row * x_stride);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        const int c = tid + 256 * i;
+        const int c = tid + TPR * i;
         v[i] = c < nchunks ? __builtin_nontemporal_load(&xr[c]) : zero;
       }
     };
@@ -117,16 +128,16 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t *__restrict__ ou
       mo_u32x4 *outr = reinterpret_cast<mo_u32x4 *>(out + row * out_stride);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
-        const int c = tid + 256 * i;
+        const int c = tid + TPR * i;
         if (c < nchunks) outr[c] = scaled(v[i], w[i], s);
       }
     };
     mo_u32x4 a[CPT], b[CPT];
-    int row = blockIdx.x;
+    int row = first;
     load_row(a, row);
 #pragma unroll
     for (int i = 0; i < CPT; ++i) {
-      const int c = tid + 256 * i;
+      const int c = tid + TPR * i;
       w[i] = c < nchunks ? wr[c] : zero;
     }
     for (; row < num_rows; row += 2 * step) {
@@ -138,13 +149,13 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(uint16_t *__restrict__ ou
     }
   } else {
     int buf = 0;
-    for (int row = blockIdx.x; row < num_rows; row += step, buf ^= 1) {
+    for (int row = first; row < num_rows; row += step, buf ^= 1) {
       const mo_u32x4 *xr = reinterpret_cast<const mo_u32x4 *>(x + row * x_stride);
       mo_u32x4 *outr = reinterpret_cast<mo_u32x4 *>(out + row * out_stride);
       float ss = 0.f;
-      for (int c = tid; c < nchunks; c += 256) ss = add_squares(xr[c], ss);
+      for (int c = tid; c < nchunks; c += TPR) ss = add_squares(xr[c], ss);
       const float s = scale_of(ss, buf);
-      for (int c = tid; c < nchunks; c += 256) outr[c] = scaled(xr[c], wr[c], s);
+      for (int c = tid; c < nchunks; c += TPR) outr[c] = scaled(xr[c], wr[c], s);
     }
   }
 }
@@ -187,7 +198,7 @@ extern "C" int32_t mux_rms_norm(void *out, int64_t out_row_stride, const void *x
     return MUXA_EINVAL;
   if (num_tokens == 0) return MUXA_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // At most kRmsWgsPerCu workgroups per CU; rows beyond that are walked in sequence.
+  // At most so many workgroups per CU; rows beyond that are walked in sequence.
   static const int cus = [] {                      // compute units of the current device, asked once
     int dev = 0, v = 0;
     if (hipGetDevice(&dev) == hipSuccess &&
@@ -195,16 +206,21 @@ extern "C" int32_t mux_rms_norm(void *out, int64_t out_row_stride, const void *x
       return v;
     return 256;
   }();
-  const dim3 grid(std::min(num_tokens, cus * kRmsWgsPerCu)), block(256);
+  const bool wave = hidden_size <= kRmsWaveHidden || (hidden_size <= 2 * kRmsWaveHidden && num_tokens > 1024);
+  const dim3 grid(wave ? std::min((num_tokens + 3) / 4, cus * kRmsWaveWgsPerCu) : std::min(num_tokens, cus * kRmsWgsPerCu));
+  const dim3 block(256);
   uint16_t *o = static_cast<uint16_t *>(out);
   const uint16_t *xi = static_cast<const uint16_t *>(x), *w = static_cast<const uint16_t *>(weight);
   const int nchunks = hidden_size / 8;
-#define MUX_RMS_LAUNCH(TT, CPT)                                                                              \
-  hipLaunchKernelGGL((rms_norm_kernel<TT, CPT>), grid, block, 0, st, o, out_row_stride, xi, x_row_stride, w, \
+#define MUX_RMS_LAUNCH(...)                                                                              \
+  hipLaunchKernelGGL((rms_norm_kernel<__VA_ARGS__>), grid, block, 0, st, o, out_row_stride, xi, x_row_stride, w, \
                      eps, hidden_size, num_tokens)
 #define MUX_RMS_PICK(TT)                              \
   do {                                                \
-    if (nchunks <= 256 * 1) MUX_RMS_LAUNCH(TT, 1);      \
+    if (wave && nchunks <= 64 * 1) MUX_RMS_LAUNCH(TT, 1, 1); \
+    else if (wave && nchunks <= 64 * 2) MUX_RMS_LAUNCH(TT, 2, 1); \
+    else if (wave) MUX_RMS_LAUNCH(TT, 4, 1);            \
+    else if (nchunks <= 256 * 1) MUX_RMS_LAUNCH(TT, 1); \
     else if (nchunks <= 256 * 2) MUX_RMS_LAUNCH(TT, 2); \
     else if (nchunks <= 256 * 3) MUX_RMS_LAUNCH(TT, 3); \
     else if (nchunks <= 256 * 4) MUX_RMS_LAUNCH(TT, 4); \

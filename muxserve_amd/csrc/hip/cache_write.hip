@@ -333,13 +333,20 @@ __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
 // lanes to a 128-byte line.
 //
 // A token by itself - no neighbour in the batch goes to the slot beside its own, as in
-// a decode step - is stored past the L2, here and in the window kernel: it leaves a few
-// bytes in each of 32 lines of V and 16 of K, and the attention behind it reads those
-// lines whole, from another XCD.  Left in the L2 they cost that launch more than the
-// write: us, write alone and with the attention, kept / past the L2: 56 tokens of three
-// models 6.1, 89.7 / 8.5, 82.7; 16 x 40 heads bf16 4.5, 34.4 / 4.9, 32.5; 256 x 32 heads (window
-// kernel) 14.3, 333 / 25, 299; 64 x 8 heads on 64 bf16 4.3, 239.5 / 4.8, 236.5.  Tokens in a run
-// (prompts) write the same lines again and keep the L2.
+// a decode step - is stored past the L2, here and in the window kernel (with rotation and
+// without): it leaves a few bytes in each of 32 lines of V and 16 of K, and left in the L2
+// those lines cost the attention behind the write more than the write itself.  us, kept /
+// past the L2, over six sets of blocks and sixteen successive steps in turn: attention
+// alone, 16 x 40 heads bf16 31.8 / 29.7, 56 tokens of three models 85.4 / 78.8, 256 x 32
+// heads 318 / 280, 64 x 8 heads on 64 bf16 235.3 / 233.9; the write alone 5.3 / 5.0, 8.3 / 8.4,
+// 22.5 / 25.1, 5.3 / 5.2; both as calls 37.8 / 35.3, 94.9 / 88.0, 341 / 307, 245.2 / 243.1; the
+// plain write of 256 x 32 heads 20.8 / 23.5, with the attention 346 / 313; a mixed step (4
+// prompts of 300, 64 decode rows, 32 heads) 128 / 120.  Blocks of 8 and 32 tokens alike (256
+// x 32 heads 326 / 305, 350 / 335); contexts of some 30 tokens gain nothing.  The attention
+// reads and writes the same bytes past the L2 either way (counters), so it is not traffic.
+// On one state again and again, where the lines of the last pass are still at hand, the
+// write alone looks worse (256 x 32 heads 13.3 / 24.1).  Tokens in a run (prompts) write
+// the same lines again and keep the L2.
 template <typename T>
 __global__ __launch_bounds__(256) void rope_scatter_kernel(const MultiCacheWriteParams P) {
   constexpr int D = kHeadSize;

@@ -1195,8 +1195,6 @@ __global__ __launch_bounds__(64 * NW, 3) void paged_decode_gqa_sweep_kernel(cons
 
 
 
-// Zero-fills the arrival counters (a kernel rather than a memset node so the
-// call can be captured into a graph).
 // ---------------------------------------------------------------------------
 // A decode step of ONE sequence with as many kv heads as query heads and a short
 // context, in one launch: rotation of its q and k rows in place, the new token's K and
@@ -1335,6 +1333,8 @@ __global__ __launch_bounds__(64 * NW) void decode_single_step_kernel(const Singl
   merge_and_write<T, 1, NW>(I, u, 0, sm.x_acc, sm.x_ml, n_active, lane);
 }
 
+// Zero-fills the arrival counters (a kernel rather than a memset node so the
+// call can be captured into a graph).
 __global__ void fill_zero_kernel(int32_t *p, int64_t n) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;

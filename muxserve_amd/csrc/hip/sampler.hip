@@ -365,11 +365,12 @@ __global__ __launch_bounds__(64 * NW) void lm_head_argmax_kernel(const LmHeadPar
 // 32 NB (a quarter less) 80, four waves of 128 x 16 NB with the hidden states straight
 // from global memory in registers (half of it) 100 before the reduction, one wave per
 // SIMD hides neither the barrier nor the latencies.
-// The reduction is the one above with 64 NB columns per table line.  One workgroup
-// reads 250 lines of 256 keys in 8 rounds of loads, so beyond 64 workgroups (4 rounds
-// in two slices) it takes two levels: groups of 16, or 32 groups (one level / two:
-// 32000 x 4096, 256 rows 84.5 / 79, 128 rows 56.2 / 54.3; 128256 x 4096, 256 rows
-// 331 / 304; 9000 rows, 71 workgroups, 62.5 / 61.8).
+// The reduction is the one above with 64 NB columns per table line.  At 256 columns one
+// workgroup reads 32 lines per round of loads (two slices of sixteen), the 250 lines of
+// 32000 rows in 8 rounds; beyond 64 workgroups, 2 rounds at that width, it takes two
+// levels: groups of 16, or 32 groups (one level / two: 32000 x 4096, 256 rows 84.5 / 79,
+// 128 rows 56.2 / 54.3; 128256 x 4096, 256 rows 331 / 304; 9000 rows, 71 workgroups, 62.5 /
+// 61.8).  Fewer columns read more lines per round, so there the line could lie higher.
 constexpr size_t kSmCounterBytes = 256;    // the arrival counters, in front of the table
 constexpr int kSmOneLevelWgs = 64, kSmGroupWgs = 16, kSmMaxGroups = 32;
 template <typename T, int NB, int NBUF>

@@ -28,6 +28,9 @@ namespace mux {
 // 9.7 / 9.4, of 128 12.9 / 12.0, 2 of 91 13.1 / 11.1, 16 of 91 25.8 / 19.3; 52 heads, 8 of 128
 // 29.1 / 21.8; 32 heads, 64 of 20 30.7 / 18.0, of 64 55.8 / 48.3, of 91 76.8 / 71.8, of 128 101 /
 // 92: the products with the split weights are hidden.
+// A few prompts on a few heads are up to a tenth slower as kernels (8 heads, f16, one prompt
+// of 70 tokens 9.8 / 10.6, 3 of 33 8.9 / 9.4) and faster as calls, which the host bounds there
+// with one launch or two: 32 heads, one prompt of 45 tokens 12.7 / 10.2.
 inline int32_t prompt_step_short_waves(const int32_t *prompt_lens_host, int32_t num_prompts, int32_t num_q_heads,
                                        int32_t num_kv_heads) {
   if (!prompt_lens_host || num_prompts <= 0 || num_q_heads != num_kv_heads) return 0;
